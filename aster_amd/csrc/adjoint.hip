@@ -251,24 +251,21 @@ int traj_forward(aster_ctx* c, double dt, int64_t nsteps, int64_t ckpt, int32_t 
   int rc;
   const int method = ASTER_ALLPAIRS_FP32_KAHAN;
   if ((rc = compute_forces(c, method))) return rc;
-  double pending = 0.0;
   int q = 0;
   for (int64_t s = 0; s < nsteps; ++s) {
-    if (s % ckpt == 0) {
-      if (pending != 0.0 && (rc = launch_kick(c, pending))) return rc;
-      pending = 0.0;
+    if (s % ckpt == 0) {  // the evaluation before applied the closing kick
       const size_t o = (size_t)(s / ckpt) * n3;
       if ((rc = dcopy(c, c->x.p, S.ckpt_x.p + o, n3)) || (rc = dcopy(c, c->v.p, S.ckpt_v.p + o, n3))) return rc;
+      if ((rc = launch_kick_drift(c, 0.0, dt))) return rc;
     }
-    if ((rc = launch_kick_drift(c, pending, dt))) return rc;
-    if ((rc = compute_forces(c, method))) return rc;
-    pending = dt;
     if (q < nsnap && snaps[q] == s + 1) {
       if ((rc = dcopy(c, c->x.p, S.snapg.p + (size_t)q * n3, n3))) return rc;
       ++q;
     }
+    const bool close = s + 1 == nsteps || (s + 1) % ckpt == 0;
+    if ((rc = compute_forces(c, method, close ? StepPost{POST_KICK, 0.0, dt} : StepPost{POST_KICK_DRIFT, dt, dt})))
+      return rc;
   }
-  if ((rc = launch_kick(c, pending))) return rc;
   if (snap_pos && nsnap > 0) {
     std::vector<double> h((size_t)nsnap * n3);
     ASTER_HIP(c, hipMemcpyAsync(h.data(), S.snapg.p, h.size() * 8, hipMemcpyDeviceToHost, c->stream));
@@ -315,6 +312,7 @@ int traj_backward(aster_ctx* c, const double* gsnap, double* gx, double* gv, dou
     if (rc) return rc;
     --q;
   }
+  c->src_ready = SrcReady{};  // the passes below move the state and use the source buffer
   int Sl = choose_split(c);
   int64_t slice = round_up((npad + Sl - 1) / Sl, kApTile);
   Sl = (int)((npad + slice - 1) / slice);

@@ -5,7 +5,9 @@
 // and feed VALU instructions directly (no LDS staging, no barriers). The
 // source range is split into slices (grid.y) so that a 64K-body problem puts
 // several waves on every SIMD; slice partials are combined in FP64 in a fixed
-// order, so results are deterministic. Per interaction the plain FP32 loop
+// order, so results are deterministic. Up to some tens of thousands of bodies
+// one launch does the whole evaluation and the integrator's update instead,
+// with the sources in LDS (k_allpairs_tiles). Per interaction the plain FP32 loop
 // issues 3 sub + 3 fma (r^2) + 1 rsq + 3 mul + 3 fma = 12 VALU + 1
 // transcendental; the mixed method forms the separation in FP64 and rounds it
 // (3 add_f64 + 3 cvt instead of 3 sub: 15 VALU + 1 transcendental) and
@@ -30,44 +32,22 @@ namespace aster {
 
 // ---------------------------------------------------------------- FP32 ----
 
-enum { ACC_PLAIN = 0, ACC_TILE_KAHAN = 1, ACC_FULL_KAHAN = 2 };
-
-__device__ __forceinline__ void kahan_add(float& s, float& c, float t) { kahan_add32(s, c, t); }
+enum { ACC_PLAIN = 0, ACC_TILE_KAHAN = 1 };
 
 // Sources, padded to npad with zero-mass bodies at the origin. Bodies outside
 // the source range [lower, upper) (Solver::set_bounds) get zero mass, which
 // adds exactly zero force. Masses are scaled by msc (Fp32Scales).
-//   k_src32: FP32 {x, y, z, m} (positions rounded to FP32 once).
-//   k_src64: FP64 {x, y, z, m}; the kernel forms x_j - x_i in FP64 and rounds
-//            the separation to FP32, so the pair force is FP32 but a close pair
-//            does not lose ~|x|/r ulps to position rounding.
-__global__ __launch_bounds__(256) void k_src32(int n, int npad, int lower, int upper, float msc,
-                                               const double* __restrict__ x, const double* __restrict__ m,
-                                               float4* __restrict__ src) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= npad) return;
-  const bool in = i >= lower && i < upper;
-  src[i] = i < n ? make_float4((float)x[i], (float)x[n + i], (float)x[2 * n + i], in ? (float)m[i] * msc : 0.f)
-                 : make_float4(0.f, 0.f, 0.f, 0.f);
-}
-
-// The w slot carries the FP32 mass in its low 32 bits, so the kernel reads it
-// straight from the low SGPR of the pair without a conversion.
+//   FP32 {x, y, z, m} (positions rounded to FP32 once) for the plain method;
+//   FP64 {x, y, z, m} for the mixed one: the kernel forms x_j - x_i in FP64 and
+//   rounds the separation to FP32, so the pair force is FP32 but a close pair
+//   does not lose ~|x|/r ulps to position rounding. The w slot carries the
+//   FP32 mass in its low 32 bits, so the kernel reads it straight from the low
+//   SGPR of the pair without a conversion.
 __device__ __forceinline__ double pack_mass(float m) {
   return __longlong_as_double((long long)(unsigned long long)__float_as_uint(m));
 }
 __device__ __forceinline__ float unpack_mass(double w) {
   return __uint_as_float((unsigned)(unsigned long long)__double_as_longlong(w));
-}
-
-__global__ __launch_bounds__(256) void k_src64(int n, int npad, int lower, int upper, float msc,
-                                               const double* __restrict__ x, const double* __restrict__ m,
-                                               double4* __restrict__ src) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= npad) return;
-  const bool in = i >= lower && i < upper;
-  src[i] = i < n ? make_double4(x[i], x[n + i], x[2 * n + i], pack_mass(in ? (float)m[i] * msc : 0.f))
-                 : make_double4(0.0, 0.0, 0.0, pack_mass(0.f));
 }
 
 __device__ __forceinline__ float src_mass(const float4& q) { return q.w; }
@@ -78,11 +58,110 @@ struct SrcT;
 template <>
 struct SrcT<false> {
   using type = float4;
+  static __device__ __forceinline__ float4 make(double x, double y, double z, float m) {
+    return make_float4((float)x, (float)y, (float)z, m);
+  }
 };
 template <>
 struct SrcT<true> {
   using type = double4;
+  static __device__ __forceinline__ double4 make(double x, double y, double z, float m) {
+    return make_double4(x, y, z, pack_mass(m));
+  }
 };
+
+// Source j: the body's record, its mass only inside [lower, upper); zeros past
+// n. The mass scale is msc, or read from the device where dmsc is given.
+struct SrcRange {
+  int n, lower, upper;
+  float msc;
+  const double* dmsc;
+  __device__ __forceinline__ float scale() const { return dmsc ? (float)dmsc[0] : msc; }
+};
+template <bool SRC64>
+__device__ __forceinline__ typename SrcT<SRC64>::type load_src(const SrcRange& r, float msc, int j,
+                                                               const double* __restrict__ x,
+                                                               const double* __restrict__ m) {
+  const int jj = min(j, r.n - 1);  // loads at a clamped index, so none waits for a branch
+  const double px = x[jj], py = x[r.n + jj], pz = x[2 * r.n + jj];
+  const float mj = (float)m[jj] * msc;
+  const bool in = j >= r.lower && j < r.upper;
+  return j < r.n ? SrcT<SRC64>::make(px, py, pz, in ? mj : 0.f) : SrcT<SRC64>::make(0.0, 0.0, 0.0, 0.f);
+}
+
+template <bool SRC64>
+__global__ __launch_bounds__(256) void k_src(SrcRange r, int npad, const double* __restrict__ x,
+                                             const double* __restrict__ m,
+                                             typename SrcT<SRC64>::type* __restrict__ src) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < npad) src[i] = load_src<SRC64>(r, r.scale(), i, x, m);
+}
+
+// One target per lane.
+template <bool MASK, bool SRC64>
+struct PairSums {
+  double px, py, pz;
+  float fx, fy, fz;
+  __device__ __forceinline__ void target(const double* __restrict__ x, int n, int i) {
+    px = x[i];
+    py = x[n + i];
+    pz = x[2 * n + i];
+    fx = (float)px;
+    fy = (float)py;
+    fz = (float)pz;
+  }
+  // Adds the pull of source q to t.
+  __device__ __forceinline__ void pair(const typename SrcT<SRC64>::type& q, float eps2, float* t) const {
+    float dx, dy, dz;
+    if (SRC64) {
+      dx = (float)(q.x - px);
+      dy = (float)(q.y - py);
+      dz = (float)(q.z - pz);
+    } else {
+      dx = q.x - fx;
+      dy = q.y - fy;
+      dz = q.z - fz;
+    }
+    float r2 = fmaf(dx, dx, eps2);
+    r2 = fmaf(dy, dy, r2);
+    r2 = fmaf(dz, dz, r2);
+    float inv = __builtin_amdgcn_rsqf(r2);
+    if (MASK) inv = (r2 > 0.f) ? inv : 0.f;
+    const float inv2 = inv * inv;
+    const float f = (src_mass(q) * inv) * inv2;
+    t[0] = fmaf(f, dx, t[0]);
+    t[1] = fmaf(f, dy, t[1]);
+    t[2] = fmaf(f, dz, t[2]);
+  }
+};
+
+// The FP32 sums of one tile of sources in LDS.
+template <class P, class T>
+__device__ __forceinline__ void tile_sums(const P& ps, const T* __restrict__ src, float eps2, float* t) {
+  t[0] = t[1] = t[2] = 0.f;
+  // The next kB sources are read before the sums over the present ones, and
+  // kept there: left alone, the compiler reads each right before its use and
+  // waits for LDS every time (leapfrog step at n = 1000, mixed: 9.1 -> 7.5 us).
+  // kB = 4 needs twice the registers and loses where many waves share a SIMD
+  // (n = 16384: 120 -> 135 us).
+  constexpr int kB = 2;
+  T q[kB], next[kB];
+#pragma unroll
+  for (int u = 0; u < kB; ++u) q[u] = src[u];
+#pragma unroll 4
+  for (int j = 0; j < kApTile; j += kB) {
+#pragma unroll
+    for (int u = 0; u < kB; ++u) next[u] = src[min(j + kB, kApTile - kB) + u];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kB; ++u) ps.pair(q[u], eps2, t);
+#pragma unroll
+    for (int u = 0; u < kB; ++u) {
+      hold_pad(q[u]);
+      q[u] = next[u];
+    }
+  }
+}
 
 // One target per lane (natural order), sources [s*slice_len, ...) of the
 // padded source array; out: [S][3][n] doubles.
@@ -91,93 +170,232 @@ __global__ __launch_bounds__(256) void k_allpairs_f32(const typename SrcT<SRC64>
                                                       const double* __restrict__ x, int n, int npad, int slice_len,
                                                       float eps2, double* __restrict__ out) {
   const int i = blockIdx.x * kApBlock + threadIdx.x;
-  const int ii = i < n ? i : n - 1;
-  const int s = blockIdx.y;
-  const int jb = s * slice_len;
+  const int jb = blockIdx.y * slice_len;
   const int je = min(jb + slice_len, npad);
-  const double px = x[ii], py = x[n + ii], pz = x[2 * n + ii];
-  const float fx = (float)px, fy = (float)py, fz = (float)pz;
-  float sx = 0.f, sy = 0.f, sz = 0.f;
-  float cx = 0.f, cy = 0.f, cz = 0.f;
+  PairSums<MASK, SRC64> p;
+  p.target(x, n, i < n ? i : n - 1);
+  float s[3] = {0.f, 0.f, 0.f}, cmp[3] = {0.f, 0.f, 0.f};
   for (int t = jb; t < je; t += kApTile) {
-    float tx = 0.f, ty = 0.f, tz = 0.f;
+    float ts[3] = {0.f, 0.f, 0.f};
 #pragma unroll 16
-    for (int k = 0; k < kApTile; ++k) {
-      const auto q = src[t + k];
-      float dx, dy, dz;
-      if (SRC64) {
-        dx = (float)(q.x - px);
-        dy = (float)(q.y - py);
-        dz = (float)(q.z - pz);
-      } else {
-        dx = q.x - fx;
-        dy = q.y - fy;
-        dz = q.z - fz;
-      }
-      float r2 = fmaf(dx, dx, eps2);
-      r2 = fmaf(dy, dy, r2);
-      r2 = fmaf(dz, dz, r2);
-      float inv = __builtin_amdgcn_rsqf(r2);
-      if (MASK) inv = (r2 > 0.f) ? inv : 0.f;
-      const float inv2 = inv * inv;
-      const float f = (src_mass(q) * inv) * inv2;
-      if (ACC == ACC_FULL_KAHAN) {
-        kahan_add(sx, cx, f * dx);
-        kahan_add(sy, cy, f * dy);
-        kahan_add(sz, cz, f * dz);
-      } else if (ACC == ACC_TILE_KAHAN) {
-        tx = fmaf(f, dx, tx);
-        ty = fmaf(f, dy, ty);
-        tz = fmaf(f, dz, tz);
-      } else {
-        sx = fmaf(f, dx, sx);
-        sy = fmaf(f, dy, sy);
-        sz = fmaf(f, dz, sz);
-      }
-    }
-    if (ACC == ACC_TILE_KAHAN) {
-      kahan_add(sx, cx, tx);
-      kahan_add(sy, cy, ty);
-      kahan_add(sz, cz, tz);
-    }
+    for (int k = 0; k < kApTile; ++k) p.pair(src[t + k], eps2, ACC == ACC_TILE_KAHAN ? ts : s);
+    if (ACC == ACC_TILE_KAHAN)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) kahan_add32(s[c], cmp[c], ts[c]);
   }
   if (i < n) {
-    double* o = out + (size_t)s * 3 * n;
-    o[i] = (double)sx - (double)cx;
-    o[n + i] = (double)sy - (double)cy;
-    o[2 * n + i] = (double)sz - (double)cz;
+    double* o = out + (size_t)blockIdx.y * 3 * n;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) o[(size_t)c * n + i] = (double)s[c] - (double)cmp[c];
+  }
+}
+
+// Small and middle-sized problems: sources in LDS, the tiles of a slice spread
+// over the waves of a block. A block owns 64 / GR targets. Its W worker waves
+// take GR 64-source tiles each per round: lane group g of 64 / GR lanes sums
+// tile GR w + g for its targets. A wave stages its tiles through LDS by itself
+// (the next round's sources are loaded during the sums) and leaves the tile
+// sums there; one more wave takes them in tile order, Kahan-compensated within
+// each slice, the slices in FP64: the bits of k_allpairs_f32 and k_combine with
+// the same slices (plain method: the tile sums are added in FP64, where
+// k_allpairs_f32 carries one FP32 sum through the slice).
+// With GR = 4 even 1000 bodies occupy some hundred SIMDs, a block takes every
+// source and the last wave applies the integrator's update too, so a step is
+// one launch; the positions then go to a second buffer, since other blocks
+// still read them. With f.part block row y takes slice y and writes its sums
+// for k_combine. Bound: launch and one tile's latency at n = 1000 (7.5 us a
+// step, mixed), VALU issue and LDS reads (32 bytes per source and wave) above.
+struct TileSpan {
+  int j0, tiles, slice_tiles;  // first source, number of tiles, tiles per slice
+};
+struct Finish {
+  double* part;      // slice sums [S][3][n] (the rest unused), or null:
+  const double* pn;  // FP64 post-Newtonian part, may be null
+  double G;          // result scale, or read from the device where dG is given
+  const double* dG;
+  double* a;         // SoA planes, or AoS-d3 if aos
+  int aos;
+  StepPost post;
+  double* x_out;
+  double* v;
+  uint32_t* flags;
+};
+
+template <int W, int GR, bool MASK, bool SRC64>
+__global__ __launch_bounds__(64 * (W + 1)) void k_allpairs_tiles(SrcRange r, const double* __restrict__ x,
+                                                                 const double* __restrict__ m, TileSpan sp,
+                                                                 float eps2, Finish f) {
+  constexpr int TG = 64 / GR;              // targets of the block, lanes of a group
+  constexpr int R = GR * W;                // tiles per round
+  constexpr int NC = (3 * TG + 63) / 64;   // sums per lane of the last wave
+  constexpr int ACC = SRC64 ? ACC_TILE_KAHAN : ACC_PLAIN;
+  // a tile's records end on another bank than they begin on, so the lane
+  // groups read different banks
+  __shared__ typename SrcT<SRC64>::type tiles[W][GR][kApTile + 1];
+  __shared__ float sums[2][R][3][TG];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = r.n, i0 = blockIdx.x * TG;
+  if (f.part) {  // this block's slice
+    const int t0 = blockIdx.y * sp.slice_tiles;
+    sp.j0 += t0 * kApTile;
+    sp.tiles = min(sp.slice_tiles, sp.tiles - t0);
+  }
+  const int rounds = (sp.tiles + R - 1) / R;
+  if (w < W) {
+    const int ti = lane % TG, g = lane / TG;
+    const float msc = r.scale();
+    typename SrcT<SRC64>::type q[GR];
+    auto fetch = [&](int rd) {
+#pragma unroll
+      for (int p = 0; p < GR; ++p)
+        q[p] = load_src<SRC64>(r, msc, sp.j0 + (rd * R + GR * w + p) * kApTile + lane, x, m);
+    };
+    fetch(0);
+    PairSums<MASK, SRC64> ps;
+    ps.target(x, n, min(i0 + ti, n - 1));
+    for (int rd = 0; rd < rounds; ++rd) {
+      if (rd * R + GR * w < sp.tiles) {  // wave-uniform
+        wave_sync();                     // the wave is done with its previous tiles
+#pragma unroll
+        for (int p = 0; p < GR; ++p) tiles[w][p][lane] = q[p];
+        wave_sync();
+        if (rd + 1 < rounds) fetch(rd + 1);
+        float t[3];
+        tile_sums(ps, tiles[w][g], eps2, t);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) sums[rd & 1][GR * w + g][c][ti] = t[c];
+      }
+      __syncthreads();  // the sums of this round are there, those of the round before are taken
+    }
+    return;
+  }
+  double xs[NC], vs[NC], tot[NC];
+  float s[NC], cmp[NC];
+#pragma unroll
+  for (int h = 0; h < NC; ++h) {
+    const int ch = lane + 64 * h, c = ch / TG, i = min(i0 + ch % TG, n - 1);
+    tot[h] = 0.0;
+    s[h] = cmp[h] = 0.f;
+    xs[h] = vs[h] = 0.0;
+    if (f.post.kind != POST_NONE && c < 3) {
+      xs[h] = x[(size_t)c * n + i];
+      vs[h] = f.v[(size_t)c * n + i];
+    }
+  }
+  int left = sp.slice_tiles;  // tiles to the end of the slice
+  for (int rd = 0; rd < rounds; ++rd) {
+    __syncthreads();
+    const int cnt = min(R, sp.tiles - rd * R);
+    for (int k = 0; k < cnt; ++k) {
+      const bool end = --left == 0 || (rd + 1 == rounds && k + 1 == cnt);
+#pragma unroll
+      for (int h = 0; h < NC; ++h) {
+        const int ch = min(lane + 64 * h, 3 * TG - 1);
+        const float t = (&sums[rd & 1][k][0][0])[ch];
+        if (ACC == ACC_TILE_KAHAN) {
+          kahan_add32(s[h], cmp[h], t);
+          if (end) {
+            tot[h] += (double)s[h] - (double)cmp[h];
+            s[h] = cmp[h] = 0.f;
+          }
+        } else {
+          tot[h] += (double)t;
+        }
+      }
+      if (end) left = sp.slice_tiles;
+    }
+  }
+  const double G = f.dG ? f.dG[0] : f.G;
+#pragma unroll
+  for (int h = 0; h < NC; ++h) {
+    const int ch = lane + 64 * h, c = ch / TG, i = i0 + ch % TG;
+    if (c >= 3 || i >= n) continue;
+    const size_t k = (size_t)c * n + i;
+    if (f.part) {
+      f.part[(size_t)blockIdx.y * 3 * n + k] = tot[h];
+      continue;
+    }
+    double acc = G * tot[h];
+    if (f.pn) acc += f.pn[k];
+    f.a[f.aos ? 3 * (size_t)i + c : k] = acc;
+    if (f.post.kind == POST_KICK) f.v[k] = kick_1(vs[h], acc, f.post.dt);
+    if (f.post.kind == POST_KICK_DRIFT || f.post.kind == POST_SABA) {
+      if (f.post.kind == POST_KICK_DRIFT) kick_drift_1(xs[h], vs[h], acc, f.post.dt_prev, f.post.dt);
+      else saba_1(xs[h], vs[h], acc, f.post.d, f.post.cd, f.post.cd_next, f.post.dt);
+      f.x_out[k] = xs[h];
+      f.v[k] = vs[h];
+      if (!(isfinite(xs[h]) && isfinite(vs[h]))) atomicOr(f.flags, (uint32_t)FLAG_NONFINITE);
+    }
   }
 }
 
 // Sum S slice partials (and the optional FP64 1PN term) in slice order, then
 // scale by G (times the mass scale's 2^k): a[c][i] = G * sum_s part[s][c][i]
-// + pn[c][i].
-__global__ void k_combine(int n, int S, const double* __restrict__ part, const double* __restrict__ pn, double G,
-                          double* __restrict__ a) {
+// + pn[c][i]. POST then applies the integrator's next update of this body
+// (StepPost) with the acceleration still in registers, the arithmetic of
+// k_kick_drift, k_kick and k_saba_stage, and after a drift the body's source
+// record of the next evaluation (src, may be null): between two evaluations
+// of a step sequence one launch instead of three, of about 4.6 us each.
+template <int POST, bool SRC64>
+__global__ __launch_bounds__(256) void k_combine(int n, int npad, int S, const double* __restrict__ part,
+                                                 const double* __restrict__ pn, double G, double* __restrict__ a,
+                                                 StepPost post, double* __restrict__ x, double* __restrict__ v,
+                                                 const double* __restrict__ m, SrcRange r,
+                                                 typename SrcT<SRC64>::type* __restrict__ src,
+                                                 uint32_t* __restrict__ flags) {
+  constexpr bool kDrifts = POST == POST_KICK_DRIFT || POST == POST_SABA;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n) {
+    if (kDrifts && src && i < npad) src[i] = SrcT<SRC64>::make(0.0, 0.0, 0.0, 0.f);
+    return;
+  }
+  double xs[3], vs[3];
+  if (POST != POST_NONE)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      if (kDrifts) xs[c] = x[(size_t)c * n + i];
+      vs[c] = v[(size_t)c * n + i];
+    }
   // 8 slices per round, their 24 loads issued before the first add (clamped
   // slice index); the adds stay in slice order
   double s[3] = {0.0, 0.0, 0.0};
   for (int k0 = 0; k0 < S; k0 += 8) {
-    double v[8][3];
+    double w[8][3];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int k = min(k0 + u, S - 1);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) v[u][c] = part[((size_t)k * 3 + c) * n + i];
+      for (int c = 0; c < 3; ++c) w[u][c] = part[((size_t)k * 3 + c) * n + i];
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       if (k0 + u < S)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) s[c] += v[u][c];
+        for (int c = 0; c < 3; ++c) s[c] += w[u][c];
   }
+  bool finite = true;
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    double r = G * s[c];
-    if (pn) r += pn[(size_t)c * n + i];
-    a[(size_t)c * n + i] = r;
+    const size_t k = (size_t)c * n + i;
+    double acc = G * s[c];
+    if (pn) acc += pn[k];
+    a[k] = acc;
+    if (POST == POST_KICK) v[k] = kick_1(vs[c], acc, post.dt);
+    if (kDrifts) {
+      if (POST == POST_KICK_DRIFT) kick_drift_1(xs[c], vs[c], acc, post.dt_prev, post.dt);
+      else saba_1(xs[c], vs[c], acc, post.d, post.cd, post.cd_next, post.dt);
+      x[k] = xs[c];
+      v[k] = vs[c];
+      finite = finite && isfinite(xs[c]) && isfinite(vs[c]);
+    }
+  }
+  if (kDrifts) {
+    if (!finite) atomicOr(flags, (uint32_t)FLAG_NONFINITE);
+    if (src) {
+      const bool in = i >= r.lower && i < r.upper;
+      src[i] = SrcT<SRC64>::make(xs[0], xs[1], xs[2], in ? (float)m[i] * r.scale() : 0.f);
+    }
   }
 }
 
@@ -502,9 +720,119 @@ int fp32_scales(aster_ctx* c, Fp32Scales* sc) {
   return ASTER_OK;
 }
 
-int launch_allpairs(aster_ctx* c, int method) {
+// Which kernel takes n bodies. A leapfrog step in us, before (k_allpairs_f32,
+// its sources, combine and update in launches of their own) / one launch, GR =
+// 4 / k_allpairs_tiles by slices, GR = 1 / k_allpairs_f32, two launches. Mixed:
+// n = 1000 156 / 7.5 / - / 152, 4096 159 / 15.2 / 19.2 / 156, 8192 158 / 47 / 37
+// / 155, 16384 164 / 175 / 120 / 160, 20011 200 / 270 / 178 / 192, 32768 437 /
+// 684 / 433 / 434, 65536 1453 / 2698 / 1712 / 1449. Plain: 1000 93 / 6.3 / - /
+// 90, 4096 95 / 11.6 / 16.9 / 89, 8192 92 / 30 / 28 / 93, 16384 110 / 130 / 85 /
+// 106, 20011 165 / 164 / 129 / 160, 32768 322 / 447 / 311 / 318, 65536 1135 /
+// 1699 / 1211 / 1127. One launch fills the 256 CUs once up to 4096 bodies (16
+// targets a block); above 32768 the scalar reads, which take no LDS bandwidth,
+// hide their latency behind enough waves.
+static bool one_launch(int64_t n) { return n <= 4096; }
+static bool in_tiles(int64_t n) { return n <= 32768; }
+
+template <int W, int GR, bool SRC64>
+static void launch_tiles_as(hipStream_t st, bool mask, const SrcRange& r, const double* x, const double* m,
+                            const TileSpan& sp, int S, float eps2, const Finish& f) {
+  auto k = mask ? k_allpairs_tiles<W, GR, true, SRC64> : k_allpairs_tiles<W, GR, false, SRC64>;
+  const int tg = 64 / GR;
+  hipLaunchKernelGGL(k, dim3((r.n + tg - 1) / tg, f.part ? S : 1), dim3(64 * (W + 1)), 0, st, r, x, m, sp, eps2, f);
+}
+
+// One launch: W = 4 waves hold 16 tiles (1024 sources) in one round.
+template <bool SRC64>
+static void launch_tiles(hipStream_t st, bool mask, const SrcRange& r, const double* x, const double* m,
+                         const TileSpan& sp, int S, float eps2, const Finish& f) {
+  if (f.part) launch_tiles_as<4, 1, SRC64>(st, mask, r, x, m, sp, S, eps2, f);
+  else if (sp.tiles <= 16) launch_tiles_as<4, 4, SRC64>(st, mask, r, x, m, sp, S, eps2, f);
+  else launch_tiles_as<8, 4, SRC64>(st, mask, r, x, m, sp, S, eps2, f);
+}
+
+template <bool SRC64>
+static void launch_slices(hipStream_t st, bool mask, int n, int npad, int S, int span, int slice, float eps2,
+                          const double* x, const typename SrcT<SRC64>::type* src, double* out) {
+  constexpr int ACC = SRC64 ? ACC_TILE_KAHAN : ACC_PLAIN;
+  auto k = mask ? k_allpairs_f32<ACC, true, SRC64> : k_allpairs_f32<ACC, false, SRC64>;
+  hipLaunchKernelGGL(k, dim3(npad / kApBlock, S), dim3(kApBlock), 0, st, src, x, n, span, slice, eps2, out);
+}
+
+// One FP32 evaluation and the update that follows: the FP64 post-Newtonian
+// part, then one launch; or sources (unless left by the update before), pair
+// sums over slices and the combine with the update.
+template <bool SRC64>
+static int allpairs_f32(aster_ctx* c, DBuf<typename SrcT<SRC64>::type>& srcbuf, int lower, int upper, int pnf,
+                        const StepPost& post) {
+  const int n = (int)c->n, npad = (int)c->npad;
+  Fp32Scales sc;
+  int rc = fp32_scales(c, &sc);
+  if (rc) return rc;
+  const SrcRange r{n, lower, upper, sc.msc, nullptr};
+  // Slices over the tiles that hold the source range (sources outside it and
+  // the padding bodies have zero mass).
+  const int j0 = lower / kApTile * kApTile;
+  const int span = std::max<int>(j0 + kApTile, (int)round_up(upper, kApTile)) - j0;
+  int S = 0, slice = 0;
+  slice_span(span, choose_split(c), &S, &slice);
+  const bool drifts = post.kind == POST_KICK_DRIFT || post.kind == POST_SABA;
+  const double* pnp = nullptr;
+  if (pnf) {
+    ASTER_HIP(c, c->apn.reserve((size_t)3 * n));
+    if ((rc = launch_allpairs_f64(c, true, 1, n, lower, upper, 1.0 / c->P.c, pnf, c->apn.p))) return rc;
+    pnp = c->apn.p;
+  }
+  const TileSpan sp{j0, span / kApTile, slice / kApTile};
+  if (one_launch(n)) {
+    if (drifts) ASTER_HIP(c, c->x_next.reserve((size_t)3 * n));
+    const Finish f{nullptr, pnp, sc.gsc, nullptr, c->a.p, 0, post, c->x_next.p, c->v.p, c->flags.p};
+    phase_begin(c, ASTER_PHASE_ALLPAIRS);
+    launch_tiles<SRC64>(c->stream, sc.mask, r, c->x.p, c->m.p, sp, S, sc.eps2, f);
+    ASTER_HIP(c, hipGetLastError());
+    phase_end(c, ASTER_PHASE_ALLPAIRS);
+    if (drifts) std::swap(c->x, c->x_next);
+    return ASTER_OK;
+  }
+  ASTER_HIP(c, c->apart.reserve((size_t)S * 3 * n));
+  typename SrcT<SRC64>::type* src = nullptr;
+  const SrcReady want{c->x.p, c->n, SRC64 ? 2 : 1, lower, upper, sc.msc};
+  const bool have = c->src_ready == want;
+  c->src_ready = SrcReady{};
+  if (in_tiles(n)) {
+    Finish f{};
+    f.part = c->apart.p;
+    phase_begin(c, ASTER_PHASE_ALLPAIRS);
+    launch_tiles<SRC64>(c->stream, sc.mask, r, c->x.p, c->m.p, sp, S, sc.eps2, f);
+  } else {
+    ASTER_HIP(c, srcbuf.reserve((size_t)npad));
+    src = srcbuf.p;
+    if (!have) {
+      phase_begin(c, ASTER_PHASE_TILES);
+      hipLaunchKernelGGL(k_src<SRC64>, dim3(npad / 256), dim3(256), 0, c->stream, r, npad, c->x.p, c->m.p, src);
+      ASTER_HIP(c, hipGetLastError());
+      phase_end(c, ASTER_PHASE_TILES);
+    }
+    phase_begin(c, ASTER_PHASE_ALLPAIRS);
+    launch_slices<SRC64>(c->stream, sc.mask, n, npad, S, span, slice, sc.eps2, c->x.p, src + j0, c->apart.p);
+  }
+  ASTER_HIP(c, hipGetLastError());
+  phase_end(c, ASTER_PHASE_ALLPAIRS);
+  phase_begin(c, ASTER_PHASE_COMBINE);
+  auto k = k_combine<POST_NONE, SRC64>;
+  if (post.kind == POST_KICK_DRIFT) k = k_combine<POST_KICK_DRIFT, SRC64>;
+  else if (post.kind == POST_KICK) k = k_combine<POST_KICK, SRC64>;
+  else if (post.kind == POST_SABA) k = k_combine<POST_SABA, SRC64>;
+  hipLaunchKernelGGL(k, dim3(npad / 256), dim3(256), 0, c->stream, n, npad, S, (const double*)c->apart.p, pnp, sc.gsc,
+                     c->a.p, post, c->x.p, c->v.p, (const double*)c->m.p, r, src, c->flags.p);
+  ASTER_HIP(c, hipGetLastError());
+  phase_end(c, ASTER_PHASE_COMBINE);
+  if (drifts && src) c->src_ready = want;
+  return ASTER_OK;
+}
+
+int launch_allpairs(aster_ctx* c, int method, const StepPost& post) {
   const int n = (int)c->n;
-  const int npad = (int)c->npad;
   const int lower = c->P.lower < 0 ? 0 : c->P.lower;
   const int upper = (c->P.upper < 0 || c->P.upper > n) ? n : c->P.upper;
   if (lower > upper) return fail(c, ASTER_ERR_INVALID, "source bounds: lower > upper");
@@ -524,78 +852,19 @@ int launch_allpairs(aster_ctx* c, int method) {
                        c->P.softening, (const double*)phi, (const double*)an, c->a.p);
     ASTER_HIP(c, hipGetLastError());
     phase_end(c, ASTER_PHASE_ALLPAIRS);
-    return ASTER_OK;
+    return launch_post(c, post, false);
   }
   if (method == ASTER_ALLPAIRS_FP64) {
     phase_begin(c, ASTER_PHASE_ALLPAIRS);
     if (const int e = launch_allpairs_f64(c, pn, 0, n, lower, upper, ic, pnf, c->a.p)) return e;
     ASTER_HIP(c, hipGetLastError());
     phase_end(c, ASTER_PHASE_ALLPAIRS);
-    return ASTER_OK;
+    return launch_post(c, post, false);
   }
   if (method != ASTER_ALLPAIRS_FP32 && method != ASTER_ALLPAIRS_FP32_KAHAN)
     return fail(c, ASTER_ERR_INVALID, "unknown all-pairs method");
-  Fp32Scales sc;
-  int rc = fp32_scales(c, &sc);
-  if (rc) return rc;
-  // Padded source array: FP32 for the plain method, FP64 for the mixed one.
-  const bool src64 = method == ASTER_ALLPAIRS_FP32_KAHAN;
-  phase_begin(c, ASTER_PHASE_TILES);
-  if (src64) {
-    ASTER_HIP(c, c->src64.reserve((size_t)npad));
-    hipLaunchKernelGGL(k_src64, dim3(npad / 256), dim3(256), 0, c->stream, n, npad, lower, upper, sc.msc, c->x.p,
-                       c->m.p, c->src64.p);
-  } else {
-    hipLaunchKernelGGL(k_src32, dim3(npad / 256), dim3(256), 0, c->stream, n, npad, lower, upper, sc.msc, c->x.p,
-                       c->m.p, c->sh.p);
-  }
-  ASTER_HIP(c, hipGetLastError());
-  phase_end(c, ASTER_PHASE_TILES);
-  // Slices over the tiles that hold the source range (sources outside it and
-  // the padding bodies have zero mass).
-  const int jb = lower / kApTile * kApTile;
-  const int je = std::max<int>(jb + kApTile, (int)round_up(upper, kApTile));
-  const int span = je - jb;
-  int S = 0, slice = 0;
-  slice_span(span, choose_split(c), &S, &slice);
-  ASTER_HIP(c, c->apart.reserve((size_t)S * 3 * n));
-  const float eps2 = sc.eps2;
-  const bool mask = sc.mask;
-  dim3 grid(npad / kApBlock, S);
-  double* out = c->apart.p;
-  phase_begin(c, ASTER_PHASE_ALLPAIRS);
-  if (src64) {
-    const double4* sp = c->src64.p + jb;
-    if (mask)
-      hipLaunchKernelGGL((k_allpairs_f32<ACC_TILE_KAHAN, true, true>), grid, dim3(kApBlock), 0, c->stream, sp,
-                         c->x.p, n, span, (int)slice, eps2, out);
-    else
-      hipLaunchKernelGGL((k_allpairs_f32<ACC_TILE_KAHAN, false, true>), grid, dim3(kApBlock), 0, c->stream, sp,
-                         c->x.p, n, span, (int)slice, eps2, out);
-  } else {
-    const float4* sp = c->sh.p + jb;
-    if (mask)
-      hipLaunchKernelGGL((k_allpairs_f32<ACC_PLAIN, true, false>), grid, dim3(kApBlock), 0, c->stream, sp, c->x.p, n,
-                         span, (int)slice, eps2, out);
-    else
-      hipLaunchKernelGGL((k_allpairs_f32<ACC_PLAIN, false, false>), grid, dim3(kApBlock), 0, c->stream, sp, c->x.p,
-                         n, span, (int)slice, eps2, out);
-  }
-  ASTER_HIP(c, hipGetLastError());
-  phase_end(c, ASTER_PHASE_ALLPAIRS);
-  const double* pnp = nullptr;
-  if (pn) {
-    ASTER_HIP(c, c->apn.reserve((size_t)3 * n));
-    if ((rc = launch_allpairs_f64(c, true, 1, n, lower, upper, ic, pnf, c->apn.p))) return rc;
-    ASTER_HIP(c, hipGetLastError());
-    pnp = c->apn.p;
-  }
-  phase_begin(c, ASTER_PHASE_COMBINE);
-  hipLaunchKernelGGL(k_combine, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, S, c->apart.p, pnp, sc.gsc,
-                     c->a.p);
-  ASTER_HIP(c, hipGetLastError());
-  phase_end(c, ASTER_PHASE_COMBINE);
-  return ASTER_OK;
+  if (method == ASTER_ALLPAIRS_FP32) return allpairs_f32<false>(c, c->sh, lower, upper, pnf, post);
+  return allpairs_f32<true>(c, c->src64, lower, upper, pnf, post);
 }
 
 }  // namespace aster
@@ -646,17 +915,6 @@ __global__ void k_na_scales(const double* __restrict__ sums, float eps2, int mas
   if (k > kMaxMassShift) k = kMaxMassShift;
   scale[0] = (double)ldexpf(1.0f, -k);
   scale[1] = ldexp(G, k);
-}
-
-// k_src64 with the mass scale read from the device.
-__global__ __launch_bounds__(256) void k_na_src(int n, int npad, const double* __restrict__ scale,
-                                                const double* __restrict__ x, const double* __restrict__ m,
-                                                double4* __restrict__ src) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= npad) return;
-  const float msc = (float)scale[0];
-  src[i] = i < n ? make_double4(x[i], x[n + i], x[2 * n + i], pack_mass((float)m[i] * msc))
-                 : make_double4(0.0, 0.0, 0.0, pack_mass(0.f));
 }
 
 // k_combine (no post-Newtonian term) writing AoS-d3.
@@ -737,16 +995,22 @@ extern "C" int aster_forces_noalloc(int64_t n, const double* d_pos, const double
   hipLaunchKernelGGL(k_com_partial, dim3(rblocks), b256, 0, st, n, (const double*)x, d_mass, red);
   hipLaunchKernelGGL(k_com_final, dim3(1), dim3(64), 0, st, rblocks, (const double*)red, sums);
   hipLaunchKernelGGL(k_na_scales, dim3(1), dim3(64), 0, st, (const double*)sums, eps2, mask ? 1 : 0, G, scale);
-  hipLaunchKernelGGL(k_na_src, dim3(npad / 256), b256, 0, st, ni, npad, (const double*)scale, (const double*)x,
-                     d_mass, src);
-  const dim3 grid(npad / kApBlock, S);
-  if (mask)
-    hipLaunchKernelGGL((k_allpairs_f32<ACC_TILE_KAHAN, true, true>), grid, dim3(kApBlock), 0, st,
-                       (const double4*)src, (const double*)x, ni, span, slice, eps2, part);
-  else
-    hipLaunchKernelGGL((k_allpairs_f32<ACC_TILE_KAHAN, false, true>), grid, dim3(kApBlock), 0, st,
-                       (const double4*)src, (const double*)x, ni, span, slice, eps2, part);
-  hipLaunchKernelGGL(k_na_combine, gn, b256, 0, st, ni, S, (const double*)part, (const double*)scale, d_acc);
+  const SrcRange r{ni, 0, ni, 1.f, scale};
+  const TileSpan sp{0, span / kApTile, slice / kApTile};
+  if (one_launch(n)) {
+    const Finish f{nullptr, nullptr, 0.0, scale + 1, d_acc, 1, StepPost{}, nullptr, nullptr, nullptr};
+    launch_tiles<true>(st, mask, r, x, d_mass, sp, S, eps2, f);
+  } else {
+    if (in_tiles(n)) {
+      Finish f{};
+      f.part = part;
+      launch_tiles<true>(st, mask, r, x, d_mass, sp, S, eps2, f);
+    } else {
+      hipLaunchKernelGGL(k_src<true>, dim3(npad / 256), b256, 0, st, r, npad, (const double*)x, d_mass, src);
+      launch_slices<true>(st, mask, ni, npad, S, span, slice, eps2, x, src, part);
+    }
+    hipLaunchKernelGGL(k_na_combine, gn, b256, 0, st, ni, S, (const double*)part, (const double*)scale, d_acc);
+  }
   if ((e = hipGetLastError()) != hipSuccess)
     return na_fail(ASTER_ERR_HIP, std::string("aster_forces_noalloc launch: ") + hipGetErrorString(e));
   return ASTER_OK;

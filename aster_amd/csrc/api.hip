@@ -49,15 +49,20 @@ static bool is_allpairs(int m) {
 }
 static bool is_bh(int m) { return m == ASTER_BH_PARITY || m == ASTER_BH_GEOMETRIC || m == ASTER_BH_GROUP; }
 
-int compute_forces(aster_ctx* c, int method) {
+int compute_forces(aster_ctx* c, int method, const StepPost& post) {
   int rc;
-  if (is_allpairs(method))
-    rc = launch_allpairs(c, method);
-  else if (is_bh(method))
+  if (is_allpairs(method)) {
+    if ((rc = launch_allpairs(c, method, post))) return rc;
+  } else if (is_bh(method)) {
     rc = bh_forces(c, method);
-  else
+    c->box_parts = 0;
+    if (rc) return rc;
+    // the drift also forms the first stage of the next tree's automatic box,
+    // consumed by the force evaluation that follows alone
+    if ((rc = launch_post(c, post, true))) return rc;
+  } else {
     return fail(c, ASTER_ERR_INVALID, "unknown force method");
-  if (rc) return rc;
+  }
   c->acc_valid = true;
   c->acc_stale = false;
   c->acc_method = method;
@@ -144,7 +149,7 @@ int aster_destroy(aster_ctx* c) {
     if (e) (void)hipEventDestroy(e);
   if (c->tree_ev) (void)hipEventDestroy(c->tree_ev);
   if (c->host_words) (void)hipHostFree(c->host_words);
-  c->x.release(); c->v.release(); c->m.release(); c->a.release(); c->sh.release(); c->src64.release();
+  c->x.release(); c->x_next.release(); c->v.release(); c->m.release(); c->a.release(); c->sh.release(); c->src64.release();
   c->apart.release(); c->apn.release(); c->ework.release(); c->eout.release(); c->flags.release();
   c->boxpart.release(); c->boxd.release(); c->stage.release();
   c->codes.release(); c->xm4.release(); c->idx.release(); c->codes2.release(); c->idx2.release(); c->hist.release();
@@ -355,26 +360,25 @@ int aster_step(aster_ctx* c, int method, int integrator, double dt, int64_t nste
   // previous step's second evaluation: re-evaluate, as update_leapfrog does.
   // Newtonian forces depend on positions only and are reused.
   const bool vdep = (c->P.pn_flags & ASTER_PN_TERMS) != 0;
-  if (!vdep && (!c->acc_valid || c->acc_stale || c->acc_method != method))
-    if ((rc = compute_forces(c, method))) return rc;
-  double pending = 0.0;
+  auto weight = [&](int k) { return (integrator == ASTER_YOSHIDA4) ? w[k] * dt : dt; };
+  // Every update is handed to the force evaluation before it (the all-pairs
+  // FP32 methods apply it with their last launch).
+  if (vdep || !c->acc_valid || c->acc_stale || c->acc_method != method) {
+    if ((rc = compute_forces(c, method, StepPost{POST_KICK_DRIFT, 0.0, weight(0)}))) return rc;
+  } else if ((rc = launch_kick_drift(c, 0.0, weight(0), is_bh(method)))) {
+    return rc;
+  }
   for (int64_t s = 0; s < nsteps; ++s)
     for (int k = 0; k < nsub; ++k) {
-      const double h = (integrator == ASTER_YOSHIDA4) ? w[k] * dt : dt;
-      if (vdep) {
-        if (pending != 0.0 && (rc = launch_kick(c, pending))) return rc;
-        if ((rc = compute_forces(c, method))) return rc;
-        pending = 0.0;
+      const double h = weight(k), next = weight(k + 1 < nsub ? k + 1 : 0);
+      const bool last = s + 1 == nsteps && k + 1 == nsub;
+      if (last || vdep) {
+        if ((rc = compute_forces(c, method, StepPost{POST_KICK, 0.0, h}))) return rc;
+        if (!last && (rc = compute_forces(c, method, StepPost{POST_KICK_DRIFT, 0.0, next}))) return rc;
+      } else if ((rc = compute_forces(c, method, StepPost{POST_KICK_DRIFT, h, next}))) {
+        return rc;
       }
-      // Barnes-Hut: the drift also forms the first stage of the next tree's
-      // automatic box, consumed by that force evaluation alone
-      if ((rc = launch_kick_drift(c, pending, h, is_bh(method)))) return rc;
-      rc = compute_forces(c, method);
-      c->box_parts = 0;
-      if (rc) return rc;
-      pending = h;
     }
-  if ((rc = launch_kick(c, pending))) return rc;
   c->adj.ready = false;
   return ASTER_OK;
 }
@@ -394,16 +398,15 @@ int aster_integrate(aster_ctx* c, int method, int integrator, int order, double 
   int rc;
   for (int64_t s = 0; s < nsteps; ++s) {
     if (order == 1) {
-      if ((rc = compute_forces(c, method))) return rc;
-      if ((rc = launch_saba_stage(c, true, 1.0, 1.0, dt))) return rc;
+      if ((rc = compute_forces(c, method, StepPost{POST_SABA, 0.0, dt, 1.0, 1.0}))) return rc;
       continue;
     }
     const double* cs = kSabaC[order];
     const double* ds = kSabaD[order];
-    if ((rc = launch_saba_stage(c, false, 0.0, cs[0], dt))) return rc;
+    if (s == 0 && (rc = launch_saba_stage(c, false, 0.0, cs[0], dt))) return rc;
     for (int st = 0; st < order; ++st) {
-      if ((rc = compute_forces(c, method))) return rc;
-      if ((rc = launch_saba_stage(c, true, ds[st], cs[st + 1], dt))) return rc;
+      const double open = st + 1 == order && s + 1 < nsteps ? cs[0] : 0.0;
+      if ((rc = compute_forces(c, method, StepPost{POST_SABA, 0.0, dt, ds[st], cs[st + 1], open}))) return rc;
     }
   }
   // every stage ends with a drift: the accelerations are those of the last

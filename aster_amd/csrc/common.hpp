@@ -76,6 +76,27 @@ struct BatchState {
   bool traj_ready = false;
 };
 
+// What source records of the all-pairs kernels a context holds: written with
+// the drift to the positions of state buffer x (kind 1: FP32, 2: FP64; 0: none).
+struct SrcReady {
+  const double* x = nullptr;
+  int64_t n = 0;
+  int kind = 0, lower = 0, upper = 0;
+  float msc = 0.f;
+  bool operator==(const SrcReady& o) const {
+    return kind != 0 && kind == o.kind && x == o.x && n == o.n && lower == o.lower && upper == o.upper && msc == o.msc;
+  }
+};
+
+// The integrator's update that follows a force evaluation with the new
+// accelerations (k_kick_drift, k_kick, k_saba_stage).
+enum { POST_NONE = 0, POST_KICK_DRIFT = 1, POST_KICK = 2, POST_SABA = 3 };
+struct StepPost {
+  int kind = POST_NONE;
+  double dt_prev = 0.0, dt = 0.0, d = 0.0, cd = 0.0;
+  double cd_next = 0.0;  // POST_SABA: the next step's opening drift, when not 0
+};
+
 struct AdjointState {
   int64_t nsteps = 0, ckpt_every = 0;
   int32_t nsnap = 0;
@@ -109,6 +130,8 @@ struct aster_ctx {
   aster::DBuf<double> x, v, m, a;
   aster::DBuf<float4> sh;       // FP32 sources {x, y, z, m}, npad entries
   aster::DBuf<double4> src64;   // FP64 sources {x, y, z, m}, npad entries
+  aster::DBuf<double> x_next;   // positions after the update of a one-launch all-pairs evaluation [3][n]
+  aster::SrcReady src_ready;    // which of the two holds the next evaluation's sources
   aster::DBuf<double> apart;    // all-pairs slice partials [S][3][n]
   aster::DBuf<double> apn;      // FP64 1PN correction [3][n]
   aster::DBuf<double> ework;    // energy work [6][n] + reduction scratch
@@ -230,10 +253,11 @@ __host__ __device__ inline int fp32_mass_shift(double mtot, double extent, float
 }
 constexpr int kMaxMassShift = 126;  // 2^-k must stay a normal FP32 number
 // Launchers (each returns an aster_status).
-int launch_allpairs(aster_ctx* c, int method);           // writes c->a
+int launch_allpairs(aster_ctx* c, int method, const StepPost& post);  // writes c->a, then applies the update
+int launch_post(aster_ctx* c, const StepPost& post, bool box);
 int launch_kick_drift(aster_ctx* c, double dt_prev, double dt, bool box = false);
 int launch_kick(aster_ctx* c, double dt);
-int launch_saba_stage(aster_ctx* c, bool kick, double d, double cdrift, double dt);
+int launch_saba_stage(aster_ctx* c, bool kick, double d, double cdrift, double dt, double cd_next = 0.0);
 int launch_energy(aster_ctx* c, double* out6_host);
 int import_state(aster_ctx* c, int64_t n, const double* d_pos, const double* d_vel, const double* d_mass);
 int export_plane(aster_ctx* c, const double* soa, double* d_aos);
@@ -268,7 +292,8 @@ __global__ void k_com_final(int nparts, const double* __restrict__ part, double*
 int choose_split(aster_ctx* c);
 int default_split(int64_t npad);                           // source slices of the FP32 all-pairs kernels
 void set_global_error(const std::string& msg);            // aster_last_error(NULL) for calls without a context
-int compute_forces(aster_ctx* c, int method);             // all-pairs or Barnes-Hut into c->a
+// all-pairs or Barnes-Hut into c->a, then the update that follows
+int compute_forces(aster_ctx* c, int method, const StepPost& post = StepPost{});
 void phase_begin(aster_ctx* c, int phase);
 void phase_end(aster_ctx* c, int phase);
 

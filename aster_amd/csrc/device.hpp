@@ -18,6 +18,23 @@ __device__ __forceinline__ void kick_drift_1(double& x, double& v, double a, dou
   v = vc + 0.5 * a * dt;
 }
 
+// The closing half-kick alone.
+__device__ __forceinline__ double kick_1(double v, double a, double dt) {
+#pragma clang fp contract(off)
+  return v + 0.5 * a * dt;
+}
+
+// One coordinate of a SABA stage (src/integrators/SABA.cpp:19-553): v += (a d)
+// dt, then x += (v c) dt with the kicked v; after a step's last stage also the
+// next step's opening drift (cd_next, when not 0), as an addition of its own.
+__device__ __forceinline__ void saba_1(double& x, double& v, double a, double d, double cd, double cd_next,
+                                       double dt) {
+#pragma clang fp contract(off)
+  v = v + a * d * dt;
+  x = x + v * cd * dt;
+  if (cd_next != 0.0) x = x + v * cd_next * dt;
+}
+
 // get_pn1 (src/physics/tool_chain_impl.cpp:110-118) evaluated in the
 // reference's operation order; `n` is the caller's -norm (:133).
 __device__ __forceinline__ void pn1_term64(double m1, double m2, double v1x, double v1y, double v1z, double v2x,
@@ -190,6 +207,14 @@ __device__ __forceinline__ double rsqrt64_n(double x) {
   return y;
 }
 __device__ __forceinline__ double rsqrt64(double x) { return rsqrt64_n<2>(x); }
+
+// The unused high word of a mass slot that was read counts as used here, so that
+// its register is not taken for another value while the read is in flight (the
+// wait on it would end the read-ahead of tile_sums). No instruction.
+__device__ __forceinline__ void hold_pad(const float4&) {}
+__device__ __forceinline__ void hold_pad(const double4& q) {
+  asm volatile("" ::"v"((unsigned)((unsigned long long)__double_as_longlong(q.w) >> 32)));
+}
 
 // Kahan-compensated FP32 accumulation: s + (-c) carries the running sum.
 __device__ __forceinline__ void kahan_add32(float& s, float& c, float t) {

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) void k_kick_drift(int n, double* __restrict__ 
 // (v 1) dt round exactly like a dt and v dt.
 __global__ __launch_bounds__(256) void k_saba_stage(int n, double* __restrict__ x, double* __restrict__ v,
                                                     const double* __restrict__ a, int kick, double d, double cdrift,
-                                                    double dt, uint32_t* __restrict__ flags) {
+                                                    double cd_next, double dt, uint32_t* __restrict__ flags) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -72,12 +72,13 @@ __global__ __launch_bounds__(256) void k_saba_stage(int n, double* __restrict__ 
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     const size_t k = (size_t)c * n + i;
-    double vc = v[k];
+    double xc = x[k], vc = v[k];
     if (kick) {
-      vc = vc + a[k] * d * dt;
+      saba_1(xc, vc, a[k], d, cdrift, cd_next, dt);
       v[k] = vc;
+    } else {
+      xc = xc + vc * cdrift * dt;
     }
-    const double xc = x[k] + vc * cdrift * dt;
     x[k] = xc;
     finite = finite && isfinite(xc) && isfinite(vc);
   }
@@ -92,7 +93,7 @@ __global__ __launch_bounds__(256) void k_kick(int n, double* __restrict__ v, con
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     const size_t k = (size_t)c * n + i;
-    v[k] = v[k] + 0.5 * a[k] * dt;
+    v[k] = kick_1(v[k], a[k], dt);
   }
 }
 
@@ -233,6 +234,7 @@ int launch_kick_drift(aster_ctx* c, double dt_prev, double dt, bool box) {
   const int n = (int)c->n;
   const int blocks = (n + 255) / 256;
   c->box_parts = 0;
+  c->src_ready = SrcReady{};
   // (at least what launch_box reserves, so that it never reallocates the partials)
   if (box) ASTER_HIP(c, c->boxpart.reserve((size_t)3 * std::max(blocks, kBoxBlocks)));
   phase_begin(c, ASTER_PHASE_KICKDRIFT);
@@ -252,11 +254,12 @@ int launch_kick_drift(aster_ctx* c, double dt_prev, double dt, bool box) {
   return ASTER_OK;
 }
 
-int launch_saba_stage(aster_ctx* c, bool kick, double d, double cdrift, double dt) {
+int launch_saba_stage(aster_ctx* c, bool kick, double d, double cdrift, double dt, double cd_next) {
   const int n = (int)c->n;
+  c->src_ready = SrcReady{};
   phase_begin(c, ASTER_PHASE_KICKDRIFT);
   hipLaunchKernelGGL(k_saba_stage, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, c->x.p, c->v.p, c->a.p,
-                     kick ? 1 : 0, d, cdrift, dt, c->flags.p);
+                     kick ? 1 : 0, d, cdrift, cd_next, dt, c->flags.p);
   ASTER_HIP(c, hipGetLastError());
   phase_end(c, ASTER_PHASE_KICKDRIFT);
   return ASTER_OK;
@@ -267,6 +270,15 @@ int launch_kick(aster_ctx* c, double dt) {
   hipLaunchKernelGGL(k_kick, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, c->v.p, c->a.p, dt);
   ASTER_HIP(c, hipGetLastError());
   return ASTER_OK;
+}
+
+int launch_post(aster_ctx* c, const StepPost& post, bool box) {
+  switch (post.kind) {
+    case POST_KICK_DRIFT: return launch_kick_drift(c, post.dt_prev, post.dt, box);
+    case POST_KICK: return launch_kick(c, post.dt);
+    case POST_SABA: return launch_saba_stage(c, true, post.d, post.cd, post.dt, post.cd_next);
+    default: return ASTER_OK;
+  }
 }
 
 int launch_energy(aster_ctx* c, double* out6) {

@@ -137,6 +137,7 @@ int import_state(aster_ctx* c, int64_t n, const double* d_pos, const double* d_v
   c->e0_valid = false;
   c->mass_total_valid = false;
   c->box_parts = 0;
+  c->src_ready = SrcReady{};
   return ASTER_OK;
 }
 
@@ -186,6 +187,7 @@ int grow_state(aster_ctx* c, int64_t add, int64_t* base) {
   c->e0_valid = false;
   c->mass_total_valid = false;
   c->box_parts = 0;
+  c->src_ready = SrcReady{};
   *base = n0;
   return ASTER_OK;
 }

@@ -1,0 +1,55 @@
+"""The all-pairs FP32 paths over small and middle sizes, through the C ABI: the
+sizes at which the kernel, the number of rounds or the last tile changes. The
+updates fused into the evaluation give the bits of separate calls."""
+import numpy as np
+import pytest
+
+import aster_amd as A
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [1, 15, 16, 17, 64, 65, 1000, 1024, 1025, 2112, 4095, 4096, 4097, 20481, 32768, 32769]
+
+
+def state(n, seed=3):
+    pos, vel, mass = A.ic_plummer(n, seed, mass_mode=1)
+    return pos, vel, mass
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("soft", [2.5e-5, 0.0])
+def test_fp32_forces_against_fp64(ctx, n, soft):
+    """The FP32 bars (mixed 1e-5, plain 1e-4) of every body relative to max(|a_i|, median |a|), full range and a source
+    range that starts and ends inside tiles."""
+    pos, vel, mass = state(n)
+    ranges = [(0, -1)] + ([(n // 3, n - n // 5)] if n > 10 else [])
+    for lower, upper in ranges:
+        ctx.set_params(G=1.3, softening=soft, lower=lower, upper=upper)
+        ctx.set_state(pos, vel, mass)
+        ref = ctx.forces(A.ALLPAIRS_FP64)
+        scale = np.linalg.norm(ref, axis=1)
+        scale = np.maximum(scale, np.median(scale)) + 1e-300
+        for method, bar in ((A.ALLPAIRS_FP32_KAHAN, 1e-5), (A.ALLPAIRS_FP32, 1e-4)):
+            err = np.linalg.norm(ctx.forces(method) - ref, axis=1) / scale
+            assert err.max() <= bar, (lower, upper, method, err.max())
+
+
+@pytest.mark.parametrize("n", [1, 17, 1025, 4096, 4097, 33000])
+@pytest.mark.parametrize("method", [A.ALLPAIRS_FP32_KAHAN, A.ALLPAIRS_FP32])
+def test_fused_updates_same_bits_as_separate_calls(ctx, n, method):
+    """Several steps in one call against one step per call (whose closing kick and opening drift are launches of their
+    own), for every integrator, with and without velocity-dependent terms."""
+    pos, vel, mass = state(n)
+    runs = [(A.LEAPFROG, 0, A.NEWTON), (A.YOSHIDA4, 0, A.NEWTON), (A.EULER, 1, A.NEWTON), (A.SABA, 3, A.NEWTON)]
+    if n < 5000:
+        runs.append((A.LEAPFROG, 0, A.NEWTON | A.PN1))
+    for integrator, order, flags in runs:
+        out = []
+        for parts in ((3,), (1, 1, 1)):
+            ctx.set_params(G=1.0, softening=1e-4, c=10.0, pn_flags=flags)
+            ctx.set_state(pos, vel, mass)
+            for k in parts:
+                ctx.integrate(method, integrator, order, 1e-3, k)
+            out.append(ctx.get_state() + (ctx.get_acc(),))
+        for a, b in zip(*out):
+            assert np.all(np.isfinite(a)) and np.array_equal(a, b), (integrator, order, flags)
