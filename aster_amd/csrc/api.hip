@@ -165,8 +165,12 @@ int aster_destroy(aster_ctx* c) {
   Bt.doff.release(); Bt.lane_body.release(); Bt.lane_seg.release(); Bt.wave_max.release();
   Bt.traj.release(); Bt.x0.release(); Bt.v0.release(); Bt.tgrad.release(); Bt.tout.release(); Bt.tsnap.release();
   auto& A = c->adj;
-  A.ckpt_x.release(); A.ckpt_v.release(); A.lx.release(); A.lv.release(); A.lm.release(); A.w.release();
-  A.snapg.release(); A.g.release(); A.wsrc.release(); A.part.release();
+  A.ckpt_x.release(); A.ckpt_v.release(); A.lx.release(); A.lv.release(); A.lm.release();
+  A.snapg.release(); A.part.release();
+  for (int b = 0; b < 2; ++b) {
+    A.src[b].release();
+    A.wsrc[b].release();
+  }
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return ASTER_OK;

@@ -104,10 +104,9 @@ struct AdjointState {
   std::vector<int64_t> snap_steps;
   DBuf<double> ckpt_x, ckpt_v;  // (nsteps/ckpt_every + 1) * 3n each
   DBuf<double> lx, lv, lm;      // adjoint accumulators (3n, 3n, n)
-  DBuf<double> w;               // weights for the fused VJP (3n)
   DBuf<double> snapg;           // snapshot positions, then their gradients (nsnap * 3n)
-  DBuf<double> g;               // J^T w (3n) and M^T w (n) of the current step
-  DBuf<float4> wsrc;            // FP32 {w, m} per source, npad
+  DBuf<double4> src[2];         // sources of the current step (and the next): FP64 position, FP32 mass; npad
+  DBuf<float4> wsrc[2];         // FP32 {w, m} per source, npad
   DBuf<double> part;            // slice partials: slices * 7 * n
   bool ready = false;
 };

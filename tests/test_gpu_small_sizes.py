@@ -53,3 +53,21 @@ def test_fused_updates_same_bits_as_separate_calls(ctx, n, method):
             out.append(ctx.get_state() + (ctx.get_acc(),))
         for a, b in zip(*out):
             assert np.all(np.isfinite(a)) and np.array_equal(a, b), (integrator, order, flags)
+
+
+@pytest.mark.parametrize("n", [2, 16, 17, 100, 1025, 4097])
+def test_gradient_against_oracle(ctx, orc, n):
+    """Relative 2-norm of each gradient block against the FP64 oracle adjoint: 1e-4, the bar of the adjoint's own tests."""
+    pos, vel, mass = A.ic_plummer(n, 5)
+    steps, snaps = (12, [4, 5, 12]) if n < 1000 else (4, [1, 4])
+    rng = np.random.default_rng(n)
+    ctx.set_params(G=1.0, softening=1e-2)
+    ctx.set_state(pos, vel, mass)
+    s = ctx.traj_forward(1e-2, steps, 4 if n < 1000 else 3, snaps)
+    target = s + rng.normal(scale=1e-2, size=s.shape)
+    got = ctx.traj_backward(2.0 * (s - target) / (n * len(snaps)))
+    _, *ref = orc.traj_grad(pos, vel, mass, 1e-2, steps, np.array(snaps), target, soft=1e-2)
+    for g, r in zip(got, ref):
+        assert np.linalg.norm(g - r) <= 1e-4 * np.linalg.norm(r)
+    p, v = ctx.get_state()
+    assert np.array_equal(p, pos) and np.array_equal(v, vel)
