@@ -24,6 +24,7 @@
 #include <cmath>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "common.hpp"
 #include "device.hpp"
@@ -408,134 +409,207 @@ __global__ __launch_bounds__(256) void k_combine(int n, int npad, int S, const d
 // division and square root, no contraction. MODE 0: Newton (+ the
 // post-Newtonian terms pnf selects if PN); MODE 1: only the post-Newtonian
 // terms (added to an FP32 Newtonian result). x, v: SoA planes [3][n]; ic = 1/c.
-// A block owns kF64Targets targets and walks the sources in chunks of
-// kF64Chunk: all 256 threads form the chunk's pair contributions f/m_i
-// (4 each) into LDS, then each target's thread adds its row in j order (the
-// self pair and sources past upper are skipped by a select). Every target sums
-// the same doubles in the same order as a sequential loop would, so the
-// result is bit-identical; a 4096-body problem runs 256 blocks instead of 16
-// wavefronts of long dependent chains.
-constexpr int kF64Targets = 16;
+//
+// Every target's sum is one dependent chain over its sources; the pair
+// contributions are independent. A block owns 16 targets and walks the sources
+// in chunks of 64, one per lane: its 8 worker waves form the chunk's
+// contributions f/m_i for two targets each (the targets' values are uniform,
+// the next chunk's sources load during the arithmetic) and put them in LDS
+// rows, one per target and coordinate; a ninth wave adds the chunk before, one
+// row per lane, in j order. A contribution that does not count (the target's
+// own, sources past upper) is written as 0: adding +0 changes no sum that
+// began at +0, so every sum has the bits of a sequential loop.
+// Bound: FP64 issue (45 FP64 instructions and a v_rsq_f64 per pair, 57 VALU in
+// all, the adding wave's share included); few bodies: the adding wave's chain.
+// Per evaluation, against 256 threads that formed a chunk with IEEE square
+// root and division and then waited for 16 of them to add it (above 32768
+// bodies: one target per lane): n = 1000 70 -> 16 us, 4096 264 -> 55 us, 16384
+// 1.89 -> 0.64 ms, 65536 15.4 -> 9.2 ms; with the 1PN term 79 -> 31 us, 297 ->
+// 114 us, 2.60 -> 1.78 ms, 31.6 -> 28.1 ms.
 constexpr int kF64Chunk = 64;
 
-template <bool PN, int MODE>
-__global__ __launch_bounds__(256) void k_allpairs_f64_tiled(int n, int lower, int upper,
-                                                            const double* __restrict__ x,
-                                                            const double* __restrict__ v,
-                                                            const double* __restrict__ m, double G, double ic,
-                                                            int pnf, double soft, double* __restrict__ a) {
+template <int W, int kPer, bool PN, int MODE>
+__global__ __launch_bounds__(64 * (W + 1)) void k_allpairs_f64(int n, int lower, int upper,
+                                                                        const double* __restrict__ x,
+                                                                        const double* __restrict__ v,
+                                                                        const double* __restrict__ m, double G,
+                                                                        double ic, int pnf, double soft,
+                                                                        double* __restrict__ a) {
 #pragma clang fp contract(off)
-  __shared__ double cf[3][kF64Targets][kF64Chunk + 1];
-  const int t = threadIdx.x;
-  const int ti = t % kF64Targets, sj = t / kF64Targets;  // this thread's target and first source slot
-  const int i = blockIdx.x * kF64Targets + ti;
-  const int ii = i < n ? i : n - 1;
-  const double p1x = x[ii], p1y = x[n + ii], p1z = x[2 * n + ii];
-  const double m1 = m[ii];
-  double v1x = 0.0, v1y = 0.0, v1z = 0.0;
-  if (PN) {
-    v1x = v[ii];
-    v1y = v[n + ii];
-    v1z = v[2 * n + ii];
-  }
-  double ax = 0.0, ay = 0.0, az = 0.0;  // the sums (threads t < kF64Targets)
-  for (int jb = lower; jb < upper; jb += kF64Chunk) {
+  constexpr int kF64Targets = W * kPer;
+  static_assert(3 * kF64Targets <= 64, "one row per lane of the adding wave");
+  // rows start on different banks (16-byte reads of the adding wave)
+  __shared__ double cf[2][3 * kF64Targets][kF64Chunk + 2];
+  __shared__ int in_range[2][W];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i0 = blockIdx.x * kF64Targets;
+  const int chunks = (upper - lower + kF64Chunk - 1) / kF64Chunk;
+  if (w < W) {
+    double p1x[kPer], p1y[kPer], p1z[kPer], v1x[kPer], v1y[kPer], v1z[kPer];
+    Divisor64 m1[kPer];
+    bool range1 = law_in_range64(G, soft);
 #pragma unroll
-    for (int q = 0; q < kF64Chunk * kF64Targets / 256; ++q) {
-      const int s = sj + q * (256 / kF64Targets);
-      const int j = min(jb + s, upper - 1);
-      const double p2x = x[j], p2y = x[n + j], p2z = x[2 * n + j];
-      const double m2 = m[j];
-      const double dx = p2x - p1x, dy = p2y - p1y, dz = p2z - p1z;
-      const double r2 = dx * dx + dy * dy + dz * dz + soft;
-      const double inv_r = 1.0 / sqrt(r2);
-      const double inv_r2 = inv_r * inv_r;
-      const double nx = dx * inv_r, ny = dy * inv_r, nz = dz * inv_r;
-      double fx = 0.0, fy = 0.0, fz = 0.0;
-      if (MODE == 0) {
-        const double scal = G * m2 * m1 * inv_r2;
-        fx = nx * scal;
-        fy = ny * scal;
-        fz = nz * scal;
-      }
+    for (int q = 0; q < kPer; ++q) {
+      const int i = min(i0 + w * kPer + q, n - 1);
+      p1x[q] = x[i];
+      p1y[q] = x[n + i];
+      p1z[q] = x[2 * n + i];
+      m1[q] = divisor64(m[i]);
+      v1x[q] = PN ? v[i] : 0.0;
+      v1y[q] = PN ? v[n + i] : 0.0;
+      v1z[q] = PN ? v[2 * n + i] : 0.0;
+      range1 = range1 && coord_in_range64(p1x[q]) && coord_in_range64(p1y[q]) && coord_in_range64(p1z[q]) &&
+               mass_in_range64(m1[q].b);
+    }
+    // byte offsets of 32 bits from uniform plane addresses (n <= 2^28)
+    auto at = [](const double* plane, uint32_t off) {
+      return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(plane) + off);
+    };
+    const double *xp = x, *yp = x + n, *zp = x + 2 * (size_t)n;
+    const uint32_t last = 8u * (uint32_t)(upper - 1);
+    auto chunk_off = [&](int ch) { return min(8u * (uint32_t)(lower + ch * kF64Chunk + lane), last); };
+    double sx, sy, sz, sm, svx = 0.0, svy = 0.0, svz = 0.0;
+    auto fetch = [&](int ch) {
+      const uint32_t o = chunk_off(ch);
+      sx = at(xp, o);
+      sy = at(yp, o);
+      sz = at(zp, o);
+      sm = at(m, o);
       if (PN) {
-        const double v2x = v[j], v2y = v[n + j], v2z = v[2 * n + j];
-        pn_add64(pnf, m1, m2, v1x, v1y, v1z, v2x, v2y, v2z, inv_r, -nx, -ny, -nz, G, ic, fx, fy, fz);
+        svx = at(v, o);
+        svy = at(v + n, o);
+        svz = at(v + 2 * (size_t)n, o);
       }
-      cf[0][ti][s] = fx / m1;
-      cf[1][ti][s] = fy / m1;
-      cf[2][ti][s] = fz / m1;
+    };
+    // Each worker looks at the range of one chunk's sources of the next W and
+    // leaves the verdict in LDS.
+    double cx, cy, cz, cm;
+    auto check_fetch = [&](int group) {
+      const uint32_t o = chunk_off(min(group * W + w, chunks - 1));
+      cx = at(xp, o);
+      cy = at(yp, o);
+      cz = at(zp, o);
+      cm = at(m, o);
+    };
+    auto check_leave = [&](int group) {
+      const bool ok = __all(coord_in_range64(cx) && coord_in_range64(cy) && coord_in_range64(cz) && mass_in_range64(cm));
+      if (lane == 0) in_range[group & 1][w] = ok ? 1 : 0;
+    };
+    if (chunks > 0) {
+      check_fetch(0);
+      fetch(0);
+      check_leave(0);
+      check_fetch(1);
     }
     __syncthreads();
-    if (t < kF64Targets) {
-      const int cnt = min(kF64Chunk, upper - jb);
-      for (int s = 0; s < kF64Chunk; ++s) {
-        const bool take = s < cnt && jb + s != ii;
-        const double nax = ax + cf[0][t][s], nay = ay + cf[1][t][s], naz = az + cf[2][t][s];
-        ax = take ? nax : ax;
-        ay = take ? nay : ay;
-        az = take ? naz : az;
+    for (int ch = 0; ch < chunks; ++ch) {
+      const double p2x = sx, p2y = sy, p2z = sz, m2 = sm, v2x = svx, v2y = svy, v2z = svz;
+      if (ch + 1 < chunks) fetch(ch + 1);
+      const int jb = lower + ch * kF64Chunk;
+      const int group = ch / W;
+      const bool fast = range1 && __builtin_amdgcn_readfirstlane(in_range[group & 1][ch % W]) != 0;
+      if (ch % W == 0) {  // the next group's verdicts, seen after this chunk's barrier
+        check_leave(group + 1);
+        check_fetch(group + 2);
+      }
+      // one straight stretch of code for the targets of a wave, so that their
+      // chains overlap
+      auto chunk = [&](auto fast_tag) {
+        constexpr bool FAST = decltype(fast_tag)::value;
+        double dx[kPer], dy[kPer], dz[kPer], r2[kPer], inv_r[kPer], f[kPer][3];
+        bool odd = false, fdiv = FAST;
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+          dx[q] = p2x - p1x[q];
+          dy[q] = p2y - p1y[q];
+          dz[q] = p2z - p1z[q];
+          r2[q] = dx[q] * dx[q] + dy[q] * dy[q] + dz[q] * dz[q] + soft;
+        }
+        if (FAST)
+          odd = inv_sqrt64_fast<kPer>(r2, inv_r);
+        else
+#pragma unroll
+          for (int q = 0; q < kPer; ++q) inv_r[q] = 1.0 / sqrt(r2[q]);
+        if (FAST && __builtin_expect(__any(odd), 0)) {
+#pragma unroll
+          for (int q = 0; q < kPer; ++q) inv_r[q] = 1.0 / sqrt(r2[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+          const double inv_r2 = inv_r[q] * inv_r[q];
+          const double nx = dx[q] * inv_r[q], ny = dy[q] * inv_r[q], nz = dz[q] * inv_r[q];
+          f[q][0] = f[q][1] = f[q][2] = 0.0;
+          if (MODE == 0) {
+            const double scal = G * m2 * m1[q].b * inv_r2;
+            f[q][0] = nx * scal;
+            f[q][1] = ny * scal;
+            f[q][2] = nz * scal;
+          }
+          if (PN) {
+            pn_add64(pnf, m1[q].b, m2, v1x[q], v1y[q], v1z[q], v2x, v2y, v2z, inv_r[q], -nx, -ny, -nz, G, ic, f[q][0], f[q][1],
+                     f[q][2]);
+            // the post-Newtonian terms have no bounds of their own
+            fdiv = fdiv && zero_or_within64(f[q][0], 1023 - 800, 1023 + 800) &&
+                   zero_or_within64(f[q][1], 1023 - 800, 1023 + 800) && zero_or_within64(f[q][2], 1023 - 800, 1023 + 800);
+          }
+        }
+        if (FAST && (!PN || __all(fdiv))) {
+#pragma unroll
+          for (int q = 0; q < kPer; ++q) div64_fast<3>(f[q], m1[q]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < kPer; ++q) {
+            f[q][0] = f[q][0] / m1[q].b;
+            f[q][1] = f[q][1] / m1[q].b;
+            f[q][2] = f[q][2] / m1[q].b;
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+          const int t = w * kPer + q, i = i0 + t;
+          if (jb + kF64Chunk > upper || (i >= jb && i < jb + kF64Chunk)) {  // wave-uniform
+            const bool take = jb + lane < upper && jb + lane != i;
+            f[q][0] = take ? f[q][0] : 0.0;
+            f[q][1] = take ? f[q][1] : 0.0;
+            f[q][2] = take ? f[q][2] : 0.0;
+          }
+          cf[ch & 1][t][lane] = f[q][0];
+          cf[ch & 1][kF64Targets + t][lane] = f[q][1];
+          cf[ch & 1][2 * kF64Targets + t][lane] = f[q][2];
+        }
+      };
+      if (fast) chunk(std::true_type{});
+      else chunk(std::false_type{});
+      __syncthreads();  // this chunk's contributions are there, the chunk before is added
+    }
+    return;
+  }
+  const int row = min(lane, 3 * kF64Targets - 1);
+  double acc = 0.0;
+  __syncthreads();
+  for (int ch = 0; ch < chunks; ++ch) {
+    __syncthreads();
+    const double2* __restrict__ c = reinterpret_cast<const double2*>(cf[ch & 1][row]);
+    constexpr int kB = 8;  // values read ahead of the adds, and kept there
+    double2 d[kB], next[kB];
+#pragma unroll
+    for (int u = 0; u < kB; ++u) d[u] = c[u];
+#pragma unroll
+    for (int s = 0; s < kF64Chunk / 2; s += kB) {
+#pragma unroll
+      for (int u = 0; u < kB; ++u) next[u] = c[min(s + kB, kF64Chunk / 2 - kB) + u];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        acc += d[u].x;
+        acc += d[u].y;
+        d[u] = next[u];
       }
     }
-    __syncthreads();  // the next chunk rewrites the contributions
   }
-  if (t < kF64Targets && i < n) {
-    a[i] = ax;
-    a[n + i] = ay;
-    a[2 * n + i] = az;
-  }
-}
-
-// One target per thread, the sources in j order (the same sums as
-// k_allpairs_f64_tiled, which is faster when there are few targets): four
-// sources per iteration, whose pair forces are independent, added one by one.
-template <bool PN, int MODE>
-__global__ __launch_bounds__(256) void k_allpairs_f64(int n, int lower, int upper, const double* __restrict__ x,
-                                                      const double* __restrict__ v, const double* __restrict__ m,
-                                                      double G, double ic, int pnf, double soft,
-                                                      double* __restrict__ a) {
-#pragma clang fp contract(off)
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int ii = i < n ? i : n - 1;
-  const double p1x = x[ii], p1y = x[n + ii], p1z = x[2 * n + ii];
-  const double m1 = m[ii];
-  double v1x = 0.0, v1y = 0.0, v1z = 0.0;
-  if (PN) {
-    v1x = v[ii];
-    v1y = v[n + ii];
-    v1z = v[2 * n + ii];
-  }
-  double ax = 0.0, ay = 0.0, az = 0.0;
-#pragma unroll 4
-  for (int j = lower; j < upper; ++j) {
-    const double p2x = x[j], p2y = x[n + j], p2z = x[2 * n + j];
-    const double m2 = m[j];
-    const double dx = p2x - p1x, dy = p2y - p1y, dz = p2z - p1z;
-    const double r2 = dx * dx + dy * dy + dz * dz + soft;
-    const double inv_r = 1.0 / sqrt(r2);
-    const double inv_r2 = inv_r * inv_r;
-    const double nx = dx * inv_r, ny = dy * inv_r, nz = dz * inv_r;
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-    if (MODE == 0) {
-      const double scal = G * m2 * m1 * inv_r2;
-      fx = nx * scal;
-      fy = ny * scal;
-      fz = nz * scal;
-    }
-    if (PN) {
-      const double v2x = v[j], v2y = v[n + j], v2z = v[2 * n + j];
-      pn_add64(pnf, m1, m2, v1x, v1y, v1z, v2x, v2y, v2z, inv_r, -nx, -ny, -nz, G, ic, fx, fy, fz);
-    }
-    const double nax = ax + fx / m1, nay = ay + fy / m1, naz = az + fz / m1;
-    ax = j == ii ? ax : nax;
-    ay = j == ii ? ay : nay;
-    az = j == ii ? az : naz;
-  }
-  if (i < n) {
-    a[i] = ax;
-    a[n + i] = ay;
-    a[2 * n + i] = az;
-  }
+  const int i = i0 + lane % kF64Targets;
+  if (lane < 3 * kF64Targets && i < n) a[(size_t)(lane / kF64Targets) * n + i] = acc;
 }
 
 // ----------------------------------------------------------------- EIH ----
@@ -564,7 +638,7 @@ __global__ __launch_bounds__(256) void k_eih_pass1(int n, const double* __restri
     if (j == i) continue;
     const double dx = x[j] - p1x, dy = x[n + j] - p1y, dz = x[2 * n + j] - p1z;
     const double r2 = dx * dx + dy * dy + dz * dz + soft;
-    const double inv_r = 1.0 / sqrt(r2);
+    const double inv_r = inv_sqrt64(r2);
     const double inv_r3 = inv_r * inv_r * inv_r;
     const double mu = G * m[j];
     ph += mu * inv_r;
@@ -595,7 +669,7 @@ __global__ __launch_bounds__(256) void k_eih_pass2(int n, const double* __restri
     if (j == i) continue;
     const double dx = x[j] - p1x, dy = x[n + j] - p1y, dz = x[2 * n + j] - p1z;
     const double r2 = dx * dx + dy * dy + dz * dz + soft;
-    const double inv_r = 1.0 / sqrt(r2);
+    const double inv_r = inv_sqrt64(r2);
     const double inv_r3 = inv_r * inv_r * inv_r;
     const double mu = G * m[j];
     const double v2x = v[j], v2y = v[n + j], v2z = v[2 * n + j];
@@ -627,40 +701,25 @@ __global__ __launch_bounds__(256) void k_eih_pass2(int n, const double* __restri
 
 // --------------------------------------------------------------- launch ----
 
-// Bit-exact FP64 sums: the tiled kernel below kF64TiledMax targets (few
-// wavefronts of one target per lane would leave most SIMDs idle), one target
-// per lane above.
-#ifndef ASTER_F64_TILED_MAX
-#define ASTER_F64_TILED_MAX 32768
-#endif
-constexpr int kF64TiledMax = ASTER_F64_TILED_MAX;
+template <int W, int PER>
+static void launch_allpairs_f64_as(aster_ctx* c, bool pn, int mode, int n, int lower, int upper, double ic, int pnf,
+                                   double* out) {
+  auto k = mode == 1 ? k_allpairs_f64<W, PER, true, 1>
+                     : pn ? k_allpairs_f64<W, PER, true, 0> : k_allpairs_f64<W, PER, false, 0>;
+  const int targets = W * PER;
+  hipLaunchKernelGGL(k, dim3((n + targets - 1) / targets), dim3(64 * (W + 1)), 0, c->stream, n, lower, upper, c->x.p,
+                     c->v.p, c->m.p, c->P.G, ic, pnf, c->P.softening, out);
+}
 
+// 16 targets a block fill the 256 CUs once at 4096 bodies and twice at 8192;
+// seven workers and the adding wave load the four SIMDs evenly, which counts
+// with many blocks: 8 and 7 workers ran 55 and 80 us at n = 4096, 165 and 205 at
+// 8192, 797 and 672 at 16384, 10.9 and 9.9 ms at 65536 (with the 1PN term 28.5
+// and 33.3 ms), both before the division took four steps instead of five.
 static int launch_allpairs_f64(aster_ctx* c, bool pn, int mode, int n, int lower, int upper, double ic, int pnf,
                                double* out) {
-  const bool tiled = n <= kF64TiledMax;
-  const dim3 grid(tiled ? (n + kF64Targets - 1) / kF64Targets : (n + 255) / 256), block(256);
-  const double G = c->P.G, soft = c->P.softening;
-  if (tiled) {
-    if (mode == 1)
-      hipLaunchKernelGGL((k_allpairs_f64_tiled<true, 1>), grid, block, 0, c->stream, n, lower, upper, c->x.p,
-                         c->v.p, c->m.p, G, ic, pnf, soft, out);
-    else if (pn)
-      hipLaunchKernelGGL((k_allpairs_f64_tiled<true, 0>), grid, block, 0, c->stream, n, lower, upper, c->x.p,
-                         c->v.p, c->m.p, G, ic, pnf, soft, out);
-    else
-      hipLaunchKernelGGL((k_allpairs_f64_tiled<false, 0>), grid, block, 0, c->stream, n, lower, upper, c->x.p,
-                         c->v.p, c->m.p, G, ic, pnf, soft, out);
-  } else {
-    if (mode == 1)
-      hipLaunchKernelGGL((k_allpairs_f64<true, 1>), grid, block, 0, c->stream, n, lower, upper, c->x.p, c->v.p,
-                         c->m.p, G, ic, pnf, soft, out);
-    else if (pn)
-      hipLaunchKernelGGL((k_allpairs_f64<true, 0>), grid, block, 0, c->stream, n, lower, upper, c->x.p, c->v.p,
-                         c->m.p, G, ic, pnf, soft, out);
-    else
-      hipLaunchKernelGGL((k_allpairs_f64<false, 0>), grid, block, 0, c->stream, n, lower, upper, c->x.p, c->v.p,
-                         c->m.p, G, ic, pnf, soft, out);
-  }
+  if (pn || n <= 8192) launch_allpairs_f64_as<8, 2>(c, pn, mode, n, lower, upper, ic, pnf, out);
+  else launch_allpairs_f64_as<7, 2>(c, pn, mode, n, lower, upper, ic, pnf, out);
   ASTER_HIP(c, hipGetLastError());
   return ASTER_OK;
 }

@@ -35,6 +35,107 @@ __device__ __forceinline__ void saba_1(double& x, double& v, double a, double d,
   if (cd_next != 0.0) x = x + v * cd_next * dt;
 }
 
+// ---- correctly rounded FP64 reciprocal square root and division ----------
+//
+// The reference's 1.0 / sqrt(r2) and f / m1 round twice and once; the results
+// here are those doubles, at 14 + v_rsq_f64 and 4 instructions instead of
+// about 30 and 10. Newton-Raphson with fused multiply-adds and an exact
+// residual at the end (Markstein, IBM J. Res. Dev. 34, 111 (1990)): a quotient
+// or root within one unit in the last place, corrected by its exact residual
+// times a reciprocal that is good to half a unit, is the correctly rounded
+// one. Ranges are the caller's business: no scaling is done.
+
+__device__ __forceinline__ uint32_t hi32(double x) {
+  return (uint32_t)((unsigned long long)__double_as_longlong(x) >> 32);
+}
+__device__ __forceinline__ uint32_t lo32(double x) { return (uint32_t)(unsigned long long)__double_as_longlong(x); }
+
+// 1 / sqrt(x), both rounded, for N values x in [2^-700, 2^700], step by step
+// together (their chains overlap; left alone the compiler runs one after the
+// other). A root whose mantissa is all ones is the reciprocal's exception (the
+// residual step would see a tie): returns whether a root ends in 32 ones; such
+// results must not be used.
+template <int N>
+__device__ __forceinline__ bool inv_sqrt64_fast(const double* x, double* r) {
+#pragma clang fp contract(off)
+  double g[N], h[N], e[N], s[N];
+#define ASTER_EACH(expr)                      \
+  _Pragma("unroll") for (int q = 0; q < N; ++q) { expr; } \
+  if (N > 1) __builtin_amdgcn_sched_barrier(0);
+  ASTER_EACH(e[q] = __builtin_amdgcn_rsq(x[q]))  // to 2^-24
+  ASTER_EACH(g[q] = x[q] * e[q])                 // sqrt(x)
+  ASTER_EACH(h[q] = 0.5 * e[q])                  // 1 / (2 sqrt(x))
+  ASTER_EACH(e[q] = fma(-h[q], g[q], 0.5))
+  ASTER_EACH(g[q] = fma(g[q], e[q], g[q]))
+  ASTER_EACH(h[q] = fma(h[q], e[q], h[q]))  // both to 2^-47
+  ASTER_EACH(e[q] = fma(-g[q], g[q], x[q]))
+  ASTER_EACH(g[q] = fma(e[q], h[q], g[q]))  // to one unit
+  ASTER_EACH(e[q] = fma(-h[q], g[q], 0.5))
+  ASTER_EACH(s[q] = fma(-g[q], g[q], x[q]))
+  ASTER_EACH(h[q] = fma(h[q], e[q], h[q]))  // to half a unit
+  ASTER_EACH(s[q] = fma(s[q], h[q], g[q]))  // the root
+  ASTER_EACH(r[q] = h[q] + h[q])
+  ASTER_EACH(e[q] = fma(-s[q], r[q], 1.0))
+  ASTER_EACH(r[q] = fma(e[q], r[q], r[q]))
+#undef ASTER_EACH
+  bool odd = false;
+#pragma unroll
+  for (int q = 0; q < N; ++q) odd = odd || lo32(s[q]) == 0xffffffffu;
+  return odd;
+}
+
+__device__ __forceinline__ double inv_sqrt64(double x) {
+#pragma clang fp contract(off)
+  double r;
+  const bool odd = inv_sqrt64_fast<1>(&x, &r);
+  // [2^-700, 2^700] by the exponent; also 0, negative numbers, infinity, NaN
+  if (__builtin_expect(odd || hi32(x) - 0x14300000u >= 0x6bb00000u - 0x14300000u, 0)) r = 1.0 / sqrt(x);
+  return r;
+}
+
+// A divisor with its reciprocal in two parts: y = 1 / b rounded, yl = 1 / b - y.
+struct Divisor64 {
+  double b, y, yl;
+};
+__device__ __forceinline__ Divisor64 divisor64(double b) {
+#pragma clang fp contract(off)
+  const double y = 1.0 / b;
+  return {b, y, fma(-b, y, 1.0) * y};
+}
+
+// a / b in place for N values a, step by step together; a = 0 or |a| in
+// [2^-960, 2^960], the quotient normal or 0. (A zero quotient may lose its
+// sign.) The quotient of the first two steps is off by at most one unit.
+template <int N>
+__device__ __forceinline__ void div64_fast(double* a, const Divisor64& d) {
+#pragma clang fp contract(off)
+  double u[N], e[N];
+#define ASTER_EACH(expr)                      \
+  _Pragma("unroll") for (int q = 0; q < N; ++q) { expr; } \
+  if (N > 1) __builtin_amdgcn_sched_barrier(0);
+  ASTER_EACH(u[q] = a[q] * d.y)
+  ASTER_EACH(u[q] = fma(a[q], d.yl, u[q]))
+  ASTER_EACH(e[q] = fma(-u[q], d.b, a[q]))
+  ASTER_EACH(a[q] = fma(e[q], d.y, u[q]))
+#undef ASTER_EACH
+}
+
+// |x| = 0 or in [2^(lo - 1023), 2^(hi - 1023)): by the exponent field.
+__device__ __forceinline__ bool zero_or_within64(double x, uint32_t lo, uint32_t hi) {
+  return x == 0.0 || (hi32(x) & 0x7fffffffu) - (lo << 20) < ((hi - lo) << 20);
+}
+
+// Inputs for which the Newtonian pair force and its division by m1 stay inside
+// the ranges above: coordinates 0 or 2^-100..2^100, masses 2^-150..2^150, |G|
+// 2^-100..2^100 or 0, softening 0 or 2^-300..2^200. Then a separation is 0 or
+// 2^-152..2^102, r^2 2^-304..2^205 (or 0: the result is NaN either way), the
+// force 0 or 2^-860..2^705 and the quotient 0 or 2^-1010..2^855.
+__device__ __forceinline__ bool coord_in_range64(double x) { return zero_or_within64(x, 1023 - 100, 1023 + 100); }
+__device__ __forceinline__ bool mass_in_range64(double m) { return m > 0.0 && zero_or_within64(m, 1023 - 150, 1023 + 150); }
+__device__ __forceinline__ bool law_in_range64(double G, double soft) {
+  return zero_or_within64(G, 1023 - 100, 1023 + 100) && zero_or_within64(soft, 1023 - 300, 1023 + 200);
+}
+
 // get_pn1 (src/physics/tool_chain_impl.cpp:110-118) evaluated in the
 // reference's operation order; `n` is the caller's -norm (:133).
 __device__ __forceinline__ void pn1_term64(double m1, double m2, double v1x, double v1y, double v1z, double v2x,
@@ -181,7 +282,7 @@ __device__ __forceinline__ void grav64(double m1, double m2, double v1x, double 
 #pragma clang fp contract(off)
   const double dx = p2x - p1x, dy = p2y - p1y, dz = p2z - p1z;
   const double r2 = dx * dx + dy * dy + dz * dz + soft;
-  const double inv_r = 1.0 / sqrt(r2);
+  const double inv_r = inv_sqrt64(r2);
   const double inv_r2 = inv_r * inv_r;
   const double nx = dx * inv_r, ny = dy * inv_r, nz = dz * inv_r;
   const double scal = G * m2 * m1 * inv_r2;

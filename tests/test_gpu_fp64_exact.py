@@ -1,0 +1,84 @@
+"""The FP64 paths in the reference's arithmetic, bit for bit against the oracle, where their reciprocal square root and
+division change method: roots whose mantissa is all ones, values at and beyond the ranges of the short forms, planar
+systems (zero components), and body counts at the edges of blocks, chunks and of the kernel choice."""
+import numpy as np
+import pytest
+
+import aster_amd as A
+
+pytestmark = pytest.mark.gpu
+
+
+def plummer(n, seed=1):
+    return A.ic_plummer(n, seed, mass_mode=1)
+
+
+@pytest.mark.parametrize("n", [1, 2, 13, 14, 15, 16, 17, 63, 64, 65, 129, 1000, 8192, 8193, 8207])
+def test_allpairs_sizes(ctx, orc, n):
+    pos, vel, mass = plummer(n)
+    for lower, upper in [(0, -1)] + ([(n // 3, n - n // 7), (n // 2, n // 2)] if n > 10 else []):
+        ctx.set_params(G=1.7, softening=1e-4, lower=lower, upper=upper)
+        ctx.set_state(pos, vel, mass)
+        ref = orc.allpairs(pos, vel, mass, G=1.7, soft=1e-4, lower=lower, upper=upper)
+        assert np.array_equal(ctx.forces(A.ALLPAIRS_FP64), ref), (lower, upper)
+
+
+def states():
+    pos, vel, mass = plummer(200, 2)
+    yield "plain", pos, mass, 1.0, 1e-4
+    yield "unsoftened", pos, mass, 1.0, 0.0
+    yield "planar", pos * [1.0, 1.0, 0.0], mass, 1.0, 0.0
+    # separations whose square root ends in ones: 2 - 2^-52 and neighbours, at several powers of four
+    x = np.zeros((64, 3))
+    x[1::2, 0] = np.array([np.nextafter(2.0, 0.0), 2.0 - 2.0 ** -51, 2.0 - 2.0 ** -50, 2.0, np.nextafter(2.0, 3.0),
+                           2.0 - 2.0 ** -20, 1.0, 3.0] * 4) * 2.0 ** np.repeat([0, 4, -4, 30], 8)
+    x[::2, 1] = np.arange(32) * 2.0 ** 40
+    x[1::2, 1] = np.arange(32) * 2.0 ** 40
+    yield "all-ones roots", x, np.linspace(0.5, 1.5, 64), 1.0, 0.0
+    yield "SI", pos * 1e11, mass * 1e31, 6.674e-11, 1e-14
+    for e in (-105, -100, -99, 99, 101):  # about the coordinates' range
+        yield f"coordinates 2^{e}", pos * 2.0 ** e, mass, 1.0, 0.0
+    for e in (-160, -140, 140, 160):  # about the masses' range
+        yield f"masses 2^{e}", pos, mass * 2.0 ** e, 1.0, 1e-4
+    yield "G 2^-120", pos, mass, 2.0 ** -120, 1e-4
+    yield "softening 2^-320", pos, mass, 1.0, 2.0 ** -320
+    q = pos.copy()
+    q[:7] *= 1e-300  # a few bodies beyond the range among ordinary ones
+    q[3, 1] = 5e-324
+    yield "some tiny", q, mass, 1.0, 1e-4
+    m = mass.copy()
+    m[11] = np.nextafter(2.0, 0.0)  # divisors whose mantissa is all ones
+    m[12] = np.nextafter(1.0, 0.0)
+    yield "all-ones masses", pos, m, 1.0, 1e-4
+
+
+@pytest.mark.parametrize("flags", [A.NEWTON, A.NEWTON | A.PN1])
+def test_allpairs_ranges(ctx, orc, flags):
+    for name, pos, mass, G, soft in states():
+        vel = np.random.default_rng(3).normal(size=pos.shape) * 0.1
+        ctx.set_params(G=G, softening=soft, c=30.0, pn_flags=flags)
+        ctx.set_state(pos, vel, mass)
+        ref = orc.allpairs(pos, vel, mass, G=G, soft=soft, pn=flags, c=30.0)
+        assert np.array_equal(ctx.forces(A.ALLPAIRS_FP64), ref, equal_nan=True), name
+
+
+@pytest.mark.parametrize("flags", [A.NEWTON, A.NEWTON | A.PN1, A.NEWTON | A.EIH])
+def test_ensembles_ranges(ctx, orc, flags):
+    """The same states in systems of up to 64 bodies, three leapfrog steps in the exact mode."""
+    for name, pos, mass, G, soft in states():
+        rng = np.random.default_rng(4)
+        vel = rng.normal(size=pos.shape) * 0.1
+        off, k = [0], 0
+        while off[-1] < len(mass):
+            off.append(min(len(mass), off[-1] + [64, 3, 1, 40, 17][k % 5]))
+            k += 1
+        ctx.set_params(G=G, softening=soft, c=30.0, pn_flags=flags, precision=A.FP64)
+        ctx.batch_set(np.array(off), pos, vel, mass)
+        dt = 1e-3 * min(1.0, float(np.abs(pos).max()))
+        ctx.batch_step(A.LEAPFROG, dt, 3)
+        p, v = ctx.batch_get()
+        for a, b in zip(off[:-1], off[1:]):
+            s = slice(a, b)
+            rp, rv, _ = orc.integrate(pos[s], vel[s], mass[s], dt, 3, integrator=2, G=G, soft=soft, c=30.0,
+                                      pn=flags)
+            assert np.array_equal(p[s], rp, equal_nan=True) and np.array_equal(v[s], rv, equal_nan=True), (name, a)
