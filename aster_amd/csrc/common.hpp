@@ -133,7 +133,7 @@ struct aster_ctx {
   aster::SrcReady src_ready;    // which of the two holds the next evaluation's sources
   aster::DBuf<double> apart;    // all-pairs slice partials [S][3][n]
   aster::DBuf<double> apn;      // FP64 1PN correction [3][n]
-  aster::DBuf<double> ework;    // energy work [6][n] + reduction scratch
+  aster::DBuf<double> ework;    // partial sums of the energies and of the mass sums
   aster::DBuf<double> eout;     // 8 doubles
   aster::DBuf<uint32_t> flags;  // device error word(s), 4 words
   aster::DBuf<double> boxpart;  // per-block |x| maxima for the auto box [blocks][3]

@@ -97,51 +97,118 @@ __global__ __launch_bounds__(256) void k_kick(int n, double* __restrict__ v, con
   }
 }
 
-// Per-body energy terms: out[0][i] = kinetic, out[1][i] = sum_j G m_i m_j /
-// (|r| + soft), out[2][i] = sum_j G m_i m_j / sqrt(r^2 + soft), out[3..5][i] =
-// m x cross v. Pair sums run over all j != i (each pair counted twice).
-__global__ __launch_bounds__(256) void k_energy_terms(int n, const double* __restrict__ x,
-                                                      const double* __restrict__ v, const double* __restrict__ m,
-                                                      double G, double soft, double* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int ii = i < n ? i : n - 1;
-  const double px = x[ii], py = x[n + ii], pz = x[2 * n + ii];
-  const double mi = m[ii];
+// Energy sums. Tile a of 64 bodies meets the tiles b >= a, so every pair counts
+// once: block (a, y) of one wavefront takes the `strip` tiles from a + y strip
+// on, one target per lane, the sources through LDS. It writes the wavefront's
+// sums of G m_i m_j / (|r| + soft) and G m_i m_j / sqrt(r^2 + soft) to
+// part[0/1][y ntiles + a], and for y = 0 those of the kinetic energy and of m x
+// cross v to rows[0..3][a]. Every sum has a fixed order. Bound: FP64 issue at
+// many bodies, latency at few. An aster_energy call (with its two readbacks of
+// about 25 us), against one thread per body over all sources (every pair twice):
+// n = 1000 331 -> 70 us, 4096 1205 -> 91 us, 20011 5.83 -> 0.47 ms, 65536 20.6 ->
+// 4.3 ms (2.5 ms unsoftened, where the two pair terms are one).
+__device__ __forceinline__ double wave_sum64(double v) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// sqrt(x) and 1 / x to about one unit in the last place.
+__device__ __forceinline__ double sqrt64_near(double x) {
+  if (__builtin_expect(hi32(x) - 0x14300000u >= 0x6bb00000u - 0x14300000u, 0)) return sqrt(x);  // beyond 2^+-700, or 0
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  return fma(fma(-g, g, x), h, g);
+}
+__device__ __forceinline__ double rcp64_near(double x) {
+  if (__builtin_expect(hi32(x) - 0x14300000u >= 0x6bb00000u - 0x14300000u, 0)) return 1.0 / x;
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
+
+template <bool SOFT>
+__global__ __launch_bounds__(64) void k_energy_pairs(int n, int ntiles, int strip, const double* __restrict__ x,
+                                                     const double* __restrict__ v, const double* __restrict__ m,
+                                                     double G, double soft, double* __restrict__ part,
+                                                     double* __restrict__ rows) {
+  __shared__ double4 tile[64];
+  const int lane = threadIdx.x, a = blockIdx.x;
+  const int i = a * 64 + lane, ii = min(i, n - 1);
+  const double px = x[ii], py = x[n + ii], pz = x[2 * (size_t)n + ii];
+  const double mi = i < n ? m[ii] : 0.0;
+  const int b0 = a + (int)blockIdx.y * strip, b1 = min(b0 + strip, ntiles);
+  auto fetch = [&](int b) {
+    const int j = b * 64 + lane, jj = min(j, n - 1);
+    return make_double4(x[jj], x[n + jj], x[2 * (size_t)n + jj], j < n ? m[jj] : 0.0);
+  };
   double pref = 0.0, ppl = 0.0;
-  for (int j = 0; j < n; ++j) {
-    const double dx = x[j] - px, dy = x[n + j] - py, dz = x[2 * n + j] - pz;
-    const double mj = m[j];
-    if (j == ii) continue;
-    const double r2 = dx * dx + dy * dy + dz * dz;
-    pref += mj / (sqrt(r2) + soft);
-    ppl += mj / sqrt(r2 + soft);
+  double4 q = b0 < b1 ? fetch(b0) : make_double4(0.0, 0.0, 0.0, 0.0);
+  for (int b = b0; b < b1; ++b) {
+    wave_sync();
+    tile[lane] = q;
+    wave_sync();
+    if (b + 1 < b1) q = fetch(b + 1);
+    const int cnt = min(64, n - b * 64);
+    const int from = b == a ? lane : -1;  // the pairs i < j of the tile with itself
+#pragma unroll 4
+    for (int k = 0; k < cnt; ++k) {
+      const double4 s = tile[k];
+      const double dx = s.x - px, dy = s.y - py, dz = s.z - pz;
+      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+      const double pl = inv_sqrt64(r2 + soft);
+      const bool take = k > from;
+      ppl += take ? s.w * pl : 0.0;
+      if (SOFT) pref += take ? s.w * rcp64_near(sqrt64_near(r2) + soft) : 0.0;
+    }
   }
-  if (i < n) {
-    const double vx = v[i], vy = v[n + i], vz = v[2 * n + i];
-    out[i] = 0.5 * mi * (vx * vx + vy * vy + vz * vz);
-    out[(size_t)n + i] = G * mi * pref;
-    out[(size_t)2 * n + i] = G * mi * ppl;
-    out[(size_t)3 * n + i] = mi * (py * vz - pz * vy);
-    out[(size_t)4 * n + i] = mi * (pz * vx - px * vz);
-    out[(size_t)5 * n + i] = mi * (px * vy - py * vx);
+  const double gm = G * mi;
+  const double sp = wave_sum64(i < n ? gm * ppl : 0.0);
+  const double sr = SOFT ? wave_sum64(i < n ? gm * pref : 0.0) : sp;
+  const size_t slot = (size_t)blockIdx.y * ntiles + a, slots = (size_t)gridDim.y * ntiles;
+  if (lane == 0) {
+    part[slot] = sr;
+    part[slots + slot] = sp;
+  }
+  if (blockIdx.y == 0) {
+    const double vx = v[ii], vy = v[n + ii], vz = v[2 * (size_t)n + ii];
+    const double t[4] = {0.5 * mi * (vx * vx + vy * vy + vz * vz), mi * (py * vz - pz * vy), mi * (pz * vx - px * vz),
+                         mi * (px * vy - py * vx)};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const double w = wave_sum64(t[c]);
+      if (lane == 0) rows[(size_t)c * ntiles + a] = w;
+    }
   }
 }
 
-// Deterministic reduction of `rows` rows of length n: one block, fixed
-// strided order, fixed tree.
-__global__ __launch_bounds__(1024) void k_reduce_rows(int n, int rows, const double* __restrict__ in,
-                                                      double* __restrict__ out) {
+// out = {kinetic, 2 sum_{i<j} of the two pair terms, L}: one block, fixed
+// strided order, fixed tree. 8 loads per thread are in flight.
+__global__ __launch_bounds__(1024) void k_energy_reduce(int slots, int ntiles, const double* __restrict__ part,
+                                                        const double* __restrict__ rows, double* __restrict__ out) {
   __shared__ double sm[1024];
-  for (int r = 0; r < rows; ++r) {
+  const int t = threadIdx.x;
+  for (int r = 0; r < 6; ++r) {
+    const bool pair = r == 1 || r == 2;
+    const double* __restrict__ in = pair ? part + (size_t)(r - 1) * slots : rows + (size_t)(r == 0 ? 0 : r - 2) * ntiles;
+    const int len = pair ? slots : ntiles;
     double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += 1024) s += in[(size_t)r * n + i];
-    sm[threadIdx.x] = s;
+    for (int i0 = t; i0 < len; i0 += 8 * 1024) {
+      double w[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) w[u] = in[min(i0 + u * 1024, len - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += i0 + u * 1024 < len ? w[u] : 0.0;
+    }
+    sm[t] = s;
     __syncthreads();
     for (int w = 512; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) sm[threadIdx.x] += sm[threadIdx.x + w];
+      if (t < w) sm[t] += sm[t + w];
       __syncthreads();
     }
-    if (threadIdx.x == 0) out[r] = sm[0];
+    if (t == 0) out[r] = pair ? 2.0 * sm[0] : sm[0];
     __syncthreads();
   }
 }
@@ -283,12 +350,21 @@ int launch_post(aster_ctx* c, const StepPost& post, bool box) {
 
 int launch_energy(aster_ctx* c, double* out6) {
   const int n = (int)c->n;
-  ASTER_HIP(c, c->ework.reserve((size_t)6 * n));
+  const int ntiles = (n + 63) / 64;
+  // one tile per wavefront up to 128 tiles; above, strips that keep about 16384
+  // of the 32768 blocks busy (half of them lie past the last tile)
+  const int strip = ntiles <= 128 ? 1 : (int)(((int64_t)ntiles * ntiles + 32767) / 32768);
+  const int ny = (ntiles + strip - 1) / strip;
+  const size_t slots = (size_t)ny * ntiles;
+  ASTER_HIP(c, c->ework.reserve(2 * slots + 4 * (size_t)ntiles));
   ASTER_HIP(c, c->eout.reserve(8));
-  hipLaunchKernelGGL(k_energy_terms, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, c->x.p, c->v.p, c->m.p,
-                     c->P.G, c->P.softening, c->ework.p);
+  double* rows = c->ework.p + 2 * slots;
+  auto k = c->P.softening != 0.0 ? k_energy_pairs<true> : k_energy_pairs<false>;
+  hipLaunchKernelGGL(k, dim3(ntiles, ny), dim3(64), 0, c->stream, n, ntiles, strip, c->x.p, c->v.p, c->m.p, c->P.G,
+                     c->P.softening, c->ework.p, rows);
   ASTER_HIP(c, hipGetLastError());
-  hipLaunchKernelGGL(k_reduce_rows, dim3(1), dim3(1024), 0, c->stream, n, 6, c->ework.p, c->eout.p);
+  hipLaunchKernelGGL(k_energy_reduce, dim3(1), dim3(1024), 0, c->stream, (int)slots, ntiles, (const double*)c->ework.p,
+                     (const double*)rows, c->eout.p);
   ASTER_HIP(c, hipGetLastError());
   ASTER_HIP(c, hipMemcpyAsync(out6, c->eout.p, 6 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   ASTER_HIP(c, hipStreamSynchronize(c->stream));

@@ -71,3 +71,20 @@ def test_gradient_against_oracle(ctx, orc, n):
         assert np.linalg.norm(g - r) <= 1e-4 * np.linalg.norm(r)
     p, v = ctx.get_state()
     assert np.array_equal(p, pos) and np.array_equal(v, vel)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1000, 8192, 8193, 8300])
+@pytest.mark.parametrize("soft", [1e-4, 0.0])
+def test_energy_against_oracle(ctx, orc, n, soft):
+    """One tile, its edges, one tile per strip and the first longer strips: 1e-12 relative, the bar of the energy's own
+    test (sums in another order), and the same bits on a second call."""
+    pos, vel, mass = state(n)
+    ctx.set_params(G=1.3, softening=soft)
+    ctx.set_state(pos, vel, mass)
+    e, ep, L = ctx.energy()
+    re, rep, rL = orc.energy(pos, vel, mass, G=1.3, soft=soft)
+    kin = 0.5 * float((mass[:, None] * vel * vel).sum())  # e is kinetic minus potential: bound by the larger part
+    assert abs(e - re) <= 1e-12 * (abs(re) + 2 * kin) and abs(ep - rep) <= 1e-12 * (abs(rep) + 2 * kin)
+    np.testing.assert_allclose(L, rL, rtol=1e-10, atol=1e-14)
+    e2, ep2, L2 = ctx.energy()
+    assert (e, ep) == (e2, ep2) and np.array_equal(L, L2)
