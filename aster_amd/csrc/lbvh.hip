@@ -1393,10 +1393,70 @@ __device__ __forceinline__ void group_piece_sum(const float4* __restrict__ p, in
   }
 }
 
-// Post-Newtonian terms of the group traversal (PN): with every list flush each
-// body's lane also adds, in FP64, the terms of each list entry (NodePn). The
-// list keeps its node ids in LDS for this.
-template <bool MASK, bool PN>
+// Post-Newtonian terms of the group traversal (PN): with every list flush the
+// lanes also evaluate, in FP64, the terms of each list entry (NodePn), in the
+// same pieces as the Newtonian sums. The list keeps its node ids in LDS; their
+// FP64 records are loaded during the Newtonian passes (the next batch's during
+// this one's terms) and put in LDS beside the group's bodies. Bound: FP64 issue
+// (about 52 instructions and a v_rsq_f64 per pair, the SIMDs issue in 83% of
+// their cycles). Traversal at theta 0.5 (Newtonian sums included), against one
+// lane per body, which left a third of the lanes idle and waited for the
+// gather, and 61 instructions: 1PN, 5000 bodies 352 -> 219 us, 100003 1219 ->
+// 766 us, 2^20 9.8 -> 6.3 ms; 1PN + 2PN + 2.5PN 1023 -> 986 us, 4.62 -> 4.16 ms,
+// 36.8 -> 30.3 ms. More waves (3 or 4 per SIMD by launch bounds) gained nothing.
+constexpr int kPnBatch = 64;  // entries in LDS at a time
+struct PnLds {                // behind the list, the stack and the node ids
+  double4 com[kPnBatch];      // entries: centre of mass, mass
+  double4 vel[kPnBatch];      // velocity, -2 |v|^2
+  double4 bpos[64];           // bodies: position, mass
+  double4 bvel[64];           // velocity, -|v|^2
+};
+static_assert(kPieceMaxPasses * 64 * sizeof(double) <= (kGrpList + kGrpListPad) * sizeof(float4),
+              "one coordinate of the pieces' sums takes the list's place");
+
+// get_pn1 (tool_chain_impl.cpp:110-118) as an acceleration of the body at pb
+// by the node at nc, over G / c^2, n = (x_i - x_node)/r, grouped for fused
+// multiply-adds:
+//   m2/r^2 [n (-v1^2 - 2 v2^2 + 4 v1.v2 + 3/2 (n.v2)^2 + (5 G m1 + 4 G m2)/r)
+//           + (v1 - v2)(4 n.v1 - 3 n.v2)]
+// N entries step by step together, so that their chains overlap. Every term
+// carries n, so a node at distance 0 adds 0, as long as 1/r and the products
+// with it (up to m G m / r^4) stay finite: r^2 is kept above 1e-100.
+template <int N>
+__device__ __forceinline__ void pn1_pairs(const double4* nc, const double4* nv, const double4& pb, const double4& vb,
+                                          double g5m1, double g4, double soft, double* a) {
+  double d[N][3], x[N], y[N], e[N], n1[N], n2[N], sc[N], k[N];
+#define ASTER_EACH(...)                                          \
+  _Pragma("unroll") for (int q = 0; q < N; ++q) { __VA_ARGS__; } \
+  __builtin_amdgcn_sched_barrier(0);
+  ASTER_EACH(d[q][0] = nc[q].x - pb.x; d[q][1] = nc[q].y - pb.y; d[q][2] = nc[q].z - pb.z)
+  ASTER_EACH(x[q] = fma(d[q][0], d[q][0], fma(d[q][1], d[q][1], fma(d[q][2], d[q][2], soft))))
+  ASTER_EACH(x[q] = fmax(x[q], 1e-100))
+  ASTER_EACH(y[q] = __builtin_amdgcn_rsq(x[q]))
+  // meanwhile what needs no 1 / r: d.v1, d.v2 and the velocity terms
+  ASTER_EACH(n1[q] = fma(d[q][0], vb.x, fma(d[q][1], vb.y, d[q][2] * vb.z)))
+  ASTER_EACH(n2[q] = fma(d[q][0], nv[q].x, fma(d[q][1], nv[q].y, d[q][2] * nv[q].z)))
+  ASTER_EACH(sc[q] = fma(vb.x, nv[q].x, fma(vb.y, nv[q].y, vb.z * nv[q].z)))
+  ASTER_EACH(sc[q] = fma(4.0, sc[q], vb.w) + nv[q].w)
+  // 1 / r: one third-order step from the estimate (rsqrt64)
+  ASTER_EACH(e[q] = x[q] * y[q])
+  ASTER_EACH(e[q] = fma(-e[q], y[q], 1.0))
+  ASTER_EACH(k[q] = fma(0.375, e[q], 0.5); e[q] = e[q] * y[q])
+  ASTER_EACH(y[q] = fma(e[q], k[q], y[q]))
+  // n = -d / r: n.v = -(d.v) / r
+  ASTER_EACH(n2[q] = n2[q] * y[q]; n1[q] = n1[q] * y[q])
+  ASTER_EACH(sc[q] = fma(1.5 * n2[q], n2[q], sc[q]); x[q] = fma(g4, nc[q].w, g5m1))
+  ASTER_EACH(sc[q] = fma(x[q], y[q], sc[q]); k[q] = nc[q].w * (y[q] * y[q]); e[q] = fma(4.0, n1[q], -3.0 * n2[q]))
+  ASTER_EACH(sc[q] = sc[q] * y[q]; e[q] = e[q] * k[q])
+  ASTER_EACH(sc[q] = sc[q] * k[q])
+  // a -= k (d sc / r + (v1 - v2) (4 d.v1 - 3 d.v2) / r)
+  ASTER_EACH(a[0] = fma(-sc[q], d[q][0], a[0]); a[1] = fma(-sc[q], d[q][1], a[1]); a[2] = fma(-sc[q], d[q][2], a[2]))
+  ASTER_EACH(a[0] = fma(-e[q], vb.x - nv[q].x, a[0]); a[1] = fma(-e[q], vb.y - nv[q].y, a[1]);
+             a[2] = fma(-e[q], vb.z - nv[q].z, a[2]))
+#undef ASTER_EACH
+}
+
+template <bool MASK, int PN>  // PN: 0 none, 1 the 1PN term alone, 2 any terms
 __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restrict__ gstart,
                                                  const uint32_t* __restrict__ gcount, const float4* __restrict__ gsh,
                                                  const float4* __restrict__ kids, const uint32_t* __restrict__ perm,
@@ -1407,9 +1467,7 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
   float4* lst = grp_lds;                                              // kGrpList + kGrpListPad entries
   int* stk = reinterpret_cast<int*>(grp_lds + kGrpList + kGrpListPad);  // stack_cap entries
   int* lid = stk + stack_cap;  // PN: node id of each list entry (kGrpList entries)
-  // PN: the entries' FP64 node records, gathered once per flush (kGrpList each)
-  double4* pnc = reinterpret_cast<double4*>(grp_lds + kGrpList + kGrpListPad + (stack_cap + kGrpList + 3) / 4);
-  double4* pnv = pnc + kGrpList;
+  PnLds* pl = reinterpret_cast<PnLds*>(grp_lds + kGrpList + kGrpListPad + (stack_cap + kGrpList + 3) / 4);  // PN
   const int lane = threadIdx.x;
   const int ngroups = (int)*gcount;
   const int per_xcd = (ngroups + 7) >> 3;
@@ -1425,18 +1483,18 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
     const int k = lo + lane;
     const bool live = k <= hi;
     const float4 me = gsh[live ? k : hi];
-    // PN: this body's FP64 position, mass and velocity (leaf k's records)
-    double4 pme = make_double4(0.0, 0.0, 0.0, 1.0), vme = make_double4(0.0, 0.0, 0.0, 0.0);
-    double pax = 0.0, pay = 0.0, paz = 0.0;
-    if (PN) {
-      pme = pnp.nmc[live ? k : hi];
-      vme = pnp.nvel[live ? k : hi];
+    double pacc[3] = {0.0, 0.0, 0.0};  // PN: the body's terms
+    if (PN) {  // the bodies' FP64 positions, masses and velocities (the leaves' records)
+      double4 vme = pnp.nvel[live ? k : hi];
+      vme.w = -fma(vme.x, vme.x, fma(vme.y, vme.y, vme.z * vme.z));
+      pl->bpos[lane] = pnp.nmc[live ? k : hi];
+      pl->bvel[lane] = vme;
     }
     // this lane's piece in each pass
     const int npass = __builtin_amdgcn_readfirstlane((int)kPieces.passes[gsz]);
     const int npc = __builtin_amdgcn_readfirstlane((int)kPieces.pieces[gsz]);
     float4 ppos[kPieceMaxPasses];
-    int pidx[kPieceMaxPasses];
+    int pidx[kPieceMaxPasses], pbody[kPieceMaxPasses];
 #pragma unroll
     for (int p = 0; p < kPieceMaxPasses; ++p) {
       const int j = 64 * p + lane;
@@ -1447,6 +1505,7 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
       }
       ppos[p] = make_float4(__shfl(me.x, b, 64), __shfl(me.y, b, 64), __shfl(me.z, b, 64), 0.f);
       pidx[p] = pc;
+      pbody[p] = b;
     }
     float blo[3] = {me.x, me.y, me.z}, bhi[3] = {me.x, me.y, me.z};
 #pragma unroll
@@ -1474,6 +1533,16 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
       const int lam = __builtin_amdgcn_readfirstlane((m + npc - 1) / npc);
       const int mp = npc * lam;  // m <= mp < m + npc <= m + 64
       if (lane < mp - m) lst[m + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+      double4 ec, ev;
+      auto gather = [&](int first) {
+        const int node = lid[min(first + lane, m - 1)];
+        ec = pnp.nmc[node];
+        ev = pnp.nvel[node];
+        if (first + lane >= m) ec.w = 0.0;  // padding: adds exactly zero
+      };
+      // whole pieces of at most kPnBatch entries
+      const int batch = PN ? __builtin_amdgcn_readfirstlane(kPnBatch / npc * npc) : 0;
+      if (PN) gather(0);  // in flight during the Newtonian passes
       wave_sync();
       float px[kPieceMaxPasses], py[kPieceMaxPasses], pz[kPieceMaxPasses];
 #pragma unroll
@@ -1500,17 +1569,55 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
         kahan_add32(sz, cz, tz);
       }
       if (PN) {
-        // gather the list's node records into LDS (one round per 64 entries),
-        // then every body's lane reads them as broadcasts
-        for (int e = lane; e < m; e += 64) {
-          const int node = lid[e];
-          pnc[e] = pnp.nmc[node];
-          pnv[e] = pnp.nvel[node];
+        double pa[kPieceMaxPasses][3];
+#pragma unroll
+        for (int p = 0; p < kPieceMaxPasses; ++p) pa[p][0] = pa[p][1] = pa[p][2] = 0.0;
+        const double g4 = 4.0 * pnp.G;
+        for (int first = 0; first < m; first += batch) {
+          const int cntb = min(batch, m - first);
+          const int lamb = __builtin_amdgcn_readfirstlane((cntb + npc - 1) / npc);
+          pl->com[lane] = ec;
+          ev.w = -2.0 * fma(ev.x, ev.x, fma(ev.y, ev.y, ev.z * ev.z));
+          pl->vel[lane] = ev;
+          wave_sync();
+          if (first + batch < m) gather(first + batch);
+#pragma unroll
+          for (int p = 0; p < kPieceMaxPasses; ++p) {
+            if (p >= npass) continue;
+            const double4 pb = pl->bpos[pbody[p]], vb = pl->bvel[pbody[p]];
+            const int e0 = pidx[p] * lamb;
+            if constexpr (PN == 1) {
+              const double g5m1 = 5.0 * pnp.G * pb.w;
+              int e = 0;
+              for (; e + 2 <= lamb; e += 2) {
+                const double4 nc[2] = {pl->com[e0 + e], pl->com[e0 + e + 1]};
+                const double4 nv[2] = {pl->vel[e0 + e], pl->vel[e0 + e + 1]};
+                pn1_pairs<2>(nc, nv, pb, vb, g5m1, g4, pnp.soft, pa[p]);
+              }
+              if (e < lamb) pn1_pairs<1>(&pl->com[e0 + e], &pl->vel[e0 + e], pb, vb, g5m1, g4, pnp.soft, pa[p]);
+            } else {
+              const double inv_m = 1.0 / pb.w;
+              for (int e = 0; e < lamb; ++e)  // every term carries the node's mass: padding adds 0
+                node_pn_rec(pnp, pl->com[e0 + e], pl->vel[e0 + e], pb, vb, inv_m, pa[p][0], pa[p][1], pa[p][2]);
+            }
+          }
+          wave_sync();  // every lane is done with these entries
         }
-        wave_sync();
-        if (live) {
-          const double inv_m = 1.0 / pme.w;
-          for (int e = 0; e < m; ++e) node_pn_rec(pnp, pnc[e], pnv[e], pme, vme, inv_m, pax, pay, paz);
+        // a body adds its pieces in order, one coordinate at a time through the
+        // list's LDS
+        double* ps = reinterpret_cast<double*>(lst);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+#pragma unroll
+          for (int p = 0; p < kPieceMaxPasses; ++p)
+            if (p < npass) ps[64 * p + lane] = pa[p][c];
+          wave_sync();
+          if (live) {
+            double t = 0.0;
+            for (int q = 0; q < npc; ++q) t += ps[lane * npc + q];
+            pacc[c] += PN == 1 ? t * (pnp.G * (pnp.ic * pnp.ic)) : t;
+          }
+          wave_sync();
         }
       }
       wave_sync();  // the partial sums are read before the list is refilled
@@ -1592,9 +1699,9 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
     wave_sync();
     if (live) {
       const int b = (int)perm[k];
-      a[b] = G * ((double)sx - (double)cx) + pax;
-      a[n + b] = G * ((double)sy - (double)cy) + pay;
-      a[2 * n + b] = G * ((double)sz - (double)cz) + paz;
+      a[b] = G * ((double)sx - (double)cx) + pacc[0];
+      a[n + b] = G * ((double)sy - (double)cy) + pacc[1];
+      a[2 * n + b] = G * ((double)sz - (double)cz) + pacc[2];
     }
     // every body's own leaf is in its group's list (distance 0, no force)
     const unsigned long long nlive = (unsigned long long)(hi - lo + 1);
@@ -1929,11 +2036,12 @@ static int bh_forces_all(aster_ctx* c, int method) {
       const int cap = grp_stack_cap(c->tree_levels);
       // PN: node ids, then (16-byte aligned) FP64 records and velocities of the list
       const size_t lds = (kGrpList + kGrpListPad) * sizeof(float4) +
-                         (pn ? (size_t)(cap + kGrpList + 3) / 4 * sizeof(float4) + 2 * kGrpList * sizeof(double4)
+                         (pn ? (size_t)(cap + kGrpList + 3) / 4 * sizeof(float4) + sizeof(PnLds)
                              : (size_t)cap * sizeof(int));
       const NodePn gp{c->nmc.p, c->nvel.p, c->P.G, ic, c->P.softening, pnf};
-      auto kern = pn ? (mask ? k_bh_group<true, true> : k_bh_group<false, true>)
-                     : (mask ? k_bh_group<true, false> : k_bh_group<false, false>);
+      auto kern = !pn ? (mask ? k_bh_group<true, 0> : k_bh_group<false, 0>)
+                  : pnf == ASTER_PN1 ? (mask ? k_bh_group<true, 1> : k_bh_group<false, 1>)
+                                     : (mask ? k_bh_group<true, 2> : k_bh_group<false, 2>);
       hipLaunchKernelGGL(kern, grid, block, lds, c->stream, n, c->gstart.p, c->gcount.p, c->gsh.p, c->kids.p,
                          c->idx.p, eps2, sc.msc, sc.gsc, c->a.p, c->bh_counters.p, c->flags.p, cap, gp);
     } else {

@@ -88,3 +88,22 @@ def test_energy_against_oracle(ctx, orc, n, soft):
     np.testing.assert_allclose(L, rL, rtol=1e-10, atol=1e-14)
     e2, ep2, L2 = ctx.energy()
     assert (e, ep) == (e2, ep2) and np.array_equal(L, L2)
+
+
+@pytest.mark.parametrize("n", [4, 37, 64, 65, 66, 200, 1500])
+@pytest.mark.parametrize("soft", [2.5e-5, 0.0])
+@pytest.mark.parametrize("flags", [A.NEWTON | A.PN1, A.NEWTON | A.PN1 | A.PN25])
+def test_group_traversal_pn_small_groups(ctx, orc, n, soft, flags):
+    """Post-Newtonian part of the group traversal at the edges of groups, pieces and list batches, with two bodies at one
+    place: against the oracle's lists, the bars of the traversal's own test."""
+    pos, vel, mass = A.ic_mixed(n, n)
+    pos[n // 2] = pos[0]
+    part = []
+    for f in (A.NEWTON, flags):
+        ctx.set_params(G=1.0, softening=soft, theta=0.6, c=30.0, pn_flags=f)
+        ctx.set_state(pos, vel, mass)
+        part.append(ctx.forces(A.BH_GROUP))
+    ref = orc.bh_group_pn(pos, vel, mass, orc.box_auto(pos), 0.6, c=30.0, soft=soft, pn=flags)
+    scale = np.linalg.norm(ref, axis=1)
+    err = np.linalg.norm(part[1] - part[0] - ref, axis=1)
+    assert np.all(err <= 1e-9 * np.maximum(scale, np.median(scale)) + 1e-15 * np.abs(part[1]).max())
