@@ -147,17 +147,14 @@ int aster_destroy(aster_ctx* c) {
     if (e) (void)hipEventDestroy(e);
   for (auto& e : c->prof_pool)
     if (e) (void)hipEventDestroy(e);
-  if (c->tree_ev) (void)hipEventDestroy(c->tree_ev);
-  if (c->host_words) (void)hipHostFree(c->host_words);
   c->x.release(); c->x_next.release(); c->v.release(); c->m.release(); c->a.release(); c->sh.release(); c->src64.release();
   c->apart.release(); c->apn.release(); c->ework.release(); c->eout.release(); c->flags.release();
   c->boxpart.release(); c->boxd.release(); c->stage.release();
   c->codes.release(); c->xm4.release(); c->idx.release(); c->codes2.release(); c->idx2.release(); c->hist.release();
   c->left.release(); c->right.release(); c->parent.release(); c->escape.release(); c->scanpart.release();
   c->depth.release(); c->nmc.release(); c->nvel.release(); c->nbox.release();
-  c->levels.release(); c->bucket.release(); c->grange.release(); c->gscan.release();
-  c->gstart.release(); c->gcount.release(); c->splitnode.release(); c->groot.release(); c->climb.release();
-  c->dmax.release(); c->censusctr.release();
+  c->above.release(); c->units.release(); c->top.release(); c->grange.release(); c->gscan.release();
+  c->gstart.release(); c->gcount.release(); c->splitnode.release();
   c->nrec.release(); c->nlink.release(); c->kids.release(); c->topslot.release(); c->bh_counters.release(); c->gsh.release();
   c->sub_x.release(); c->sub_v.release(); c->sub_a.release(); c->sub_m.release();
   auto& Bt = c->batch;

@@ -158,12 +158,9 @@ struct aster_ctx {
   aster::DBuf<uint32_t> scanpart;                  // per-chunk totals of the device scan
   aster::DBuf<int32_t> depth;                      // 2n-1
   aster::DBuf<int32_t> splitnode;                  // internal node whose split lies after sorted position k (n-1)
-  aster::DBuf<int32_t> groot;                      // at a group's first position: the group's root node (n)
-  aster::DBuf<int32_t> climb;                      // leaf k: levels from the leaf up to its group's root (n)
-  aster::DBuf<int32_t> dmax;                       // per-block largest internal-node depth
-  aster::DBuf<uint32_t> censusctr;                 // census: per-depth counts and cursors (256)
-  aster::DBuf<int32_t> levels;                     // per-depth bucket offsets, level count, max depth
-  aster::DBuf<int32_t> bucket;                     // internal nodes grouped by depth, in-group ones last (n-1)
+  aster::DBuf<uint32_t> above;                     // lengths of the lists units, top (2)
+  aster::DBuf<int32_t> units;                      // largest nodes above the groups of at most kUnit leaves
+  aster::DBuf<int32_t> top;                        // nodes of more than kUnit leaves (n)
   aster::DBuf<int2> grange;                        // sorted-position range of internal node n+i
   aster::DBuf<uint32_t> gscan;                     // group-start flags, then their exclusive scan (n)
   aster::DBuf<int32_t> gstart;                     // first sorted position of each group (+ n)
@@ -173,16 +170,13 @@ struct aster_ctx {
   aster::DBuf<float4> nbox;                        // FP32 AABB: {lo, 0}, {hi, 0} per node (2 (2n-1))
   aster::DBuf<float4> nrec;                        // FP32 node record: com, mass (2n-1)
   aster::DBuf<int4> nlink;                         // right, escape, crit2 bits, leaf body (2n-1)
-  aster::DBuf<int32_t> topslot;                    // top-levels moments: node - n -> list position (n)
+  aster::DBuf<int32_t> topslot;                    // node - n -> position in top (n)
   aster::DBuf<float4> kids;                        // group traversal: per child slot {record}, {node, crit2} (2(2n-1))
   aster::DBuf<unsigned long long> bh_counters;     // BHC_COUNT
   aster::DBuf<float4> gsh;                         // bodies in sorted order (FP32), n
   aster::DBuf<double> sub_x, sub_v, sub_a, sub_m;  // body range [lower, upper) of a bounded Barnes-Hut evaluation
   bool tree_valid = false;
   int tree_mac = -1;
-  int tree_levels = 0;                             // depths of internal nodes: 0 .. tree_levels-1
-  int32_t* host_words = nullptr;                   // pinned: census level bounds + largest depth
-  hipEvent_t tree_ev = nullptr;                    // recorded after their readback
 
   // Timers.
   hipEvent_t ev[16] = {};

@@ -33,6 +33,7 @@ constexpr int kRsTile = 2048;  // keys per block (8 per thread)
 // Depth bound of the radix tree: an internal node's split bit strictly
 // increases with depth over 30 code bits + 32 tie-break bits, so depth <= 63.
 constexpr int kMaxLevels = 128;
+constexpr int kUnit = 4096;  // leaves per unit of the moments above the groups
 // Traversal groups (and the moment kernel's per-wavefront subtrees): subtrees
 // of at most kGroup leaves whose parent has more.
 constexpr int kGroup = 64;
@@ -64,9 +65,10 @@ __device__ __forceinline__ uint32_t cell_of(double p, double b, uint32_t* bad) {
 __global__ __launch_bounds__(256) void k_morton(int n, const double* __restrict__ x, const double* __restrict__ m,
                                                 const double* __restrict__ box, uint32_t* __restrict__ codes,
                                                 uint32_t* __restrict__ idx, double4* __restrict__ xm,
-                                                uint32_t* __restrict__ flags) {
+                                                uint32_t* __restrict__ above, uint32_t* __restrict__ flags) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  if (i < 2) above[i] = 0u;  // lengths of the lists that k_build writes
   uint32_t bad = 0;
   const double px = x[i], py = x[n + i], pz = x[2 * n + i];
   xm[i] = make_double4(px, py, pz, m[i]);
@@ -375,6 +377,11 @@ __device__ __forceinline__ int kdelta(const uint32_t* __restrict__ codes, int n,
 // Thread k initialises leaf k (body perm[k]) and, for k < n-1, the internal
 // node n+k with its sorted-position range. Also writes parent links. VEL
 // also gathers the velocities (only the 1PN traversal reads node velocities).
+// A node of more than kGroup leaves splits between two traversal groups:
+// gflag marks the position behind its split as a group's first (every
+// boundary is one node's split). Nodes of more than kUnit leaves are listed in
+// `top`, the largest nodes of at most kUnit leaves above the groups in
+// `units`, in any order (lengths above[1] and above[0]; k_moments_above).
 template <bool VEL>
 __global__ __launch_bounds__(256) void k_build(int n, const uint32_t* __restrict__ codes,
                                                const uint32_t* __restrict__ perm, const double4* __restrict__ xm,
@@ -384,6 +391,8 @@ __global__ __launch_bounds__(256) void k_build(int n, const uint32_t* __restrict
                                                double4* __restrict__ nmc, double4* __restrict__ nvel,
                                                float4* __restrict__ nbox, float4* __restrict__ nrec,
                                                float4* __restrict__ gsh, int32_t* __restrict__ splitnode,
+                                               uint32_t* __restrict__ gflag, uint32_t* __restrict__ above,
+                                               int32_t* __restrict__ units, int32_t* __restrict__ top,
                                                uint32_t* __restrict__ flags, int leaf_records) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
@@ -405,7 +414,11 @@ __global__ __launch_bounds__(256) void k_build(int n, const uint32_t* __restrict
     left[k] = -1;
     right[k] = -1;
   }
-  if (k == 0) parent[n] = -1;
+  if (k == 0) {
+    parent[n] = -1;
+    gflag[0] = 1u;
+    if (n > kGroup && n <= kUnit) units[atomicAdd(&above[0], 1u)] = n;
+  }
   if (k >= n - 1) return;
   const int i = k;
   const int d_left = (i == 0) ? -1 : kdelta(codes, n, i, i - 1);
@@ -438,6 +451,13 @@ __global__ __launch_bounds__(256) void k_build(int n, const uint32_t* __restrict
   parent[R] = n + i;
   grange[i] = make_int2(lo, hi);
   splitnode[gamma] = n + i;  // every split position belongs to exactly one internal node
+  gflag[gamma + 1] = l + 1 > kGroup ? 1u : 0u;
+  if (l + 1 > kUnit) {
+    top[atomicAdd(&above[1], 1u)] = n + i;
+    const int cl = gamma - lo + 1, cr = hi - gamma;
+    if (cl > kGroup && cl <= kUnit) units[atomicAdd(&above[0], 1u)] = L;
+    if (cr > kGroup && cr <= kUnit) units[atomicAdd(&above[0], 1u)] = R;
+  }
 }
 
 // Depth of every node and its escape link in the right-first preorder (the
@@ -464,179 +484,6 @@ __global__ __launch_bounds__(256) void k_depth(int n, const int32_t* __restrict_
   }
   depth[node] = dep;
   escape[node] = esc;
-}
-
-// Depths of the nodes above the traversal groups, whose moments the band
-// kernels form level by level. They are exactly the internal nodes whose
-// split lies at a boundary between consecutive groups (a node above the
-// groups splits between two of them, and each boundary is one node's
-// split), so thread t < ngroups - 1 takes boundary t, walks up for the
-// node's depth and writes entry t of the compact (depth, node) list. Thread
-// ngroups - 1 + g walks up from group
-// g's root instead: with the deepest climb of the group's leaves
-// (k_group_flags) that gives the group's deepest internal node. The block's
-// largest internal-node depth goes to dmax[block].
-__device__ __forceinline__ int walk_depth(int node, const int32_t* __restrict__ parent, uint32_t* __restrict__ flags) {
-  int d = 0;
-  for (int p = parent[node]; p >= 0; p = parent[p]) {
-    if (++d >= kMaxLevels - 1) {
-      atomicOr(flags, (uint32_t)FLAG_TREE);
-      break;
-    }
-  }
-  return d;
-}
-
-__global__ __launch_bounds__(256) void k_above_census(int n, const int32_t* __restrict__ gstart,
-                                                      const uint32_t* __restrict__ gcount,
-                                                      const int32_t* __restrict__ splitnode,
-                                                      const int32_t* __restrict__ groot,
-                                                      const int32_t* __restrict__ climb,
-                                                      const int32_t* __restrict__ parent, int32_t* __restrict__ depth,
-                                                      uint32_t* __restrict__ cdep, uint32_t* __restrict__ cnode,
-                                                      int32_t* __restrict__ dmax, uint32_t* __restrict__ gcnt,
-                                                      uint32_t* __restrict__ flags) {
-  __shared__ int wmax[4];
-  if (blockIdx.x == 0) gcnt[threadIdx.x] = 0u;  // the 2 kMaxLevels = 256 census counters and cursors
-  const int ng = (int)*gcount;
-  int mx = 0;
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < 2 * ng - 1; t += gridDim.x * blockDim.x) {
-    if (t < ng - 1) {
-      const int node = splitnode[gstart[t + 1] - 1];
-      const int d = walk_depth(node, parent, flags);
-      depth[node] = d;
-      cdep[t] = (uint32_t)d;  // one entry per node above the groups
-      cnode[t] = (uint32_t)node;
-      mx = max(mx, d);
-    } else {
-      const int g = t - (ng - 1);
-      const int lo = gstart[g], hi = gstart[g + 1] - 1;
-      // a group has at most kGroup leaves: all their loads are issued at once
-      // (indices clamped to the group) rather than one round trip per leaf
-      int cm = 0;
-#pragma unroll
-      for (int k = 0; k < kGroup; ++k) cm = max(cm, climb[min(lo + k, hi)]);
-      if (cm > 0) mx = max(mx, walk_depth(groot[lo], parent, flags) + cm - 1);
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1) mx = max(mx, __shfl_xor(mx, off, 64));
-  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  if (threadIdx.x == 0) dmax[blockIdx.x] = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
-}
-
-// The census list ordered by level, in two passes over tiles of kRsTile
-// entries (8 per thread, 256 threads). k_census_count: per-tile depth counts
-// in LDS, added into gcnt[0..127]. k_census_place: every tile derives the
-// level offsets from gcnt, reserves a range of each level for its entries
-// with one atomic per depth on the cursors gcnt[128..255], and writes its
-// nodes there; tile 0 also writes levels[] (offsets, level count, largest
-// depth over the census blocks' maxima). The order inside a level is
-// arbitrary: each node's moments depend on its children only. Lanes of a
-// wavefront with equal depths (few distinct values, many nodes each) are
-// counted with one LDS atomic per distinct depth.
-static_assert(kMaxLevels == 128, "depth_match compares 7 bits; the census keeps 2 x 128 counters");
-__device__ __forceinline__ uint64_t depth_match(bool valid, uint32_t d, uint64_t lt, uint32_t& rank) {
-  uint64_t m = __ballot(valid);
-#pragma unroll
-  for (int b = 0; b < 7; ++b) {  // depth < kMaxLevels = 2^7
-    const bool bit = (d >> b) & 1u;
-    const uint64_t bal = __ballot(bit);
-    m &= bit ? bal : ~bal;
-  }
-  rank = (uint32_t)__popcll(m & lt);
-  return m;
-}
-
-__global__ __launch_bounds__(kRsThreads) void k_census_count(const uint32_t* __restrict__ gcount,
-                                                             const uint32_t* __restrict__ cdep,
-                                                             uint32_t* __restrict__ gcnt) {
-  __shared__ uint32_t lcnt[kMaxLevels];
-  const int t = threadIdx.x, lane = t & 63;
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const int cnt = (int)*gcount - 1;  // one node above the groups per boundary between groups
-  const int base = blockIdx.x * kRsTile;
-  if (base >= cnt) return;  // uniform over the block
-  if (t < kMaxLevels) lcnt[t] = 0u;
-  __syncthreads();
-  uint32_t d[kRsTile / kRsThreads];
-#pragma unroll
-  for (int r = 0; r < kRsTile / kRsThreads; ++r) {
-    const int i = base + r * kRsThreads + t;
-    d[r] = i < cnt ? cdep[i] : 0u;
-  }
-#pragma unroll
-  for (int r = 0; r < kRsTile / kRsThreads; ++r) {
-    const bool valid = base + r * kRsThreads + t < cnt;
-    uint32_t rank;
-    const uint64_t m = depth_match(valid, d[r], lt, rank);
-    if (valid && rank == 0) atomicAdd(&lcnt[d[r]], (uint32_t)__popcll(m));
-  }
-  __syncthreads();
-  if (t < kMaxLevels && lcnt[t]) atomicAdd(&gcnt[t], lcnt[t]);
-}
-
-__global__ __launch_bounds__(kRsThreads) void k_census_place(const uint32_t* __restrict__ gcount,
-                                                             const uint32_t* __restrict__ cdep,
-                                                             const uint32_t* __restrict__ cnode,
-                                                             uint32_t* __restrict__ gcnt,
-                                                             const int32_t* __restrict__ dmax, int cblocks,
-                                                             int32_t* __restrict__ bucket,
-                                                             int32_t* __restrict__ levels) {
-  constexpr int R = kRsTile / kRsThreads;
-  __shared__ uint32_t off[kMaxLevels], lcnt[kMaxLevels], lbase[kMaxLevels];
-  __shared__ int wmax[kRsThreads / 64];
-  const int t = threadIdx.x, lane = t & 63;
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const int cnt = (int)*gcount - 1;
-  const int base = blockIdx.x * kRsTile;
-  if (blockIdx.x > 0 && base >= cnt) return;  // uniform over the block; tile 0 always writes levels[]
-  if (t < kMaxLevels) lcnt[t] = 0u;
-  if (t == 0) {
-    uint32_t run = 0;
-    for (int q = 0; q < kMaxLevels; ++q) {
-      off[q] = run;
-      run += gcnt[q];
-    }
-  }
-  __syncthreads();
-  uint32_t d[R], node[R], pos[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int i = base + r * kRsThreads + t;
-    d[r] = i < cnt ? cdep[i] : 0u;
-    node[r] = i < cnt ? cnode[i] : 0u;
-  }
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const bool valid = base + r * kRsThreads + t < cnt;
-    uint32_t rank, first = 0;
-    const uint64_t m = depth_match(valid, d[r], lt, rank);
-    if (valid && rank == 0) first = atomicAdd(&lcnt[d[r]], (uint32_t)__popcll(m));
-    first = __shfl(first, (int)__builtin_ctzll(m | (1ull << lane)), 64);  // from the group's lowest lane
-    pos[r] = first + rank;
-  }
-  __syncthreads();
-  if (t < kMaxLevels && lcnt[t]) lbase[t] = off[t] + atomicAdd(&gcnt[kMaxLevels + t], lcnt[t]);
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-    if (base + r * kRsThreads + t < cnt) bucket[lbase[d[r]] + pos[r]] = (int32_t)node[r];
-  if (blockIdx.x == 0) {
-    int mx = 0;
-    for (int i = t; i < cblocks; i += kRsThreads) mx = max(mx, dmax[i]);
-    for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o, 64));
-    if (lane == 0) wmax[t >> 6] = mx;
-    __syncthreads();
-    if (t < kMaxLevels) levels[t] = (int32_t)off[t];
-    if (t == 0) {
-      int nlev = 0;
-      for (int q = 0; q < kMaxLevels; ++q)
-        if (gcnt[q]) nlev = q + 1;
-      levels[kMaxLevels + 1] = nlev;
-      levels[kMaxLevels + 2] = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
-    }
-  }
 }
 
 // A node's moments: FP64 centre of mass and mass (and centre-of-mass velocity),
@@ -733,176 +580,6 @@ __device__ __forceinline__ MomRec shfl_xor_rec(const MomRec& r, int m) {
   o.lo = make_float4(__shfl_xor(r.lo.x, m, 64), __shfl_xor(r.lo.y, m, 64), __shfl_xor(r.lo.z, m, 64), 0.f);
   o.hi = make_float4(__shfl_xor(r.hi.x, m, 64), __shfl_xor(r.hi.y, m, 64), __shfl_xor(r.hi.z, m, 64), 0.f);
   return o;
-}
-
-// Band of up to H <= 6 levels above the groups, formed by a team of 2^H lanes
-// per node at the band's top depth. Lane s of a team stands for slot s of the
-// band's bottom level: a node at band level l covers the slots
-// [k 2^(H-l), (k+1) 2^(H-l)) and is handled by the first of them, its leader.
-// Going down, the leaders of the nodes formed here load their children and
-// leaf ranges (one round of loads per level; the ranges tell which children
-// lie above the groups) and the other lanes of the node take theirs by
-// shuffle. Then the leader of every child that is already complete (group
-// roots, leaves, nodes of the band below) loads its record, all in one round.
-// Going up, a leader unites its own record (its node's left child) with the
-// one held half its span away (the right child). H levels cost H + 2
-// dependent load rounds (the band top, H levels of children, the records)
-// and one launch; a team is at most one wavefront, so
-// no barrier is needed. Bottom-up order is what unite (barnes_hut.cpp:137-152)
-// needs: kernel boundaries order the bands.
-template <bool VEL, int H>
-__global__ __launch_bounds__(256) void k_moments_band(int n, const int32_t* __restrict__ bucket, int count,
-                                                      const int32_t* __restrict__ left,
-                                                      const int32_t* __restrict__ right,
-                                                      const int2* __restrict__ grange, double4* __restrict__ nmc,
-                                                      double4* __restrict__ nvel, float4* __restrict__ nbox,
-                                                      float4* __restrict__ nrec, double theta,
-                                                      float4* __restrict__ kids) {
-  static_assert(H >= 1 && H <= 6, "a band's team is at most one wavefront");
-  constexpr int S = 1 << H;
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  const int team = g >> H;
-  if (team >= count) return;  // teams are aligned to S lanes and leave whole
-  const int lane = threadIdx.x & 63;
-  const int s = g & (S - 1);
-  int ids[H];            // node covering this slot at band level l
-  uint32_t inmask = 0;   // bit l: that node is formed here
-  int cur = bucket[team];
-  bool cin = true;
-  int clev = 0;  // band level at which the complete node covering this slot appears
-#pragma unroll
-  for (int l = 0; l < H; ++l) {
-    const int span = S >> l;
-    ids[l] = cur;
-    if (cin) inmask |= 1u << l;
-    int L = 0, R = 0, fl = 0;
-    if (cin && (s & (span - 1)) == 0) {
-      L = left[cur];
-      R = right[cur];
-      const int2 r = grange[cur - n];  // children cover [r.x, gamma] and [gamma + 1, r.y]
-      const int gamma = L < n ? L : L - n;
-      if (l + 1 < H)
-        fl = (L >= n && gamma - r.x + 1 > kGroup ? 1 : 0) | (R >= n && r.y - gamma > kGroup ? 2 : 0);
-    }
-    const int src = lane & ~(span - 1);
-    L = __shfl(L, src, 64);
-    R = __shfl(R, src, 64);
-    fl = __shfl(fl, src, 64);
-    if (cin) {
-      const bool rt = (s & (span >> 1)) != 0;
-      cur = rt ? R : L;
-      cin = ((rt ? fl >> 1 : fl) & 1) != 0;
-      clev = l + 1;
-    }
-  }
-  MomRec rec{};
-  if ((s & ((S >> clev) - 1)) == 0) rec = load_moments<VEL>(n, cur, nmc, nvel, nbox);
-  int cid = cur;  // node whose record this lane holds
-#pragma unroll
-  for (int l = H - 1; l >= 0; --l) {
-    const int half = S >> (l + 1);
-    const MomRec o = shfl_xor_rec<VEL>(rec, half);
-    const int oid = __shfl_xor(cid, half, 64);
-    if (((inmask >> l) & 1u) && (s & (2 * half - 1)) == 0) {
-      const int node = ids[l];
-      const MomRec me = unite_moments<VEL>(rec, o);
-      nmc[node] = me.com;
-      if (VEL) nvel[node] = me.vel;
-      nbox[2 * node] = me.lo;
-      nbox[2 * node + 1] = me.hi;
-      if (!kids) nrec[node] = node_rec(me.com);
-      if (kids) {  // this node's child slots (and the root's own slot)
-        put_kid(kids, kid_slot(n, node, 0), cid, rec.com, rec.lo, rec.hi, theta);
-        put_kid(kids, kid_slot(n, node, 1), oid, o.com, o.lo, o.hi, theta);
-        if (node == n) put_kid(kids, 2 * (n - 1), n, me.com, me.lo, me.hi, theta);
-      }
-      rec = me;
-      cid = node;
-    }
-  }
-}
-
-// The top levels above the groups (at most kTopNodes nodes in all) in one
-// workgroup: thread p owns the p-th node of the depth-sorted list. Its
-// children's ids and leaf ranges, then the records of the children that are
-// already complete (formed by the bands below, group roots, leaves), are
-// loaded up front; the levels are then formed bottom-up through LDS, one
-// barrier per level, instead of one band launch per 3 levels.
-constexpr int kTopNodes = 512;
-constexpr int kTopMaxLevels = 32;
-struct TopLevels {
-  int nlev;                    // levels 0 .. nlev - 1
-  int off[kTopMaxLevels + 1];  // their offsets in the depth-sorted list
-};
-
-template <bool VEL>
-__global__ __launch_bounds__(kTopNodes) void k_moments_top(int n, const int32_t* __restrict__ bucket, TopLevels tl,
-                                                           const int32_t* __restrict__ left,
-                                                           const int32_t* __restrict__ right,
-                                                           const int2* __restrict__ grange, double4* __restrict__ nmc,
-                                                           double4* __restrict__ nvel, float4* __restrict__ nbox,
-                                                           float4* __restrict__ nrec, double theta,
-                                                           float4* __restrict__ kids, int32_t* __restrict__ topslot) {
-  __shared__ double4 scom[kTopNodes];
-  __shared__ double4 svel[VEL ? kTopNodes : 1];
-  __shared__ float4 slo[kTopNodes], shi[kTopNodes];
-  const int p = threadIdx.x;
-  const bool mine = p < tl.off[tl.nlev];
-  int node = n, L = 0, R = 0, lev = 0;
-  bool inL = false, inR = false;
-  if (mine) {
-    node = bucket[p];
-    while (tl.off[lev + 1] <= p) ++lev;
-    L = left[node];
-    R = right[node];
-    const int2 r = grange[node - n];  // children cover [r.x, gamma] and [gamma + 1, r.y]
-    const int gamma = L < n ? L : L - n;
-    const bool below = lev + 1 < tl.nlev;  // children at a level formed here
-    inL = below && L >= n && gamma - r.x + 1 > kGroup;
-    inR = below && R >= n && r.y - gamma > kGroup;
-    topslot[node - n] = p;
-  }
-  __syncthreads();
-  MomRec cl{}, cr{};
-  int sl = -1, sr = -1;
-  if (mine) {
-    if (inL) sl = topslot[L - n];
-    else cl = load_moments<VEL>(n, L, nmc, nvel, nbox);
-    if (inR) sr = topslot[R - n];
-    else cr = load_moments<VEL>(n, R, nmc, nvel, nbox);
-  }
-  for (int d = tl.nlev - 1; d >= 0; --d) {
-    if (mine && lev == d) {
-      if (sl >= 0) {
-        cl.com = scom[sl];
-        if (VEL) cl.vel = svel[sl];
-        cl.lo = slo[sl];
-        cl.hi = shi[sl];
-      }
-      if (sr >= 0) {
-        cr.com = scom[sr];
-        if (VEL) cr.vel = svel[sr];
-        cr.lo = slo[sr];
-        cr.hi = shi[sr];
-      }
-      const MomRec me = unite_moments<VEL>(cl, cr);
-      scom[p] = me.com;
-      if (VEL) svel[p] = me.vel;
-      slo[p] = me.lo;
-      shi[p] = me.hi;
-      nmc[node] = me.com;
-      if (VEL) nvel[node] = me.vel;
-      nbox[2 * node] = me.lo;
-      nbox[2 * node + 1] = me.hi;
-      if (!kids) nrec[node] = node_rec(me.com);
-      if (kids) {  // this node's child slots (and the root's own slot)
-        put_kid(kids, kid_slot(n, node, 0), L, cl.com, cl.lo, cl.hi, theta);
-        put_kid(kids, kid_slot(n, node, 1), R, cr.com, cr.lo, cr.hi, theta);
-        if (node == n) put_kid(kids, 2 * (n - 1), n, me.com, me.lo, me.hi, theta);
-      }
-    }
-    __syncthreads();
-  }
 }
 
 // Moments of every internal node inside a traversal group, one wavefront per
@@ -1028,6 +705,170 @@ __global__ __launch_bounds__(256) void k_group_moments(int n, const int32_t* __r
         if (node == n) put_kid(kids, 2 * (n - 1), n, com, blo, bhi, theta);
       }
     }
+  }
+}
+
+// Moments of the nodes above the groups, a workgroup per unit: first the nodes
+// of the subtrees of at most kUnit leaves (TOP = false; their splits are the
+// boundaries between the groups inside), then all larger nodes in one workgroup
+// (TOP = true, from the list `top`). A thread takes a node, loads the records
+// of its children that are complete (group roots, leaves, units' roots) and
+// polls the other children's flags, one barrier per sweep; records pass through
+// LDS. A flag holds the sweep its node was formed in, and only earlier sweeps
+// count, so a sweep needs no second barrier and the records' order never
+// depends on timing. More nodes than threads (a unit of many small groups, more
+// than ~1.4 million bodies): the threads take turns and the records pass
+// through global memory. Bound: latency, ~4 dependent loads and a sweep per
+// level (at most 47 levels up to 2^17 bodies: 30 code bits, 17 of position).
+// Neither the host nor a level census is needed to order the launches: against
+// the census (four launches, a readback and a wait), bands of levels and a top
+// pass, the tree's part of a step falls from 167 to 127 us at 50000 bodies
+// (these two launches 16 + 9 us) and from 331 to 280 us at 2^20 (15 + 30 us).
+template <bool VEL, int CAP>
+struct MomLds {
+  double4 com[CAP];
+  double4 vel[VEL ? CAP : 1];
+  float4 lo[CAP], hi[CAP];
+  int done[CAP];
+  __device__ void put(int s, const MomRec& r) {
+    com[s] = r.com;
+    if (VEL) vel[s] = r.vel;
+    lo[s] = r.lo;
+    hi[s] = r.hi;
+  }
+  __device__ void get(int s, MomRec& r) const {
+    r.com = com[s];
+    if (VEL) r.vel = vel[s];
+    r.lo = lo[s];
+    r.hi = hi[s];
+  }
+};
+
+constexpr int kUnitThreads = 256;
+constexpr int kTopThreads = 512;
+
+template <bool VEL, bool TOP>
+__global__ __launch_bounds__(TOP ? kTopThreads : kUnitThreads) void k_moments_above(
+    int n, const uint32_t* __restrict__ above, const int32_t* __restrict__ units, const int32_t* __restrict__ top,
+    const int32_t* __restrict__ gstart, const uint32_t* __restrict__ gcount, const uint32_t* __restrict__ gscan,
+    const int32_t* __restrict__ splitnode, const int32_t* __restrict__ left, const int32_t* __restrict__ right,
+    const int2* __restrict__ grange, double4* nmc, double4* nvel, float4* nbox, float4* __restrict__ nrec,
+    double theta, float4* __restrict__ kids, int32_t* topslot, uint32_t* __restrict__ flags) {
+  constexpr int T = TOP ? kTopThreads : kUnitThreads;
+  constexpr int kNever = 0xFFFF;
+  constexpr int kSmall = TOP ? kUnit : kGroup;  // children of at most so many leaves are complete
+  __shared__ MomLds<VEL, T> lds;
+  __shared__ uint16_t uslot[TOP ? 1 : kUnit];  // unit: node - n - lo -> thread, or its sweep
+  __shared__ int rslot;
+  const int t = threadIdx.x;
+  const int nunits = TOP ? 1 : (int)above[0];
+  for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
+    int root = n, ulo = 0, g0 = 0, m = 0;
+    if (TOP) {
+      m = (int)above[1];
+    } else {
+      root = units[u];
+      const int2 r = grange[root - n];
+      ulo = r.x;
+      g0 = (int)gscan[r.x];
+      m = (r.y + 1 < n ? (int)gscan[r.y + 1] : (int)*gcount) - g0 - 1;
+    }
+    // a node's entry: TOP in global memory, otherwise in LDS
+    auto state_put = [&](int node, int v) {
+      if (TOP) topslot[node - n] = v;
+      else uslot[node - n - ulo] = (uint16_t)v;
+    };
+    auto state_get = [&](int node) -> int { return TOP ? topslot[node - n] : (int)uslot[node - n - ulo]; };
+    auto node_at = [&](int e) { return TOP ? top[e] : splitnode[gstart[g0 + e + 1] - 1]; };
+    struct Kids {
+      int L, R;
+      bool inL, inR;  // formed here
+    };
+    auto kids_of = [&](int node) {
+      Kids k;
+      k.L = left[node];
+      k.R = right[node];
+      const int2 r = grange[node - n];  // children cover [r.x, gamma] and [gamma + 1, r.y]
+      const int gamma = k.L < n ? k.L : k.L - n;
+      k.inL = k.L >= n && gamma - r.x + 1 > kSmall;
+      k.inR = k.R >= n && r.y - gamma > kSmall;
+      return k;
+    };
+    auto store = [&](int node, const Kids& k, const MomRec& cl, const MomRec& cr, const MomRec& me) {
+      nmc[node] = me.com;
+      if (VEL) nvel[node] = me.vel;
+      nbox[2 * node] = me.lo;
+      nbox[2 * node + 1] = me.hi;
+      if (!kids) nrec[node] = node_rec(me.com);
+      if (kids) {  // this node's child slots (and the root's own slot)
+        put_kid(kids, kid_slot(n, node, 0), k.L, cl.com, cl.lo, cl.hi, theta);
+        put_kid(kids, kid_slot(n, node, 1), k.R, cr.com, cr.lo, cr.hi, theta);
+        if (node == n) put_kid(kids, 2 * (n - 1), n, me.com, me.lo, me.hi, theta);
+      }
+    };
+    if (m <= 0) continue;  // uniform; cannot happen for a valid tree
+    if (m <= T) {
+      const bool mine = t < m;
+      int node = root;
+      Kids k{};
+      MomRec cl{}, cr{};
+      if (mine) {
+        node = node_at(t);
+        state_put(node, t);
+        if (node == root) rslot = t;
+        k = kids_of(node);
+      }
+      lds.done[t] = kNever;
+      __syncthreads();
+      int sl = -1, sr = -1;
+      if (mine) {
+        if (k.inL) sl = state_get(k.L);
+        else cl = load_moments<VEL>(n, k.L, nmc, nvel, nbox);
+        if (k.inR) sr = state_get(k.R);
+        else cr = load_moments<VEL>(n, k.R, nmc, nvel, nbox);
+      }
+      bool wait = mine;
+      for (int it = 1;; ++it) {
+        if (wait && (sl < 0 || lds.done[sl] < it) && (sr < 0 || lds.done[sr] < it)) {
+          if (sl >= 0) lds.get(sl, cl);
+          if (sr >= 0) lds.get(sr, cr);
+          const MomRec me = unite_moments<VEL>(cl, cr);
+          lds.put(t, me);
+          lds.done[t] = it;
+          store(node, k, cl, cr, me);
+          wait = false;
+        }
+        __syncthreads();
+        if (lds.done[rslot] <= it) break;
+        if (it >= kMaxLevels) {  // cannot happen for a valid tree
+          if (t == 0) atomicOr(flags, (uint32_t)FLAG_TREE);
+          break;
+        }
+      }
+    } else {
+      for (int e = t; e < m; e += T) state_put(node_at(e), kNever);
+      __syncthreads();
+      for (int it = 1;; ++it) {
+        for (int e = t; e < m; e += T) {
+          const int node = node_at(e);
+          if (state_get(node) != kNever) continue;
+          const Kids k = kids_of(node);
+          if ((k.inL && state_get(k.L) >= it) || (k.inR && state_get(k.R) >= it)) continue;
+          const MomRec cl = load_moments<VEL>(n, k.L, nmc, nvel, nbox);
+          const MomRec cr = load_moments<VEL>(n, k.R, nmc, nvel, nbox);
+          store(node, k, cl, cr, unite_moments<VEL>(cl, cr));
+          state_put(node, it);
+        }
+        __syncthreads();
+        const int rs = state_get(root);
+        if (rs <= it) break;
+        if (it >= kMaxLevels) {
+          if (t == 0) atomicOr(flags, (uint32_t)FLAG_TREE);
+          break;
+        }
+      }
+    }
+    __syncthreads();  // the unit's entries are read before the next unit's are written
   }
 }
 
@@ -1274,31 +1115,6 @@ __global__ __launch_bounds__(256) void k_bh_f64(int n, const double* __restrict_
 // Morton cell (the subtree's common code prefix), so the group box is compact
 // wherever the curve jumps. Groups partition the sorted bodies.
 
-// Leaf k climbs while the parent still has at most kGroup leaves; k starts a
-// group when it is the first position of the subtree it stops at.
-// The climb's length (the leaf's depth below its group's root) and, at the
-// group's first position, the root itself are kept for the depth census.
-__global__ __launch_bounds__(256) void k_group_flags(int n, const int32_t* __restrict__ parent,
-                                                     const int2* __restrict__ grange, uint32_t* __restrict__ flag,
-                                                     int32_t* __restrict__ climb, int32_t* __restrict__ groot) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  int v = k, lo = k, steps = 0;
-  for (;;) {
-    const int p = parent[v];
-    if (p < 0) break;
-    const int2 r = grange[p - n];
-    if (r.y - r.x + 1 > kGroup) break;
-    v = p;
-    lo = r.x;
-    ++steps;
-  }
-  flag[k] = (lo == k) ? 1u : 0u;
-  climb[k] = steps;
-  if (lo == k) groot[k] = v;
-}
-
-
 // Wavefront-cooperative traversal, one group per wavefront (lanes = the
 // group's bodies, at most 64). The wavefront walks the tree once for the
 // whole group with a shared LDS stack of opened nodes, testing up to 64
@@ -1311,12 +1127,12 @@ __global__ __launch_bounds__(256) void k_group_flags(int n, const int32_t* __res
 // Accepted nodes are appended to an LDS interaction list that the lanes then
 // evaluate in pieces (below; 12 VALU + 1 rsq per entry and lane), FP32 sums
 // per list flush, Kahan-compensated across flushes.
-// Stack bound: each iteration pops the top min(sp, 32) entries and pushes
-// their opened children (at most 64) in order, so the stack stays sorted by
-// depth from bottom to top and a pop only ever leaves behind part of one
-// pushed batch: at most 32 entries per depth below a top batch of at most 64.
-// With internal nodes at depths 0..L-1 that is fewer than 32 L + 64 entries;
-// the stack is sized from L of the tree at hand (dynamic LDS).
+// Stack bound: an iteration pops up to 32 entries and pushes their opened
+// children, at most one more each than it popped. It pops no more than leave
+// kGrpDeep entries free, but at least one: single entries walk depth first,
+// which adds at most one entry per level, and internal nodes have at most 61
+// levels (their common prefix grows by a bit or more per level: 30 bits of
+// code, then 31 of the position). So the stack suffices for every tree.
 // Scheduling: the 8 XCDs take workgroups round-robin, so workgroup b works on
 // the groups of chunk (b mod 8), consecutive in Morton order, and neighbouring
 // groups (which open the same nodes) share an L2.
@@ -1344,7 +1160,8 @@ constexpr int kGrpListPad = 64;  // room for that padding
 constexpr int kPieceMaxPasses = 3;
 static_assert(kPieceMaxPasses * 64 <= kGrpList + kGrpListPad, "partial sums must fit the list LDS");
 
-__host__ __device__ constexpr int grp_stack_cap(int levels) { return 32 * levels + 64; }
+constexpr int kGrpStack = 384;
+constexpr int kGrpDeep = 62;
 
 struct PieceTable {
   uint8_t passes[65];
@@ -1462,12 +1279,12 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
                                                  const float4* __restrict__ kids, const uint32_t* __restrict__ perm,
                                                  float eps2, float msc, double G,
                                                  double* __restrict__ a, unsigned long long* __restrict__ counters,
-                                                 uint32_t* __restrict__ flags, int stack_cap, NodePn pnp) {
+                                                 uint32_t* __restrict__ flags, NodePn pnp) {
   extern __shared__ float4 grp_lds[];
   float4* lst = grp_lds;                                              // kGrpList + kGrpListPad entries
-  int* stk = reinterpret_cast<int*>(grp_lds + kGrpList + kGrpListPad);  // stack_cap entries
-  int* lid = stk + stack_cap;  // PN: node id of each list entry (kGrpList entries)
-  PnLds* pl = reinterpret_cast<PnLds*>(grp_lds + kGrpList + kGrpListPad + (stack_cap + kGrpList + 3) / 4);  // PN
+  int* stk = reinterpret_cast<int*>(grp_lds + kGrpList + kGrpListPad);  // kGrpStack entries
+  int* lid = stk + kGrpStack;  // PN: node id of each list entry (kGrpList entries)
+  PnLds* pl = reinterpret_cast<PnLds*>(grp_lds + kGrpList + kGrpListPad + (kGrpStack + kGrpList) / 4);  // PN
   const int lane = threadIdx.x;
   const int ngroups = (int)*gcount;
   const int per_xcd = (ngroups + 7) >> 3;
@@ -1639,7 +1456,7 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
       }
     }
     wave_sync();
-    // The children of the next batch (the top min(sp, 32) stack entries) are
+    // The children of the next batch (the top of the stack) are
     // loaded before a pending flush evaluates the list, so the load's latency
     // overlaps that arithmetic. Lane 2 i + s takes child s of entry i: the two
     // children of a node are 64 contiguous bytes. Lanes past the batch load a
@@ -1650,7 +1467,7 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
     float2 na;
     // With an empty stack (the walk is over) it loads the root's children.
     auto fetch = [&]() {
-      take = min(sp, 32);
+      take = min(min(sp, 32), max(kGrpStack - kGrpDeep - sp, 1));
       const int e = max(min(lane >> 1, take - 1), 0);
       const int opened = sp > 0 ? stk[sp - take + e] : n;
       const int slot = kid_slot(n, opened, lane & 1);
@@ -1674,7 +1491,7 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
       const int nopen = (int)__popcll(om);
       // cannot happen for a valid tree (see bound above); the walk then ends
       // here (no early exit from the loop, which keeps its control flow simple)
-      const bool over = sp + nopen > stack_cap;
+      const bool over = sp + nopen > kGrpStack;
       if (over) {
         if (lane == 0) atomicOr(flags, (uint32_t)FLAG_TREE);
         overflow = true;
@@ -1729,6 +1546,7 @@ static int reserve_sort(aster_ctx* c) {
   ASTER_HIP(c, c->codes2.reserve(n));
   ASTER_HIP(c, c->idx2.reserve(n));
   ASTER_HIP(c, c->xm4.reserve(n));
+  ASTER_HIP(c, c->above.reserve(2));
   ASTER_HIP(c, c->hist.reserve(256 * (size_t)rs_stride((int)nblocks)));
   ASTER_HIP(c, c->scanpart.reserve((n + kScanChunk - 1) / kScanChunk + 1));
   return ASTER_OK;
@@ -1756,12 +1574,13 @@ static int reserve_tree(aster_ctx* c, bool full) {
   ASTER_HIP(c, c->parent.reserve(nn));
   ASTER_HIP(c, c->escape.reserve(nn));
   ASTER_HIP(c, c->depth.reserve(nn));
-  ASTER_HIP(c, c->levels.reserve(kMaxLevels + 3));
-  ASTER_HIP(c, c->bucket.reserve(n));
   ASTER_HIP(c, c->splitnode.reserve(n));
-  ASTER_HIP(c, c->groot.reserve(n));
-  ASTER_HIP(c, c->climb.reserve(n));
+  ASTER_HIP(c, c->units.reserve(n / kGroup + 1));
+  ASTER_HIP(c, c->top.reserve(n));
   ASTER_HIP(c, c->topslot.reserve(n));
+  ASTER_HIP(c, c->gscan.reserve(n));
+  ASTER_HIP(c, c->gstart.reserve(n + 1));
+  ASTER_HIP(c, c->gcount.reserve(1));
   ASTER_HIP(c, c->grange.reserve(n));
   ASTER_HIP(c, c->nmc.reserve(nn));
   ASTER_HIP(c, c->nbox.reserve(2 * nn));
@@ -1784,7 +1603,7 @@ static int morton_codes(aster_ctx* c, bool user_box) {
   if (rc) return rc;
   const int n = (int)c->n;
   hipLaunchKernelGGL(k_morton, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, c->x.p, c->m.p, c->boxd.p,
-                     c->codes.p, c->idx.p, c->xm4.p, c->flags.p);
+                     c->codes.p, c->idx.p, c->xm4.p, c->above.p, c->flags.p);
   ASTER_HIP(c, hipGetLastError());
   phase_end(c, ASTER_PHASE_MORTON);
   c->tree_valid = false;
@@ -1852,54 +1671,6 @@ int morton_sort(aster_ctx* c, bool user_box) {
   return ASTER_OK;
 }
 
-// Groups for the wavefront traversal (subtrees of at most kGroup leaves whose
-// parent has more), as first sorted positions gstart[0..ngroups] in Morton
-// order; the count stays on the device.
-static int build_groups(aster_ctx* c) {
-  const int n = (int)c->n;
-  ASTER_HIP(c, c->gscan.reserve((size_t)n));
-  ASTER_HIP(c, c->gstart.reserve((size_t)n + 1));
-  ASTER_HIP(c, c->gcount.reserve(1));
-  hipLaunchKernelGGL(k_group_flags, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, c->parent.p, c->grange.p,
-                     c->gscan.p, c->climb.p, c->groot.p);
-  // the scan of the start flags also writes the group starts and the sentinel n
-  int rc = device_scan(c, c->gscan.p, n, c->gcount.p, c->gstart.p);
-  if (rc) return rc;
-  ASTER_HIP(c, hipGetLastError());
-  return ASTER_OK;
-}
-
-constexpr int kBand = 6;  // levels per moments launch above the groups (a team of 2^6 lanes)
-
-static int launch_moments_band(aster_ctx* c, bool vel, int h, int off, int cnt, float4* kids) {
-  const int n = (int)c->n;
-  if (h < 1 || h > kBand) return fail(c, ASTER_ERR_STATE, "moments band height out of range");
-  const int64_t threads = (int64_t)cnt << h;
-  if (threads > INT32_MAX) return fail(c, ASTER_ERR_STATE, "moments band too wide");
-  const dim3 grid((unsigned)((threads + 255) / 256)), block(256);
-  const int32_t* b = c->bucket.p + off;
-#define ASTER_BAND(V, H)                                                                                          \
-  hipLaunchKernelGGL((k_moments_band<V, H>), grid, block, 0, c->stream, n, b, cnt, c->left.p, c->right.p,        \
-                     c->grange.p, c->nmc.p, c->nvel.p, c->nbox.p, c->nrec.p, c->P.theta, kids)
-#define ASTER_BAND_H(H)                 \
-  case H:                               \
-    if (vel) ASTER_BAND(true, H);       \
-    else ASTER_BAND(false, H);          \
-    break;
-  switch (h) {
-    ASTER_BAND_H(1)
-    ASTER_BAND_H(2)
-    ASTER_BAND_H(3)
-    ASTER_BAND_H(4)
-    ASTER_BAND_H(5)
-    ASTER_BAND_H(6)
-  }
-#undef ASTER_BAND_H
-#undef ASTER_BAND
-  ASTER_HIP(c, hipGetLastError());
-  return ASTER_OK;
-}
-
 // full: also the depth and escape link of every node (the per-body
 // traversals and the reference MAC need them; the group traversal does not).
 static int build_tree(aster_ctx* c, int mac, bool vel, bool full) {
@@ -1913,77 +1684,32 @@ static int build_tree(aster_ctx* c, int mac, bool vel, bool full) {
   auto build = vel ? k_build<true> : k_build<false>;
   hipLaunchKernelGGL(build, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, c->codes.p, c->idx.p, c->xm4.p,
                      c->v.p, c->left.p, c->right.p, c->parent.p, c->grange.p, c->nmc.p, c->nvel.p, c->nbox.p,
-                     c->nrec.p, c->gsh.p, c->splitnode.p, c->flags.p, full ? 1 : 0);
+                     c->nrec.p, c->gsh.p, c->splitnode.p, c->gscan.p, c->above.p, c->units.p, c->top.p, c->flags.p,
+                     full ? 1 : 0);
   ASTER_HIP(c, hipGetLastError());
-  // traversal groups (also the per-wavefront subtrees of the moment pass)
-  if ((rc = build_groups(c))) return rc;
+  // Groups of the wavefront traversal, also the subtrees of the first moment
+  // pass: the scan of the start flags writes their first sorted positions in
+  // Morton order and the sentinel n; the count stays on the device.
+  if ((rc = device_scan(c, c->gscan.p, n, c->gcount.p, c->gstart.p))) return rc;
   phase_end(c, ASTER_PHASE_BUILD);
   const int nn = 2 * n - 1;
   phase_begin(c, ASTER_PHASE_MOMENTS);
-  // Depth census of the nodes above the groups: their depths (walks from the
-  // group boundaries, and from the group roots for the largest depth) as a
-  // compact (depth, node) list, then two passes list them level by level
-  // (depth < 128). The sort scratch of the Morton pass holds the list.
-  const int cblocks = (int)std::min<int64_t>((2 * (int64_t)n / 32 + 2 + 255) / 256, 4096);
-  ASTER_HIP(c, c->dmax.reserve((size_t)cblocks));
-  ASTER_HIP(c, c->censusctr.reserve(2 * kMaxLevels));
-  hipLaunchKernelGGL(k_above_census, dim3(cblocks), dim3(256), 0, c->stream, n, c->gstart.p, c->gcount.p,
-                     c->splitnode.p, c->groot.p, c->climb.p, c->parent.p, c->depth.p, c->codes2.p, c->idx2.p,
-                     c->dmax.p, c->censusctr.p, c->flags.p);
-  const int ctiles = (n + kRsTile - 1) / kRsTile;  // the list has fewer than n entries
-  hipLaunchKernelGGL(k_census_count, dim3(ctiles), dim3(kRsThreads), 0, c->stream, c->gcount.p, c->codes2.p,
-                     c->censusctr.p);
-  hipLaunchKernelGGL(k_census_place, dim3(ctiles), dim3(kRsThreads), 0, c->stream, c->gcount.p, c->codes2.p,
-                     c->idx2.p, c->censusctr.p, c->dmax.p, cblocks, c->bucket.p, c->levels.p);
   if (full)
     hipLaunchKernelGGL(k_depth, dim3((nn + 255) / 256), dim3(256), 0, c->stream, n, c->left.p, c->right.p,
                        c->parent.p, c->depth.p, c->escape.p, c->flags.p);
-  ASTER_HIP(c, hipGetLastError());
-  // The level bounds and the largest depth go to pinned host memory
-  // asynchronously; the host waits for them only after the group kernel below
-  // is queued, so the device keeps working meanwhile.
-  if (!c->host_words) {
-    ASTER_HIP(c, hipHostMalloc((void**)&c->host_words, (kMaxLevels + 3) * sizeof(int32_t), hipHostMallocDefault));
-    ASTER_HIP(c, hipEventCreateWithFlags(&c->tree_ev, hipEventDisableTiming));
-  }
-  ASTER_HIP(c, hipMemcpyAsync(c->host_words, c->levels.p, (kMaxLevels + 3) * sizeof(int32_t), hipMemcpyDeviceToHost,
-                              c->stream));
-  ASTER_HIP(c, hipEventRecord(c->tree_ev, c->stream));
-  // every node inside a group: one wavefront per group, bottom-up in LDS
+  // the nodes inside the groups, then those above: units, then the top
   const int gblocks = ((n / 32 + 1) + 3) / 4;
   auto gmom = vel ? k_group_moments<true> : k_group_moments<false>;
   hipLaunchKernelGGL(gmom, dim3(gblocks), dim3(256), 0, c->stream, n, c->gstart.p, c->gcount.p, c->grange.p, c->left.p,
                      c->right.p, c->nmc.p, c->nvel.p, c->nbox.p, c->nrec.p, c->P.theta, kids);
-  ASTER_HIP(c, hipGetLastError());
-  ASTER_HIP(c, hipEventSynchronize(c->tree_ev));
-  const int32_t* lv = c->host_words;
-  const int nlev = lv[kMaxLevels + 1];  // depths above the groups
-  const int maxdep = lv[kMaxLevels + 2];
-  if (nlev < 0 || nlev >= kMaxLevels || maxdep < nlev - 1 || maxdep >= kMaxLevels - 1 || (nlev > 0 && lv[0] != 0))
-    return fail(c, ASTER_ERR_STATE, "radix tree depth census is inconsistent");
-  c->tree_levels = maxdep + 1;
-  // the nodes above the groups: the top levels holding at most kTopNodes
-  // nodes in one workgroup, the rest in bands of up to kBand levels, deepest
-  // band first (the children of a band's deepest nodes are group roots,
-  // leaves or nodes of the band below)
-  int ntop = 0;
-  while (ntop < nlev && ntop < kTopMaxLevels && lv[ntop + 1] <= kTopNodes) ++ntop;
-  for (int d = nlev - 1; d >= ntop;) {
-    const int top = d - kBand + 1 > ntop ? d - kBand + 1 : ntop;
-    const int h = d - top + 1;
-    const int off = lv[top], cnt = lv[top + 1] - off;
-    if (cnt <= 0) return fail(c, ASTER_ERR_STATE, "radix tree depth census has an empty level");
-    if ((rc = launch_moments_band(c, vel, h, off, cnt, kids))) return rc;
-    d = top - 1;
-  }
-  if (ntop > 0) {
-    TopLevels tl;
-    tl.nlev = ntop;
-    for (int d = 0; d <= ntop; ++d) tl.off[d] = lv[d];
-    auto topk = vel ? k_moments_top<true> : k_moments_top<false>;
-    hipLaunchKernelGGL(topk, dim3(1), dim3(kTopNodes), 0, c->stream, n, c->bucket.p, tl, c->left.p, c->right.p,
-                       c->grange.p, c->nmc.p, c->nvel.p, c->nbox.p, c->nrec.p, c->P.theta, kids, c->topslot.p);
-  }
+  auto above = [&](auto kern, int blocks, int threads) {
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(threads), 0, c->stream, n, c->above.p, c->units.p, c->top.p,
+                       c->gstart.p, c->gcount.p, c->gscan.p, c->splitnode.p, c->left.p, c->right.p, c->grange.p,
+                       c->nmc.p, c->nvel.p, c->nbox.p, c->nrec.p, c->P.theta, kids, c->topslot.p, c->flags.p);
+  };
+  const int ublocks = n / 1024 + 1;  // units hold ~2700 leaves each; the workgroups loop over more
+  if (n > kGroup) above(vel ? k_moments_above<true, false> : k_moments_above<false, false>, ublocks, kUnitThreads);
+  if (n > kUnit) above(vel ? k_moments_above<true, true> : k_moments_above<false, true>, 1, kTopThreads);
   ASTER_HIP(c, hipGetLastError());
   phase_end(c, ASTER_PHASE_MOMENTS);
   phase_begin(c, ASTER_PHASE_LINKS);
@@ -2033,17 +1759,15 @@ static int bh_forces_all(aster_ctx* c, int method) {
       // count is a multiple of 8 for the XCD-interleaved group order.
       const int blocks = ((n / 32 + 1) + 7) & ~7;
       const dim3 grid(blocks), block(64);
-      const int cap = grp_stack_cap(c->tree_levels);
       // PN: node ids, then (16-byte aligned) FP64 records and velocities of the list
       const size_t lds = (kGrpList + kGrpListPad) * sizeof(float4) +
-                         (pn ? (size_t)(cap + kGrpList + 3) / 4 * sizeof(float4) + sizeof(PnLds)
-                             : (size_t)cap * sizeof(int));
+                         (pn ? (kGrpStack + kGrpList) * sizeof(int) + sizeof(PnLds) : kGrpStack * sizeof(int));
       const NodePn gp{c->nmc.p, c->nvel.p, c->P.G, ic, c->P.softening, pnf};
       auto kern = !pn ? (mask ? k_bh_group<true, 0> : k_bh_group<false, 0>)
                   : pnf == ASTER_PN1 ? (mask ? k_bh_group<true, 1> : k_bh_group<false, 1>)
                                      : (mask ? k_bh_group<true, 2> : k_bh_group<false, 2>);
       hipLaunchKernelGGL(kern, grid, block, lds, c->stream, n, c->gstart.p, c->gcount.p, c->gsh.p, c->kids.p,
-                         c->idx.p, eps2, sc.msc, sc.gsc, c->a.p, c->bh_counters.p, c->flags.p, cap, gp);
+                         c->idx.p, eps2, sc.msc, sc.gsc, c->a.p, c->bh_counters.p, c->flags.p, gp);
     } else {
       const NodePn gp{c->nmc.p, c->nvel.p, c->P.G, ic, c->P.softening, pnf};
       auto kern = pn ? (mask ? k_bh_f32<true, true> : k_bh_f32<false, true>)
