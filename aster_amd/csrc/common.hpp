@@ -151,9 +151,11 @@ struct aster_ctx {
   aster::DBuf<double> boxd;     // box half-extent used (3) + |box| (1)
 
   // Barnes-Hut / LBVH.
-  aster::DBuf<uint32_t> codes, idx, codes2, idx2;  // sort ping-pong, n
+  aster::DBuf<uint32_t> codes, idx;                // Morton codes and, once sorted, the body at each position (n)
+  aster::DBuf<uint2> kv;                           // the sort's {code, body} pairs between passes (2 n)
   aster::DBuf<double4> xm4;                        // {x, y, z, m} per body (body order), n
-  aster::DBuf<uint32_t> hist;                      // per-block digit counts
+  aster::DBuf<uint32_t> rows;                      // the sort's digit counts per pass and tile
+  aster::DBuf<uint2> rowsum;                       // their sums over groups of tiles
   aster::DBuf<int32_t> left, right, parent, escape;// 2n-1
   aster::DBuf<uint32_t> scanpart;                  // per-chunk totals of the device scan
   aster::DBuf<int32_t> depth;                      // 2n-1

@@ -21,6 +21,7 @@
 //    every accepted/skipped node continues at its escape link, which is the
 //    next node of that same order, so the FP64 traversal accumulates in the
 //    reference's order and is bit-identical to get_node_body (:202-261).
+#include <type_traits>
 #include <utility>
 
 #include "common.hpp"
@@ -28,8 +29,6 @@
 
 namespace aster {
 
-constexpr int kRsThreads = 256;
-constexpr int kRsTile = 2048;  // keys per block (8 per thread)
 // Depth bound of the radix tree: an internal node's split bit strictly
 // increases with depth over 30 code bits + 32 tie-break bits, so depth <= 63.
 constexpr int kMaxLevels = 128;
@@ -59,68 +58,377 @@ __device__ __forceinline__ uint32_t cell_of(double p, double b, uint32_t* bad) {
   return c < 1023u ? c : 1023u;
 }
 
-// Also packs {x, y, z, m} of each body into one 32-byte record, so the leaf
-// initialisation gathers one record through the sort permutation instead of
-// four scattered planes.
-__global__ __launch_bounds__(256) void k_morton(int n, const double* __restrict__ x, const double* __restrict__ m,
-                                                const double* __restrict__ box, uint32_t* __restrict__ codes,
-                                                uint32_t* __restrict__ idx, double4* __restrict__ xm,
-                                                uint32_t* __restrict__ above, uint32_t* __restrict__ flags) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  if (i < 2) above[i] = 0u;  // lengths of the lists that k_build writes
-  uint32_t bad = 0;
-  const double px = x[i], py = x[n + i], pz = x[2 * n + i];
-  xm[i] = make_double4(px, py, pz, m[i]);
-  const uint32_t ix = cell_of(px, box[0], &bad);
-  const uint32_t iy = cell_of(py, box[1], &bad);
-  const uint32_t iz = cell_of(pz, box[2], &bad);
-  codes[i] = (part1by2(iz) << 2) | (part1by2(iy) << 1) | part1by2(ix);
-  idx[i] = (uint32_t)i;
-  if (bad) atomicOr(flags, (uint32_t)FLAG_OUT_OF_BOX);
-}
-
 // -------------------------------------------------------- radix sort ------
 
-// LSD radix sort of (Morton code, body) pairs, 4 passes of 8 bits. A block
-// handles a tile of kRsPer * THREADS keys. Per pass, k_rs_hist writes each
-// tile's digit counts (hist[d * stride + b]); the scatter needs every digit's
-// start, i.e. the keys of smaller digits in all tiles plus those of the same
-// digit in earlier tiles. With at most kRsRawMaxBlocks tiles the scatter
-// forms these starts itself from the raw counts (two launches per pass); with
-// more, an exclusive scan of the count matrix runs between the two kernels.
-constexpr int kRsPer = 8;
-constexpr int kRsRawMaxBlocks = 128;
+// LSD radix sort of (Morton code, body) pairs, 3 passes of 10 bits. A
+// workgroup takes a tile of consecutive keys: it forms its digits' starts
+// from the tiles' digit counts (the keys of smaller digits in all tiles, those
+// of the same digit in earlier tiles), ranks its keys, reorders them in LDS and
+// writes them out. Counts are two digits to a word, at most a tile's keys each:
+// row b of a pass's table holds tile b's 512 words. The first pass's rows come
+// with the codes (k_morton), the later ones from k_rs_hist. With many tiles the
+// rows are first summed over groups of kRsGroup (k_rs_groups), so that a tile
+// reads the groups' sums and at most kRsGroup rows. Bound: latency below ~2^19
+// keys (a scatter is one chain of loads, ranks and stores), with launches as
+// long as they can be short. Against 4 passes of 8 bits with counts and keys in
+// separate arrays: sort 54 -> 31 us at 50000 keys, 84 -> 72 us at 2^20. (Adding
+// each key to its next tile's counts while scattering, instead of k_rs_hist,
+// was slower: 50000 bodies +25 us, many equal keys +200 us at 20000.)
+constexpr int kDigBits = 10;
+constexpr int kDigits = 1 << kDigBits;
+constexpr int kRsWords = kDigits / 2;
+constexpr int kRsPasses = 3;
+constexpr int kRsThreads = 512;
+constexpr int kRsGroup = 64;
+constexpr int kRsSmall = 4096;  // keys that one workgroup sorts by itself
+constexpr int kRsMaxRows = 128;  // more tiles: in groups
+constexpr int kRsAhead = 8;
 
-__host__ __device__ constexpr int rs_stride(int nblocks) { return (nblocks + 3) & ~3; }
+__device__ __forceinline__ uint32_t rs_digit(uint32_t key, int pass) {
+  return (key >> (pass * kDigBits)) & (uint32_t)(kDigits - 1);
+}
 
-template <int THREADS>
-__global__ __launch_bounds__(THREADS) void k_rs_hist(const uint32_t* __restrict__ keys, int n, int shift,
-                                                     uint32_t* __restrict__ hist, int stride) {
-  constexpr int TILE = kRsPer * THREADS, H = THREADS / 256;  // H copies of the counters
-  static_assert(THREADS % 256 == 0, "one counter per thread and copy");
-  __shared__ uint32_t cnt[H][256];
+template <int K>
+__global__ __launch_bounds__(kRsThreads) void k_rs_hist(const uint2* __restrict__ kv, int n, int pass,
+                                               uint32_t* __restrict__ rows) {
+  constexpr int T = kRsThreads;
+  __shared__ uint32_t cnt[kRsWords];
   const int t = threadIdx.x;
-  const int base = blockIdx.x * TILE;
+  const int base = blockIdx.x * (T * K);
   // every load of the thread is issued before the first is used (clamped
-  // addresses, no branch around a load), so the tile costs one memory
-  // round trip rather than kRsPer
-  uint32_t key[kRsPer];
+  // addresses, no branch around a load), so the tile costs one memory round
+  // trip rather than K
+  uint32_t key[K];
 #pragma unroll
-  for (int r = 0; r < kRsPer; ++r) key[r] = keys[min(base + r * THREADS + t, n - 1)];
-  cnt[t >> 8][t & 255] = 0;
+  for (int r = 0; r < K; ++r) key[r] = kv[min(base + r * T + t, n - 1)].x;
+  for (int i = t; i < kRsWords; i += T) cnt[i] = 0;
   __syncthreads();
-  uint32_t* mine = cnt[(t >> 6) % H];  // wavefront w counts into copy w mod H
 #pragma unroll
-  for (int r = 0; r < kRsPer; ++r)
-    if (base + r * THREADS + t < n) atomicAdd(&mine[(key[r] >> shift) & 255u], 1u);
-  __syncthreads();
-  if (t < 256) {
-    uint32_t s = 0;
-#pragma unroll
-    for (int h = 0; h < H; ++h) s += cnt[h][t];
-    hist[(size_t)t * stride + blockIdx.x] = s;
+  for (int r = 0; r < K; ++r) {
+    const uint32_t d = rs_digit(key[r], pass);
+    if (base + r * T + t < n) atomicAdd(&cnt[d >> 1], 1u << (16 * (d & 1)));
   }
+  __syncthreads();
+  for (int i = t; i < kRsWords; i += T) rows[(size_t)blockIdx.x * kRsWords + i] = cnt[i];
+}
+
+// Sums of kRsGroup rows: {even digit, odd digit} per word.
+__global__ __launch_bounds__(kRsWords) void k_rs_groups(const uint32_t* __restrict__ rows, int ntiles,
+                                                        uint2* __restrict__ groups) {
+  const int t = threadIdx.x, b0 = blockIdx.x * kRsGroup, b1 = min(b0 + kRsGroup, ntiles);
+  uint2 s = make_uint2(0u, 0u);
+  for (int b = b0; b < b1; b += 8) {
+    uint32_t c[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) c[u] = rows[(size_t)min(b + u, b1 - 1) * kRsWords + t];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (b + u < b1) {
+        s.x += c[u] & 0xffffu;
+        s.y += c[u] >> 16;
+      }
+  }
+  groups[(size_t)blockIdx.x * kRsWords + t] = s;
+}
+
+// Inclusive sum over the lanes of a wavefront.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v, int lane) {
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t y = __shfl_up(v, off, 64);
+    if (lane >= off) v += y;
+  }
+  return v;
+}
+
+// Ranks of the keys of a tile. Each wavefront owns 64 K consecutive keys (K
+// rounds of 64, the first `left` of them valid) and ranks them among equal
+// digits with its own running counters in LDS: rank = the wavefront's earlier
+// keys of the digit (mine) + earlier lanes of the round (ballot match mask).
+// LDS operations of one wavefront execute in order, so the rounds need no
+// workgroup barrier.
+typedef uint16_t __attribute__((may_alias)) Count16;
+constexpr uint32_t kRsNone = 0xFFFFFFFFu;
+
+template <int K>
+__device__ __forceinline__ void rs_rank(const uint2 (&kv)[K], int left, int pass, int lane, Count16* mine,
+                                        uint32_t (&pos)[K]) {
+  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+  for (int r = 0; r < K; ++r) {
+    const bool valid = r * 64 + lane < left;
+    const uint32_t d = rs_digit(kv[r].x, pass);
+    uint64_t m = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < kDigBits; ++b) {
+      const bool bit = (d >> b) & 1u;
+      const uint64_t bal = __ballot(bit);
+      m &= bit ? bal : ~bal;
+    }
+    const uint32_t rank = (uint32_t)__popcll(m & lt);
+    const uint32_t prev = mine[d];
+    wave_sync();  // every lane has read its digit's count before the leaders update it
+    if (valid && rank == 0) mine[d] = (Count16)(prev + (uint32_t)__popcll(m));
+    wave_sync();
+    pos[r] = valid ? prev + rank : kRsNone;  // rank among this wavefront's keys of digit d
+  }
+}
+
+// A word's two digits: their totals in the tile (packed), each wavefront's
+// counts turned into its offsets inside them.
+template <int W>
+__device__ __forceinline__ uint32_t rs_totals(uint32_t (*wcnt)[kRsWords], int word) {
+  uint32_t run = 0;
+#pragma unroll
+  for (int v = 0; v < W; ++v) {
+    const uint32_t c = wcnt[v][word];
+    wcnt[v][word] = run;
+    run += c;
+  }
+  return run;
+}
+
+// The whole sort in one workgroup, for up to T K keys: three passes through LDS
+// instead of five launches. Step of the group method: 4096 bodies 117 -> 111 us,
+// 2000 132 -> 125 us; at 8192 the five launches are as fast (129 and 130 us).
+template <int T, int K>
+__global__ __launch_bounds__(T) void k_rs_small(uint32_t* __restrict__ codes, uint32_t* __restrict__ idx, int n) {
+  constexpr int W = T / 64;
+  static_assert(T >= kRsWords && T * K <= 0xffff, "a word per thread, 16 bits per count");
+  __shared__ uint32_t wcnt[W][kRsWords];
+  __shared__ uint32_t lpre[kDigits];
+  __shared__ uint32_t lsum[W];
+  __shared__ uint2 skv[T * K];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int base = w * (64 * K);
+  uint2 kv[K];
+#pragma unroll
+  for (int r = 0; r < K; ++r) {
+    const int p = min(base + r * 64 + lane, n - 1);
+    kv[r] = make_uint2(codes[p], (uint32_t)p);
+  }
+  Count16* mine = reinterpret_cast<Count16*>(wcnt[w]);
+  for (int pass = 0; pass < kRsPasses; ++pass) {
+    for (int i = lane; i < kRsWords; i += 64) wcnt[w][i] = 0;
+    wave_sync();
+    uint32_t pos[K];
+    rs_rank<K>(kv, n - base, pass, lane, mine, pos);
+    __syncthreads();
+    const bool owner = t < kRsWords;
+    const uint32_t run = owner ? rs_totals<W>(wcnt, t) : 0u;
+    const uint32_t both = (run & 0xffffu) + (run >> 16);
+    const uint32_t inc = wave_scan(both, lane);
+    if (lane == 63) lsum[w] = inc;
+    __syncthreads();
+    if (owner) {
+      uint32_t l = inc - both;
+      for (int v = 0; v < w; ++v) l += lsum[v];
+      lpre[2 * t] = l;
+      lpre[2 * t + 1] = l + (run & 0xffffu);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+      if (pos[r] == kRsNone) continue;
+      const uint32_t d = rs_digit(kv[r].x, pass);
+      skv[lpre[d] + mine[d] + pos[r]] = kv[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < K; ++r) kv[r] = skv[min(base + r * 64 + lane, n - 1)];
+    // (the next pass writes skv only behind further barriers)
+  }
+#pragma unroll
+  for (int r = 0; r < K; ++r) {
+    const int p = base + r * 64 + lane;
+    if (p >= n) continue;
+    codes[p] = kv[r].x;
+    idx[p] = kv[r].y;
+  }
+}
+
+// Stable scatter. The tile's digit totals give each digit's start in the tile
+// (lpre) and each wavefront's offset inside it; the tile is reordered by digit
+// in LDS and written out with consecutive lanes on consecutive addresses within
+// each digit's run.
+template <int K, bool GROUPS>
+__global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const uint32_t* __restrict__ codes, const uint2* __restrict__ kin,
+                                                  uint2* __restrict__ kout, uint32_t* __restrict__ codes_out,
+                                                  uint32_t* __restrict__ idx_out, int n, int pass,
+                                                  const uint32_t* __restrict__ rows,
+                                                  const uint2* __restrict__ groups, int ntiles) {
+  constexpr int T = kRsThreads;
+  constexpr int W = T / 64;        // wavefronts per tile
+  constexpr int TILE = T * K;
+  constexpr int Q = T / (kRsWords / 4);  // threads that share 4 words of the rows
+  static_assert(TILE <= 0xffff, "16 bits per count");
+  __shared__ uint32_t wcnt[W][kRsWords];
+  __shared__ uint32_t gbase[kDigits];
+  __shared__ uint32_t lpre[kDigits];
+  __shared__ uint32_t gsum[W], lsum[W];
+  __shared__ uint2 skv[TILE];
+  const int t = threadIdx.x;
+  const int lane = t & 63, w = t >> 6;
+  const int blk = (int)blockIdx.x;
+  // This wavefront's keys, loaded first (clamped addresses, no branch around a
+  // load) so that their latency overlaps the digit starts. The first pass
+  // takes the codes in body order.
+  const int base = blk * TILE + w * (64 * K);
+  uint2 kv[K];
+  if (pass == 0) {
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+      const int p = min(base + r * 64 + lane, n - 1);
+      kv[r] = make_uint2(codes[p], (uint32_t)p);
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < K; ++r) kv[r] = kin[min(base + r * 64 + lane, n - 1)];
+  }
+  // Digit starts: totals over all rows and what precedes this tile. Q threads
+  // share 4 words (16 bytes) of every row and take the rows in turns, kRsAhead
+  // loads at a time; adjacent lanes, so they add up by shuffles, and the first
+  // four keep a word each.
+  const int wg = t / Q, q = t - wg * Q;
+  uint32_t pre[8] = {}, tot[8] = {};
+  if (GROUPS) {
+    const int ng = (ntiles + kRsGroup - 1) / kRsGroup, g = blk / kRsGroup;
+    const uint4* __restrict__ gs = reinterpret_cast<const uint4*>(groups) + 2 * wg;
+    for (int b = q; b < ng; b += Q) {
+      const uint4 c0 = gs[(size_t)b * (kDigits / 4)], c1 = gs[(size_t)b * (kDigits / 4) + 1];
+      const uint32_t e[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        tot[v] += e[v];
+        pre[v] += b < g ? e[v] : 0u;
+      }
+    }
+  }
+  const int b0 = GROUPS ? blk / kRsGroup * kRsGroup : 0, b1 = GROUPS ? blk : ntiles;
+  const uint4* __restrict__ rw = reinterpret_cast<const uint4*>(rows) + wg;
+  for (int b = b0 + q; b < b1; b += kRsAhead * Q) {
+    uint4 c[kRsAhead];
+#pragma unroll
+    for (int u = 0; u < kRsAhead; ++u) c[u] = rw[(size_t)min(b + u * Q, b1 - 1) * (kRsWords / 4)];
+#pragma unroll
+    for (int u = 0; u < kRsAhead; ++u) {
+      const bool in = b + u * Q < b1, before = b + u * Q < blk;
+      const uint32_t e[4] = {c[u].x, c[u].y, c[u].z, c[u].w};
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        const uint32_t d = v & 1 ? e[v >> 1] >> 16 : e[v >> 1] & 0xffffu;
+        if (!GROUPS) tot[v] += in ? d : 0u;
+        pre[v] += before && in ? d : 0u;
+      }
+    }
+  }
+  for (int i = t; i < W * kRsWords; i += T) (&wcnt[0][0])[i] = 0;
+#pragma unroll
+  for (int off = 1; off < Q; off <<= 1)
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      pre[v] += __shfl_xor(pre[v], off, 64);
+      tot[v] += __shfl_xor(tot[v], off, 64);
+    }
+  const bool owner = q < 4;
+  const int word = 4 * wg + (q & 3);
+  uint32_t pre0 = 0, pre1 = 0, tot0 = 0, tot1 = 0;
+#pragma unroll
+  for (int v = 0; v < 4; ++v)
+    if (q == v) {
+      pre0 = pre[2 * v];
+      pre1 = pre[2 * v + 1];
+      tot0 = tot[2 * v];
+      tot1 = tot[2 * v + 1];
+    }
+  __syncthreads();
+  Count16* mine = reinterpret_cast<Count16*>(wcnt[w]);
+  uint32_t pos[K];
+  rs_rank<K>(kv, n - base, pass, lane, mine, pos);
+  __syncthreads();
+  // the exclusive sums over the digits, in the tile and over all keys
+  const uint32_t run = owner ? rs_totals<W>(wcnt, word) : 0u;
+  const uint32_t linc = wave_scan((run & 0xffffu) + (run >> 16), lane);
+  const uint32_t ginc = wave_scan(tot0 + tot1, lane);
+  if (lane == 63) {
+    lsum[w] = linc;
+    gsum[w] = ginc;
+  }
+  __syncthreads();
+  if (owner) {
+    uint32_t l = linc - (run & 0xffffu) - (run >> 16), g = ginc - tot0 - tot1;
+    for (int v = 0; v < w; ++v) {
+      l += lsum[v];
+      g += gsum[v];
+    }
+    lpre[2 * word] = l;
+    lpre[2 * word + 1] = l + (run & 0xffffu);
+    gbase[2 * word] = g + pre0;
+    gbase[2 * word + 1] = g + tot0 + pre1;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < K; ++r) {
+    if (pos[r] == kRsNone) continue;
+    const uint32_t d = rs_digit(kv[r].x, pass);
+    skv[lpre[d] + mine[d] + pos[r]] = kv[r];
+  }
+  __syncthreads();
+  const int valid_here = min(TILE, n - blk * TILE);
+#pragma unroll
+  for (int r = 0; r < K; ++r) {
+    const int j = r * T + t;
+    if (j >= valid_here) continue;
+    const uint2 e = skv[j];
+    const uint32_t d = rs_digit(e.x, pass);
+    const uint32_t g = gbase[d] + ((uint32_t)j - lpre[d]);
+    if (pass + 1 == kRsPasses) {
+      codes_out[g] = e.x;
+      idx_out[g] = e.y;
+    } else {
+      kout[g] = e;
+    }
+  }
+}
+
+// Also packs {x, y, z, m} of each body into one 32-byte record, so the leaf
+// initialisation gathers one record through the sort permutation instead of
+// four scattered planes. A workgroup takes a tile of the sort: it counts its
+// codes' first digits into the tile's row.
+template <int K>
+__global__ __launch_bounds__(kRsThreads) void k_morton(int n, const double* __restrict__ x, const double* __restrict__ m,
+                                              const double* __restrict__ box, uint32_t* __restrict__ codes,
+                                              double4* __restrict__ xm, uint32_t* __restrict__ above,
+                                              uint32_t* __restrict__ rows, uint32_t* __restrict__ flags) {
+  constexpr int T = kRsThreads;
+  __shared__ uint32_t cnt[kRsWords];
+  const int t = threadIdx.x, base = blockIdx.x * (T * K);
+  if (blockIdx.x == 0 && t < 2) above[t] = 0u;  // lengths of the lists that k_build writes
+  for (int i = t; i < kRsWords; i += T) cnt[i] = 0u;
+  double4 p[K];
+#pragma unroll
+  for (int r = 0; r < K; ++r) {
+    const int i = min(base + r * T + t, n - 1);
+    p[r] = make_double4(x[i], x[n + i], x[2 * n + i], m[i]);
+  }
+  const double b[3] = {box[0], box[1], box[2]};
+  __syncthreads();
+  uint32_t bad = 0;
+#pragma unroll
+  for (int r = 0; r < K; ++r) {
+    const int i = base + r * T + t;
+    if (i >= n) continue;
+    const uint32_t ix = cell_of(p[r].x, b[0], &bad);
+    const uint32_t iy = cell_of(p[r].y, b[1], &bad);
+    const uint32_t iz = cell_of(p[r].z, b[2], &bad);
+    const uint32_t code = (part1by2(iz) << 2) | (part1by2(iy) << 1) | part1by2(ix);
+    xm[i] = p[r];
+    codes[i] = code;
+    const uint32_t d = rs_digit(code, 0);
+    atomicAdd(&cnt[d >> 1], 1u << (16 * (d & 1)));
+  }
+  if (bad) atomicOr(flags, (uint32_t)FLAG_OUT_OF_BOX);
+  __syncthreads();
+  for (int i = t; i < kRsWords; i += T) rows[(size_t)blockIdx.x * kRsWords + i] = cnt[i];
 }
 
 // Exclusive prefix sum of a u32 array, in place, in two passes over chunks of
@@ -200,168 +508,6 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(uint32_t* __restric
   if (total && base < count && base + kScanPer >= count) {
     *total = run;
     if (emit) emit[run] = count;
-  }
-}
-
-// Stable scatter. Each wavefront owns 512 consecutive keys of the tile (8
-// rounds of 64) and ranks its keys among equal digits with its own running
-// counters in LDS: rank = the wavefront's earlier keys of the digit
-// (wcnt[w][d]) + earlier lanes of the round (ballot match mask). LDS
-// operations of one wavefront execute in order, so the rounds need no
-// workgroup barrier. Then the tile's digit totals give each digit's start in
-// the tile (lpre) and each wavefront's offset inside it; the tile is
-// reordered by digit in LDS and written out with consecutive lanes on
-// consecutive addresses within each digit's run.
-// RAW: hist holds the raw tile counts and the block forms its digit starts:
-// Q = THREADS / 256 threads per digit sum the digit's row (16-byte loads),
-// then a scan over the 256 digit totals. Otherwise hist holds the starts
-// (the exclusive scan of the count matrix).
-template <int THREADS, bool RAW>
-__global__ __launch_bounds__(THREADS) void k_rs_scatter(const uint32_t* __restrict__ kin,
-                                                        const uint32_t* __restrict__ vin,
-                                                        uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
-                                                        int n, int shift, const uint32_t* __restrict__ hist,
-                                                        int nblocks, int stride) {
-  constexpr int W = THREADS / 64;       // wavefronts per tile
-  constexpr int TILE = kRsPer * THREADS;
-  constexpr int C = TILE / W;           // keys per wavefront
-  constexpr int R = C / 64;             // rounds per wavefront
-  __shared__ uint32_t gbase[256];
-  __shared__ uint32_t wcnt[W][256];
-  __shared__ uint32_t wsum[4];
-  __shared__ uint32_t lpre[256];
-  __shared__ uint32_t skey[TILE], sval[TILE];
-  const int t = threadIdx.x;
-  const int lane = t & 63, w = t >> 6;
-  const int blk = (int)blockIdx.x;
-  // This wavefront's keys and values, loaded first (clamped addresses, no
-  // branch around a load) so that their latency overlaps the digit starts.
-  const int base = blk * TILE + w * C;
-  uint32_t key[R], val[R], pos[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int p = min(base + r * 64 + lane, n - 1);
-    key[r] = kin[p];
-    val[r] = vin[p];
-  }
-  if constexpr (RAW) {
-    constexpr int Q = THREADS / 256;
-    // 16-byte loads per thread for the most tiles the raw form takes, all
-    // issued before the sums (entries past nblocks re-read entry 0 and count
-    // nothing)
-    constexpr int KMAX = (kRsRawMaxBlocks / 4 + Q - 1) / Q;
-    const int d = t / Q, q = t - d * Q;
-    const uint4* __restrict__ row = reinterpret_cast<const uint4*>(hist + (size_t)d * stride);
-    uint4 rv[KMAX];
-#pragma unroll
-    for (int k = 0; k < KMAX; ++k) {
-      const int i = q + k * Q;
-      rv[k] = row[4 * i < nblocks ? i : 0];
-    }
-    uint32_t pre = 0, tot = 0;
-#pragma unroll
-    for (int k = 0; k < KMAX; ++k) {
-      const uint32_t e[4] = {rv[k].x, rv[k].y, rv[k].z, rv[k].w};
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int b = 4 * (q + k * Q) + u;
-        const uint32_t c = b < nblocks ? e[u] : 0u;
-        tot += c;
-        pre += b < blk ? c : 0u;
-      }
-    }
-#pragma unroll
-    for (int off = 1; off < Q; off <<= 1) {  // the Q threads of a digit are adjacent lanes
-      pre += __shfl_xor(pre, off, 64);
-      tot += __shfl_xor(tot, off, 64);
-    }
-    if (q == 0) {
-      gbase[d] = pre;
-      lpre[d] = tot;
-    }
-    __syncthreads();
-    uint32_t v = 0, inc = 0;
-    if (t < 256) {
-      v = lpre[t];
-      inc = v;
-      for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = __shfl_up(inc, off, 64);
-        if (lane >= off) inc += y;
-      }
-      if (lane == 63) wsum[w] = inc;
-    }
-    __syncthreads();
-    if (t < 256) {
-      uint32_t p = inc - v;
-      for (int q2 = 0; q2 < w; ++q2) p += wsum[q2];
-      gbase[t] += p;
-    }
-  } else {
-    if (t < 256) gbase[t] = hist[(size_t)t * stride + blk];
-  }
-  for (int i = t; i < W * 256; i += THREADS) (&wcnt[0][0])[i] = 0;
-  __syncthreads();
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const bool valid = base + r * 64 + lane < n;
-    const uint32_t d = (key[r] >> shift) & 255u;
-    uint64_t m = __ballot(valid);
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const bool bit = (d >> b) & 1u;
-      const uint64_t bal = __ballot(bit);
-      m &= bit ? bal : ~bal;
-    }
-    const uint32_t rank = (uint32_t)__popcll(m & lt);
-    const uint32_t prev = wcnt[w][d];
-    wave_sync();  // every lane has read its digit's count before the leaders update it
-    if (valid && rank == 0) wcnt[w][d] = prev + (uint32_t)__popcll(m);
-    wave_sync();
-    pos[r] = valid ? prev + rank : 0xFFFFFFFFu;  // rank among this wavefront's keys of digit d
-  }
-  __syncthreads();
-  // digit t: its total in the tile, each wavefront's offset inside it, and
-  // the exclusive prefix of the totals over the digits
-  uint32_t tot = 0, inc = 0;
-  if (t < 256) {
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-      const uint32_t c = wcnt[q][t];
-      wcnt[q][t] = tot;
-      tot += c;
-    }
-    inc = tot;
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t y = __shfl_up(inc, off, 64);
-      if (lane >= off) inc += y;
-    }
-    if (lane == 63) wsum[w] = inc;
-  }
-  __syncthreads();
-  if (t < 256) {
-    uint32_t pre = inc - tot;
-    for (int q = 0; q < w; ++q) pre += wsum[q];
-    lpre[t] = pre;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (pos[r] != 0xFFFFFFFFu) {
-      const uint32_t d = (key[r] >> shift) & 255u;
-      const uint32_t slot = lpre[d] + wcnt[w][d] + pos[r];
-      skey[slot] = key[r];
-      sval[slot] = val[r];
-    }
-  }
-  __syncthreads();
-  const int valid_here = min(TILE, n - blk * TILE);
-  for (int j = t; j < valid_here; j += THREADS) {
-    const uint32_t k = skey[j];
-    const uint32_t d = (k >> shift) & 255u;
-    const uint32_t g = gbase[d] + ((uint32_t)j - lpre[d]);
-    kout[g] = k;
-    vout[g] = sval[j];
   }
 }
 
@@ -1539,18 +1685,45 @@ __global__ void k_zero_counters(unsigned long long* p) {
 
 // --------------------------------------------------------------- launch ----
 
+// Tiles of the sort: kRsThreads times `keys` keys.
+struct SortPlan {
+  int keys, tiles;
+  bool groups;
+};
+
+// Few keys per thread shorten the serial ranking of a tile, many tiles lengthen
+// the sums of their rows. Leapfrog step of the group method, us, with 2 / 4 / 8
+// keys: 20000 bodies 137 / 140 / 150, 50000 163 / 164 / 174, 262144 343 / 337 /
+// 336, 524288 550 / 546 / 529 (16 keys: 538). Summing the rows themselves beyond
+// 128 tiles would be 40 rounds of loads at 2^20 keys.
+static SortPlan sort_plan(int64_t n) {
+  SortPlan p{};
+  p.keys = n <= (1 << 15) ? 2 : n <= (1 << 18) ? 4 : 8;
+  p.tiles = (int)((n + p.keys * kRsThreads - 1) / (p.keys * kRsThreads));
+  p.groups = p.tiles > kRsMaxRows;
+  return p;
+}
+
 static int reserve_sort(aster_ctx* c) {
   const size_t n = (size_t)c->n;
-  const size_t nblocks = (n + kRsTile - 1) / kRsTile;  // the most tiles any pass layout uses
+  const size_t tiles = (size_t)sort_plan(c->n).tiles;
   ASTER_HIP(c, c->codes.reserve(n));
   ASTER_HIP(c, c->idx.reserve(n));
-  ASTER_HIP(c, c->codes2.reserve(n));
-  ASTER_HIP(c, c->idx2.reserve(n));
+  ASTER_HIP(c, c->kv.reserve(2 * n));
   ASTER_HIP(c, c->xm4.reserve(n));
   ASTER_HIP(c, c->above.reserve(2));
-  ASTER_HIP(c, c->hist.reserve(256 * (size_t)rs_stride((int)nblocks)));
+  ASTER_HIP(c, c->rows.reserve(tiles * kRsWords));
+  ASTER_HIP(c, c->rowsum.reserve((tiles / kRsGroup + 1) * kRsWords));
   ASTER_HIP(c, c->scanpart.reserve((n + kScanChunk - 1) / kScanChunk + 1));
   return ASTER_OK;
+}
+
+// f with the plan's keys per thread as a compile-time constant.
+template <class F>
+static void with_keys(const SortPlan& p, F f) {
+  if (p.keys == 2) f(std::integral_constant<int, 2>{});
+  else if (p.keys == 4) f(std::integral_constant<int, 4>{});
+  else f(std::integral_constant<int, 8>{});
 }
 
 // In-place exclusive scan of data[0, count); the total goes to *total when
@@ -1603,8 +1776,11 @@ static int morton_codes(aster_ctx* c, bool user_box) {
   int rc = launch_box(c, user_box);
   if (rc) return rc;
   const int n = (int)c->n;
-  hipLaunchKernelGGL(k_morton, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, c->x.p, c->m.p, c->boxd.p,
-                     c->codes.p, c->idx.p, c->xm4.p, c->above.p, c->flags.p);
+  const SortPlan p = sort_plan(n);
+  with_keys(p, [&](auto K) {
+    hipLaunchKernelGGL(k_morton<K()>, dim3(p.tiles), dim3(kRsThreads), 0, c->stream, n, c->x.p, c->m.p, c->boxd.p,
+                       c->codes.p, c->xm4.p, c->above.p, c->rows.p, c->flags.p);
+  });
   ASTER_HIP(c, hipGetLastError());
   phase_end(c, ASTER_PHASE_MORTON);
   c->tree_valid = false;
@@ -1625,50 +1801,28 @@ int morton_sort(aster_ctx* c, bool user_box) {
   if (rc) return rc;
   if ((rc = morton_codes(c, user_box))) return rc;
   const int n = (int)c->n;
-  uint32_t *kin = c->codes.p, *vin = c->idx.p, *kout = c->codes2.p, *vout = c->idx2.p;
-  // The smaller tile (4096 or 8192 keys) that needs at most kRsRawMaxBlocks
-  // tiles; beyond 2^20 keys, 2048-key tiles and the scan. (2048-key tiles
-  // with the offsets formed in the scatter were slower at 2^18 keys: each
-  // block then sums twice the count matrix with half the threads.)
-  int threads = 0;
-  for (int th = 512; th <= 1024 && !threads; th *= 2)
-    if ((n + kRsPer * th - 1) / (kRsPer * th) <= kRsRawMaxBlocks) threads = th;
-  const bool raw = threads != 0;
-  if (!raw) threads = kRsThreads;
-  const int tile = kRsPer * threads;
-  const int nblocks = (n + tile - 1) / tile;
-  const int stride = raw ? rs_stride(nblocks) : nblocks;  // the scan runs over 256 * nblocks contiguous counts
+  const SortPlan p = sort_plan(n);
   phase_begin(c, ASTER_PHASE_SORT);
-  for (int shift = 0; shift < 32; shift += 8) {
-    const dim3 grid(nblocks), block(threads);
-    switch (threads) {
-      case 256:
-        hipLaunchKernelGGL(k_rs_hist<256>, grid, block, 0, c->stream, kin, n, shift, c->hist.p, stride);
-        break;
-      case 512:
-        hipLaunchKernelGGL(k_rs_hist<512>, grid, block, 0, c->stream, kin, n, shift, c->hist.p, stride);
-        break;
-      default:
-        hipLaunchKernelGGL(k_rs_hist<1024>, grid, block, 0, c->stream, kin, n, shift, c->hist.p, stride);
-        break;
-    }
-    if (!raw) {
-      if ((rc = device_scan(c, c->hist.p, 256 * nblocks, nullptr))) return rc;
-      hipLaunchKernelGGL((k_rs_scatter<kRsThreads, false>), grid, block, 0, c->stream, kin, vin, kout, vout, n, shift,
-                         c->hist.p, nblocks, stride);
-    } else if (threads == 512) {
-      hipLaunchKernelGGL((k_rs_scatter<512, true>), grid, block, 0, c->stream, kin, vin, kout, vout, n, shift,
-                         c->hist.p, nblocks, stride);
-    } else {
-      hipLaunchKernelGGL((k_rs_scatter<1024, true>), grid, block, 0, c->stream, kin, vin, kout, vout, n, shift,
-                         c->hist.p, nblocks, stride);
-    }
-    std::swap(kin, kout);
-    std::swap(vin, vout);
+  if (n <= kRsSmall) {
+    hipLaunchKernelGGL((k_rs_small<1024, kRsSmall / 1024>), dim3(1), dim3(1024), 0, c->stream, c->codes.p, c->idx.p, n);
+  }
+  for (int pass = 0; pass < kRsPasses && n > kRsSmall; ++pass) {
+    const uint2* kin = c->kv.p + (pass == 2 ? n : 0);  // pass 0: the codes -> kv, then -> kv + n -> codes, idx
+    uint2* kout = c->kv.p + (pass == 1 ? n : 0);
+    with_keys(p, [&](auto K) {
+      const dim3 grid(p.tiles), block(kRsThreads);
+      if (pass > 0)
+        hipLaunchKernelGGL((k_rs_hist<K()>), grid, block, 0, c->stream, kin, n, pass, c->rows.p);
+      if (p.groups)
+        hipLaunchKernelGGL(k_rs_groups, dim3((p.tiles + kRsGroup - 1) / kRsGroup), dim3(kRsWords), 0, c->stream,
+                           c->rows.p, p.tiles, c->rowsum.p);
+      auto kern = p.groups ? k_rs_scatter<K(), true> : k_rs_scatter<K(), false>;
+      hipLaunchKernelGGL(kern, grid, block, 0, c->stream, c->codes.p, kin, kout, c->codes.p, c->idx.p, n, pass,
+                         c->rows.p, c->rowsum.p, p.tiles);
+    });
   }
   ASTER_HIP(c, hipGetLastError());
   phase_end(c, ASTER_PHASE_SORT);
-  // Four passes: sorted codes are back in c->codes, permutation in c->idx.
   return ASTER_OK;
 }
 

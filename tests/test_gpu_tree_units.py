@@ -108,3 +108,21 @@ def test_stack_at_its_limit(ctx):
     scale = np.linalg.norm(ref, axis=1)
     err = np.linalg.norm(acc - ref, axis=1) / np.maximum(scale, np.median(scale))
     assert inter == n * (n - 1) and np.median(err) < 1e-6 and err.max() < 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 1025, 4095, 4096, 4097, 32768, 32769, 131073, 262144, 262145, 524288,
+                               524289, 2097151])
+@pytest.mark.parametrize("cells", ["spread", "few", "one"])
+def test_sort_order_at_the_tiles_edges(ctx, n, cells):
+    """(code, body) order against numpy where the tile, the kernel or the way to the digit starts changes, also with most
+    or all keys equal."""
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(-1.0, 1.0, (n, 3)) * {"spread": 1.0, "few": 0.004, "one": 1e-9}[cells] + 1e-3
+    ctx.set_params(G=1.0, softening=1e-2, theta=1.5, box=(1.0, 1.0, 1.0))
+    ctx.set_state(pos, np.zeros_like(pos), np.ones(n))
+    codes, _ = ctx.morton()
+    ctx.forces(A.BH_GROUP, out=False)
+    tree = ctx.tree()
+    ref = np.lexsort((np.arange(n), codes))
+    assert np.array_equal(tree["perm"], ref) and np.array_equal(tree["codes"], codes[ref])
