@@ -1262,8 +1262,10 @@ __global__ __launch_bounds__(256) void k_bh_f64(int n, const double* __restrict_
 // Morton cell (the subtree's common code prefix), so the group box is compact
 // wherever the curve jumps. Groups partition the sorted bodies.
 
-// Wavefront-cooperative traversal, one group per wavefront (lanes = the
-// group's bodies, at most 64). The wavefront walks the tree once for the
+// Cooperative traversal, one group (at most 64 bodies) per workgroup of W
+// wavefronts; W = 1 in what follows, more in bh_forces_all's rule: W times the
+// candidates per iteration, the list, the stack and the lanes that share its
+// evaluation, by workgroup barriers. The wavefront walks the tree once for the
 // whole group with a shared LDS stack of opened nodes, testing up to 64
 // candidate nodes per iteration: lane 2 i + s takes child s of the i-th popped
 // node from that node's child slots (record, id and threshold of both
@@ -1315,14 +1317,14 @@ struct PieceTable {
   uint8_t pieces[65];
 };
 
-constexpr PieceTable make_piece_table() {
+constexpr PieceTable make_piece_table(int waves) {
   PieceTable t{};
   for (int g = 1; g <= 64; ++g) {
     int best = 1 << 30, bp = 1, bq = 1;
     for (int p = 1; p <= kPieceMaxPasses; ++p) {
-      int q = (64 * p) / g;
+      int q = (64 * waves * p) / g;
       if (q > 64) q = 64;
-      const int cost = p * ((96 + q - 1) / q + 1);
+      const int cost = p * ((96 * waves + q - 1) / q + 1);
       if (cost < best) {
         best = cost;
         bp = p;
@@ -1335,7 +1337,8 @@ constexpr PieceTable make_piece_table() {
   return t;
 }
 
-__constant__ PieceTable kPieces = make_piece_table();
+template <int W>
+__constant__ PieceTable kPieces = make_piece_table(W);
 
 // One piece: lam list entries from `p` against the body at `me`.
 template <bool MASK>
@@ -1367,13 +1370,14 @@ __device__ __forceinline__ void group_piece_sum(const float4* __restrict__ p, in
 // lane per body, which left a third of the lanes idle and waited for the
 // gather, and 61 instructions: 1PN, 5000 bodies 352 -> 219 us, 100003 1219 ->
 // 766 us, 2^20 9.8 -> 6.3 ms; 1PN + 2PN + 2.5PN 1023 -> 986 us, 4.62 -> 4.16 ms,
-// 36.8 -> 30.3 ms. More waves (3 or 4 per SIMD by launch bounds) gained nothing.
-constexpr int kPnBatch = 64;  // entries in LDS at a time
-struct PnLds {                // behind the list, the stack and the node ids
-  double4 com[kPnBatch];      // entries: centre of mass, mass
-  double4 vel[kPnBatch];      // velocity, -2 |v|^2
-  double4 bpos[64];           // bodies: position, mass
-  double4 bvel[64];           // velocity, -|v|^2
+// 36.8 -> 30.3 ms (a wavefront per group; several: bh_forces_all).
+constexpr int kPnBatch = 64;  // entries in LDS at a time, per wavefront
+template <int W>
+struct PnLds {                  // behind the list, the stack and the node ids
+  double4 com[W * kPnBatch];    // entries: centre of mass, mass
+  double4 vel[W * kPnBatch];    // velocity, -2 |v|^2
+  double4 bpos[64];             // bodies: position, mass
+  double4 bvel[64];             // velocity, -|v|^2
 };
 static_assert(kPieceMaxPasses * 64 * sizeof(double) <= (kGrpList + kGrpListPad) * sizeof(float4),
               "one coordinate of the pieces' sums takes the list's place");
@@ -1420,19 +1424,25 @@ __device__ __forceinline__ void pn1_pairs(const double4* nc, const double4* nv, 
 #undef ASTER_EACH
 }
 
-template <bool MASK, int PN>  // PN: 0 none, 1 the 1PN term alone, 2 any terms
-__global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restrict__ gstart,
+template <bool MASK, int PN, int W>  // PN: 0 none, 1 the 1PN term alone, 2 any terms; W: wavefronts per group
+__global__ __launch_bounds__(64 * W, PN == 1 ? 3 : 1) void k_bh_group(int n, const int32_t* __restrict__ gstart,
                                                  const uint32_t* __restrict__ gcount, const float4* __restrict__ gsh,
                                                  const float4* __restrict__ kids, const uint32_t* __restrict__ perm,
                                                  float eps2, float msc, double G,
                                                  double* __restrict__ a, unsigned long long* __restrict__ counters,
                                                  uint32_t* __restrict__ flags, NodePn pnp) {
   extern __shared__ float4 grp_lds[];
-  float4* lst = grp_lds;                                              // kGrpList + kGrpListPad entries
-  int* stk = reinterpret_cast<int*>(grp_lds + kGrpList + kGrpListPad);  // kGrpStack entries
-  int* lid = stk + kGrpStack;  // PN: node id of each list entry (kGrpList entries)
-  PnLds* pl = reinterpret_cast<PnLds*>(grp_lds + kGrpList + kGrpListPad + (kGrpStack + kGrpList) / 4);  // PN
-  const int lane = threadIdx.x;
+  constexpr int kList = W * kGrpList, kPad = W * kGrpListPad, kStack = W * kGrpStack;
+  float4* lst = grp_lds;                                   // kList + kPad entries
+  int* stk = reinterpret_cast<int*>(grp_lds + kList + kPad);  // kStack entries
+  int* lid = stk + kStack;  // PN: node id of each list entry (kList entries)
+  PnLds<W>* pl = reinterpret_cast<PnLds<W>*>(grp_lds + kList + kPad + (kStack + kList) / 4);  // PN
+  __shared__ int2 wsum[W];  // W > 1: each wavefront's accepted and opened candidates
+  const int tid = threadIdx.x, lane = tid & 63, w = W > 1 ? tid >> 6 : 0;
+  auto sync = [] {
+    if (W > 1) __syncthreads();
+    else wave_sync();
+  };
   const int ngroups = (int)*gcount;
   const int per_xcd = (ngroups + 7) >> 3;
   const int xcd = blockIdx.x & 7;
@@ -1448,20 +1458,20 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
     const bool live = k <= hi;
     const float4 me = gsh[live ? k : hi];
     double pacc[3] = {0.0, 0.0, 0.0};  // PN: the body's terms
-    if (PN) {  // the bodies' FP64 positions, masses and velocities (the leaves' records)
+    if (PN && w == 0) {  // the bodies' FP64 positions, masses and velocities (the leaves' records)
       double4 vme = pnp.nvel[live ? k : hi];
       vme.w = -fma(vme.x, vme.x, fma(vme.y, vme.y, vme.z * vme.z));
       pl->bpos[lane] = pnp.nmc[live ? k : hi];
       pl->bvel[lane] = vme;
     }
     // this lane's piece in each pass
-    const int npass = __builtin_amdgcn_readfirstlane((int)kPieces.passes[gsz]);
-    const int npc = __builtin_amdgcn_readfirstlane((int)kPieces.pieces[gsz]);
+    const int npass = __builtin_amdgcn_readfirstlane((int)kPieces<W>.passes[gsz]);
+    const int npc = __builtin_amdgcn_readfirstlane((int)kPieces<W>.pieces[gsz]);
     float4 ppos[kPieceMaxPasses];
     int pidx[kPieceMaxPasses], pbody[kPieceMaxPasses];
 #pragma unroll
     for (int p = 0; p < kPieceMaxPasses; ++p) {
-      const int j = 64 * p + lane;
+      const int j = 64 * W * p + tid;
       int b = j / npc, pc = j - b * npc;
       if (b >= gsz) {
         b = gsz - 1;
@@ -1496,30 +1506,30 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
       const int m = __builtin_amdgcn_readfirstlane(cnt);
       const int lam = __builtin_amdgcn_readfirstlane((m + npc - 1) / npc);
       const int mp = npc * lam;  // m <= mp < m + npc <= m + 64
-      if (lane < mp - m) lst[m + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (tid < mp - m) lst[m + tid] = make_float4(0.f, 0.f, 0.f, 0.f);
       double4 ec, ev;
       auto gather = [&](int first) {
-        const int node = lid[min(first + lane, m - 1)];
+        const int node = lid[min(first + tid, m - 1)];
         ec = pnp.nmc[node];
         ev = pnp.nvel[node];
-        if (first + lane >= m) ec.w = 0.0;  // padding: adds exactly zero
+        if (first + tid >= m) ec.w = 0.0;  // padding: adds exactly zero
       };
       // whole pieces of at most kPnBatch entries
-      const int batch = PN ? __builtin_amdgcn_readfirstlane(kPnBatch / npc * npc) : 0;
+      const int batch = PN ? __builtin_amdgcn_readfirstlane(W * kPnBatch / npc * npc) : 0;
       if (PN) gather(0);  // in flight during the Newtonian passes
-      wave_sync();
+      sync();
       float px[kPieceMaxPasses], py[kPieceMaxPasses], pz[kPieceMaxPasses];
 #pragma unroll
       for (int p = 0; p < kPieceMaxPasses; ++p) {
         px[p] = py[p] = pz[p] = 0.f;
         if (p < npass) group_piece_sum<MASK>(lst + pidx[p] * lam, lam, ppos[p], eps2, px[p], py[p], pz[p]);
       }
-      wave_sync();  // every lane is done with the list: its LDS takes the partial sums
+      sync();  // every lane is done with the list: its LDS takes the partial sums
 #pragma unroll
       for (int p = 0; p < kPieceMaxPasses; ++p)
-        if (p < npass) lst[64 * p + lane] = make_float4(px[p], py[p], pz[p], 0.f);
-      wave_sync();
-      if (live) {
+        if (p < npass) lst[64 * W * p + tid] = make_float4(px[p], py[p], pz[p], 0.f);
+      sync();
+      if (live && w == 0) {
         float tx = 0.f, ty = 0.f, tz = 0.f;
         const float4* __restrict__ mine = lst + lane * npc;
         for (int c = 0; c < npc; ++c) {
@@ -1540,10 +1550,10 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
         for (int first = 0; first < m; first += batch) {
           const int cntb = min(batch, m - first);
           const int lamb = __builtin_amdgcn_readfirstlane((cntb + npc - 1) / npc);
-          pl->com[lane] = ec;
+          pl->com[tid] = ec;
           ev.w = -2.0 * fma(ev.x, ev.x, fma(ev.y, ev.y, ev.z * ev.z));
-          pl->vel[lane] = ev;
-          wave_sync();
+          pl->vel[tid] = ev;
+          sync();
           if (first + batch < m) gather(first + batch);
 #pragma unroll
           for (int p = 0; p < kPieceMaxPasses; ++p) {
@@ -1565,7 +1575,7 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
                 node_pn_rec(pnp, pl->com[e0 + e], pl->vel[e0 + e], pb, vb, inv_m, pa[p][0], pa[p][1], pa[p][2]);
             }
           }
-          wave_sync();  // every lane is done with these entries
+          sync();  // every lane is done with these entries
         }
         // a body adds its pieces in order, one coordinate at a time through the
         // list's LDS
@@ -1574,17 +1584,17 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
         for (int c = 0; c < 3; ++c) {
 #pragma unroll
           for (int p = 0; p < kPieceMaxPasses; ++p)
-            if (p < npass) ps[64 * p + lane] = pa[p][c];
-          wave_sync();
-          if (live) {
+            if (p < npass) ps[64 * W * p + tid] = pa[p][c];
+          sync();
+          if (live && w == 0) {
             double t = 0.0;
             for (int q = 0; q < npc; ++q) t += ps[lane * npc + q];
             pacc[c] += PN == 1 ? t * (pnp.G * (pnp.ic * pnp.ic)) : t;
           }
-          wave_sync();
+          sync();
         }
       }
-      wave_sync();  // the partial sums are read before the list is refilled
+      sync();  // the partial sums are read before the list is refilled
       listed += (unsigned long long)cnt;
       cnt = 0;
     };
@@ -1592,17 +1602,17 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
       const int root = n, rs = 2 * (n - 1);
       const float4 r = kids[2 * rs];
       if (dmin2(r) > kids[2 * rs + 1].y) {
-        if (lane == 0) {
+        if (tid == 0) {
           lst[0] = make_float4(r.x, r.y, r.z, r.w * msc);
           if (PN) lid[0] = root;
         }
         cnt = 1;
       } else {
-        if (lane == 0) stk[0] = root;
+        if (tid == 0) stk[0] = root;
         sp = 1;
       }
     }
-    wave_sync();
+    sync();
     // The children of the next batch (the top of the stack) are
     // loaded before a pending flush evaluates the list, so the load's latency
     // overlaps that arithmetic. Lane 2 i + s takes child s of entry i: the two
@@ -1614,10 +1624,10 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
     float2 na;
     // With an empty stack (the walk is over) it loads the root's children.
     auto fetch = [&]() {
-      take = min(min(sp, 32), max(kGrpStack - kGrpDeep - sp, 1));
-      const int e = max(min(lane >> 1, take - 1), 0);
+      take = min(min(sp, 32 * W), max(kStack - kGrpDeep - sp, 1));
+      const int e = max(min(tid >> 1, take - 1), 0);
       const int opened = sp > 0 ? stk[sp - take + e] : n;
-      const int slot = kid_slot(n, opened, lane & 1);
+      const int slot = kid_slot(n, opened, tid & 1);
       nr = kids[2 * slot];
       na = *reinterpret_cast<const float2*>(kids + 2 * slot + 1);
     };
@@ -1629,39 +1639,53 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
       // both terms evaluated (no short circuit): the id and the threshold
       // arrive with the record in one round trip
       const bool take_it = (node < n) | (dmin2(r) > na.y);
-      const bool mine = lane < 2 * take;
+      const bool mine = tid < 2 * take;
       const bool acc = mine & take_it, opn = mine & !take_it;
       sp -= take;
       visits += 2 * take;
-      wave_sync();
       const uint64_t am = __ballot(acc), om = __ballot(opn);
-      const int nopen = (int)__popcll(om);
+      int nacc = (int)__popcll(am), nopen = (int)__popcll(om);  // of all wavefronts
+      int e = cnt + (int)__popcll(am & lt), f = sp + (int)__popcll(om & lt);
+      if (W > 1 && lane == 0) wsum[w] = make_int2(nacc, nopen);
+      sync();  // also: every candidate's entry has been read off the stack
+      if (W > 1) {
+        nacc = nopen = 0;
+#pragma unroll
+        for (int v = 0; v < W; ++v) {
+          const int2 c = wsum[v];
+          e += v < w ? c.x : 0;
+          f += v < w ? c.y : 0;
+          nacc += c.x;
+          nopen += c.y;
+        }
+        nacc = __builtin_amdgcn_readfirstlane(nacc);
+        nopen = __builtin_amdgcn_readfirstlane(nopen);
+      }
       // cannot happen for a valid tree (see bound above); the walk then ends
       // here (no early exit from the loop, which keeps its control flow simple)
-      const bool over = sp + nopen > kGrpStack;
+      const bool over = sp + nopen > kStack;
       if (over) {
-        if (lane == 0) atomicOr(flags, (uint32_t)FLAG_TREE);
+        if (tid == 0) atomicOr(flags, (uint32_t)FLAG_TREE);
         overflow = true;
       }
       // list entries carry the scaled mass (one multiply per entry, not per pair)
       if (acc) {
-        const int e = cnt + (int)__popcll(am & lt);
         lst[e] = make_float4(r.x, r.y, r.z, r.w * msc);
         if (PN) lid[e] = node;
       }
-      if (opn && !over) stk[sp + __popcll(om & lt)] = node;
-      cnt += (int)__popcll(am);
+      if (opn && !over) stk[f] = node;
+      cnt += nacc;
       sp = over ? 0 : sp + nopen;
-      wave_sync();
+      sync();
       fetch();
-      if (cnt > kGrpList - 64) {
+      if (cnt > kList - 64 * W) {
         flush();
-        wave_sync();
+        sync();
       }
     }
     if (cnt > 0) flush();
-    wave_sync();
-    if (live) {
+    sync();
+    if (live && w == 0) {
       const int b = (int)perm[k];
       a[b] = G * ((double)sx - (double)cx) + pacc[0];
       a[n + b] = G * ((double)sy - (double)cy) + pacc[1];
@@ -1673,7 +1697,7 @@ __global__ __launch_bounds__(64) void k_bh_group(int n, const int32_t* __restric
     tot_visits += visits;
     if (overflow) break;
   }
-  if (lane == 0 && (tot_inter | tot_visits)) {
+  if (tid == 0 && (tot_inter | tot_visits)) {
     atomicAdd(&counters[BHC_INTERACTIONS], tot_inter);
     atomicAdd(&counters[BHC_VISITS], tot_visits);
   }
@@ -1913,16 +1937,35 @@ static int bh_forces_all(aster_ctx* c, int method) {
       // (the usual case); workgroups loop when there are more groups. The
       // count is a multiple of 8 for the XCD-interleaved group order.
       const int blocks = ((n / 32 + 1) + 7) & ~7;
-      const dim3 grid(blocks), block(64);
-      // PN: node ids, then (16-byte aligned) FP64 records and velocities of the list
-      const size_t lds = (kGrpList + kGrpListPad) * sizeof(float4) +
-                         (pn ? (kGrpStack + kGrpList) * sizeof(int) + sizeof(PnLds) : kGrpStack * sizeof(int));
       const NodePn gp{c->nmc.p, c->nvel.p, c->P.G, ic, c->P.softening, pnf};
-      auto kern = !pn ? (mask ? k_bh_group<true, 0> : k_bh_group<false, 0>)
-                  : pnf == ASTER_PN1 ? (mask ? k_bh_group<true, 1> : k_bh_group<false, 1>)
-                                     : (mask ? k_bh_group<true, 2> : k_bh_group<false, 2>);
-      hipLaunchKernelGGL(kern, grid, block, lds, c->stream, n, c->gstart.p, c->gcount.p, c->gsh.p, c->kids.p,
-                         c->idx.p, eps2, sc.msc, sc.gsc, c->a.p, c->bh_counters.p, c->flags.p, gp);
+      // Wavefronts per group. Below ~2^18 bodies the ~n/42 groups leave SIMDs
+      // idle (there are 1024) and the longest walk decides. Evaluation at
+      // theta 0.5 with 1 / 2 / 4 wavefronts, us: 2000 bodies 162 / 129 / 115,
+      // 50000 222 / 180 / 164, 100000 273 / 239 / 235, 200000 374 / 349 / 365,
+      // 400000 572 / 577 / 605, 2^20 1199 / 1285 / 1444. With the 1PN term: 5000
+      // 298 / 209 / 204, 20000 417 / 322 / 341, 50000 580 / 479 / 485, 100000
+      // 849 / 734 / 792, 2^20 6.5 / 6.4 ms; several wavefronts wait at barriers, so
+      // registers are kept to three waves per SIMD there (785 / 868 without at
+      // 100000). All terms: 5000 1073 / 667 / 390, 131072 5251 / 4285 / 3534, 2^20
+      // 29.8 / 30.7 / 28.8 ms. The same line for all, so that the Newtonian sums
+      // have the same bits with and without the terms.
+      auto launch = [&](auto waves, auto terms) {
+        constexpr int W = waves(), PN = terms();
+        // PN: node ids, then (16-byte aligned) FP64 records and velocities of the list
+        const size_t lds = W * ((kGrpList + kGrpListPad) * sizeof(float4) + kGrpStack * sizeof(int)) +
+                           (PN ? W * kGrpList * sizeof(int) + sizeof(PnLds<W>) : 0);
+        auto kern = mask ? k_bh_group<true, PN, W> : k_bh_group<false, PN, W>;
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * W), lds, c->stream, n, c->gstart.p, c->gcount.p, c->gsh.p,
+                           c->kids.p, c->idx.p, eps2, sc.msc, sc.gsc, c->a.p, c->bh_counters.p, c->flags.p, gp);
+      };
+      auto waves = [&](auto terms) {
+        if (n <= 1 << 16) launch(std::integral_constant<int, 4>{}, terms);
+        else if (n <= 1 << 18) launch(std::integral_constant<int, 2>{}, terms);
+        else launch(std::integral_constant<int, 1>{}, terms);
+      };
+      if (!pn) waves(std::integral_constant<int, 0>{});
+      else if (pnf == ASTER_PN1) waves(std::integral_constant<int, 1>{});
+      else waves(std::integral_constant<int, 2>{});
     } else {
       const NodePn gp{c->nmc.p, c->nvel.p, c->P.G, ic, c->P.softening, pnf};
       auto kern = pn ? (mask ? k_bh_f32<true, true> : k_bh_f32<false, true>)

@@ -126,3 +126,28 @@ def test_sort_order_at_the_tiles_edges(ctx, n, cells):
     tree = ctx.tree()
     ref = np.lexsort((np.arange(n), codes))
     assert np.array_equal(tree["perm"], ref) and np.array_equal(tree["codes"], codes[ref])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,flags", [(65536, 0), (65537, 0), (262145, 0), (65536, A.PN1), (65537, A.PN1), (262145, A.PN1),
+                                     (9000, A.PN1 | A.PN2)])
+def test_wavefronts_per_group(ctx, orc, n, flags):
+    """The oracle's lists and forces on both sides of the rule's lines (bars of the traversal's own tests)."""
+    pos, vel, mass = A.ic_mixed(n, 5)
+    box = orc.box_auto(pos)
+    ctx.set_params(G=1.0, softening=2.5e-5, theta=0.7, c=30.0)
+    ctx.set_state(pos, vel, mass)
+    newton = ctx.forces(A.BH_GROUP)
+    if not flags:
+        ref, inter, visits = orc.bh_group(pos, mass, box, 0.7, soft=2.5e-5)
+        assert ctx.bh_stats() == (inter, visits)
+        scale = np.linalg.norm(ref, axis=1)
+        err = np.linalg.norm(newton - ref, axis=1) / np.maximum(scale, np.median(scale))
+        assert np.median(err) < 1e-6 and err.max() < 1e-4
+        return
+    ctx.set_params(G=1.0, softening=2.5e-5, theta=0.7, c=30.0, pn_flags=A.NEWTON | flags)
+    both = ctx.forces(A.BH_GROUP)
+    ref = orc.bh_group_pn(pos, vel, mass, box, 0.7, c=30.0, soft=2.5e-5, pn=A.NEWTON | flags)
+    scale = np.linalg.norm(ref, axis=1)
+    err = np.linalg.norm(both - newton - ref, axis=1)
+    assert np.all(err <= 1e-9 * np.maximum(scale, np.median(scale)) + 1e-15 * np.abs(both).max())
