@@ -1011,137 +1011,302 @@ int batch_autotune(aster_ctx* c, int integrator, double dt, int32_t* spb, int32_
 //   J^T w : G sum_j [u/s^3 - 3 d (d.u)/s^5],  u = m_k w_j - m_j w_k
 //   M^T w : -G sum_j (w_j . d)/s^3
 
-__global__ __launch_bounds__(256) void k_batch_traj_fwd(BatchArgs P, double* __restrict__ traj, int64_t nbodies) {
-  __shared__ double sx[kBatchMaxWpb][64], sy[kBatchMaxWpb][64], sz[kBatchMaxWpb][64], sm[kBatchMaxWpb][64];
+// Both kernels evaluate every pair once: in round r = 1 .. n/2 a lane takes the
+// pair of its body with the body r places on (cyclically in its system; an even
+// system's last round covers each pair twice, the first half keeps theirs) and
+// passes the partner's part over LDS. A three-body system, one round, needs
+// one pair per lane and step instead of three sources of which one is the body
+// itself. Bound: latency (4096 three-body systems are some 200 wavefronts on
+// 1024 SIMDs, a serial chain per step), so the backward pass loads positions
+// kTrajAhead steps ahead and nothing in the loop waits for loads or stores.
+// 200 steps of 4096 three-body systems, forward / backward: three sources per
+// lane 112 / 222 us; pairs once 90 / 97; snapshot steps kept as scalars and the
+// look-ahead kept through the loop 66 / 93; in quads of lanes 36 / 50.
+constexpr int kTrajAhead = 4;
+
+// A lane's partner and the lane it receives from in round r.
+struct CyclicPair {
+  int to, from;
+  bool own;  // this lane evaluates the pair
+};
+__device__ __forceinline__ CyclicPair cyclic_pair(int lane, int base, int cnt, int r, bool live) {
+  const int i = lane - base;
+  CyclicPair p;
+  const bool in = live && 2 * r <= cnt;
+  p.own = in && (2 * r < cnt || i < r);
+  p.to = in ? (i + r < cnt ? lane + r : lane + r - cnt) : lane;
+  p.from = in ? (i >= r ? lane - r : lane - r + cnt) : lane;
+  return p;
+}
+
+// Systems of three bodies in quads of lanes (TRIPLES): the exchanges with the
+// next and the previous body are lane permutations within the quad instead of
+// LDS round trips; a quad's last lane is idle.
+__device__ __forceinline__ double quad_next(double x) {  // lanes 0, 1, 2 <- 1, 2, 0
+  const int lo = __builtin_amdgcn_mov_dpp((int)lo32(x), 0xC9, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)hi32(x), 0xC9, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double quad_prev(double x) {  // lanes 0, 1, 2 <- 2, 0, 1
+  const int lo = __builtin_amdgcn_mov_dpp((int)lo32(x), 0xD2, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)hi32(x), 0xD2, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+
+// A lane's body, its system's first lane and size, and the wavefront's rounds.
+struct TrajLane {
+  int b, base, cnt, rounds;
+};
+template <bool TRIPLES>
+__device__ __forceinline__ TrajLane traj_lane(const BatchArgs& P, int64_t nbodies, int wave, int lane) {
+  if (TRIPLES) {
+    const int64_t b = (int64_t)(wave * 16 + (lane >> 2)) * 3 + (lane & 3);
+    return {(lane & 3) < 3 && b < nbodies ? (int)b : -1, lane & ~3, 3, 1};
+  }
+  const int slot = wave * 64 + lane, seg = P.lane_seg[slot];
+  return {P.lane_body[slot], seg >> 8, seg & 255, __builtin_amdgcn_readfirstlane(P.wave_max[wave]) >> 1};
+}
+
+// 1 / sqrt(x) by one third-order step from the estimate.
+__device__ __forceinline__ double rsqrt64_cubic(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// Snapshot step q as a scalar: kept as a loaded vector, every comparison would
+// wait for all earlier stores or loads of the wavefront.
+__device__ __forceinline__ int64_t snap_step(const int64_t* snaps, int q) {
+  const int64_t s = snaps[q];
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)s);
+  const int hi = __builtin_amdgcn_readfirstlane((int)(s >> 32));
+  return (int64_t)(((uint64_t)(uint32_t)hi << 32) | lo);
+}
+
+struct TrajArgs {
+  double* traj;          // positions of every step
+  double* v0;            // initial velocities
+  const int64_t* snaps;  // snapshot steps
+  int nsnap;
+  double* snap_pos;  // positions of the snapshots, forward; gradients, backward
+  int64_t nbodies, nsteps;
+  double dt;
+  double* out;  // gradients: positions, velocities, masses
+  int nwaves;
+};
+
+// Launch shape: quads of lanes where every system has three bodies, otherwise
+// the batch's own packing.
+struct TrajShape {
+  bool triples;
+  int nwaves, wpb;
+};
+static TrajShape traj_shape(const BatchState& B) {
+  if (B.triples) return {true, (int)((B.nsys + 15) / 16), 1};
+  return {false, B.nwaves, B.waves_per_block};
+}
+
+template <bool TRIPLES>
+__global__ __launch_bounds__(256) void k_batch_traj_fwd(BatchArgs P, TrajArgs Q) {
+  constexpr int kLds = TRIPLES ? 1 : kBatchMaxWpb;
+  __shared__ double4 sbody[kLds][64];  // position, mass
+  __shared__ double4 spart[kLds][64];
   const int wl = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wave = blockIdx.x * (blockDim.x >> 6) + wl;
-  if (wave >= P.nwaves) return;
-  const int slot = wave * 64 + lane;
-  const int b = P.lane_body[slot];
-  const int seg = P.lane_seg[slot];
-  const int base = seg >> 8, cnt = seg & 255;
-  const int maxcnt = P.wave_max[wave];
+  if (wave >= Q.nwaves) return;
+  const TrajLane me = traj_lane<TRIPLES>(P, Q.nbodies, wave, lane);
+  const int b = me.b, base = me.base, cnt = me.cnt;
   const bool live = b >= 0;
-  double X[3] = {0.0, 0.0, 0.0}, V[3] = {0.0, 0.0, 0.0}, A[3] = {0.0, 0.0, 0.0};
+  double X[3] = {0.0, 0.0, 0.0}, V[3] = {0.0, 0.0, 0.0}, a[3];
   double mi = 0.0;
   if (live) {
     for (int c = 0; c < 3; ++c) {
       X[c] = P.x[3 * (size_t)b + c];
       V[c] = P.v[3 * (size_t)b + c];
+      Q.v0[3 * (size_t)b + c] = V[c];
     }
     mi = P.m[b];
   }
-  sm[wl][lane] = mi;
-  auto publish = [&]() {
-    sx[wl][lane] = X[0];
-    sy[wl][lane] = X[1];
-    sz[wl][lane] = X[2];
+  const double mnext = quad_next(mi);
+  const CyclicPair first = cyclic_pair(lane, base, cnt, 1, live);
+  auto pair = [&](const CyclicPair& p) {
+    const double4 q = TRIPLES ? make_double4(quad_next(X[0]), quad_next(X[1]), quad_next(X[2]), mnext)
+                              : sbody[wl][p.to];
+    const double d[3] = {q.x - X[0], q.y - X[1], q.z - X[2]};
+    const double r2 = fma(d[0], d[0], fma(d[1], d[1], fma(d[2], d[2], P.soft)));
+    const double inv = rsqrt64_cubic(r2);
+    const double inv3 = p.own ? inv * inv * inv : 0.0;
+    const double fk = q.w * inv3, fj = mi * inv3;
+    if (TRIPLES) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) a[c] = fma(fk, d[c], -quad_prev(fj * d[c]));
+      return;
+    }
+    spart[wl][lane] = make_double4(fj * d[0], fj * d[1], fj * d[2], 0.0);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) a[c] = fma(fk, d[c], a[c]);
+    wave_sync();
+    const double4 o = spart[wl][p.from];
+    a[0] -= o.x;
+    a[1] -= o.y;
+    a[2] -= o.z;
     wave_sync();
   };
+  auto accel = [&]() {  // over G
+    if (!TRIPLES) {
+      sbody[wl][lane] = make_double4(X[0], X[1], X[2], mi);
+      wave_sync();
+    }
+    a[0] = a[1] = a[2] = 0.0;
+    pair(first);
+    for (int r = 2; r <= me.rounds; ++r) pair(cyclic_pair(lane, base, cnt, r, live));
+  };
+  int q = 0;
+  int64_t next = Q.nsnap > 0 ? snap_step(Q.snaps, 0) : -1;
+  double* at = Q.traj + 3 * (size_t)(live ? b : 0);
   auto store = [&](int64_t s) {
     if (live)
-      for (int c = 0; c < 3; ++c) traj[((size_t)s * nbodies + b) * 3 + c] = X[c];
+      for (int c = 0; c < 3; ++c) at[c] = X[c];
+    at += 3 * Q.nbodies;
+    if (s == next) {
+      if (live)
+        for (int c = 0; c < 3; ++c) Q.snap_pos[((size_t)q * Q.nbodies + b) * 3 + c] = X[c];
+      next = ++q < Q.nsnap ? snap_step(Q.snaps, q) : -1;
+    }
   };
-  publish();
-  batch_accel<false, false>(lane, base, cnt, maxcnt, live, sx[wl], sy[wl], sz[wl], sm[wl], nullptr, nullptr,
-                            nullptr, nullptr, X, V, mi, P.G, P.ic2, P.ic, P.pnf, P.soft, Divisor64{}, false, A);
-  wave_sync();
+  accel();
   store(0);
-  const double dt = P.h[0];
-  double pending = 0.0;
-  for (int64_t s = 0; s < P.nsteps; ++s) {
-    kick_drift_reg(X, V, A, pending, dt);
-    publish();
-    batch_accel<false, false>(lane, base, cnt, maxcnt, live, sx[wl], sy[wl], sz[wl], sm[wl], nullptr, nullptr,
-                              nullptr, nullptr, X, V, mi, P.G, P.ic2, P.ic, P.pnf, P.soft, Divisor64{}, false, A);
-    wave_sync();
-    pending = dt;
+  // kick-drift-kick, the kicks between two drifts as one
+  const double dt = Q.dt, gdt = P.G * dt;
+  double kick = 0.5 * gdt;
+  for (int64_t s = 0; s < Q.nsteps; ++s) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      V[c] = fma(kick, a[c], V[c]);
+      X[c] = fma(dt, V[c], X[c]);
+    }
+    accel();
+    kick = gdt;
     store(s + 1);
   }
-  if (P.nsteps > 0) kick_reg(V, A, pending);
   if (live)
     for (int c = 0; c < 3; ++c) {
       P.x[3 * (size_t)b + c] = X[c];
-      P.v[3 * (size_t)b + c] = V[c];
-      P.a[3 * (size_t)b + c] = A[c];
+      P.v[3 * (size_t)b + c] = Q.nsteps > 0 ? fma(0.5 * gdt, a[c], V[c]) : V[c];
+      P.a[3 * (size_t)b + c] = P.G * a[c];
     }
 }
 
-__global__ __launch_bounds__(256) void k_batch_traj_bwd(BatchArgs P, const double* __restrict__ traj,
-                                                        int64_t nbodies, int64_t nsteps, double dt,
-                                                        const double* __restrict__ gsnap,
-                                                        const int64_t* __restrict__ snaps, int nsnap,
-                                                        double* __restrict__ out) {
-  __shared__ double sx[kBatchMaxWpb][64], sy[kBatchMaxWpb][64], sz[kBatchMaxWpb][64], sm[kBatchMaxWpb][64];
-  __shared__ double swx[kBatchMaxWpb][64], swy[kBatchMaxWpb][64], swz[kBatchMaxWpb][64];
+// Also puts the initial state back.
+template <bool TRIPLES>
+__global__ __launch_bounds__(256) void k_batch_traj_bwd(BatchArgs P, TrajArgs Q) {
+  constexpr int kLds = TRIPLES ? 1 : kBatchMaxWpb;
+  __shared__ double4 sbody[kLds][64];  // position, mass
+  __shared__ double4 sw[kLds][64];
+  __shared__ double4 spart[kLds][64];
   const int wl = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wave = blockIdx.x * (blockDim.x >> 6) + wl;
-  if (wave >= P.nwaves) return;
-  const int slot = wave * 64 + lane;
-  const int b = P.lane_body[slot];
-  const int seg = P.lane_seg[slot];
-  const int base = seg >> 8, cnt = seg & 255;
-  const int maxcnt = P.wave_max[wave];
+  if (wave >= Q.nwaves) return;
+  const TrajLane me = traj_lane<TRIPLES>(P, Q.nbodies, wave, lane);
+  const int b = me.b, base = me.base, cnt = me.cnt;
   const bool live = b >= 0;
   const double mk = live ? P.m[b] : 0.0;
-  sm[wl][lane] = mk;
   double lx[3] = {0.0, 0.0, 0.0}, lv[3] = {0.0, 0.0, 0.0}, lm = 0.0;
-  int q = nsnap - 1;
-  if (q >= 0 && snaps[q] == nsteps) {
+  int q = Q.nsnap - 1;
+  int64_t next = q >= 0 ? snap_step(Q.snaps, q) : -1;
+  auto snapshot = [&](int64_t s) {  // dL/dx at step s
+    if (s != next) return;
     if (live)
-      for (int c = 0; c < 3; ++c) lx[c] = gsnap[((size_t)q * nbodies + b) * 3 + c];
-    --q;
-  }
-  for (int64_t s = nsteps - 1; s >= 0; --s) {
-    const double cw = (s > 0) ? dt : 0.5 * dt;
-    double w[3], X[3];
+      for (int c = 0; c < 3; ++c) lx[c] += Q.snap_pos[((size_t)q * Q.nbodies + b) * 3 + c];
+    next = --q >= 0 ? snap_step(Q.snaps, q) : -1;
+  };
+  const double mnext = quad_next(mk);
+  const CyclicPair first = cyclic_pair(lane, base, cnt, 1, live);
+  // J^T w and M^T w of the pair over G c_s (w = lv) for body k = this lane's,
+  // with u and d; both change sign for the partner, whose M^T w has the other w
+  double g[3], gm;
+  auto pair = [&](const CyclicPair& p, const double* X) {
+    const double4 o = TRIPLES ? make_double4(quad_next(X[0]), quad_next(X[1]), quad_next(X[2]), mnext)
+                              : sbody[wl][p.to];
+    const double4 wo = TRIPLES ? make_double4(quad_next(lv[0]), quad_next(lv[1]), quad_next(lv[2]), 0.0)
+                               : sw[wl][p.to];
+    const double d[3] = {o.x - X[0], o.y - X[1], o.z - X[2]};
+    const double r2 = fma(d[0], d[0], fma(d[1], d[1], fma(d[2], d[2], P.soft)));
+    const double inv = rsqrt64_cubic(r2);
+    const double inv2 = p.own ? inv * inv : 0.0;
+    const double inv3 = p.own ? inv2 * inv : 0.0;
+    const double u[3] = {fma(mk, wo.x, -(o.w * lv[0])), fma(mk, wo.y, -(o.w * lv[1])), fma(mk, wo.z, -(o.w * lv[2]))};
+    const double du = 3.0 * inv2 * fma(d[0], u[0], fma(d[1], u[1], d[2] * u[2]));
+    double t[3];
+#pragma unroll
     for (int c = 0; c < 3; ++c) {
-      lv[c] = lv[c] + dt * lx[c];
-      w[c] = cw * lv[c];
-      X[c] = live ? traj[((size_t)s * nbodies + b) * 3 + c] : 0.0;
+      t[c] = inv3 * fma(-d[c], du, u[c]);
+      g[c] += t[c];
     }
-    sx[wl][lane] = X[0];
-    sy[wl][lane] = X[1];
-    sz[wl][lane] = X[2];
-    swx[wl][lane] = w[0];
-    swy[wl][lane] = w[1];
-    swz[wl][lane] = w[2];
-    wave_sync();
-    double gx = 0.0, gy = 0.0, gz = 0.0, gm = 0.0;
-    for (int j = 0; j < maxcnt; ++j) {
-      const int src = min(base + j, 63);
-      const bool valid = live && j < cnt && src != lane;
-      const double dx = sx[wl][src] - X[0], dy = sy[wl][src] - X[1], dz = sz[wl][src] - X[2];
-      const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, P.soft)));
-      const double inv = rsqrt64(valid ? r2 : 1.0);
-      const double inv3 = valid ? inv * inv * inv : 0.0;
-      const double inv5 = inv3 * inv * inv;
-      const double mj = sm[wl][src];
-      const double wjx = swx[wl][src], wjy = swy[wl][src], wjz = swz[wl][src];
-      const double ux = mk * wjx - mj * w[0], uy = mk * wjy - mj * w[1], uz = mk * wjz - mj * w[2];
-      const double du = dx * ux + dy * uy + dz * uz;
-      gx += ux * inv3 - 3.0 * dx * du * inv5;
-      gy += uy * inv3 - 3.0 * dy * du * inv5;
-      gz += uz * inv3 - 3.0 * dz * du * inv5;
-      gm -= (wjx * dx + wjy * dy + wjz * dz) * inv3;
+    const double tm = inv3 * fma(d[0], lv[0], fma(d[1], lv[1], d[2] * lv[2]));
+    gm = fma(-inv3, fma(d[0], wo.x, fma(d[1], wo.y, d[2] * wo.z)), gm);
+    if (TRIPLES) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) g[c] -= quad_prev(t[c]);
+      gm += quad_prev(tm);
+      return;
     }
+    spart[wl][lane] = make_double4(t[0], t[1], t[2], tm);
     wave_sync();
-    lx[0] += P.G * gx;
-    lx[1] += P.G * gy;
-    lx[2] += P.G * gz;
-    lm += P.G * gm;
-    if (q >= 0 && snaps[q] == s) {
-      if (live)
-        for (int c = 0; c < 3; ++c) lx[c] += gsnap[((size_t)q * nbodies + b) * 3 + c];
-      --q;
+    const double4 q = spart[wl][p.from];
+    g[0] -= q.x;
+    g[1] -= q.y;
+    g[2] -= q.z;
+    gm += q.w;
+    wave_sync();
+  };
+  const double dt = Q.dt, gdt = P.G * dt;
+  auto step = [&](int64_t s, const double* X) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) lv[c] = fma(dt, lx[c], lv[c]);
+    if (!TRIPLES) {
+      sbody[wl][lane] = make_double4(X[0], X[1], X[2], mk);
+      sw[wl][lane] = make_double4(lv[0], lv[1], lv[2], 0.0);
+      wave_sync();
+    }
+    g[0] = g[1] = g[2] = gm = 0.0;
+    pair(first, X);
+    for (int r = 2; r <= me.rounds; ++r) pair(cyclic_pair(lane, base, cnt, r, live), X);
+    const double gc = s > 0 ? gdt : 0.5 * gdt;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) lx[c] = fma(gc, g[c], lx[c]);
+    lm = fma(gc, gm, lm);
+    snapshot(s);
+  };
+  double ahead[kTrajAhead][3];
+  auto load = [&](int64_t s, double* X) {
+    const size_t at = ((size_t)(s > 0 ? s : 0) * Q.nbodies + (live ? b : 0)) * 3;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) X[c] = Q.traj[at + c];
+  };
+#pragma unroll
+  for (int k = 0; k < kTrajAhead; ++k) load(Q.nsteps - 1 - k, ahead[k]);
+  snapshot(Q.nsteps);
+  int64_t s = Q.nsteps - 1;
+  for (; s >= kTrajAhead - 1; s -= kTrajAhead) {
+#pragma unroll
+    for (int k = 0; k < kTrajAhead; ++k) {
+      step(s - k, ahead[k]);
+      load(s - k - kTrajAhead, ahead[k]);
     }
   }
+#pragma unroll
+  for (int k = 0; k < kTrajAhead - 1; ++k)
+    if (s - k >= 0) step(s - k, ahead[k]);
   if (live) {
     for (int c = 0; c < 3; ++c) {
-      out[3 * (size_t)b + c] = lx[c];
-      out[3 * (size_t)nbodies + 3 * (size_t)b + c] = lv[c];
+      const size_t i = 3 * (size_t)b + c;
+      Q.out[i] = lx[c];
+      Q.out[3 * (size_t)Q.nbodies + i] = lv[c];
+      P.x[i] = Q.traj[i];
+      P.v[i] = Q.v0[i];
     }
-    out[6 * (size_t)nbodies + b] = lm;
+    Q.out[6 * (size_t)Q.nbodies + b] = lm;
   }
 }
 
@@ -1159,21 +1324,20 @@ int batch_traj_forward(aster_ctx* c, double dt, int64_t nsteps, int32_t nsnap, c
   const size_t nb3 = (size_t)3 * B.nbodies;
   if ((double)(nsteps + 1) * nb3 * 8.0 > 64e9) return fail(c, ASTER_ERR_CAPACITY, "trajectory would exceed 64 GB");
   ASTER_HIP(c, B.traj.reserve((size_t)(nsteps + 1) * nb3));
-  ASTER_HIP(c, B.x0.reserve(nb3));
   ASTER_HIP(c, B.v0.reserve(nb3));
-  ASTER_HIP(c, hipMemcpyAsync(B.x0.p, B.x.p, nb3 * 8, hipMemcpyDeviceToDevice, c->stream));
-  ASTER_HIP(c, hipMemcpyAsync(B.v0.p, B.v.p, nb3 * 8, hipMemcpyDeviceToDevice, c->stream));
+  ASTER_HIP(c, B.tgrad.reserve(std::max<size_t>(1, nsnap * nb3)));
+  ASTER_HIP(c, B.tsnap.reserve(std::max(1, nsnap)));
+  if (nsnap > 0) ASTER_HIP(c, hipMemcpyAsync(B.tsnap.p, snaps, nsnap * 8, hipMemcpyHostToDevice, c->stream));
   const double h[3] = {dt, 0.0, 0.0};
   const BatchArgs P = make_args(c, nsteps, 1, h, 0);
-  const int wpb = B.waves_per_block;
-  hipLaunchKernelGGL(k_batch_traj_fwd, dim3((P.nwaves + wpb - 1) / wpb), dim3(64 * wpb), 0, c->stream, P, B.traj.p,
-                     B.nbodies);
+  const TrajShape t = traj_shape(B);
+  const TrajArgs Q{B.traj.p, B.v0.p, B.tsnap.p, nsnap, B.tgrad.p, B.nbodies, nsteps, dt, nullptr, t.nwaves};
+  hipLaunchKernelGGL(t.triples ? k_batch_traj_fwd<true> : k_batch_traj_fwd<false>,
+                     dim3((t.nwaves + t.wpb - 1) / t.wpb), dim3(64 * t.wpb), 0, c->stream, P, Q);
   ASTER_HIP(c, hipGetLastError());
   B.a_valid = true;
-  if (snap_pos)
-    for (int q = 0; q < nsnap; ++q)
-      ASTER_HIP(c, hipMemcpyAsync(snap_pos + (size_t)q * nb3, B.traj.p + (size_t)snaps[q] * nb3, nb3 * 8,
-                                  hipMemcpyDeviceToHost, c->stream));
+  if (snap_pos && nsnap > 0)
+    ASTER_HIP(c, hipMemcpyAsync(snap_pos, B.tgrad.p, nsnap * nb3 * 8, hipMemcpyDeviceToHost, c->stream));
   ASTER_HIP(c, hipStreamSynchronize(c->stream));
   B.traj_snaps.assign(snaps, snaps + nsnap);
   B.traj_steps = nsteps;
@@ -1188,25 +1352,20 @@ int batch_traj_backward(aster_ctx* c, const double* gsnap, double* gx, double* g
   const int nsnap = (int)B.traj_snaps.size();
   if (nsnap > 0 && !gsnap) return fail(c, ASTER_ERR_INVALID, "snapshot gradients required");
   const size_t nb3 = (size_t)3 * B.nbodies;
-  ASTER_HIP(c, B.tgrad.reserve(std::max<size_t>(1, nsnap * nb3)));
-  ASTER_HIP(c, B.tsnap.reserve(std::max(1, nsnap)));
   ASTER_HIP(c, B.tout.reserve(7 * (size_t)B.nbodies));
-  if (nsnap > 0) {
+  if (nsnap > 0)
     ASTER_HIP(c, hipMemcpyAsync(B.tgrad.p, gsnap, nsnap * nb3 * 8, hipMemcpyHostToDevice, c->stream));
-    ASTER_HIP(c, hipMemcpyAsync(B.tsnap.p, B.traj_snaps.data(), nsnap * 8, hipMemcpyHostToDevice, c->stream));
-  }
   const double h0[3] = {0.0, 0.0, 0.0};
   const BatchArgs P = make_args(c, 0, 1, h0, 0);
-  const int wpb = B.waves_per_block;
-  hipLaunchKernelGGL(k_batch_traj_bwd, dim3((P.nwaves + wpb - 1) / wpb), dim3(64 * wpb), 0, c->stream, P, B.traj.p,
-                     B.nbodies, B.traj_steps, B.traj_dt, B.tgrad.p, B.tsnap.p, nsnap, B.tout.p);
+  const TrajShape t = traj_shape(B);
+  const TrajArgs Q{B.traj.p, B.v0.p, B.tsnap.p, nsnap, B.tgrad.p, B.nbodies, B.traj_steps, B.traj_dt, B.tout.p,
+                   t.nwaves};
+  hipLaunchKernelGGL(t.triples ? k_batch_traj_bwd<true> : k_batch_traj_bwd<false>,
+                     dim3((t.nwaves + t.wpb - 1) / t.wpb), dim3(64 * t.wpb), 0, c->stream, P, Q);
   ASTER_HIP(c, hipGetLastError());
   if (gx) ASTER_HIP(c, hipMemcpyAsync(gx, B.tout.p, nb3 * 8, hipMemcpyDeviceToHost, c->stream));
   if (gv) ASTER_HIP(c, hipMemcpyAsync(gv, B.tout.p + nb3, nb3 * 8, hipMemcpyDeviceToHost, c->stream));
   if (gm) ASTER_HIP(c, hipMemcpyAsync(gm, B.tout.p + 2 * nb3, B.nbodies * 8, hipMemcpyDeviceToHost, c->stream));
-  // restore the initial state
-  ASTER_HIP(c, hipMemcpyAsync(B.x.p, B.x0.p, nb3 * 8, hipMemcpyDeviceToDevice, c->stream));
-  ASTER_HIP(c, hipMemcpyAsync(B.v.p, B.v0.p, nb3 * 8, hipMemcpyDeviceToDevice, c->stream));
   ASTER_HIP(c, hipStreamSynchronize(c->stream));
   B.a_valid = false;
   B.traj_ready = false;
@@ -1224,9 +1383,11 @@ int aster_batch_set(aster_ctx* c, int64_t nsys, const int64_t* offsets, const do
   if (!c) return ASTER_ERR_INVALID;
   if (nsys < 1 || !offsets || !pos || !mass) return fail(c, ASTER_ERR_INVALID, "need nsys >= 1, offsets, pos, mass");
   if (offsets[0] != 0) return fail(c, ASTER_ERR_INVALID, "offsets[0] must be 0");
+  bool triples = true;
   for (int64_t s = 0; s < nsys; ++s) {
     const int64_t k = offsets[s + 1] - offsets[s];
     if (k < 1 || k > 64) return fail(c, ASTER_ERR_CAPACITY, "each system needs 1..64 bodies");
+    triples = triples && k == 3;
   }
   const int64_t nb = offsets[nsys];
   if (nb > (int64_t(1) << 28)) return fail(c, ASTER_ERR_CAPACITY, "at most 2^28 bodies per batch");
@@ -1242,6 +1403,7 @@ int aster_batch_set(aster_ctx* c, int64_t nsys, const int64_t* offsets, const do
   B.nsys = nsys;
   B.nbodies = nb;
   B.offsets.assign(offsets, offsets + nsys + 1);
+  B.triples = triples;
   ASTER_HIP(c, B.x.reserve(3 * nb));
   ASTER_HIP(c, B.v.reserve(3 * nb));
   ASTER_HIP(c, B.a.reserve(3 * nb));

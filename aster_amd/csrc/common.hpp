@@ -45,6 +45,7 @@ enum { BHC_INTERACTIONS = 0, BHC_VISITS = 1, BHC_COUNT = 4 };
 
 struct BatchState {
   int64_t nsys = 0, nbodies = 0;
+  bool triples = false;              // every system has three bodies
   std::vector<int64_t> offsets;      // host copy, nsys+1
   DBuf<double> x, v, a, m;           // AoS-d3 over bodies (x, v, a), m per body
   DBuf<double> ebody;                // per-body energy terms [4][nbodies]
@@ -66,7 +67,7 @@ struct BatchState {
   double g_dt = 0.0, g_G = 0.0, g_c = 0.0, g_soft = -1.0;
   // Trajectory adjoint of the ensemble: positions at every step are kept.
   DBuf<double> traj;                 // (nsteps + 1) * 3 * nbodies, AoS-d3 per step
-  DBuf<double> x0, v0;               // initial state, restored after the backward pass
+  DBuf<double> v0;                   // initial velocities, put back by the backward pass
   DBuf<double> tgrad;                // snapshot gradients, nsnap * 3 * nbodies
   DBuf<double> tout;                 // gx, gv (AoS-d3) and gm per body
   DBuf<int64_t> tsnap;               // snapshot steps on the device

@@ -107,3 +107,27 @@ def test_group_traversal_pn_small_groups(ctx, orc, n, soft, flags):
     scale = np.linalg.norm(ref, axis=1)
     err = np.linalg.norm(part[1] - part[0] - ref, axis=1)
     assert np.all(err <= 1e-9 * np.maximum(scale, np.median(scale)) + 1e-15 * np.abs(part[1]).max())
+
+
+@pytest.mark.parametrize("sizes", [[1], [2], [3], [3] * 16, [3] * 50, [4] * 20, [1, 2, 3, 4, 5, 8, 21, 32, 33, 63, 64]])
+@pytest.mark.parametrize("snaps", [[1, 2, 7], [4], [9, 10]])
+def test_batch_gradient_against_oracle(ctx, orc, sizes, snaps):
+    """Odd and even systems, alone and packed, more and fewer steps than are loaded ahead: the bars of the three-body test."""
+    n, steps = sum(sizes), snaps[-1] + (len(snaps) == 3)
+    rng = np.random.default_rng(n)
+    pos, vel = rng.normal(size=(n, 3)), 0.1 * rng.normal(size=(n, 3))
+    mass = rng.uniform(0.5, 1.5, n)
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    ctx.set_params(G=1.3, softening=1e-2, precision=A.FP32)
+    ctx.batch_set(off, pos, vel, mass)
+    s = ctx.batch_traj_forward(1e-2, steps, snaps)
+    target = s + rng.normal(scale=1e-2, size=s.shape)
+    gsnap = 2.0 * (s - target)
+    got = ctx.batch_traj_backward(gsnap)
+    p, v = ctx.batch_get()
+    assert np.array_equal(p, pos) and np.array_equal(v, vel)
+    for a, b in zip(off[:-1], off[1:]):
+        loss, *ref = orc.traj_grad(pos[a:b], vel[a:b], mass[a:b], 1e-2, steps, np.array(snaps), target[:, a:b], G=1.3, soft=1e-2)
+        assert loss * (b - a) * len(snaps) == pytest.approx(((s - target)[:, a:b] ** 2).sum(), rel=1e-10)
+        for g, r in zip(got, ref):
+            assert np.linalg.norm(g[a:b] - r * (b - a) * len(snaps)) <= 1e-8 * np.linalg.norm(r) * (b - a) * len(snaps)
