@@ -82,6 +82,50 @@ __device__ __forceinline__ void batch_separations(int first, const double* lx, c
   }
 }
 
+// The accelerations f of the lane's body by sources j0 .. j0 + kU - 1 of its
+// system; 0 for a pair that does not count.
+template <bool PN, bool FAST>
+__device__ __forceinline__ void batch_exact_pairs(int lane, int base, int cnt, int j0, bool live, const double* lx,
+                                                  const double* ly, const double* lz, const double* lm,
+                                                  const double* lvx, const double* lvy, const double* lvz,
+                                                  const double* X, const double* V, const Divisor64& mi, double G,
+                                                  double ic, int pnf, double soft, double (*f)[3]) {
+#pragma clang fp contract(off)
+  double d[kU][3], inv[kU];
+  batch_separations<FAST>(base + j0, lx, ly, lz, X, soft, d, inv);
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    const int src = min(base + j0 + u, 63);
+    const double m2 = lm[src];
+    const double scal = G * m2 * mi.b * (inv[u] * inv[u]);
+    double n[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      n[c] = d[u][c] * inv[u];
+      f[u][c] = n[c] * scal;
+    }
+    if (PN) {
+      pn_add64(pnf, mi.b, m2, V[0], V[1], V[2], lvx[src], lvy[src], lvz[src], inv[u], -n[0], -n[1], -n[2], G, ic,
+               f[u][0], f[u][1], f[u][2]);
+    }
+  }
+  if (FAST && !PN) {  // the post-Newtonian terms have no bounds of their own
+    div64_fast<3 * kU>(&f[0][0], mi);
+  } else {
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) f[u][c] = f[u][c] / mi.b;
+  }
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    const int src = min(base + j0 + u, 63);
+    const bool valid = live && j0 + u < cnt && src != lane;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) f[u][c] = valid ? f[u][c] : 0.0;
+  }
+}
+
 template <bool PN, bool FAST>
 __device__ __forceinline__ void batch_exact(int lane, int base, int cnt, int maxcnt, bool live, const double* lx,
                                             const double* ly, const double* lz, const double* lm, const double* lvx,
@@ -91,42 +135,76 @@ __device__ __forceinline__ void batch_exact(int lane, int base, int cnt, int max
 #pragma clang fp contract(off)
   double a[3] = {0.0, 0.0, 0.0};
   for (int j0 = 0; j0 < maxcnt; j0 += kU) {
-    double d[kU][3], inv[kU], f[kU][3];
-    batch_separations<FAST>(base + j0, lx, ly, lz, X, soft, d, inv);
+    double f[kU][3];
+    batch_exact_pairs<PN, FAST>(lane, base, cnt, j0, live, lx, ly, lz, lm, lvx, lvy, lvz, X, V, mi, G, ic, pnf, soft,
+                                f);
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int src = min(base + j0 + u, 63);
-      const double m2 = lm[src];
-      const double scal = G * m2 * mi.b * (inv[u] * inv[u]);
-      double n[3];
+    for (int u = 0; u < kU; ++u)
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        n[c] = d[u][c] * inv[u];
-        f[u][c] = n[c] * scal;
-      }
-      if (PN) {
-        pn_add64(pnf, mi.b, m2, V[0], V[1], V[2], lvx[src], lvy[src], lvz[src], inv[u], -n[0], -n[1], -n[2], G, ic,
-                 f[u][0], f[u][1], f[u][2]);
-      }
-    }
-    if (FAST && !PN) {  // the post-Newtonian terms have no bounds of their own
-      div64_fast<3 * kU>(&f[0][0], mi);
-    } else {
-#pragma unroll
-      for (int u = 0; u < kU; ++u)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) f[u][c] = f[u][c] / mi.b;
-    }
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int src = min(base + j0 + u, 63);
-      const bool valid = live && j0 + u < cnt && src != lane;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) a[c] += valid ? f[u][c] : 0.0;
-    }
+      for (int c = 0; c < 3; ++c) a[c] += f[u][c];
   }
 #pragma unroll
   for (int c = 0; c < 3; ++c) A[c] = a[c];
+}
+
+// Fast mode: the parts of a pair's acceleration, f d (d) and, with 1PN terms,
+// g k (g): {f, d, k, g}.
+template <bool PN>
+constexpr int kFastVals = PN ? 8 : 4;
+
+template <bool PN>
+__device__ __forceinline__ void batch_fast_pair(int src, bool valid, const double* lx, const double* ly,
+                                                const double* lz, const double* lm, const double* lvx,
+                                                const double* lvy, const double* lvz, const double* lv22,
+                                                const double* X, const double* V, double v11, double g5m1, double G,
+                                                double ic2, double soft, double* q) {
+  const double m2 = lm[src];
+  const double dx = lx[src] - X[0], dy = ly[src] - X[1], dz = lz[src] - X[2];
+  const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, soft)));
+  // one Newton step: 1/r to 4.1e-15 (two steps, 1.4e-16, cost 4 more
+  // instructions per pair; the exact mode divides as the reference does)
+  const double inv = rsqrt64_n<1>(valid ? r2 : 1.0);
+  const double inv2 = inv * inv;
+  // a pair that does not count gets G m2 = 0 (its inv is finite), so
+  // both force terms vanish without selects of their own
+  const double gm2 = valid ? G * m2 : 0.0;
+  q[0] = gm2 * (inv2 * inv);
+  q[1] = dx;
+  q[2] = dy;
+  q[3] = dz;
+  if constexpr (PN) {
+    const double v2x = lvx[src], v2y = lvy[src], v2z = lvz[src];
+    // get_pn1 (tool_chain_impl.cpp:110-118) with n = (x1 - x2)/r, the same
+    // terms grouped for fused multiply-adds:
+    //   G m2/r^2 [n (-v1^2 - 2 v2^2 + 4 v1.v2 + 3/2 (n.v2)^2 + (5 G m1 + 4 G m2)/r)
+    //             + (v1 - v2)(4 n.v1 - 3 n.v2)]
+    const double nx = -dx * inv, ny = -dy * inv, nz = -dz * inv;
+    const double nv1 = fma(nx, V[0], fma(ny, V[1], nz * V[2]));
+    const double nv2 = fma(nx, v2x, fma(ny, v2y, nz * v2z));
+    const double v12 = fma(V[0], v2x, fma(V[1], v2y, V[2] * v2z));
+    const double v22 = lv22[src];  // |v2|^2, formed once per body when published
+    double sc = fma(4.0, v12, -v11);
+    sc = fma(-2.0, v22, sc);
+    sc = fma(1.5 * nv2, nv2, sc);
+    sc = fma(fma(4.0 * G, m2, g5m1), inv, sc);
+    const double t = fma(4.0, nv1, -3.0 * nv2);
+    q[4] = gm2 * inv2 * ic2;
+    q[5] = fma(nx, sc, (V[0] - v2x) * t);
+    q[6] = fma(ny, sc, (V[1] - v2y) * t);
+    q[7] = fma(nz, sc, (V[2] - v2z) * t);
+  }
+}
+
+template <bool PN>
+__device__ __forceinline__ void batch_fast_add(const double* q, double& ax, double& ay, double& az) {
+  ax = fma(q[0], q[1], ax);
+  ay = fma(q[0], q[2], ay);
+  az = fma(q[0], q[3], az);
+  if constexpr (PN) {
+    ax = fma(q[5], q[4], ax);
+    ay = fma(q[6], q[4], ay);
+    az = fma(q[7], q[4], az);
+  }
 }
 
 template <bool PN, bool EXACT>
@@ -148,53 +226,14 @@ __device__ __forceinline__ void batch_accel(int lane, int base, int cnt, int max
   const double v11 = V[0] * V[0] + V[1] * V[1] + V[2] * V[2];
   const double g5m1 = 5.0 * G * mi;
   // Four sources per iteration: independent pair forces, sums still taken
-  // one by one in j order (the exact mode's results are unchanged)
+  // one by one in j order
 #pragma unroll 4
   for (int j = 0; j < maxcnt; ++j) {
     const int src = min(base + j, 63);
     const bool valid = live && j < cnt && src != lane;
-    const double x2 = lx[src], y2 = ly[src], z2 = lz[src], m2 = lm[src];
-    double v2x = 0.0, v2y = 0.0, v2z = 0.0;
-    if (PN) {
-      v2x = lvx[src];
-      v2y = lvy[src];
-      v2z = lvz[src];
-    }
-    {
-      const double dx = x2 - X[0], dy = y2 - X[1], dz = z2 - X[2];
-      const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, soft)));
-      // one Newton step: 1/r to 4.1e-15 (two steps, 1.4e-16, cost 4 more
-      // instructions per pair; the exact mode divides as the reference does)
-      const double inv = rsqrt64_n<1>(valid ? r2 : 1.0);
-      const double inv2 = inv * inv;
-      // a pair that does not count gets G m2 = 0 (its inv is finite), so
-      // both force terms vanish without selects of their own
-      const double gm2 = valid ? G * m2 : 0.0;
-      const double f = gm2 * (inv2 * inv);
-      ax = fma(f, dx, ax);
-      ay = fma(f, dy, ay);
-      az = fma(f, dz, az);
-      if (PN) {
-        // get_pn1 (tool_chain_impl.cpp:110-118) with n = (x1 - x2)/r, the same
-        // terms grouped for fused multiply-adds:
-        //   G m2/r^2 [n (-v1^2 - 2 v2^2 + 4 v1.v2 + 3/2 (n.v2)^2 + (5 G m1 + 4 G m2)/r)
-        //             + (v1 - v2)(4 n.v1 - 3 n.v2)]
-        const double nx = -dx * inv, ny = -dy * inv, nz = -dz * inv;
-        const double nv1 = fma(nx, V[0], fma(ny, V[1], nz * V[2]));
-        const double nv2 = fma(nx, v2x, fma(ny, v2y, nz * v2z));
-        const double v12 = fma(V[0], v2x, fma(V[1], v2y, V[2] * v2z));
-        const double v22 = lv22[src];  // |v2|^2, formed once per body when published
-        double sc = fma(4.0, v12, -v11);
-        sc = fma(-2.0, v22, sc);
-        sc = fma(1.5 * nv2, nv2, sc);
-        sc = fma(fma(4.0 * G, m2, g5m1), inv, sc);
-        const double t = fma(4.0, nv1, -3.0 * nv2);
-        const double k = gm2 * inv2 * ic2;
-        ax = fma(fma(nx, sc, (V[0] - v2x) * t), k, ax);
-        ay = fma(fma(ny, sc, (V[1] - v2y) * t), k, ay);
-        az = fma(fma(nz, sc, (V[2] - v2z) * t), k, az);
-      }
-    }
+    double q[kFastVals<PN>];
+    batch_fast_pair<PN>(src, valid, lx, ly, lz, lm, lvx, lvy, lvz, lv22, X, V, v11, g5m1, G, ic2, soft, q);
+    batch_fast_add<PN>(q, ax, ay, az);
   }
   A[0] = ax;
   A[1] = ay;
@@ -283,10 +322,11 @@ __device__ __forceinline__ void batch_eih(int lane, int base, int cnt, int maxcn
   A[2] = az;
 }
 
+template <int N = 3>
 __device__ __forceinline__ void kick_drift_reg(double* X, double* V, const double* A, double dt_prev, double dt) {
 #pragma clang fp contract(off)
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
+  for (int c = 0; c < N; ++c) {
     double vc = V[c];
     if (dt_prev != 0.0) vc = vc + 0.5 * A[c] * dt_prev;
     X[c] = X[c] + (vc * dt + 0.5 * A[c] * dt * dt);
@@ -294,10 +334,11 @@ __device__ __forceinline__ void kick_drift_reg(double* X, double* V, const doubl
   }
 }
 
+template <int N = 3>
 __device__ __forceinline__ void kick_reg(double* V, const double* A, double dt) {
 #pragma clang fp contract(off)
 #pragma unroll
-  for (int c = 0; c < 3; ++c) V[c] = V[c] + 0.5 * A[c] * dt;
+  for (int c = 0; c < N; ++c) V[c] = V[c] + 0.5 * A[c] * dt;
 }
 
 template <bool PN, bool EXACT>
@@ -411,6 +452,136 @@ __global__ __launch_bounds__(256) void k_batch(BatchArgs P) {
       P.a[3 * (size_t)b + c] = A[c];
     }
   }
+}
+
+// Few wavefronts of systems (team_size): W worker wavefronts form a wavefront's
+// pair forces, kU sources each at a time, and pass them through LDS to three
+// adding wavefronts, one per coordinate, which sum them in j order and advance
+// the bodies; the workers are a chunk of W kU sources ahead. Same operations as
+// batch_accel in the same order, so the same bits (the fast mode passes the
+// factors of its last fused multiply-adds).
+template <bool PN, bool EXACT, int W>
+__global__ __launch_bounds__(64 * (W + 3)) void k_batch_team(BatchArgs P) {
+#pragma clang fp contract(off)
+  constexpr int kChunk = W * kU;
+  constexpr int kVals = EXACT ? 3 : kFastVals<PN>;
+  __shared__ double planes[PN ? 7 : 4][64];
+  __shared__ double v22[PN && !EXACT ? 64 : 1];
+  __shared__ double force[2][kChunk][kVals][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const bool adder = w >= W;
+  const int ax = __builtin_amdgcn_readfirstlane(adder ? w - W : 0);  // an adder's coordinate
+  const int slot = blockIdx.x * 64 + lane;
+  const int b = P.lane_body[slot];
+  const int seg = P.lane_seg[slot];
+  const int base = seg >> 8, cnt = seg & 255;
+  const int maxcnt = __builtin_amdgcn_readfirstlane(P.wave_max[blockIdx.x]);
+  const bool live = b >= 0;
+  const double mi = live ? P.m[b] : 0.0;
+  double x = 0.0, v = 0.0, a = 0.0;  // adder: its coordinate of the body
+  const size_t at = 3 * (size_t)(live ? b : 0) + ax;
+  if (live && adder) {
+    x = P.x[at];
+    v = P.v[at];
+    a = P.a[at];
+  }
+  double X[3] = {0.0, 0.0, 0.0}, V[3] = {0.0, 0.0, 0.0};  // worker: the body
+  if (w == 0) planes[3][lane] = mi;
+  const Divisor64 md = divisor64(EXACT && live ? mi : 1.0);
+  const bool ranges = EXACT && __all(!live || mass_in_range64(mi)) && law_in_range64(P.G, P.soft);
+  // sources past maxcnt add 0, so that a chunk always has the same length
+  auto work = [&](int j0, bool fast, double (*out)[kVals][64]) {
+    double f[kU][kVals] = {};
+    const double* p = &planes[0][0];
+    const double* vx = PN ? p + 4 * 64 : p;
+    const double* vy = PN ? p + 5 * 64 : p;
+    const double* vz = PN ? p + 6 * 64 : p;
+    if constexpr (EXACT) {
+      if (j0 < maxcnt && fast)
+        batch_exact_pairs<PN, true>(lane, base, cnt, j0, live, p, p + 64, p + 128, p + 192, vx, vy, vz, X, V, md, P.G,
+                                    P.ic, P.pnf, P.soft, f);
+      else if (j0 < maxcnt)
+        batch_exact_pairs<PN, false>(lane, base, cnt, j0, live, p, p + 64, p + 128, p + 192, vx, vy, vz, X, V, md, P.G,
+                                     P.ic, P.pnf, P.soft, f);
+    } else if (j0 < maxcnt) {
+      const double v11 = V[0] * V[0] + V[1] * V[1] + V[2] * V[2];
+      const double g5m1 = 5.0 * P.G * mi;
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const int src = min(base + j0 + u, 63);
+        batch_fast_pair<PN>(src, live && j0 + u < cnt && src != lane, p, p + 64, p + 128, p + 192, vx, vy, vz, v22, X,
+                            V, v11, g5m1, P.G, P.ic2, P.soft, f[u]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+#pragma unroll
+      for (int c = 0; c < kVals; ++c) out[u][c][lane] = f[u][c];
+  };
+  // the adders' bodies to the workers, then the accelerations to the adders
+  auto accel = [&]() {
+    if (adder) {
+      planes[ax][lane] = x;
+      if (PN) planes[4 + ax][lane] = v;
+    }
+    __syncthreads();
+    if (!adder) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        X[c] = planes[c][lane];
+        if (PN) V[c] = planes[4 + c][lane];
+      }
+    }
+    if (PN && !EXACT) {
+      if (w == 0) v22[lane] = fma(V[0], V[0], fma(V[1], V[1], V[2] * V[2]));
+      __syncthreads();
+    }
+    double sum = 0.0;
+    auto add = [&](int j0) {
+      const auto& f = force[(j0 / kChunk) & 1];
+#pragma unroll
+      for (int u = 0; u < kChunk; ++u) {
+        if constexpr (EXACT) {
+          sum += f[u][ax][lane];
+        } else {
+          sum = fma(f[u][0][lane], f[u][1 + ax][lane], sum);
+          if constexpr (PN) sum = fma(f[u][5 + ax][lane], f[u][4][lane], sum);
+        }
+      }
+    };
+    const bool fast =
+        ranges && __all(!live || (coord_in_range64(X[0]) && coord_in_range64(X[1]) && coord_in_range64(X[2])));
+    int j0 = 0;
+    for (; j0 < maxcnt; j0 += kChunk) {
+      if (!adder) work(j0 + w * kU, fast, &force[(j0 / kChunk) & 1][w * kU]);
+      else if (j0 > 0) add(j0 - kChunk);
+      __syncthreads();
+    }
+    if (adder) {
+      add(j0 - kChunk);
+      a = sum;
+    }
+  };
+  if (P.init) accel();
+  double pending = 0.0;
+  for (int64_t s = 0; s < P.nsteps; ++s) {
+    for (int k = 0; k < P.nsub; ++k) {
+      const double h = P.h[k];
+      if (PN) {  // as k_batch
+        if (adder && pending != 0.0) kick_reg<1>(&v, &a, pending);
+        pending = 0.0;
+        accel();
+      }
+      if (adder) kick_drift_reg<1>(&x, &v, &a, pending, h);
+      accel();
+      pending = h;
+    }
+  }
+  if (!adder || !live) return;
+  if (P.nsteps > 0) kick_reg<1>(&v, &a, pending);
+  P.x[at] = x;
+  P.v[at] = v;
+  P.a[at] = a;
 }
 
 // Per-body energy terms: kinetic - 1/2 G m_i sum_j m_j / sqrt(r^2 + soft),
@@ -742,6 +913,7 @@ static int upload_plan(aster_ctx* c) {
         while (used + sz <= 64 && next[sz] < by_size[sz].size()) used = place(by_size[sz][next[sz]++], used);
   }
   B.nwaves = (int)wm.size();
+  B.max_size = *std::max_element(wm.begin(), wm.end());
   B.lane_slots = 0;
   for (int32_t mx : wm) B.lane_slots += 64 * (int64_t)mx;
   ASTER_HIP(c, B.lane_body.reserve(lb.size()));
@@ -793,6 +965,29 @@ static BatchArgs make_args(aster_ctx* c, int64_t nsteps, int nsub, const double*
   return P;
 }
 
+// Workers per wavefront of systems (k_batch_team), 0 for k_batch: while the
+// chip has more SIMDs than such wavefronts, their serial chains are what a step
+// waits for; small systems leave workers without sources. Leapfrog step, us,
+// k_batch / 4 / 8 workers, by the largest system and the wavefronts. Exact mode,
+// Newtonian: 64 bodies, 36 wavefronts 11.5 / 4.5 / 3.6, 520 12.0 / 6.3 / 6.3, 1045
+// 12.6 / 10.7 / 11.0, 4276 31.9 / 39 / 46; 16, 148 3.35 / 1.58 / 1.33, 604 3.47 /
+// 2.21 / 2.61, 1213 3.74 / 4.14; 8, 703 2.05 / 1.65; 4, 224 1.28 / 1.05, 448
+// 1.29 / 1.29. 1PN: 64, 520 58 / 39 / 33, 1045 67 / 67 / 57, 2126 107 / 124 / 105;
+// 32, 546 29.9 / 20.6 / 18.7, 1111 31.3 / 37 / 32.6; 16, 604 15.5 / 13.9 / 12.8; 8,
+// 350 8.2 / 6.4, 703 8.5 / 9.7; 4, 224 4.5 / 3.3, 448 4.6 / 6.3. Fast mode,
+// Newtonian: 64, 153 5.3 / 3.8 / 2.95, 520 5.4 / 5.2 / 5.3, 1045 6.2 / 8.6; 16, 148
+// 1.64 / 1.28 / 1.07, 604 1.70 / 1.77; 8, 172 1.04 / 0.86; 4 0.72 / 0.83. 1PN: 64,
+// 153 23.8 / 12.4, 520 24.2 / 20.3, 1045 25.7 / 35.6; 16, 296 6.6 / 4.4, 604 6.7 /
+// 7.6; 8, 172 3.5 / 2.6; 4, 110 2.1 / 2.4.
+static int team_size(int nwaves, int largest, bool pn, bool exact) {
+  int most;
+  if (exact) most = largest <= 4 ? 256 : !pn || largest > 32 ? 1024 : largest > 8 ? 768 : 512;
+  else most = largest <= 4 ? 0 : largest <= 8 ? 256 : 512;
+  if (nwaves > most) return 0;
+  const bool wide = exact && pn ? true : nwaves <= 256 && !pn;
+  return largest > 8 && wide ? 8 : 4;
+}
+
 static int launch_batch(aster_ctx* c, const BatchArgs& P) {
   if ((c->P.pn_flags & ASTER_EIH) && c->P.precision != ASTER_FP64)
     return fail(c, ASTER_ERR_INVALID, "ASTER_EIH in ensembles needs precision ASTER_FP64 (exact mode)");
@@ -800,7 +995,14 @@ static int launch_batch(aster_ctx* c, const BatchArgs& P) {
   const dim3 grid((P.nwaves + wpb - 1) / wpb), block(64 * wpb);
   const bool pn = (c->P.pn_flags & ASTER_PN_TERMS) != 0;
   const bool exact = c->P.precision == ASTER_FP64;
-  if (pn && exact) hipLaunchKernelGGL((k_batch<true, true>), grid, block, 0, c->stream, P);
+  const int team = P.pnf & ASTER_EIH ? 0 : team_size(P.nwaves, c->batch.max_size, pn, exact);
+  if (team) {
+    auto kern = exact ? (team == 8 ? (pn ? k_batch_team<true, true, 8> : k_batch_team<false, true, 8>)
+                                   : (pn ? k_batch_team<true, true, 4> : k_batch_team<false, true, 4>))
+                      : (pn ? k_batch_team<true, false, 4>
+                            : team == 8 ? k_batch_team<false, false, 8> : k_batch_team<false, false, 4>);
+    hipLaunchKernelGGL(kern, dim3(P.nwaves), dim3(64 * (team + 3)), 0, c->stream, P);
+  } else if (pn && exact) hipLaunchKernelGGL((k_batch<true, true>), grid, block, 0, c->stream, P);
   else if (pn) hipLaunchKernelGGL((k_batch<true, false>), grid, block, 0, c->stream, P);
   else if (exact) hipLaunchKernelGGL((k_batch<false, true>), grid, block, 0, c->stream, P);
   else hipLaunchKernelGGL((k_batch<false, false>), grid, block, 0, c->stream, P);

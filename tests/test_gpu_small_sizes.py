@@ -131,3 +131,29 @@ def test_batch_gradient_against_oracle(ctx, orc, sizes, snaps):
         assert loss * (b - a) * len(snaps) == pytest.approx(((s - target)[:, a:b] ** 2).sum(), rel=1e-10)
         for g, r in zip(got, ref):
             assert np.linalg.norm(g[a:b] - r * (b - a) * len(snaps)) <= 1e-8 * np.linalg.norm(r) * (b - a) * len(snaps)
+
+
+@pytest.mark.parametrize("largest", [2, 4, 5, 8, 9, 16, 17, 33, 64])
+@pytest.mark.parametrize("flags", [A.NEWTON, A.NEWTON | A.PN1])
+@pytest.mark.parametrize("precision", [A.FP64, A.FP32])
+def test_ensembles_same_bits_whatever_their_number(ctx, largest, flags, precision):
+    """A few systems, a few hundred wavefronts and more wavefronts than the teams take: the same systems give the same
+    bits (each rule's kernel against the one for large ensembles, itself tested against the oracle)."""
+    rng = np.random.default_rng(largest)
+    sizes = [largest] + [int(k) for k in rng.integers(1, largest + 1, 6)]
+    n = sum(sizes)
+    pos, vel = rng.normal(size=(n, 3)), 0.3 * rng.normal(size=(n, 3))
+    mass = 10.0 ** rng.uniform(-3.0, 0.0, n)
+    out = []
+    for waves in (1, 300, 450, 1100):
+        k = -(-64 * waves // n)
+        off = np.concatenate([[0], np.cumsum(sizes * k)])
+        ctx.set_params(G=1.2, softening=1e-3, c=20.0, pn_flags=flags, precision=precision)
+        ctx.batch_set(off, np.tile(pos, (k, 1)), np.tile(vel, (k, 1)), np.tile(mass, k))
+        ctx.batch_step(A.YOSHIDA4, 1e-2, 2)
+        ctx.batch_step(A.LEAPFROG, 1e-2, 3)
+        p, v = ctx.batch_get()
+        assert np.array_equal(p, np.tile(p[:n], (k, 1))) and np.array_equal(v, np.tile(v[:n], (k, 1))), waves
+        out.append((p[:n], v[:n]))
+    for p, v in out:
+        assert np.all(np.isfinite(p)) and np.array_equal(p, out[-1][0]) and np.array_equal(v, out[-1][1])
