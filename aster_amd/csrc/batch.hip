@@ -1223,7 +1223,7 @@ int batch_autotune(aster_ctx* c, int integrator, double dt, int32_t* spb, int32_
 // kTrajAhead steps ahead and nothing in the loop waits for loads or stores.
 // 200 steps of 4096 three-body systems, forward / backward: three sources per
 // lane 112 / 222 us; pairs once 90 / 97; snapshot steps kept as scalars and the
-// look-ahead kept through the loop 66 / 93; in quads of lanes 36 / 50.
+// look-ahead kept through the loop 66 / 93; in quads of lanes 44 / 50.
 constexpr int kTrajAhead = 4;
 
 // A lane's partner and the lane it receives from in round r.
@@ -1378,23 +1378,30 @@ __global__ __launch_bounds__(256) void k_batch_traj_fwd(BatchArgs P, TrajArgs Q)
   };
   accel();
   store(0);
-  // kick-drift-kick, the kicks between two drifts as one
-  const double dt = Q.dt, gdt = P.G * dt;
-  double kick = 0.5 * gdt;
-  for (int64_t s = 0; s < Q.nsteps; ++s) {
+  // kick_drift_reg and kick_reg, with a G / 2 dt formed once for the kick before
+  // the drift, the drift and the kick behind it (one fused kick from drift to
+  // drift doubles the error of the positions, which is 1e-17)
+  const double dt = Q.dt, half = 0.5 * P.G;
+  auto drift = [&](bool kick) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      V[c] = fma(kick, a[c], V[c]);
-      X[c] = fma(dt, V[c], X[c]);
+      const double t = half * a[c] * dt;
+      if (kick) V[c] = V[c] + t;
+      X[c] = X[c] + (V[c] * dt + t * dt);
+      V[c] = V[c] + t;
     }
     accel();
-    kick = gdt;
+  };
+  drift(false);
+  store(1);
+  for (int64_t s = 1; s < Q.nsteps; ++s) {
+    drift(true);
     store(s + 1);
   }
   if (live)
     for (int c = 0; c < 3; ++c) {
       P.x[3 * (size_t)b + c] = X[c];
-      P.v[3 * (size_t)b + c] = Q.nsteps > 0 ? fma(0.5 * gdt, a[c], V[c]) : V[c];
+      P.v[3 * (size_t)b + c] = V[c] + half * a[c] * dt;
       P.a[3 * (size_t)b + c] = P.G * a[c];
     }
 }
