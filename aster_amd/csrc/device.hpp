@@ -387,7 +387,8 @@ __device__ inline void kepler_drift64(double* q, double* u, double mu, double dt
   double lo = 0.0, hi;
   if (beta > 0.0) {
     const double sq = sqrt(beta);
-    dt = fmod(dt, 6.283185307179586 * mu / (beta * sq));
+    const double period = 6.283185307179586 * mu / (beta * sq);
+    if (!(fabs(dt) < period)) dt = fmod(dt, period);
     hi = sgn * (6.283185307179586 / sq);
   } else {
     hi = dt / r0;
