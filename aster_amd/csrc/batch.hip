@@ -147,51 +147,76 @@ __device__ __forceinline__ void batch_exact(int lane, int base, int cnt, int max
   for (int c = 0; c < 3; ++c) A[c] = a[c];
 }
 
-// Fast mode: the parts of a pair's acceleration, f d (d) and, with 1PN terms,
-// g k (g): {f, d, k, g}.
+// Fast mode. A body's record in LDS: {position, mass} and, with 1PN terms,
+// {velocity, |v|^2}. Behind a wavefront's 64 bodies lies a record of mass 0 far
+// away: a lane that has no more sources takes it, and both force terms vanish
+// without any selects on values.
+template <bool PN>
+constexpr int kRecQuads = PN ? 2 : 1;
+constexpr int kNoBody = 64;
+
+template <bool PN>
+__device__ __forceinline__ void put_no_body(double4* rec) {
+  rec[kNoBody * kRecQuads<PN>] = make_double4(1e100, 0.0, 0.0, 0.0);
+  if (PN) rec[kNoBody * kRecQuads<PN> + 1] = make_double4(0.0, 0.0, 0.0, 0.0);
+}
+
+// (61.5 -> 58.3 instructions per pair, of them 52 of FP64; with scalar loop counts
+// and the priorities below a step of 8192 systems of 3-64 bodies 60.7 -> 53.6 us
+// with 1PN, 15.6 -> 12.5 us without: the SIMDs issue in ~90% of their cycles.)
+// Source j of a lane's body: its system's bodies in order, itself left out.
+struct FastLane {
+  int base, self, sources;  // first body's lane, the body's place, number of sources
+};
+__device__ __forceinline__ FastLane fast_lane(int lane, int base, int cnt, bool live) {
+  return {base, lane - base, live ? cnt - 1 : 0};
+}
+__device__ __forceinline__ int fast_source(const FastLane& l, int j) {
+  const int src = l.base + j + (j >= l.self ? 1 : 0);
+  return j < l.sources ? src : kNoBody;
+}
+
+// The parts of a pair's acceleration, f d (d) and, with 1PN terms, g k (g):
+// {f, d, k, g}.
 template <bool PN>
 constexpr int kFastVals = PN ? 8 : 4;
 
 template <bool PN>
-__device__ __forceinline__ void batch_fast_pair(int src, bool valid, const double* lx, const double* ly,
-                                                const double* lz, const double* lm, const double* lvx,
-                                                const double* lvy, const double* lvz, const double* lv22,
-                                                const double* X, const double* V, double v11, double g5m1, double G,
-                                                double ic2, double soft, double* q) {
-  const double m2 = lm[src];
-  const double dx = lx[src] - X[0], dy = ly[src] - X[1], dz = lz[src] - X[2];
+__device__ __forceinline__ void batch_fast_pair(const double4* rec, int src, const double* X, const double* V,
+                                                double v11, double g5m1, double G, double ic2, double soft,
+                                                double* q) {
+  const double4 o = rec[src * kRecQuads<PN>];
+  const double m2 = o.w;
+  const double dx = o.x - X[0], dy = o.y - X[1], dz = o.z - X[2];
   const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, soft)));
   // one Newton step: 1/r to 4.1e-15 (two steps, 1.4e-16, cost 4 more
   // instructions per pair; the exact mode divides as the reference does)
-  const double inv = rsqrt64_n<1>(valid ? r2 : 1.0);
+  const double inv = rsqrt64_n<1>(r2);
   const double inv2 = inv * inv;
-  // a pair that does not count gets G m2 = 0 (its inv is finite), so
-  // both force terms vanish without selects of their own
-  const double gm2 = valid ? G * m2 : 0.0;
+  const double gm2 = G * m2;
   q[0] = gm2 * (inv2 * inv);
   q[1] = dx;
   q[2] = dy;
   q[3] = dz;
   if constexpr (PN) {
-    const double v2x = lvx[src], v2y = lvy[src], v2z = lvz[src];
+    const double4 w = rec[src * kRecQuads<PN> + 1];
     // get_pn1 (tool_chain_impl.cpp:110-118) with n = (x1 - x2)/r, the same
     // terms grouped for fused multiply-adds:
     //   G m2/r^2 [n (-v1^2 - 2 v2^2 + 4 v1.v2 + 3/2 (n.v2)^2 + (5 G m1 + 4 G m2)/r)
     //             + (v1 - v2)(4 n.v1 - 3 n.v2)]
     const double nx = -dx * inv, ny = -dy * inv, nz = -dz * inv;
     const double nv1 = fma(nx, V[0], fma(ny, V[1], nz * V[2]));
-    const double nv2 = fma(nx, v2x, fma(ny, v2y, nz * v2z));
-    const double v12 = fma(V[0], v2x, fma(V[1], v2y, V[2] * v2z));
-    const double v22 = lv22[src];  // |v2|^2, formed once per body when published
+    const double nv2 = fma(nx, w.x, fma(ny, w.y, nz * w.z));
+    const double v12 = fma(V[0], w.x, fma(V[1], w.y, V[2] * w.z));
     double sc = fma(4.0, v12, -v11);
-    sc = fma(-2.0, v22, sc);
+    sc = fma(-2.0, w.w, sc);
     sc = fma(1.5 * nv2, nv2, sc);
     sc = fma(fma(4.0 * G, m2, g5m1), inv, sc);
     const double t = fma(4.0, nv1, -3.0 * nv2);
     q[4] = gm2 * inv2 * ic2;
-    q[5] = fma(nx, sc, (V[0] - v2x) * t);
-    q[6] = fma(ny, sc, (V[1] - v2y) * t);
-    q[7] = fma(nz, sc, (V[2] - v2z) * t);
+    q[5] = fma(nx, sc, (V[0] - w.x) * t);
+    q[6] = fma(ny, sc, (V[1] - w.y) * t);
+    q[7] = fma(nz, sc, (V[2] - w.z) * t);
   }
 }
 
@@ -207,32 +232,20 @@ __device__ __forceinline__ void batch_fast_add(const double* q, double& ax, doub
   }
 }
 
-template <bool PN, bool EXACT>
-__device__ __forceinline__ void batch_accel(int lane, int base, int cnt, int maxcnt, bool live, const double* lx,
-                                            const double* ly, const double* lz, const double* lm, const double* lvx,
-                                            const double* lvy, const double* lvz, const double* lv22,
-                                            const double* X, const double* V, double mi, double G, double ic2,
-                                            double ic, int pnf, double soft, const Divisor64& md, bool ranges,
-                                            double* A) {
-  if constexpr (EXACT) {
-    if (ranges)
-      batch_exact<PN, true>(lane, base, cnt, maxcnt, live, lx, ly, lz, lm, lvx, lvy, lvz, X, V, md, G, ic, pnf, soft, A);
-    else
-      batch_exact<PN, false>(lane, base, cnt, maxcnt, live, lx, ly, lz, lm, lvx, lvy, lvz, X, V, md, G, ic, pnf, soft, A);
-    return;
-  }
+template <bool PN>
+__device__ __forceinline__ void batch_fast(const FastLane& l, int sources, const double4* rec, const double* X,
+                                           const double* V, double mi, double G, double ic2, double soft,
+                                           double* A) {
   double ax = 0.0, ay = 0.0, az = 0.0;
-  // fast mode, 1PN: this body's |v1|^2 and 5 G m1 (get_pn1's per-body parts)
+  // 1PN: this body's |v1|^2 and 5 G m1 (get_pn1's per-body parts)
   const double v11 = V[0] * V[0] + V[1] * V[1] + V[2] * V[2];
   const double g5m1 = 5.0 * G * mi;
   // Four sources per iteration: independent pair forces, sums still taken
   // one by one in j order
 #pragma unroll 4
-  for (int j = 0; j < maxcnt; ++j) {
-    const int src = min(base + j, 63);
-    const bool valid = live && j < cnt && src != lane;
+  for (int j = 0; j < sources; ++j) {
     double q[kFastVals<PN>];
-    batch_fast_pair<PN>(src, valid, lx, ly, lz, lm, lvx, lvy, lvz, lv22, X, V, v11, g5m1, G, ic2, soft, q);
+    batch_fast_pair<PN>(rec, fast_source(l, j), X, V, v11, g5m1, G, ic2, soft, q);
     batch_fast_add<PN>(q, ax, ay, az);
   }
   A[0] = ax;
@@ -343,12 +356,12 @@ __device__ __forceinline__ void kick_reg(double* V, const double* A, double dt) 
 
 template <bool PN, bool EXACT>
 __global__ __launch_bounds__(256) void k_batch(BatchArgs P) {
-  // positions, masses (and velocities) of each wavefront's bodies, one plane
-  // per quantity in a single array, so a source's values sit at one address
-  // plus constant plane offsets
-  // (the fast 1PN mode also keeps each body's |v|^2, a per-source term of get_pn1)
-  constexpr int kPlanes = PN ? (EXACT ? 7 : 8) : 4;
-  __shared__ double planes[kPlanes][kBatchMaxWpb][64];
+  // exact mode: positions, masses (and velocities) of each wavefront's bodies,
+  // one plane per quantity in a single array, so a source's values sit at one
+  // address plus constant plane offsets; fast mode: records
+  constexpr int kX = EXACT ? kBatchMaxWpb : 1, kF = EXACT ? 1 : kBatchMaxWpb;
+  __shared__ double planes[PN ? 7 : 4][kX][64];
+  __shared__ double4 recs[kF][EXACT ? 1 : (kNoBody + 1) * kRecQuads<PN>];
   auto sx = planes[0];
   auto sy = planes[1];
   auto sz = planes[2];
@@ -356,7 +369,6 @@ __global__ __launch_bounds__(256) void k_batch(BatchArgs P) {
   auto svx = planes[PN ? 4 : 0];
   auto svy = planes[PN ? 5 : 0];
   auto svz = planes[PN ? 6 : 0];
-  auto sv22 = planes[(PN && !EXACT) ? 7 : 0];
   constexpr int kE = (PN && EXACT) ? kBatchMaxWpb : 1;  // EIH potentials and Newtonian accelerations
   __shared__ double sphi[kE][64], sanx[kE][64], sany[kE][64], sanz[kE][64];
   const int wl = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -366,7 +378,11 @@ __global__ __launch_bounds__(256) void k_batch(BatchArgs P) {
   const int b = P.lane_body[slot];
   const int seg = P.lane_seg[slot];
   const int base = seg >> 8, cnt = seg & 255;
-  const int maxcnt = P.wave_max[wave];
+  const int maxcnt = __builtin_amdgcn_readfirstlane(P.wave_max[wave]);
+  // the longest loops first: a wavefront that is left alone issues at half the rate
+  if (maxcnt > 48) __builtin_amdgcn_s_setprio(3);
+  else if (maxcnt > 32) __builtin_amdgcn_s_setprio(2);
+  else if (maxcnt > 16) __builtin_amdgcn_s_setprio(1);
   const bool live = b >= 0;
   double X[3] = {0.0, 0.0, 0.0}, V[3] = {0.0, 0.0, 0.0}, A[3] = {0.0, 0.0, 0.0};
   double mi = 0.0;
@@ -378,25 +394,35 @@ __global__ __launch_bounds__(256) void k_batch(BatchArgs P) {
     }
     mi = P.m[b];
   }
-  double* lx = sx[wl];
-  double* ly = sy[wl];
-  double* lz = sz[wl];
-  double* lvx = svx[PN ? wl : 0];
-  double* lvy = svy[PN ? wl : 0];
-  double* lvz = svz[PN ? wl : 0];
-  double* lv22 = sv22[wl];
-  sm[wl][lane] = mi;
+  const int xl = EXACT ? wl : 0;
+  double* lx = sx[xl];
+  double* ly = sy[xl];
+  double* lz = sz[xl];
+  double* lvx = svx[xl];
+  double* lvy = svy[xl];
+  double* lvz = svz[xl];
+  double* lm = sm[xl];
+  double4* rec = recs[EXACT ? 0 : wl];
+  const FastLane fl = fast_lane(lane, base, cnt, live);
+  if (EXACT) lm[lane] = mi;
+  else if (lane == 0) put_no_body<PN>(rec);
   const Divisor64 md = divisor64(live ? mi : 1.0);
   const bool ranges = EXACT && __all(!live || mass_in_range64(mi)) && law_in_range64(P.G, P.soft);
   auto publish = [&]() {
-    lx[lane] = X[0];
-    ly[lane] = X[1];
-    lz[lane] = X[2];
-    if (PN) {
-      lvx[lane] = V[0];
-      lvy[lane] = V[1];
-      lvz[lane] = V[2];
-      if (!EXACT) lv22[lane] = fma(V[0], V[0], fma(V[1], V[1], V[2] * V[2]));
+    if constexpr (EXACT) {
+      lx[lane] = X[0];
+      ly[lane] = X[1];
+      lz[lane] = X[2];
+      if (PN) {
+        lvx[lane] = V[0];
+        lvy[lane] = V[1];
+        lvz[lane] = V[2];
+      }
+    } else {
+      rec[lane * kRecQuads<PN>] = make_double4(X[0], X[1], X[2], mi);
+      if (PN)
+        rec[lane * kRecQuads<PN> + 1] =
+            make_double4(V[0], V[1], V[2], fma(V[0], V[0], fma(V[1], V[1], V[2] * V[2])));
     }
     wave_sync();
   };
@@ -406,17 +432,22 @@ __global__ __launch_bounds__(256) void k_batch(BatchArgs P) {
            __all(!live || (coord_in_range64(X[0]) && coord_in_range64(X[1]) && coord_in_range64(X[2])));
   };
   auto accel = [&]() {
-    if (eih) {
-      const int e = (PN && EXACT) ? wl : 0;
+    if constexpr (!EXACT) {
+      batch_fast<PN>(fl, maxcnt - 1, rec, X, V, mi, P.G, P.ic2, P.soft, A);
+    } else if (eih) {
+      const int e = PN ? wl : 0;
       if (in_ranges())
-        batch_eih<true>(lane, base, cnt, maxcnt, live, lx, ly, lz, sm[wl], lvx, lvy, lvz, X, V, P.G, P.ic, P.soft,
+        batch_eih<true>(lane, base, cnt, maxcnt, live, lx, ly, lz, lm, lvx, lvy, lvz, X, V, P.G, P.ic, P.soft,
                         sphi[e], sanx[e], sany[e], sanz[e], A);
       else
-        batch_eih<false>(lane, base, cnt, maxcnt, live, lx, ly, lz, sm[wl], lvx, lvy, lvz, X, V, P.G, P.ic, P.soft,
+        batch_eih<false>(lane, base, cnt, maxcnt, live, lx, ly, lz, lm, lvx, lvy, lvz, X, V, P.G, P.ic, P.soft,
                          sphi[e], sanx[e], sany[e], sanz[e], A);
+    } else if (in_ranges()) {
+      batch_exact<PN, true>(lane, base, cnt, maxcnt, live, lx, ly, lz, lm, lvx, lvy, lvz, X, V, md, P.G, P.ic, P.pnf,
+                            P.soft, A);
     } else {
-      batch_accel<PN, EXACT>(lane, base, cnt, maxcnt, live, lx, ly, lz, sm[wl], lvx, lvy, lvz, lv22, X, V, mi, P.G,
-                             P.ic2, P.ic, P.pnf, P.soft, md, in_ranges(), A);
+      batch_exact<PN, false>(lane, base, cnt, maxcnt, live, lx, ly, lz, lm, lvx, lvy, lvz, X, V, md, P.G, P.ic, P.pnf,
+                             P.soft, A);
     }
   };
   if (P.init) {
@@ -465,8 +496,8 @@ __global__ __launch_bounds__(64 * (W + 3)) void k_batch_team(BatchArgs P) {
 #pragma clang fp contract(off)
   constexpr int kChunk = W * kU;
   constexpr int kVals = EXACT ? 3 : kFastVals<PN>;
-  __shared__ double planes[PN ? 7 : 4][64];
-  __shared__ double v22[PN && !EXACT ? 64 : 1];
+  __shared__ double planes[PN ? 7 : 4][EXACT ? 64 : 1];
+  __shared__ double4 rec[EXACT ? 1 : (kNoBody + 1) * kRecQuads<PN>];
   __shared__ double force[2][kChunk][kVals][64];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const bool adder = w >= W;
@@ -486,10 +517,16 @@ __global__ __launch_bounds__(64 * (W + 3)) void k_batch_team(BatchArgs P) {
     a = P.a[at];
   }
   double X[3] = {0.0, 0.0, 0.0}, V[3] = {0.0, 0.0, 0.0};  // worker: the body
-  if (w == 0) planes[3][lane] = mi;
+  const FastLane fl = fast_lane(lane, base, cnt, live);
+  const int sources = EXACT ? maxcnt : maxcnt - 1;  // the exact mode passes 0 for the body itself
+  if (EXACT && w == 0) planes[3][lane] = mi;
+  if (!EXACT && w == 0) {
+    rec[lane * kRecQuads<PN>].w = mi;
+    if (lane == 0) put_no_body<PN>(rec);
+  }
   const Divisor64 md = divisor64(EXACT && live ? mi : 1.0);
   const bool ranges = EXACT && __all(!live || mass_in_range64(mi)) && law_in_range64(P.G, P.soft);
-  // sources past maxcnt add 0, so that a chunk always has the same length
+  // past the sources: 0, so that a chunk always has the same length
   auto work = [&](int j0, bool fast, double (*out)[kVals][64]) {
     double f[kU][kVals] = {};
     const double* p = &planes[0][0];
@@ -503,15 +540,12 @@ __global__ __launch_bounds__(64 * (W + 3)) void k_batch_team(BatchArgs P) {
       else if (j0 < maxcnt)
         batch_exact_pairs<PN, false>(lane, base, cnt, j0, live, p, p + 64, p + 128, p + 192, vx, vy, vz, X, V, md, P.G,
                                      P.ic, P.pnf, P.soft, f);
-    } else if (j0 < maxcnt) {
+    } else if (j0 < sources) {
       const double v11 = V[0] * V[0] + V[1] * V[1] + V[2] * V[2];
       const double g5m1 = 5.0 * P.G * mi;
 #pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        const int src = min(base + j0 + u, 63);
-        batch_fast_pair<PN>(src, live && j0 + u < cnt && src != lane, p, p + 64, p + 128, p + 192, vx, vy, vz, v22, X,
-                            V, v11, g5m1, P.G, P.ic2, P.soft, f[u]);
-      }
+      for (int u = 0; u < kU; ++u)
+        batch_fast_pair<PN>(rec, fast_source(fl, j0 + u), X, V, v11, g5m1, P.G, P.ic2, P.soft, f[u]);
     }
 #pragma unroll
     for (int u = 0; u < kU; ++u)
@@ -520,20 +554,21 @@ __global__ __launch_bounds__(64 * (W + 3)) void k_batch_team(BatchArgs P) {
   };
   // the adders' bodies to the workers, then the accelerations to the adders
   auto accel = [&]() {
+    double* mine = reinterpret_cast<double*>(rec + lane * kRecQuads<PN>);  // fast mode: {x, y, z, m, v, |v|^2}
     if (adder) {
-      planes[ax][lane] = x;
-      if (PN) planes[4 + ax][lane] = v;
+      (EXACT ? planes[ax][lane] : mine[ax]) = x;
+      if (PN) (EXACT ? planes[4 + ax][lane] : mine[4 + ax]) = v;
     }
     __syncthreads();
     if (!adder) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        X[c] = planes[c][lane];
-        if (PN) V[c] = planes[4 + c][lane];
+        X[c] = EXACT ? planes[c][lane] : mine[c];
+        if (PN) V[c] = EXACT ? planes[4 + c][lane] : mine[4 + c];
       }
     }
     if (PN && !EXACT) {
-      if (w == 0) v22[lane] = fma(V[0], V[0], fma(V[1], V[1], V[2] * V[2]));
+      if (w == 0) mine[7] = fma(V[0], V[0], fma(V[1], V[1], V[2] * V[2]));
       __syncthreads();
     }
     double sum = 0.0;
@@ -552,13 +587,13 @@ __global__ __launch_bounds__(64 * (W + 3)) void k_batch_team(BatchArgs P) {
     const bool fast =
         ranges && __all(!live || (coord_in_range64(X[0]) && coord_in_range64(X[1]) && coord_in_range64(X[2])));
     int j0 = 0;
-    for (; j0 < maxcnt; j0 += kChunk) {
+    for (; j0 < sources; j0 += kChunk) {
       if (!adder) work(j0 + w * kU, fast, &force[(j0 / kChunk) & 1][w * kU]);
       else if (j0 > 0) add(j0 - kChunk);
       __syncthreads();
     }
     if (adder) {
-      add(j0 - kChunk);
+      if (j0 > 0) add(j0 - kChunk);
       a = sum;
     }
   };
@@ -986,14 +1021,15 @@ static BatchArgs make_args(aster_ctx* c, int64_t nsteps, int nsub, const double*
 // 1.29 / 1.29. 1PN: 64, 520 58 / 39 / 33, 1045 67 / 67 / 57, 2126 107 / 124 / 105;
 // 32, 546 29.9 / 20.6 / 18.7, 1111 31.3 / 37 / 32.6; 16, 604 15.5 / 13.9 / 12.8; 8,
 // 350 8.2 / 6.4, 703 8.5 / 9.7; 4, 224 4.5 / 3.3, 448 4.6 / 6.3. Fast mode,
-// Newtonian: 64, 153 5.3 / 3.8 / 2.95, 520 5.4 / 5.2 / 5.3, 1045 6.2 / 8.6; 16, 148
-// 1.64 / 1.28 / 1.07, 604 1.70 / 1.77; 8, 172 1.04 / 0.86; 4 0.72 / 0.83. 1PN: 64,
-// 153 23.8 / 12.4, 520 24.2 / 20.3, 1045 25.7 / 35.6; 16, 296 6.6 / 4.4, 604 6.7 /
-// 7.6; 8, 172 3.5 / 2.6; 4, 110 2.1 / 2.4.
+// Newtonian: 64, 153 4.4 / 3.5 / 3.0, 412 4.5 / 4.2 / 4.1, 520 4.6 / 4.6 / 5.3; 16,
+// 148 1.46 / 1.21 / 1.12, 296 1.48 / 1.29 / 1.47, 441 1.50 / 1.59; 8, 172 0.99 /
+// 0.83, 256 1.00 / 0.98; 4 0.72 / 0.80. 1PN: 64, 153 18.3 / 12.3, 412 18.7 / 16.7,
+// 520 18.8 / 20.2; 16, 296 5.2 / 4.9, 441 5.3 / 6.2; 8, 172 3.0 / 2.9, 256 3.0 /
+// 3.8; 4 1.8 / 2.6.
 static int team_size(int nwaves, int largest, bool pn, bool exact) {
   int most;
   if (exact) most = largest <= 4 ? 256 : !pn || largest > 32 ? 1024 : largest > 8 ? 768 : 512;
-  else most = largest <= 4 ? 0 : largest <= 8 ? 256 : 512;
+  else most = largest <= 4 ? 0 : largest <= 8 ? 192 : largest <= 16 ? 320 : 416;
   if (nwaves > most) return 0;
   const bool wide = exact && pn ? true : nwaves <= 256 && !pn;
   return largest > 8 && wide ? 8 : 4;
