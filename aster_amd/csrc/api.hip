@@ -516,8 +516,11 @@ int aster_tree_dump(aster_ctx* c, uint32_t* codes, uint32_t* perm, int32_t* left
   int rc = 0;
   if (codes && (rc = cp(codes, c->codes.p, n * sizeof(uint32_t)))) return rc;
   if (perm && (rc = cp(perm, c->idx.p, n * sizeof(uint32_t)))) return rc;
-  if (left && (rc = cp(left, c->left.p, nn * sizeof(int32_t)))) return rc;
-  if (right && (rc = cp(right, c->right.p, nn * sizeof(int32_t)))) return rc;
+  for (int32_t* kid : {left, right}) {  // the device keeps those of the internal nodes
+    if (!kid) continue;
+    std::fill(kid, kid + n, -1);
+    if ((rc = cp(kid + n, (kid == left ? c->left.p : c->right.p) + n, (n - 1) * sizeof(int32_t)))) return rc;
+  }
   std::vector<double4> mc;
   if (node_mass || node_com) {
     mc.resize((size_t)nn);

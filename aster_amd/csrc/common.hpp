@@ -263,7 +263,14 @@ int center_of_mass(aster_ctx* c, double* com);
 int total_mass(aster_ctx* c, double* mtot, double* extent);  // sum of the masses, largest |coordinate| (cached)
 int fp32_scales(aster_ctx* c, Fp32Scales* s);
 int launch_reset_flags(aster_ctx* c);
-int launch_box(aster_ctx* c, bool user_box);             // fills c->boxd
+// Where the Morton box comes from: the maximum of nparts triples, or (nparts = 0)
+// one triple as it is (a user's box, or the finished one).
+struct BoxSource {
+  const double* part;
+  int nparts;
+};
+constexpr int kBoxSourceParts = 4096;  // more are reduced by a launch of their own
+int launch_box(aster_ctx* c, bool user_box, BoxSource* bs);
 int bh_forces(aster_ctx* c, int method);                 // writes c->a
 int bh_morton_only(aster_ctx* c);
 int morton_sort(aster_ctx* c, bool user_box);            // c->codes sorted, c->idx = perm

@@ -446,4 +446,53 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The Morton box's half-extents b in every thread of a workgroup of T, and with
+// `store` in box[0..2], |box| in box[3]. fmax is exact and order-independent, so
+// every workgroup finds the same.
+template <int T>
+__device__ __forceinline__ void box_final(const BoxSource& bs, double* __restrict__ box, double* b, bool store) {
+#pragma clang fp contract(off)
+  __shared__ double wm[3][T / 64];
+  const int t = threadIdx.x;
+  if (bs.nparts == 0) {
+    for (int c = 0; c < 3; ++c) b[c] = bs.part[c];
+  } else {
+    double r[3] = {0.0, 0.0, 0.0};
+    // 8 partials per thread and round, all loaded before the first is used
+    // (clamped indices), so a round costs one memory round trip
+    for (int i0 = t; i0 < bs.nparts; i0 += 8 * T) {
+      double q[8][3];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int i = min(i0 + u * T, bs.nparts - 1);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) q[u][c] = bs.part[3 * i + c];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) r[c] = fmax(r[c], q[u][c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      for (int off = 32; off > 0; off >>= 1) r[c] = fmax(r[c], __shfl_xor(r[c], off, 64));
+      if ((t & 63) == 0) wm[c][t >> 6] = r[c];
+    }
+  }
+  __syncthreads();
+  if (bs.nparts != 0)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      b[c] = 0.0;
+      for (int q = 0; q < T / 64; ++q) b[c] = fmax(b[c], wm[c][q]);
+    }
+  if (store && t == 0 && bs.part != box) {
+    box[0] = b[0];
+    box[1] = b[1];
+    box[2] = b[2];
+    // bd_size = |bounding_box| (barnes_hut.cpp:405; vec3::magnitude, vectors.h:93-99)
+    box[3] = sqrt(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
+  }
+}
+
 }  // namespace aster

@@ -238,51 +238,12 @@ __global__ __launch_bounds__(256) void k_box(int n, const double* __restrict__ x
   }
 }
 
-// One thread per partial (one round of loads), then a block maximum; fmax is
-// exact and order-independent.
+// The final maximum in a launch of its own, for more partials than every
+// workgroup of k_morton should read (kBoxSourceParts).
 constexpr int kBoxFinishThreads = 1024;
-__global__ __launch_bounds__(kBoxFinishThreads) void k_box_finish(const double* __restrict__ part, int nparts,
-                                                                  const double* __restrict__ user, int use_user,
-                                                                  double* __restrict__ box) {
-#pragma clang fp contract(off)
-  __shared__ double wm[3][kBoxFinishThreads / 64];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  double r[3] = {0.0, 0.0, 0.0};
-  // 8 partials per thread and round, all loaded before the first is used
-  // (clamped indices), so a round costs one memory round trip
-  if (!use_user)
-    for (int i0 = t; i0 < nparts; i0 += 8 * kBoxFinishThreads) {
-      double q[8][3];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int i = min(i0 + u * kBoxFinishThreads, nparts - 1);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) q[u][c] = part[3 * i + c];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) r[c] = fmax(r[c], q[u][c]);
-    }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    for (int off = 32; off > 0; off >>= 1) r[c] = fmax(r[c], __shfl_xor(r[c], off, 64));
-    if (lane == 0) wm[c][w] = r[c];
-  }
-  __syncthreads();
-  if (t != 0) return;
+__global__ __launch_bounds__(kBoxFinishThreads) void k_box_finish(BoxSource bs, double* __restrict__ box) {
   double b[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    double m = 0.0;
-    for (int q = 0; q < kBoxFinishThreads / 64; ++q) m = fmax(m, wm[c][q]);
-    b[c] = use_user ? user[c] : m;
-  }
-  box[0] = b[0];
-  box[1] = b[1];
-  box[2] = b[2];
-  // bd_size = |bounding_box| (barnes_hut.cpp:405; vec3::magnitude, vectors.h:93-99)
-  box[3] = sqrt(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
+  box_final<kBoxFinishThreads>(bs, box, b, true);
 }
 
 __global__ void k_zero_u32(uint32_t* p, int k) {
@@ -371,7 +332,7 @@ int launch_energy(aster_ctx* c, double* out6) {
   return ASTER_OK;
 }
 
-int launch_box(aster_ctx* c, bool user_box) {
+int launch_box(aster_ctx* c, bool user_box, BoxSource* bs) {
   const int n = (int)c->n;
   ASTER_HIP(c, c->boxpart.reserve(3 * kBoxBlocks));
   ASTER_HIP(c, c->boxd.reserve(8));
@@ -390,9 +351,12 @@ int launch_box(aster_ctx* c, bool user_box) {
     ASTER_HIP(c, hipGetLastError());
   }
   c->box_parts = 0;
-  hipLaunchKernelGGL(k_box_finish, dim3(1), dim3(kBoxFinishThreads), 0, c->stream, c->boxpart.p, blocks, c->boxd.p + 4,
-                     user ? 1 : 0, c->boxd.p);
-  ASTER_HIP(c, hipGetLastError());
+  *bs = user ? BoxSource{c->boxd.p + 4, 0} : BoxSource{c->boxpart.p, blocks};
+  if (blocks > kBoxSourceParts) {
+    hipLaunchKernelGGL(k_box_finish, dim3(1), dim3(kBoxFinishThreads), 0, c->stream, *bs, c->boxd.p);
+    ASTER_HIP(c, hipGetLastError());
+    *bs = BoxSource{c->boxd.p, 0};
+  }
   return ASTER_OK;
 }
 
