@@ -426,6 +426,18 @@ __global__ __launch_bounds__(256) void k_combine(int n, int npad, int S, const d
 // bodies: one target per lane): n = 1000 70 -> 16 us, 4096 264 -> 55 us, 16384
 // 1.89 -> 0.64 ms, 65536 15.4 -> 9.2 ms; with the 1PN term 79 -> 31 us, 297 ->
 // 114 us, 2.60 -> 1.78 ms, 31.6 -> 28.1 ms.
+//
+// The adding wave then applies the integrator's update (StepPost) to its
+// targets; positions go to a second buffer, since other blocks still read them
+// as sources. A launch less per step: 64 bodies
+// 7.3 -> 4.8 us, 1000 20.0 -> 17.2, 4096 58.5 -> 56.0 (SABA4 235.8 -> 223.3),
+// 16384 650 -> 639.
+struct Update64 {
+  StepPost post;
+  double* x_out;
+  double* v;
+  uint32_t* flags;
+};
 constexpr int kF64Chunk = 64;
 
 template <int W, int kPer, bool PN, int MODE>
@@ -434,7 +446,7 @@ __global__ __launch_bounds__(64 * (W + 1)) void k_allpairs_f64(int n, int lower,
                                                                         const double* __restrict__ v,
                                                                         const double* __restrict__ m, double G,
                                                                         double ic, int pnf, double soft,
-                                                                        double* __restrict__ a) {
+                                                                        double* __restrict__ a, Update64 up) {
 #pragma clang fp contract(off)
   constexpr int kF64Targets = W * kPer;
   static_assert(3 * kF64Targets <= 64, "one row per lane of the adding wave");
@@ -586,7 +598,13 @@ __global__ __launch_bounds__(64 * (W + 1)) void k_allpairs_f64(int n, int lower,
     return;
   }
   const int row = min(lane, 3 * kF64Targets - 1);
-  double acc = 0.0;
+  const int i = i0 + row % kF64Targets;
+  const size_t k = (size_t)(row / kF64Targets) * n + min(i, n - 1);
+  double acc = 0.0, xt = 0.0, vt = 0.0;
+  if (!PN && up.post.kind != POST_NONE) {
+    xt = x[k];
+    vt = up.v[k];
+  }
   __syncthreads();
   for (int ch = 0; ch < chunks; ++ch) {
     __syncthreads();
@@ -608,8 +626,18 @@ __global__ __launch_bounds__(64 * (W + 1)) void k_allpairs_f64(int n, int lower,
       }
     }
   }
-  const int i = i0 + lane % kF64Targets;
-  if (lane < 3 * kF64Targets && i < n) a[(size_t)(lane / kF64Targets) * n + i] = acc;
+  if (lane >= 3 * kF64Targets || i >= n) return;
+  a[k] = acc;
+  if (PN || up.post.kind == POST_NONE) return;
+  if (up.post.kind == POST_KICK) {
+    up.v[k] = kick_1(vt, acc, up.post.dt);
+    return;
+  }
+  if (up.post.kind == POST_KICK_DRIFT) kick_drift_1(xt, vt, acc, up.post.dt_prev, up.post.dt);
+  else saba_1(xt, vt, acc, up.post.d, up.post.cd, up.post.cd_next, up.post.dt);
+  up.x_out[k] = xt;
+  up.v[k] = vt;
+  if (!(isfinite(xt) && isfinite(vt))) atomicOr(up.flags, (uint32_t)FLAG_NONFINITE);
 }
 
 // ----------------------------------------------------------------- EIH ----
@@ -703,12 +731,12 @@ __global__ __launch_bounds__(256) void k_eih_pass2(int n, const double* __restri
 
 template <int W, int PER>
 static void launch_allpairs_f64_as(aster_ctx* c, bool pn, int mode, int n, int lower, int upper, double ic, int pnf,
-                                   double* out) {
+                                   double* out, const Update64& up) {
   auto k = mode == 1 ? k_allpairs_f64<W, PER, true, 1>
                      : pn ? k_allpairs_f64<W, PER, true, 0> : k_allpairs_f64<W, PER, false, 0>;
   const int targets = W * PER;
   hipLaunchKernelGGL(k, dim3((n + targets - 1) / targets), dim3(64 * (W + 1)), 0, c->stream, n, lower, upper, c->x.p,
-                     c->v.p, c->m.p, c->P.G, ic, pnf, c->P.softening, out);
+                     c->v.p, c->m.p, c->P.G, ic, pnf, c->P.softening, out, up);
 }
 
 // 16 targets a block fill the 256 CUs once at 4096 bodies and twice at 8192;
@@ -717,9 +745,9 @@ static void launch_allpairs_f64_as(aster_ctx* c, bool pn, int mode, int n, int l
 // 8192, 797 and 672 at 16384, 10.9 and 9.9 ms at 65536 (with the 1PN term 28.5
 // and 33.3 ms), both before the division took four steps instead of five.
 static int launch_allpairs_f64(aster_ctx* c, bool pn, int mode, int n, int lower, int upper, double ic, int pnf,
-                               double* out) {
-  if (pn || n <= 8192) launch_allpairs_f64_as<8, 2>(c, pn, mode, n, lower, upper, ic, pnf, out);
-  else launch_allpairs_f64_as<7, 2>(c, pn, mode, n, lower, upper, ic, pnf, out);
+                               double* out, const Update64& up = Update64{}) {
+  if (pn || n <= 8192) launch_allpairs_f64_as<8, 2>(c, pn, mode, n, lower, upper, ic, pnf, out, up);
+  else launch_allpairs_f64_as<7, 2>(c, pn, mode, n, lower, upper, ic, pnf, out, up);
   ASTER_HIP(c, hipGetLastError());
   return ASTER_OK;
 }
@@ -914,11 +942,22 @@ int launch_allpairs(aster_ctx* c, int method, const StepPost& post) {
     return launch_post(c, post, false);
   }
   if (method == ASTER_ALLPAIRS_FP64) {
+    // Velocity-dependent terms read every body's velocity; above 16384 bodies a
+    // launch is under 1% of the evaluation and not worth a second buffer.
+    const bool fused = !pn && n <= 16384 && post.kind != POST_NONE;
+    const bool drifts = fused && post.kind != POST_KICK;
+    Update64 up{};
+    if (drifts) ASTER_HIP(c, c->x_next.reserve((size_t)3 * n));
+    if (fused) up = Update64{post, c->x_next.p, c->v.p, c->flags.p};
     phase_begin(c, ASTER_PHASE_ALLPAIRS);
-    if (const int e = launch_allpairs_f64(c, pn, 0, n, lower, upper, ic, pnf, c->a.p)) return e;
-    ASTER_HIP(c, hipGetLastError());
+    if (const int e = launch_allpairs_f64(c, pn, 0, n, lower, upper, ic, pnf, c->a.p, up)) return e;
     phase_end(c, ASTER_PHASE_ALLPAIRS);
-    return launch_post(c, post, false);
+    if (drifts) {
+      std::swap(c->x, c->x_next);
+      c->box_parts = 0;
+      c->src_ready = SrcReady{};
+    }
+    return fused ? ASTER_OK : launch_post(c, post, false);
   }
   if (method != ASTER_ALLPAIRS_FP32 && method != ASTER_ALLPAIRS_FP32_KAHAN)
     return fail(c, ASTER_ERR_INVALID, "unknown all-pairs method");

@@ -82,3 +82,26 @@ def test_ensembles_ranges(ctx, orc, flags):
             rp, rv, _ = orc.integrate(pos[s], vel[s], mass[s], dt, 3, integrator=2, G=G, soft=soft, c=30.0,
                                       pn=flags)
             assert np.array_equal(p[s], rp, equal_nan=True) and np.array_equal(v[s], rv, equal_nan=True), (name, a)
+
+
+@pytest.mark.parametrize("n", [1, 2, 16, 17, 1000, 8193, 16384, 16385])
+@pytest.mark.parametrize("integrator,order", [(A.LEAPFROG, 0), (A.YOSHIDA4, 0), (A.EULER, 1), (A.SABA, 3)])
+def test_allpairs_updates_same_bits(ctx, n, integrator, order):
+    """Updates fused into the evaluation: several steps in one call against one per call, and against the same steps with a
+    source range that ends one body late (clamped to all) and a post-Newtonian term of weight 0, which go by launches of
+    their own."""
+    pos, vel, mass = plummer(n, 4)
+    out = []
+    for parts, flags in (((3,), A.NEWTON), ((1, 1, 1), A.NEWTON), ((3,), A.NEWTON | A.PN1)):
+        if flags != A.NEWTON and integrator in (A.LEAPFROG, A.YOSHIDA4):
+            continue  # evaluates once more per step with velocity-dependent terms
+        if flags != A.NEWTON and n > 8193:
+            continue
+        ctx.set_params(G=1.0, softening=1e-4, c=1e200, pn_flags=flags)
+        ctx.set_state(pos, vel, mass)
+        for k in parts:
+            ctx.integrate(A.ALLPAIRS_FP64, integrator, order, 1e-3, k)
+        out.append(ctx.get_state() + (ctx.get_acc(),))
+    for o in out[1:]:
+        for a, b in zip(out[0], o):
+            assert np.all(np.isfinite(a)) and np.array_equal(a, b)
