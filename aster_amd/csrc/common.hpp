@@ -255,7 +255,7 @@ int launch_post(aster_ctx* c, const StepPost& post, bool box);
 int launch_kick_drift(aster_ctx* c, double dt_prev, double dt, bool box = false);
 int launch_kick(aster_ctx* c, double dt);
 int launch_saba_stage(aster_ctx* c, bool kick, double d, double cdrift, double dt, double cd_next = 0.0);
-int launch_energy(aster_ctx* c, double* out6_host);
+int launch_energy(aster_ctx* c, double* out7_host);  // six sums and the error word
 int import_state(aster_ctx* c, int64_t n, const double* d_pos, const double* d_vel, const double* d_mass);
 int export_plane(aster_ctx* c, const double* soa, double* d_aos);
 int grow_state(aster_ctx* c, int64_t add, int64_t* base);  // appends `add` bodies; *base = first new index

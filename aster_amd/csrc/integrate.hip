@@ -9,6 +9,7 @@
 // and the first half-kick of the next use the same accelerations, so they are
 // applied in one pass (k_kick_drift with dt_prev != 0).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "device.hpp"
@@ -103,30 +104,53 @@ __global__ __launch_bounds__(256) void k_kick(int n, double* __restrict__ v, con
 // sums of G m_i m_j / (|r| + soft) and G m_i m_j / sqrt(r^2 + soft) to
 // part[0/1][y ntiles + a], and for y = 0 those of the kinetic energy and of m x
 // cross v to rows[0..3][a]. Every sum has a fixed order. Bound: FP64 issue at
-// many bodies, latency at few. An aster_energy call (with its two readbacks of
-// about 25 us), against one thread per body over all sources (every pair twice):
-// n = 1000 331 -> 70 us, 4096 1205 -> 91 us, 20011 5.83 -> 0.47 ms, 65536 20.6 ->
-// 4.3 ms (2.5 ms unsoftened, where the two pair terms are one).
+// many bodies, latency at few. An aster_energy call (with a readback of about 25
+// us), against one thread per body over all sources (every pair twice) and two
+// readbacks: n = 1000 331 -> 44 us, 4096 1205 -> 59 us, 20011 5.83 -> 0.37 ms,
+// 65536 20.6 -> 3.3 ms (1.7 ms unsoftened, where the two pair terms are one);
+// with exact roots, a range check per term and IEEE fallbacks in line 4.4 (2.5) ms.
 __device__ __forceinline__ double wave_sum64(double v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
 }
 
-// sqrt(x) and 1 / x to about one unit in the last place.
-__device__ __forceinline__ double sqrt64_near(double x) {
-  if (__builtin_expect(hi32(x) - 0x14300000u >= 0x6bb00000u - 0x14300000u, 0)) return sqrt(x);  // beyond 2^+-700, or 0
-  const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  const double e = fma(-h, g, 0.5);
-  g = fma(g, e, g);
-  h = fma(h, e, h);
-  return fma(fma(-g, g, x), h, g);
-}
-__device__ __forceinline__ double rcp64_near(double x) {
-  if (__builtin_expect(hi32(x) - 0x14300000u >= 0x6bb00000u - 0x14300000u, 0)) return 1.0 / x;
-  double y = __builtin_amdgcn_rcp(x);
-  y = fma(fma(-x, y, 1.0), y, y);
-  return fma(fma(-x, y, 1.0), y, y);
+// N pair terms 1 / sqrt(r^2 + soft) and (SOFT) 1 / (|r| + soft): to about one
+// unit in the last place by Newton and third-order steps from the estimates,
+// with one look at the range for all of a wavefront's N (r^2 within 2^+-600;
+// `plain` when the softening is beyond that).
+__device__ __forceinline__ bool energy_range(double x) { return hi32(x) - 0x1a700000u < 0x65700000u - 0x1a700000u; }
+
+template <int N, bool SOFT>
+__device__ __forceinline__ void energy_terms(const double* r2, double soft, bool plain, double* pl, double* pr) {
+  bool in = !plain;
+#pragma unroll
+  for (int u = 0; u < N; ++u) in = in && energy_range(r2[u]);
+  if (__builtin_expect(__all(in), 1)) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const double x = r2[u] + soft;
+      const double y = __builtin_amdgcn_rsq(x);
+      const double e = fma(-(x * y), y, 1.0);
+      pl[u] = fma(y * e, fma(0.375, e, 0.5), y);
+      if (SOFT) {
+        const double z = __builtin_amdgcn_rsq(r2[u]);
+        double g = r2[u] * z, h = 0.5 * z;
+        const double d = fma(-h, g, 0.5);
+        g = fma(g, d, g);
+        h = fma(h, d, h);
+        const double q = fma(fma(-g, g, r2[u]), h, g) + soft;  // |r| + soft
+        double w = __builtin_amdgcn_rcp(q);
+        w = fma(fma(-q, w, 1.0), w, w);
+        pr[u] = fma(fma(-q, w, 1.0), w, w);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      pl[u] = 1.0 / sqrt(r2[u] + soft);
+      if (SOFT) pr[u] = 1.0 / (sqrt(r2[u]) + soft);
+    }
+  }
 }
 
 template <bool SOFT>
@@ -144,6 +168,7 @@ __global__ __launch_bounds__(64) void k_energy_pairs(int n, int ntiles, int stri
     const int j = b * 64 + lane, jj = min(j, n - 1);
     return make_double4(x[jj], x[n + jj], x[2 * (size_t)n + jj], j < n ? m[jj] : 0.0);
   };
+  const bool plain = soft != 0.0 && !energy_range(soft);
   double pref = 0.0, ppl = 0.0;
   double4 q = b0 < b1 ? fetch(b0) : make_double4(0.0, 0.0, 0.0, 0.0);
   for (int b = b0; b < b1; ++b) {
@@ -153,16 +178,27 @@ __global__ __launch_bounds__(64) void k_energy_pairs(int n, int ntiles, int stri
     if (b + 1 < b1) q = fetch(b + 1);
     const int cnt = min(64, n - b * 64);
     const int from = b == a ? lane : -1;  // the pairs i < j of the tile with itself
-#pragma unroll 4
-    for (int k = 0; k < cnt; ++k) {
-      const double4 s = tile[k];
-      const double dx = s.x - px, dy = s.y - py, dz = s.z - pz;
-      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-      const double pl = inv_sqrt64(r2 + soft);
-      const bool take = k > from;
-      ppl += take ? s.w * pl : 0.0;
-      if (SOFT) pref += take ? s.w * rcp64_near(sqrt64_near(r2) + soft) : 0.0;
-    }
+    auto pairs = [&](int k, auto count) {
+      constexpr int N = count();
+      double r2[N], w[N], pl[N], pr[N];
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        const double4 s = tile[k + u];
+        const double dx = s.x - px, dy = s.y - py, dz = s.z - pz;
+        r2[u] = fma(dx, dx, fma(dy, dy, dz * dz));
+        w[u] = s.w;
+      }
+      energy_terms<N, SOFT>(r2, soft, plain, pl, pr);
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        const bool take = k + u > from;
+        ppl += take ? w[u] * pl[u] : 0.0;
+        if (SOFT) pref += take ? w[u] * pr[u] : 0.0;
+      }
+    };
+    int k = 0;
+    for (; k + 4 <= cnt; k += 4) pairs(k, std::integral_constant<int, 4>{});
+    for (; k < cnt; ++k) pairs(k, std::integral_constant<int, 1>{});
   }
   const double gm = G * mi;
   const double sp = wave_sum64(i < n ? gm * ppl : 0.0);
@@ -184,33 +220,44 @@ __global__ __launch_bounds__(64) void k_energy_pairs(int n, int ntiles, int stri
   }
 }
 
-// out = {kinetic, 2 sum_{i<j} of the two pair terms, L}: one block, fixed
-// strided order, fixed tree. 8 loads per thread are in flight.
+// out = {kinetic, 2 sum_{i<j} of the two pair terms, L}: one block, fixed order
+// (strided per thread, wavefronts by a fixed tree, then their sums). The loads
+// of a round are in flight together. (One sum after the other through LDS took
+// 10.3 us at 4096 bodies, this 5.9 us.) out[6]: the error word, so that one readback
+// serves both.
 __global__ __launch_bounds__(1024) void k_energy_reduce(int slots, int ntiles, const double* __restrict__ part,
-                                                        const double* __restrict__ rows, double* __restrict__ out) {
-  __shared__ double sm[1024];
+                                                        const double* __restrict__ rows,
+                                                        const uint32_t* __restrict__ flags,
+                                                        double* __restrict__ out) {
+  __shared__ double sm[6][16];
   const int t = threadIdx.x;
-  for (int r = 0; r < 6; ++r) {
-    const bool pair = r == 1 || r == 2;
-    const double* __restrict__ in = pair ? part + (size_t)(r - 1) * slots : rows + (size_t)(r == 0 ? 0 : r - 2) * ntiles;
-    const int len = pair ? slots : ntiles;
-    double s = 0.0;
-    for (int i0 = t; i0 < len; i0 += 8 * 1024) {
-      double w[8];
+  double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};  // two pair terms, four rows
+  for (int i0 = t; i0 < slots; i0 += 4 * 1024) {
+    double w[2][4];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) w[u] = in[min(i0 + u * 1024, len - 1)];
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int u = 0; u < 8; ++u) s += i0 + u * 1024 < len ? w[u] : 0.0;
-    }
-    sm[t] = s;
-    __syncthreads();
-    for (int w = 512; w > 0; w >>= 1) {
-      if (t < w) sm[t] += sm[t + w];
-      __syncthreads();
-    }
-    if (t == 0) out[r] = pair ? 2.0 * sm[0] : sm[0];
-    __syncthreads();
+      for (int r = 0; r < 2; ++r) w[r][u] = part[(size_t)r * slots + min(i0 + u * 1024, slots - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int r = 0; r < 2; ++r) s[r] += i0 + u * 1024 < slots ? w[r][u] : 0.0;
   }
+  for (int i = t; i < ntiles; i += 1024)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s[2 + r] += rows[(size_t)r * ntiles + i];
+#pragma unroll
+  for (int r = 0; r < 6; ++r) {
+    const double w = wave_sum64(s[r]);
+    if ((t & 63) == 0) sm[r][t >> 6] = w;
+  }
+  __syncthreads();
+  if (t == 6) out[6] = (double)flags[0];
+  if (t >= 6) return;
+  double sum = 0.0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) sum += sm[t][w];
+  out[t < 2 ? 1 + t : t == 2 ? 0 : t] = t < 2 ? 2.0 * sum : sum;
 }
 
 // Symmetric box: max |coordinate| per axis, in two stages (per-block maxima,
@@ -309,7 +356,7 @@ int launch_post(aster_ctx* c, const StepPost& post, bool box) {
   }
 }
 
-int launch_energy(aster_ctx* c, double* out6) {
+int launch_energy(aster_ctx* c, double* out7) {
   const int n = (int)c->n;
   const int ntiles = (n + 63) / 64;
   // one tile per wavefront up to 128 tiles; above, strips that keep about 16384
@@ -325,9 +372,9 @@ int launch_energy(aster_ctx* c, double* out6) {
                      c->P.softening, c->ework.p, rows);
   ASTER_HIP(c, hipGetLastError());
   hipLaunchKernelGGL(k_energy_reduce, dim3(1), dim3(1024), 0, c->stream, (int)slots, ntiles, (const double*)c->ework.p,
-                     (const double*)rows, c->eout.p);
+                     (const double*)rows, (const uint32_t*)c->flags.p, c->eout.p);
   ASTER_HIP(c, hipGetLastError());
-  ASTER_HIP(c, hipMemcpyAsync(out6, c->eout.p, 6 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  ASTER_HIP(c, hipMemcpyAsync(out7, c->eout.p, 7 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   ASTER_HIP(c, hipStreamSynchronize(c->stream));
   return ASTER_OK;
 }
