@@ -151,8 +151,8 @@ int aster_destroy(aster_ctx* c) {
   c->apart.release(); c->apn.release(); c->ework.release(); c->eout.release(); c->flags.release();
   c->boxpart.release(); c->boxd.release(); c->stage.release();
   c->codes.release(); c->xm4.release(); c->idx.release(); c->kv.release(); c->rows.release(); c->rowsum.release();
-  c->left.release(); c->right.release(); c->parent.release(); c->escape.release(); c->scanpart.release();
-  c->depth.release(); c->nmc.release(); c->nvel.release(); c->nbox.release();
+  c->left.release(); c->right.release(); c->parent.release(); c->scanpart.release();
+  c->nmc.release(); c->nvel.release(); c->nbox.release();
   c->above.release(); c->units.release(); c->top.release(); c->grange.release(); c->gscan.release();
   c->gstart.release(); c->gcount.release(); c->splitnode.release();
   c->nrec.release(); c->nlink.release(); c->kids.release(); c->topslot.release(); c->bh_counters.release(); c->gsh.release();

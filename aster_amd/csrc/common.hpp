@@ -158,9 +158,8 @@ struct aster_ctx {
   aster::DBuf<double4> xm4;                        // {x, y, z, m} per body (body order), n
   aster::DBuf<uint32_t> rows;                      // the sort's digit counts per pass and tile
   aster::DBuf<uint2> rowsum;                       // their sums over groups of tiles
-  aster::DBuf<int32_t> left, right, parent, escape;// 2n-1
+  aster::DBuf<int32_t> left, right, parent;        // 2n-1
   aster::DBuf<uint32_t> scanpart;                  // per-chunk totals of the device scan
-  aster::DBuf<int32_t> depth;                      // 2n-1
   aster::DBuf<int32_t> splitnode;                  // internal node whose split lies after sorted position k (n-1)
   aster::DBuf<uint32_t> above;                     // lengths of the lists units, top (2)
   aster::DBuf<int32_t> units;                      // largest nodes above the groups of at most kUnit leaves
@@ -173,7 +172,7 @@ struct aster_ctx {
   aster::DBuf<double4> nvel;                       // FP64 {mass-weighted velocity, 0} per node (1PN only)
   aster::DBuf<float4> nbox;                        // FP32 AABB: {lo, 0}, {hi, 0} per node (2 (2n-1))
   aster::DBuf<float4> nrec;                        // FP32 node record: com, mass (2n-1)
-  aster::DBuf<int4> nlink;                         // right, escape, crit2 bits, leaf body (2n-1)
+  aster::DBuf<int4> nlink;                         // right, escape, crit2 bits, leaf: body, else depth (2n-1)
   aster::DBuf<int32_t> topslot;                    // node - n -> position in top (n)
   aster::DBuf<float4> kids;                        // group traversal: per child slot {record}, {node, crit2} (2(2n-1))
   aster::DBuf<unsigned long long> bh_counters;     // BHC_COUNT
