@@ -32,7 +32,11 @@ namespace aster {
 // Depth bound of the radix tree: an internal node's split bit strictly
 // increases with depth over 30 code bits + 32 tie-break bits, so depth <= 63.
 constexpr int kMaxLevels = 128;
-constexpr int kUnit = 4096;  // leaves per unit of the moments above the groups
+// Leaves per unit of the moments above the groups. Step of the group method, us,
+// with units of 2048 / 4096 / 8192 / 16384 leaves: 4000 bodies 95.5 / 93.1 / 93.2 /
+// 93.6, 50000 155.7 / 155.9 / 149.4 / 154.1, 2^20 974 / 917 / 904 / 923, 2^21 1845 /
+// 1769 / 1697 / 1695.
+constexpr int kUnit = 8192;
 // Traversal groups (and the moment kernel's per-wavefront subtrees): subtrees
 // of at most kGroup leaves whose parent has more.
 constexpr int kGroup = 64;
@@ -840,14 +844,15 @@ __global__ __launch_bounds__(256) void k_group_moments(int n, const int32_t* __r
 // LDS. A flag holds the sweep its node was formed in, and only earlier sweeps
 // count, so a sweep needs no second barrier and the records' order never
 // depends on timing. More nodes than threads (a unit of many small groups, more
-// than ~1.4 million bodies): the threads take turns and the records pass
+// than ~2.7 million bodies): the threads take turns and the records pass
 // through global memory. Bound: latency, ~4 dependent loads and a sweep per
 // level (at most 47 levels up to 2^17 bodies: 30 code bits, 17 of position).
 // Neither the host nor a level census is needed to order the launches: against
 // the census (four launches, a readback and a wait), bands of levels and a top
 // pass, the tree's part of a step falls from 167 to 127 us at 50000 bodies
 // (these two launches 16 + 9 us) and from 331 to 280 us at 2^20 (15 + 30 us).
-// With the records stored after the sweeps: 12 + 7 and 12 + 23 us.
+// With the records stored after the sweeps 12 + 7 and 12 + 23 us (units of 4096
+// leaves).
 template <bool VEL, int CAP>
 struct MomLds {
   double4 com[CAP];
@@ -868,7 +873,7 @@ struct MomLds {
   }
 };
 
-constexpr int kUnitThreads = 256;
+constexpr int kUnitThreads = 512;
 constexpr int kTopThreads = 512;
 
 template <bool VEL, bool TOP>

@@ -68,8 +68,34 @@ def test_inputs_exceed_the_threads(orc, nclusters, core, in_unit, top):
     assert most > in_unit or in_unit == 0
 
 
+# more than 512 nodes above units of 8192 leaves; units of that size with more than 512 nodes
+CASES8 = [(25, 8300, 0, 512), (60, 130, 512, 0)]
+
+
+@pytest.mark.parametrize("nclusters,core,in_unit,top", CASES8)
+def test_inputs_exceed_the_threads_of_larger_units(orc, nclusters, core, in_unit, top):
+    pos, vel, mass = chains(nclusters, core)
+    n = len(mass)
+    t = orc.build_tree(pos, vel, mass, BOX)
+    size = sizes(t["left"], t["right"], n)
+    big = np.flatnonzero(size > 8192)
+    assert len(big) >= top
+    inside = [sum(1 for k in subtree(t, r) if size[k] > 64) for p in big for r in (t["left"][p], t["right"][p])
+              if 64 < size[r] <= 8192]
+    assert max(inside) > in_unit
+
+
+def subtree(t, root):
+    stack = [int(root)]
+    while stack:
+        k = stack.pop()
+        yield k
+        if t["left"][k] >= 0:
+            stack += [int(t["left"][k]), int(t["right"][k])]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("nclusters,core,in_unit,top", CASES)
+@pytest.mark.parametrize("nclusters,core,in_unit,top", CASES + CASES8[:1])
 def test_moments_of_many_nodes(ctx, orc, nclusters, core, in_unit, top):
     """The tree's bits for each traversal, the lists, and the velocity moments through the post-Newtonian part (bars of the
     traversal's own tests)."""
