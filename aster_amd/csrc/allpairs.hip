@@ -816,10 +816,15 @@ int fp32_scales(aster_ctx* c, Fp32Scales* sc) {
 // 90, 4096 95 / 11.6 / 16.9 / 89, 8192 92 / 30 / 28 / 93, 16384 110 / 130 / 85 /
 // 106, 20011 165 / 164 / 129 / 160, 32768 322 / 447 / 311 / 318, 65536 1135 /
 // 1699 / 1211 / 1127. One launch fills the 256 CUs once up to 4096 bodies (16
-// targets a block); above 32768 the scalar reads, which take no LDS bandwidth,
-// hide their latency behind enough waves.
+// targets a block); above the line the scalar reads, which take no LDS bandwidth,
+// hide their latency behind enough waves: k_allpairs_f32 against tiles by slices,
+// mixed 24000 286 / 251, 26000 312 / 287, 28000 330 / 333, 30000 358 / 378, 31610
+// 407 / 420; plain 28000 250 / 240, 32768 319 / 310.
 static bool one_launch(int64_t n) { return n <= 4096; }
-static bool in_tiles(int64_t n) { return n <= 32768; }
+template <bool SRC64>
+static bool in_tiles(int64_t n) {
+  return n <= (SRC64 ? 26624 : 32768);
+}
 
 template <int W, int GR, bool SRC64>
 static void launch_tiles_as(hipStream_t st, bool mask, const SrcRange& r, const double* x, const double* m,
@@ -886,7 +891,7 @@ static int allpairs_f32(aster_ctx* c, DBuf<typename SrcT<SRC64>::type>& srcbuf, 
   const SrcReady want{c->x.p, c->n, SRC64 ? 2 : 1, lower, upper, sc.msc};
   const bool have = c->src_ready == want;
   c->src_ready = SrcReady{};
-  if (in_tiles(n)) {
+  if (in_tiles<SRC64>(n)) {
     Finish f{};
     f.part = c->apart.p;
     phase_begin(c, ASTER_PHASE_ALLPAIRS);
@@ -1099,7 +1104,7 @@ extern "C" int aster_forces_noalloc(int64_t n, const double* d_pos, const double
     const Finish f{nullptr, nullptr, 0.0, scale + 1, d_acc, 1, StepPost{}, nullptr, nullptr, nullptr};
     launch_tiles<true>(st, mask, r, x, d_mass, sp, S, eps2, f);
   } else {
-    if (in_tiles(n)) {
+    if (in_tiles<true>(n)) {
       Finish f{};
       f.part = part;
       launch_tiles<true>(st, mask, r, x, d_mass, sp, S, eps2, f);

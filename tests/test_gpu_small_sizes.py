@@ -157,3 +157,10 @@ def test_ensembles_same_bits_whatever_their_number(ctx, largest, flags, precisio
         out.append((p[:n], v[:n]))
     for p, v in out:
         assert np.all(np.isfinite(p)) and np.array_equal(p, out[-1][0]) and np.array_equal(v, out[-1][1])
+
+
+@pytest.mark.parametrize("n", [26624, 26625])
+def test_fp32_forces_at_the_mixed_line(ctx, n):
+    """Both sides of the line between the mixed method's kernels: the bars of the other sizes, and fused updates."""
+    test_fp32_forces_against_fp64(ctx, n, 2.5e-5)
+    test_fused_updates_same_bits_as_separate_calls(ctx, n, A.ALLPAIRS_FP32_KAHAN)
