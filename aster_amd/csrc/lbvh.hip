@@ -852,7 +852,7 @@ __global__ __launch_bounds__(256) void k_group_moments(int n, const int32_t* __r
 // pass, the tree's part of a step falls from 167 to 127 us at 50000 bodies
 // (these two launches 16 + 9 us) and from 331 to 280 us at 2^20 (15 + 30 us).
 // With the records stored after the sweeps 12 + 7 and 12 + 23 us (units of 4096
-// leaves).
+// leaves), with units of 8192 13 + 16 us at 2^20.
 template <bool VEL, int CAP>
 struct MomLds {
   double4 com[CAP];

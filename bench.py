@@ -46,16 +46,17 @@ HBM_PEAK_GBPS = 8000.0    # MI355X published HBM3E bandwidth
 
 # Algorithmic HBM bytes per body of the bandwidth-bound phases of a BH step
 # (what each phase must read and write once):
-#  morton: Morton pass 24 B x + 8 B m read, 4 B code + 4 B index + 32 B
-#          {x, m} record written (the box's maxima come from the drift that
-#          wrote x; the drift reads x anyway);
-#  sort: 4 passes x (4 B histogram read + 8 B key/value read + 8 B written);
+#  morton: Morton pass 24 B x + 8 B m read, 4 B code + 32 B {x, m} record
+#          written (the box's maxima come from the drift that wrote x; the
+#          drift reads x anyway);
+#  sort: 3 passes x (8 B key/value read + 8 B written), the first without the
+#        values' read, and 8 B read for the digit counts of the other two;
 #  build: 4 B code + 4 B permutation + 32 B record read, 48 B of leaf records
 #         (FP64 {x, m}, FP32 sorted body) and 24 B of internal-node links
-#         (left, right, parent, range, split) written, plus the group pass's
-#         12 B (start flag, climb, root);
+#         (left, right, range, split, group flag) written, and the scan's two
+#         4 B reads of the flags;
 #  kickdrift: FP64 x, v, a read (72 B), x, v written (48 B).
-PHASE_BYTES_PER_BODY = {"morton": 24 + 8 + 4 + 4 + 32, "sort": 4 * (4 + 8 + 8), "build": 4 + 4 + 32 + 48 + 24 + 12,
+PHASE_BYTES_PER_BODY = {"morton": 24 + 8 + 4 + 32, "sort": 3 * (8 + 8) - 4 + 2 * 8, "build": 4 + 4 + 32 + 48 + 24 + 8,
                         "kickdrift": 72 + 48}
 
 
