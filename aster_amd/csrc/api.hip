@@ -151,7 +151,7 @@ int aster_destroy(aster_ctx* c) {
   c->apart.release(); c->apn.release(); c->ework.release(); c->eout.release(); c->flags.release();
   c->boxpart.release(); c->boxd.release(); c->stage.release();
   c->codes.release(); c->xm4.release(); c->idx.release(); c->kv.release(); c->rows.release(); c->rowsum.release();
-  c->left.release(); c->right.release(); c->parent.release(); c->scanpart.release();
+  c->left.release(); c->right.release(); c->parent.release(); c->gflag.release(); c->gpart.release();
   c->nmc.release(); c->nvel.release(); c->nbox.release();
   c->above.release(); c->units.release(); c->top.release(); c->grange.release(); c->gscan.release();
   c->gstart.release(); c->gcount.release(); c->splitnode.release();

@@ -159,13 +159,14 @@ struct aster_ctx {
   aster::DBuf<uint32_t> rows;                      // the sort's digit counts per pass and tile
   aster::DBuf<uint2> rowsum;                       // their sums over groups of tiles
   aster::DBuf<int32_t> left, right, parent;        // 2n-1
-  aster::DBuf<uint32_t> scanpart;                  // per-chunk totals of the device scan
   aster::DBuf<int32_t> splitnode;                  // internal node whose split lies after sorted position k (n-1)
   aster::DBuf<uint32_t> above;                     // lengths of the lists units, top (2)
   aster::DBuf<int32_t> units;                      // largest nodes above the groups of at most kUnit leaves
   aster::DBuf<int32_t> top;                        // nodes of more than kUnit leaves (n)
   aster::DBuf<int2> grange;                        // sorted-position range of internal node n+i
-  aster::DBuf<uint32_t> gscan;                     // group-start flags, then their exclusive scan (n)
+  aster::DBuf<uint8_t> gflag;                      // 1 where a group starts (n, to a multiple of 16)
+  aster::DBuf<uint32_t> gpart;                     // groups per chunk of positions (k_group_counts)
+  aster::DBuf<uint32_t> gscan;                     // the group that starts at a position, where one does (n)
   aster::DBuf<int32_t> gstart;                     // first sorted position of each group (+ n)
   aster::DBuf<uint32_t> gcount;                    // number of groups (1)
   aster::DBuf<double4> nmc;                        // FP64 {com, mass} per node (2n-1)

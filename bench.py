@@ -52,11 +52,11 @@ HBM_PEAK_GBPS = 8000.0    # MI355X published HBM3E bandwidth
 #  sort: 3 passes x (8 B key/value read + 8 B written), the first without the
 #        values' read, and 8 B read for the digit counts of the other two;
 #  build: 4 B code + 4 B permutation + 32 B record read, 48 B of leaf records
-#         (FP64 {x, m}, FP32 sorted body) and 24 B of internal-node links
-#         (left, right, range, split, group flag) written, and the scan's two
-#         4 B reads of the flags;
+#         (FP64 {x, m}, FP32 sorted body) and 20 B of internal-node links
+#         (left, right, range, split) and a 1 B group flag written, and the
+#         flag read twice;
 #  kickdrift: FP64 x, v, a read (72 B), x, v written (48 B).
-PHASE_BYTES_PER_BODY = {"morton": 24 + 8 + 4 + 32, "sort": 3 * (8 + 8) - 4 + 2 * 8, "build": 4 + 4 + 32 + 48 + 24 + 8,
+PHASE_BYTES_PER_BODY = {"morton": 24 + 8 + 4 + 32, "sort": 3 * (8 + 8) - 4 + 2 * 8, "build": 4 + 4 + 32 + 48 + 20 + 3,
                         "kickdrift": 72 + 48}
 
 

@@ -177,3 +177,20 @@ def test_wavefronts_per_group(ctx, orc, n, flags):
     scale = np.linalg.norm(ref, axis=1)
     err = np.linalg.norm(both - newton - ref, axis=1)
     assert np.all(err <= 1e-9 * np.maximum(scale, np.median(scale)) + 1e-15 * np.abs(both).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 16383, 16384, 16385, 131072, 131073, 147457, 1 << 20, (1 << 20) + 1, (1 << 20) + 16400])
+def test_group_starts_at_the_edges_of_chunks(ctx, orc, n):
+    """The groups decide both counts of the lists and which nodes' moments are formed where."""
+    pos, vel, mass = A.ic_mixed(n, 9)
+    box = orc.box_auto(pos)
+    ref = orc.build_tree(pos, vel, mass, box)
+    ctx.set_params(G=1.0, softening=2.5e-5, theta=0.7)
+    ctx.set_state(pos, vel, mass)
+    ctx.forces(A.BH_GROUP, out=False)
+    _, inter, visits = orc.bh_group(pos, mass, box, 0.7, soft=2.5e-5)
+    assert ctx.bh_stats() == (inter, visits)
+    tree = ctx.tree()
+    for key in ("perm", "left", "right", "mass", "com"):
+        assert np.array_equal(tree[key], ref[key]), key
