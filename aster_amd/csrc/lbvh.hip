@@ -85,7 +85,7 @@ constexpr int kRsPasses = 3;
 constexpr int kRsThreads = 512;
 constexpr int kRsGroup = 64;
 constexpr int kRsSmall = 4096;  // keys that one workgroup sorts by itself
-constexpr int kRsMaxRows = 128;  // more tiles: in groups
+constexpr int kRsMaxRows = 64;  // more tiles: in groups
 constexpr int kRsAhead = 8;
 
 __device__ __forceinline__ uint32_t rs_digit(uint32_t key, int pass) {
@@ -116,23 +116,38 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_hist(const uint2* __restrict_
   for (int i = t; i < kRsWords; i += T) rows[(size_t)blockIdx.x * kRsWords + i] = cnt[i];
 }
 
-// Sums of kRsGroup rows: {even digit, odd digit} per word.
+// Sums of kRsGroup rows: {even digit, odd digit} per word. A workgroup takes
+// kRsWords / kRsShare words; kRsShare threads share a word and take a run of
+// rows each, so that all loads of a thread are in flight at once (one thread per
+// word and 8 rounds of loads: step at 600000 bodies 578 -> 567 us, 2^20 918 ->
+// 905).
+constexpr int kRsShare = 4;
 __global__ __launch_bounds__(kRsWords) void k_rs_groups(const uint32_t* __restrict__ rows, int ntiles,
                                                         uint2* __restrict__ groups) {
-  const int t = threadIdx.x, b0 = blockIdx.x * kRsGroup, b1 = min(b0 + kRsGroup, ntiles);
+  constexpr int kWords = kRsWords / kRsShare, kRows = kRsGroup / kRsShare;
+  __shared__ uint2 part[kRsWords];
+  const int t = threadIdx.x, word = blockIdx.y * kWords + t % kWords;
+  const int b0 = blockIdx.x * kRsGroup + t / kWords * kRows;
+  uint32_t c[kRows];
+#pragma unroll
+  for (int u = 0; u < kRows; ++u) c[u] = rows[(size_t)min(b0 + u, ntiles - 1) * kRsWords + word];
   uint2 s = make_uint2(0u, 0u);
-  for (int b = b0; b < b1; b += 8) {
-    uint32_t c[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) c[u] = rows[(size_t)min(b + u, b1 - 1) * kRsWords + t];
+  for (int u = 0; u < kRows; ++u)
+    if (b0 + u < ntiles) {
+      s.x += c[u] & 0xffffu;
+      s.y += c[u] >> 16;
+    }
+  part[t] = s;
+  __syncthreads();
+  if (t < kWords) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (b + u < b1) {
-        s.x += c[u] & 0xffffu;
-        s.y += c[u] >> 16;
-      }
+    for (int q = 1; q < kRsShare; ++q) {
+      s.x += part[t + q * kWords].x;
+      s.y += part[t + q * kWords].y;
+    }
+    groups[(size_t)blockIdx.x * kRsWords + word] = s;
   }
-  groups[(size_t)blockIdx.x * kRsWords + t] = s;
 }
 
 // Inclusive sum over the lanes of a wavefront.
@@ -1723,11 +1738,13 @@ struct SortPlan {
 // Few keys per thread shorten the serial ranking of a tile, many tiles lengthen
 // the sums of their rows. Leapfrog step of the group method, us, with 2 / 4 / 8
 // keys: 20000 bodies 137 / 140 / 150, 50000 163 / 164 / 174, 262144 343 / 337 /
-// 336, 524288 550 / 546 / 529 (16 keys: 538). Summing the rows themselves beyond
-// 128 tiles would be 40 rounds of loads at 2^20 keys.
+// 336, and with the rows' groups summed by 4 threads a word 4 / 8 keys: 400000 433
+// / 433, 524288 524 / 535, 2^20 905 / 894. Rows summed in groups above 128 / 64 /
+// 32 tiles: 100000 (49 tiles) 191 / 191 / 199, 200000 273 / 268 / 269, 262144 321 /
+// 315 / 318.
 static SortPlan sort_plan(int64_t n) {
   SortPlan p{};
-  p.keys = n <= (1 << 15) ? 2 : n <= (1 << 18) ? 4 : 8;
+  p.keys = n <= (1 << 15) ? 2 : n <= (1 << 19) ? 4 : 8;
   p.tiles = (int)((n + p.keys * kRsThreads - 1) / (p.keys * kRsThreads));
   p.groups = p.tiles > kRsMaxRows;
   return p;
@@ -1842,7 +1859,7 @@ int morton_sort(aster_ctx* c, bool user_box) {
       if (pass > 0)
         hipLaunchKernelGGL((k_rs_hist<K()>), grid, block, 0, c->stream, kin, n, pass, c->rows.p);
       if (p.groups)
-        hipLaunchKernelGGL(k_rs_groups, dim3((p.tiles + kRsGroup - 1) / kRsGroup), dim3(kRsWords), 0, c->stream,
+        hipLaunchKernelGGL(k_rs_groups, dim3((p.tiles + kRsGroup - 1) / kRsGroup, kRsShare), dim3(kRsWords), 0, c->stream,
                            c->rows.p, p.tiles, c->rowsum.p);
       auto kern = p.groups ? k_rs_scatter<K(), true> : k_rs_scatter<K(), false>;
       hipLaunchKernelGGL(kern, grid, block, 0, c->stream, c->codes.p, kin, kout, c->codes.p, c->idx.p, n, pass,
