@@ -75,7 +75,7 @@ __device__ __forceinline__ uint32_t cell_of(double p, double b, uint32_t* bad) {
 // reads the groups' sums and at most kRsGroup rows. Bound: latency below ~2^19
 // keys (a scatter is one chain of loads, ranks and stores), with launches as
 // long as they can be short. Against 4 passes of 8 bits with counts and keys in
-// separate arrays: sort 54 -> 31 us at 50000 keys, 84 -> 72 us at 2^20. (Adding
+// separate arrays: sort 54 -> 31 us at 50000 keys, 84 -> 65 us at 2^20. (Adding
 // each key to its next tile's counts while scattering, instead of k_rs_hist,
 // was slower: 50000 bodies +25 us, many equal keys +200 us at 20000.)
 constexpr int kDigBits = 10;
@@ -83,7 +83,7 @@ constexpr int kDigits = 1 << kDigBits;
 constexpr int kRsWords = kDigits / 2;
 constexpr int kRsPasses = 3;
 constexpr int kRsThreads = 512;
-constexpr int kRsGroup = 64;
+constexpr int kRsGroup = 32;
 constexpr int kRsSmall = 4096;  // keys that one workgroup sorts by itself
 constexpr int kRsMaxRows = 64;  // more tiles: in groups
 constexpr int kRsAhead = 8;
@@ -118,9 +118,9 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_hist(const uint2* __restrict_
 
 // Sums of kRsGroup rows: {even digit, odd digit} per word. A workgroup takes
 // kRsWords / kRsShare words; kRsShare threads share a word and take a run of
-// rows each, so that all loads of a thread are in flight at once (one thread per
-// word and 8 rounds of loads: step at 600000 bodies 578 -> 567 us, 2^20 918 ->
-// 905).
+// rows each, so that all loads of a thread are in flight at once (64 rows, one
+// thread per word and 8 rounds of loads: the sort's kernels at 2^20 72.3 us; 64 rows
+// and 4 threads 67.1, 32 rows and 4 threads 64.5, 16 rows 65.6).
 constexpr int kRsShare = 4;
 __global__ __launch_bounds__(kRsWords) void k_rs_groups(const uint32_t* __restrict__ rows, int ntiles,
                                                         uint2* __restrict__ groups) {
@@ -312,13 +312,20 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const uint32_t* __res
   if (GROUPS) {
     const int ng = (ntiles + kRsGroup - 1) / kRsGroup, g = blk / kRsGroup;
     const uint4* __restrict__ gs = reinterpret_cast<const uint4*>(groups) + 2 * wg;
-    for (int b = q; b < ng; b += Q) {
-      const uint4 c0 = gs[(size_t)b * (kDigits / 4)], c1 = gs[(size_t)b * (kDigits / 4) + 1];
-      const uint32_t e[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+    for (int b = q; b < ng; b += 2 * Q) {
+      uint4 c[4];
 #pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        tot[v] += e[v];
-        pre[v] += b < g ? e[v] : 0u;
+      for (int u = 0; u < 4; ++u) c[u] = gs[(size_t)min(b + u / 2 * Q, ng - 1) * (kDigits / 4) + u % 2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const bool in = b + u * Q < ng, before = b + u * Q < g;
+        const uint4 &c0 = c[2 * u], &c1 = c[2 * u + 1];
+        const uint32_t e[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+#pragma unroll
+        for (int v = 0; v < 8; ++v) {
+          tot[v] += in ? e[v] : 0u;
+          pre[v] += before ? e[v] : 0u;
+        }
       }
     }
   }
@@ -1738,10 +1745,9 @@ struct SortPlan {
 // Few keys per thread shorten the serial ranking of a tile, many tiles lengthen
 // the sums of their rows. Leapfrog step of the group method, us, with 2 / 4 / 8
 // keys: 20000 bodies 137 / 140 / 150, 50000 163 / 164 / 174, 262144 343 / 337 /
-// 336, and with the rows' groups summed by 4 threads a word 4 / 8 keys: 400000 433
-// / 433, 524288 524 / 535, 2^20 905 / 894. Rows summed in groups above 128 / 64 /
-// 32 tiles: 100000 (49 tiles) 191 / 191 / 199, 200000 273 / 268 / 269, 262144 321 /
-// 315 / 318.
+// 336. The sort's kernels, us: 524288 bodies 4 / 8 keys 54.2 / 57.6; 262144 rows
+// summed in groups above 128 / 64 tiles 51.7 / 50.3 (above 32, step at 100000 191
+// -> 199).
 static SortPlan sort_plan(int64_t n) {
   SortPlan p{};
   p.keys = n <= (1 << 15) ? 2 : n <= (1 << 19) ? 4 : 8;
