@@ -180,7 +180,8 @@ def test_wavefronts_per_group(ctx, orc, n, flags):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [2, 15, 16, 17, 16383, 16384, 16385, 131072, 131073, 147457, 1 << 20, (1 << 20) + 1, (1 << 20) + 16400])
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 16383, 16384, 16385, 131072, 131073, 147457, 1 << 20, (1 << 20) + 1,
+                               (1 << 20) + 16400])
 def test_group_starts_at_the_edges_of_chunks(ctx, orc, n):
     """The groups decide both counts of the lists and which nodes' moments are formed where."""
     pos, vel, mass = A.ic_mixed(n, 9)
