@@ -1657,6 +1657,7 @@ int aster_batch_set(aster_ctx* c, int64_t nsys, const int64_t* offsets, const do
   ASTER_HIP(c, hipSetDevice(c->device));
   BatchState& B = c->batch;
   drop_graph(B);
+  B.traj_ready = false;  // a stored trajectory is that of the systems before
   B.nsys = nsys;
   B.nbodies = nb;
   B.offsets.assign(offsets, offsets + nsys + 1);

@@ -1,0 +1,29 @@
+"""What a trajectory gradient's two passes leave and expect: systems loaded, parameters changed or steps taken between or
+after them."""
+import numpy as np
+import pytest
+
+import aster_amd as A
+
+pytestmark = pytest.mark.gpu
+
+
+def systems(sizes, seed=1):
+    n, rng = sum(sizes), np.random.default_rng(seed)
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    return off, rng.normal(size=(n, 3)), 0.1 * rng.normal(size=(n, 3)), rng.uniform(0.5, 1.5, n)
+
+
+@pytest.mark.parametrize("sizes", [[3] * 4, [3] * 400, [5, 2, 64], [3]])
+def test_loading_systems_drops_the_stored_trajectory(ctx, sizes):
+    """The backward pass refuses (on the host) after other systems, fewer or more, were loaded."""
+    ctx.set_params(G=1.0, softening=1e-2)
+    ctx.batch_set(*systems([3] * 4))
+    ctx.batch_traj_forward(1e-2, 4, [4])
+    e = systems(sizes, 2)
+    ctx.batch_set(*e)
+    with pytest.raises(A.AsterError) as err:
+        ctx.batch_traj_backward(np.zeros((1, sum(sizes), 3)))
+    assert err.value.code == -6  # ASTER_ERR_STATE
+    p, v = ctx.batch_get()
+    assert np.array_equal(p, e[1]) and np.array_equal(v, e[2])
