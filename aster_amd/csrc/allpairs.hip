@@ -863,8 +863,9 @@ static int allpairs_f32(aster_ctx* c, DBuf<typename SrcT<SRC64>::type>& srcbuf, 
   if (rc) return rc;
   const SrcRange r{n, lower, upper, sc.msc, nullptr};
   // Slices over the tiles that hold the source range (sources outside it and
-  // the padding bodies have zero mass).
-  const int j0 = lower / kApTile * kApTile;
+  // the padding bodies have zero mass); an empty range behind the last body
+  // takes the last tile.
+  const int j0 = std::min(lower, npad - 1) / kApTile * kApTile;
   const int span = std::max<int>(j0 + kApTile, (int)round_up(upper, kApTile)) - j0;
   int S = 0, slice = 0;
   slice_span(span, choose_split(c), &S, &slice);
