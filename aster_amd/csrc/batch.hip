@@ -1450,7 +1450,6 @@ __global__ __launch_bounds__(256) void k_batch_traj_fwd(BatchArgs P, TrajArgs Q)
     for (int c = 0; c < 3; ++c) {
       P.x[3 * (size_t)b + c] = X[c];
       P.v[3 * (size_t)b + c] = V[c] + half * a[c] * dt;
-      P.a[3 * (size_t)b + c] = P.G * a[c];
     }
 }
 
@@ -1592,7 +1591,7 @@ int batch_traj_forward(aster_ctx* c, double dt, int64_t nsteps, int32_t nsnap, c
   hipLaunchKernelGGL(t.triples ? k_batch_traj_fwd<true> : k_batch_traj_fwd<false>,
                      dim3((t.nwaves + t.wpb - 1) / t.wpb), dim3(64 * t.wpb), 0, c->stream, P, Q);
   ASTER_HIP(c, hipGetLastError());
-  B.a_valid = true;
+  B.a_valid = false;  // this kernel's accelerations have not the bits of batch_step's
   if (snap_pos && nsnap > 0)
     ASTER_HIP(c, hipMemcpyAsync(snap_pos, B.tgrad.p, nsnap * nb3 * 8, hipMemcpyDeviceToHost, c->stream));
   ASTER_HIP(c, hipStreamSynchronize(c->stream));

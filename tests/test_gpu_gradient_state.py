@@ -27,3 +27,26 @@ def test_loading_systems_drops_the_stored_trajectory(ctx, sizes):
     assert err.value.code == -6  # ASTER_ERR_STATE
     p, v = ctx.batch_get()
     assert np.array_equal(p, e[1]) and np.array_equal(v, e[2])
+
+
+@pytest.mark.parametrize("precision", [A.FP64, A.FP32])
+@pytest.mark.parametrize("sizes", [[3] * 40, [1, 2, 3, 17, 64]])
+def test_steps_after_a_forward_pass(ctx, orc, sizes, precision):
+    """They begin with an evaluation of their own: the bits of the same state loaded afresh, in the exact mode those of the
+    oracle."""
+    off, pos, vel, mass = systems(sizes)
+    ctx.set_params(G=1.1, softening=1e-2, precision=precision)
+    ctx.batch_set(off, pos, vel, mass)
+    ctx.batch_step(A.LEAPFROG, 1e-2, 2)
+    ctx.batch_traj_forward(1e-2, 3, [3])
+    p0, v0 = ctx.batch_get()
+    ctx.batch_step(A.LEAPFROG, 1e-2, 4)
+    p, v = ctx.batch_get()
+    ctx.batch_set(off, p0, v0, mass)
+    ctx.batch_step(A.LEAPFROG, 1e-2, 4)
+    q, w = ctx.batch_get()
+    assert np.array_equal(p, q) and np.array_equal(v, w)
+    if precision == A.FP64:
+        for a, b in zip(off[:-1], off[1:]):
+            rp, rv, _ = orc.integrate(p0[a:b], v0[a:b], mass[a:b], 1e-2, 4, integrator=2, G=1.1, soft=1e-2)
+            assert np.array_equal(p[a:b], rp) and np.array_equal(v[a:b], rv)
