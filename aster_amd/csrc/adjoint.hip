@@ -440,6 +440,8 @@ int traj_forward(aster_ctx* c, double dt, int64_t nsteps, int64_t ckpt, int32_t 
   S.ckpt_every = ckpt;
   S.nsnap = nsnap;
   S.dt = dt;
+  S.G = c->P.G;
+  S.softening = c->P.softening;
   S.snap_steps.assign(snaps, snaps + nsnap);
   int rc;
   const int method = ASTER_ALLPAIRS_FP32_KAHAN;
@@ -472,7 +474,7 @@ int traj_forward(aster_ctx* c, double dt, int64_t nsteps, int64_t ckpt, int32_t 
   return ASTER_OK;
 }
 
-int traj_backward(aster_ctx* c, const double* gsnap, double* gx, double* gv, double* gm) {
+static int backward_passes(aster_ctx* c, const double* gsnap, double* gx, double* gv, double* gm) {
   AdjointState& S = c->adj;
   if (!S.ready) return fail(c, ASTER_ERR_STATE, "call aster_traj_forward first (and do not step in between)");
   if (S.nsnap > 0 && !gsnap) return fail(c, ASTER_ERR_INVALID, "snapshot gradients required");
@@ -581,6 +583,21 @@ int traj_backward(aster_ctx* c, const double* gsnap, double* gx, double* gv, dou
     ASTER_HIP(c, hipStreamSynchronize(c->stream));
   }
   return ASTER_OK;
+}
+
+// The gradient of the trajectory as it was run: with the forward pass's force
+// law, whatever parameters were set since.
+int traj_backward(aster_ctx* c, const double* gsnap, double* gx, double* gv, double* gm) {
+  const double G = c->P.G, soft = c->P.softening;
+  if (c->adj.ready) {
+    c->P.G = c->adj.G;
+    c->P.softening = c->adj.softening;
+  }
+  const int rc = backward_passes(c, gsnap, gx, gv, gm);
+  if (c->P.G != G || c->P.softening != soft) c->acc_valid = false;
+  c->P.G = G;
+  c->P.softening = soft;
+  return rc;
 }
 
 }  // namespace aster

@@ -1598,6 +1598,8 @@ int batch_traj_forward(aster_ctx* c, double dt, int64_t nsteps, int32_t nsnap, c
   B.traj_snaps.assign(snaps, snaps + nsnap);
   B.traj_steps = nsteps;
   B.traj_dt = dt;
+  B.traj_G = P.G;
+  B.traj_soft = P.soft;
   B.traj_ready = true;
   return ASTER_OK;
 }
@@ -1612,7 +1614,9 @@ int batch_traj_backward(aster_ctx* c, const double* gsnap, double* gx, double* g
   if (nsnap > 0)
     ASTER_HIP(c, hipMemcpyAsync(B.tgrad.p, gsnap, nsnap * nb3 * 8, hipMemcpyHostToDevice, c->stream));
   const double h0[3] = {0.0, 0.0, 0.0};
-  const BatchArgs P = make_args(c, 0, 1, h0, 0);
+  BatchArgs P = make_args(c, 0, 1, h0, 0);
+  P.G = B.traj_G;
+  P.soft = B.traj_soft;
   const TrajShape t = traj_shape(B);
   const TrajArgs Q{B.traj.p, B.v0.p, B.tsnap.p, nsnap, B.tgrad.p, B.nbodies, B.traj_steps, B.traj_dt, B.tout.p,
                    t.nwaves};

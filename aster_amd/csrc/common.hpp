@@ -74,6 +74,7 @@ struct BatchState {
   DBuf<int64_t> tsnap;               // snapshot steps on the device
   std::vector<int64_t> traj_snaps;
   int64_t traj_steps = 0;
+  double traj_G = 0.0, traj_soft = 0.0;  // the forward pass's
   double traj_dt = 0.0;
   bool traj_ready = false;
 };
@@ -104,6 +105,7 @@ struct AdjointState {
   int32_t nsnap = 0;
   double dt = 0.0;
   std::vector<int64_t> snap_steps;
+  double G = 0.0, softening = 0.0;  // the forward pass's
   DBuf<double> ckpt_x, ckpt_v;  // (nsteps/ckpt_every + 1) * 3n each
   DBuf<double> lx, lv, lm;      // adjoint accumulators (3n, 3n, n)
   DBuf<double> snapg;           // snapshot positions, then their gradients (nsnap * 3n)

@@ -50,3 +50,35 @@ def test_steps_after_a_forward_pass(ctx, orc, sizes, precision):
         for a, b in zip(off[:-1], off[1:]):
             rp, rv, _ = orc.integrate(p0[a:b], v0[a:b], mass[a:b], 1e-2, 4, integrator=2, G=1.1, soft=1e-2)
             assert np.array_equal(p[a:b], rp) and np.array_equal(v[a:b], rv)
+
+
+@pytest.mark.parametrize("changed", [dict(G=2.5), dict(softening=0.3), dict(theta=0.9)])
+@pytest.mark.parametrize("ensemble", [False, True])
+def test_parameters_set_between_the_passes(ctx, changed, ensemble):
+    """The gradient is that of the trajectory as it was run, and what follows uses the new parameters."""
+    off, pos, vel, mass = systems([3] * 30 + [17])
+    n = len(mass)
+    rng = np.random.default_rng(5)
+    g = rng.normal(size=(2, n, 3))
+    out = []
+    for change in (False, True):
+        ctx.set_params(G=1.0, softening=1e-2, theta=0.5)
+        if ensemble:
+            ctx.batch_set(off, pos, vel, mass)
+            ctx.batch_traj_forward(1e-2, 6, [3, 6])
+        else:
+            ctx.set_state(pos, vel, mass)
+            ctx.traj_forward(1e-2, 6, 4, [3, 6])
+        if change:
+            ctx.set_params(**changed)
+        out.append(ctx.batch_traj_backward(g) if ensemble else ctx.traj_backward(g))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    assert all(getattr(ctx.params(), k) == v for k, v in changed.items())
+    if ensemble or "theta" in changed:  # (without a new force law the backward pass's accelerations serve the next step)
+        return
+    ctx.step(A.ALLPAIRS_FP32_KAHAN, A.LEAPFROG, 1e-2, 1)
+    p, _ = ctx.get_state()
+    ctx.set_state(pos, vel, mass)
+    ctx.step(A.ALLPAIRS_FP32_KAHAN, A.LEAPFROG, 1e-2, 1)
+    assert np.array_equal(p, ctx.get_state()[0])
