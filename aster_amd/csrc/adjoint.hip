@@ -440,8 +440,7 @@ int traj_forward(aster_ctx* c, double dt, int64_t nsteps, int64_t ckpt, int32_t 
   S.ckpt_every = ckpt;
   S.nsnap = nsnap;
   S.dt = dt;
-  S.G = c->P.G;
-  S.softening = c->P.softening;
+  S.P = c->P;
   S.snap_steps.assign(snaps, snaps + nsnap);
   int rc;
   const int method = ASTER_ALLPAIRS_FP32_KAHAN;
@@ -470,6 +469,7 @@ int traj_forward(aster_ctx* c, double dt, int64_t nsteps, int64_t ckpt, int32_t 
         for (int d = 0; d < 3; ++d)
           snap_pos[(size_t)k * n3 + 3 * i + d] = h[(size_t)k * n3 + (size_t)d * n + i];
   }
+  S.own_acc = true;
   S.ready = true;
   return ASTER_OK;
 }
@@ -585,18 +585,21 @@ static int backward_passes(aster_ctx* c, const double* gsnap, double* gx, double
   return ASTER_OK;
 }
 
-// The gradient of the trajectory as it was run: with the forward pass's force
-// law, whatever parameters were set since.
+// The gradient of the trajectory as it was run: with the forward pass's
+// parameters and last accelerations, whatever was set or evaluated since.
 int traj_backward(aster_ctx* c, const double* gsnap, double* gx, double* gv, double* gm) {
-  const double G = c->P.G, soft = c->P.softening;
-  if (c->adj.ready) {
-    c->P.G = c->adj.G;
-    c->P.softening = c->adj.softening;
+  AdjointState& S = c->adj;
+  const aster_params now = c->P;
+  int rc = ASTER_OK;
+  if (S.ready) {
+    c->P = S.P;
+    if (!S.own_acc) rc = compute_forces(c, ASTER_ALLPAIRS_FP32_KAHAN);
   }
-  const int rc = backward_passes(c, gsnap, gx, gv, gm);
-  if (c->P.G != G || c->P.softening != soft) c->acc_valid = false;
-  c->P.G = G;
-  c->P.softening = soft;
+  if (!rc) rc = backward_passes(c, gsnap, gx, gv, gm);
+  c->P = now;
+  if (now.G != S.P.G || now.softening != S.P.softening || now.pn_flags != S.P.pn_flags || now.lower != S.P.lower ||
+      now.upper != S.P.upper)
+    c->acc_valid = false;
   return rc;
 }
 

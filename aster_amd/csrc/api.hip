@@ -51,6 +51,7 @@ static bool is_bh(int m) { return m == ASTER_BH_PARITY || m == ASTER_BH_GEOMETRI
 
 int compute_forces(aster_ctx* c, int method, const StepPost& post) {
   int rc;
+  c->adj.own_acc = false;
   if (is_allpairs(method)) {
     if ((rc = launch_allpairs(c, method, post))) return rc;
   } else if (is_bh(method)) {

@@ -105,7 +105,8 @@ struct AdjointState {
   int32_t nsnap = 0;
   double dt = 0.0;
   std::vector<int64_t> snap_steps;
-  double G = 0.0, softening = 0.0;  // the forward pass's
+  aster_params P{};              // the forward pass's
+  bool own_acc = false;          // c->a still holds its last evaluation
   DBuf<double> ckpt_x, ckpt_v;  // (nsteps/ckpt_every + 1) * 3n each
   DBuf<double> lx, lv, lm;      // adjoint accumulators (3n, 3n, n)
   DBuf<double> snapg;           // snapshot positions, then their gradients (nsnap * 3n)

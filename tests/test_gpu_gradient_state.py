@@ -82,3 +82,29 @@ def test_parameters_set_between_the_passes(ctx, changed, ensemble):
     ctx.set_state(pos, vel, mass)
     ctx.step(A.ALLPAIRS_FP32_KAHAN, A.LEAPFROG, 1e-2, 1)
     assert np.array_equal(p, ctx.get_state()[0])
+
+
+@pytest.mark.parametrize("n", [100, 5000])
+def test_evaluations_between_the_passes(ctx, n):
+    """Accelerations of another method, force law or source range do not enter the time reversal, nor are those of the
+    backward pass taken for the range's."""
+    pos, vel, mass = A.ic_plummer(n, 2)
+    g = np.random.default_rng(5).normal(size=(1, n, 3))
+    out = []
+    for between in (None, dict(lower=n // 2), dict(G=3.0)):
+        ctx.set_params(G=1.0, softening=1e-2, theta=0.8, lower=0)
+        ctx.set_state(pos, vel, mass)
+        ctx.traj_forward(1e-2, 6, 4, [6])
+        if between:
+            ctx.forces(A.BH_GROUP, out=False)
+            ctx.set_params(**between)
+            ctx.forces(A.ALLPAIRS_FP32_KAHAN, out=False)
+        out.append(ctx.traj_backward(g))
+        for a, b in zip(out[0], out[-1]):
+            assert np.array_equal(a, b), between
+        if between:
+            ctx.step(A.ALLPAIRS_FP32_KAHAN, A.LEAPFROG, 1e-2, 1)
+            p, _ = ctx.get_state()
+            ctx.set_state(pos, vel, mass)
+            ctx.step(A.ALLPAIRS_FP32_KAHAN, A.LEAPFROG, 1e-2, 1)
+            assert np.array_equal(p, ctx.get_state()[0])
