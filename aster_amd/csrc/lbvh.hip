@@ -72,7 +72,8 @@ __device__ __forceinline__ uint32_t cell_of(double p, double b, uint32_t* bad) {
 // row b of a pass's table holds tile b's 512 words. The first pass's rows come
 // with the codes (k_morton), the later ones from k_rs_hist. With many tiles the
 // rows are first summed over groups of kRsGroup (k_rs_groups), so that a tile
-// reads the groups' sums and at most kRsGroup rows. Bound: latency below ~2^19
+// reads the groups' sums and at most kRsGroup rows; with many groups these are
+// scanned (k_rs_group_scan) and a tile reads two of them. Bound: latency below ~2^19
 // keys (a scatter is one chain of loads, ranks and stores), with launches as
 // long as they can be short. Against 4 passes of 8 bits with counts and keys in
 // separate arrays: sort 54 -> 31 us at 50000 keys, 84 -> 65 us at 2^20. (Adding
@@ -85,7 +86,8 @@ constexpr int kRsPasses = 3;
 constexpr int kRsThreads = 512;
 constexpr int kRsGroup = 32;
 constexpr int kRsSmall = 4096;  // keys that one workgroup sorts by itself
-constexpr int kRsMaxRows = 64;  // more tiles: in groups
+constexpr int kRsMaxRows = 64;    // more tiles: in groups
+constexpr int kRsMaxGroups = 16;  // more groups: their sums scanned
 constexpr int kRsAhead = 8;
 
 __device__ __forceinline__ uint32_t rs_digit(uint32_t key, int pass) {
@@ -148,6 +150,46 @@ __global__ __launch_bounds__(kRsWords) void k_rs_groups(const uint32_t* __restri
     }
     groups[(size_t)blockIdx.x * kRsWords + word] = s;
   }
+}
+
+// The groups' sums turned into what precedes each group, their totals behind
+// them (row ng): what the tiles read would otherwise grow as the square of the
+// keys. A workgroup takes kRsScanWords words; the threads of a word take a run
+// of groups each. Bound: latency, 4.6 us at 2^24 keys, 7.1 us at 2^26. The sort with
+// the tiles summing all groups / with this: 2^21 keys (16 groups) 95 / 98 us,
+// 3 10^6 137 / 130, 2^22 174 / 155, 2^24 973 / 480 us, 2^26 11.6 / 1.8 ms.
+constexpr int kRsScanThreads = 1024;
+constexpr int kRsScanWords = 16;
+__global__ __launch_bounds__(kRsScanThreads) void k_rs_group_scan(uint2* __restrict__ groups, int ng) {
+  constexpr int kRuns = kRsScanThreads / kRsScanWords;
+  __shared__ uint2 part[kRuns][kRsScanWords];
+  const int t = threadIdx.x, wd = t % kRsScanWords, r = t / kRsScanWords;
+  const int word = blockIdx.x * kRsScanWords + wd;
+  const int len = (ng + kRuns - 1) / kRuns, g0 = min(r * len, ng), g1 = min(g0 + len, ng);
+  uint2 s = make_uint2(0u, 0u);
+  for (int g = g0; g < g1; ++g) {
+    const uint2 c = groups[(size_t)g * kRsWords + word];
+    s.x += c.x;
+    s.y += c.y;
+  }
+  part[r][wd] = s;
+  __syncthreads();
+  for (int off = 1; off < kRuns; off <<= 1) {  // inclusive sums over the runs
+    uint2 y = make_uint2(0u, 0u);
+    if (r >= off) y = part[r - off][wd];
+    __syncthreads();
+    part[r][wd].x += y.x;
+    part[r][wd].y += y.y;
+    __syncthreads();
+  }
+  uint2 run = r > 0 ? part[r - 1][wd] : make_uint2(0u, 0u);
+  for (int g = g0; g < g1; ++g) {
+    const uint2 c = groups[(size_t)g * kRsWords + word];
+    groups[(size_t)g * kRsWords + word] = run;
+    run.x += c.x;
+    run.y += c.y;
+  }
+  if (r == kRuns - 1) groups[(size_t)ng * kRsWords + word] = run;
 }
 
 // Inclusive sum over the lanes of a wavefront.
@@ -269,7 +311,9 @@ __global__ __launch_bounds__(T) void k_rs_small(uint32_t* __restrict__ codes, ui
 // (lpre) and each wavefront's offset inside it; the tile is reordered by digit
 // in LDS and written out with consecutive lanes on consecutive addresses within
 // each digit's run.
-template <int K, bool GROUPS>
+enum { RS_ROWS = 0, RS_GROUPS = 1, RS_SCANNED = 2 };  // what a tile sums: all rows, the groups, neither
+
+template <int K, int SUMS>
 __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const uint32_t* __restrict__ codes, const uint2* __restrict__ kin,
                                                   uint2* __restrict__ kout, uint32_t* __restrict__ codes_out,
                                                   uint32_t* __restrict__ idx_out, int n, int pass,
@@ -309,9 +353,23 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const uint32_t* __res
   // four keep a word each.
   const int wg = t / Q, q = t - wg * Q;
   uint32_t pre[8] = {}, tot[8] = {};
-  if (GROUPS) {
-    const int ng = (ntiles + kRsGroup - 1) / kRsGroup, g = blk / kRsGroup;
-    const uint4* __restrict__ gs = reinterpret_cast<const uint4*>(groups) + 2 * wg;
+  constexpr bool GROUPS = SUMS != RS_ROWS;
+  const int ng = (ntiles + kRsGroup - 1) / kRsGroup, g = blk / kRsGroup;
+  const uint4* __restrict__ gs = reinterpret_cast<const uint4*>(groups) + 2 * wg;
+  if (SUMS == RS_SCANNED) {
+    static_assert(Q >= 2, "a thread for the sums before the group, another for the totals");
+    if (q < 2) {
+      const size_t row = (size_t)(q == 0 ? g : ng) * (kDigits / 4);
+      const uint4 c0 = gs[row], c1 = gs[row + 1];
+      const uint32_t e[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        pre[v] = q == 0 ? e[v] : 0u;
+        tot[v] = q == 1 ? e[v] : 0u;
+      }
+    }
+  }
+  if (SUMS == RS_GROUPS) {
     for (int b = q; b < ng; b += 2 * Q) {
       uint4 c[4];
 #pragma unroll
@@ -1739,7 +1797,7 @@ __global__ void k_zero_counters(unsigned long long* p) {
 // Tiles of the sort: kRsThreads times `keys` keys.
 struct SortPlan {
   int keys, tiles;
-  bool groups;
+  int sums;  // RS_ROWS, RS_GROUPS, RS_SCANNED
 };
 
 // Few keys per thread shorten the serial ranking of a tile, many tiles lengthen
@@ -1752,7 +1810,7 @@ static SortPlan sort_plan(int64_t n) {
   SortPlan p{};
   p.keys = n <= (1 << 15) ? 2 : n <= (1 << 19) ? 4 : 8;
   p.tiles = (int)((n + p.keys * kRsThreads - 1) / (p.keys * kRsThreads));
-  p.groups = p.tiles > kRsMaxRows;
+  p.sums = p.tiles <= kRsMaxRows ? RS_ROWS : p.tiles <= kRsMaxGroups * kRsGroup ? RS_GROUPS : RS_SCANNED;
   return p;
 }
 
@@ -1765,7 +1823,7 @@ static int reserve_sort(aster_ctx* c) {
   ASTER_HIP(c, c->xm4.reserve(n));
   ASTER_HIP(c, c->above.reserve(2));
   ASTER_HIP(c, c->rows.reserve(tiles * kRsWords));
-  ASTER_HIP(c, c->rowsum.reserve((tiles / kRsGroup + 1) * kRsWords));
+  ASTER_HIP(c, c->rowsum.reserve((tiles / kRsGroup + 2) * kRsWords));
   return ASTER_OK;
 }
 
@@ -1864,10 +1922,16 @@ int morton_sort(aster_ctx* c, bool user_box) {
       const dim3 grid(p.tiles), block(kRsThreads);
       if (pass > 0)
         hipLaunchKernelGGL((k_rs_hist<K()>), grid, block, 0, c->stream, kin, n, pass, c->rows.p);
-      if (p.groups)
-        hipLaunchKernelGGL(k_rs_groups, dim3((p.tiles + kRsGroup - 1) / kRsGroup, kRsShare), dim3(kRsWords), 0, c->stream,
-                           c->rows.p, p.tiles, c->rowsum.p);
-      auto kern = p.groups ? k_rs_scatter<K(), true> : k_rs_scatter<K(), false>;
+      const int ng = (p.tiles + kRsGroup - 1) / kRsGroup;
+      if (p.sums != RS_ROWS)
+        hipLaunchKernelGGL(k_rs_groups, dim3(ng, kRsShare), dim3(kRsWords), 0, c->stream, c->rows.p, p.tiles,
+                           c->rowsum.p);
+      if (p.sums == RS_SCANNED)
+        hipLaunchKernelGGL(k_rs_group_scan, dim3(kRsWords / kRsScanWords), dim3(kRsScanThreads), 0, c->stream,
+                           c->rowsum.p, ng);
+      auto kern = p.sums == RS_ROWS     ? k_rs_scatter<K(), RS_ROWS>
+                  : p.sums == RS_GROUPS ? k_rs_scatter<K(), RS_GROUPS>
+                                        : k_rs_scatter<K(), RS_SCANNED>;
       hipLaunchKernelGGL(kern, grid, block, 0, c->stream, c->codes.p, kin, kout, c->codes.p, c->idx.p, n, pass,
                          c->rows.p, c->rowsum.p, p.tiles);
     });
