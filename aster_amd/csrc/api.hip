@@ -154,7 +154,7 @@ int aster_destroy(aster_ctx* c) {
   c->codes.release(); c->xm4.release(); c->idx.release(); c->kv.release(); c->rows.release(); c->rowsum.release();
   c->left.release(); c->right.release(); c->parent.release(); c->gflag.release(); c->gpart.release();
   c->nmc.release(); c->nvel.release(); c->nbox.release();
-  c->above.release(); c->units.release(); c->top.release(); c->grange.release(); c->gscan.release();
+  c->above.release(); c->units.release(); c->top.release(); c->big.release(); c->crown.release(); c->grange.release(); c->gscan.release();
   c->gstart.release(); c->gcount.release(); c->splitnode.release();
   c->nrec.release(); c->nlink.release(); c->kids.release(); c->topslot.release(); c->bh_counters.release(); c->gsh.release();
   c->sub_x.release(); c->sub_v.release(); c->sub_a.release(); c->sub_m.release();

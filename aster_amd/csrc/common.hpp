@@ -163,9 +163,11 @@ struct aster_ctx {
   aster::DBuf<uint2> rowsum;                       // their sums over groups of tiles
   aster::DBuf<int32_t> left, right, parent;        // 2n-1
   aster::DBuf<int32_t> splitnode;                  // internal node whose split lies after sorted position k (n-1)
-  aster::DBuf<uint32_t> above;                     // lengths of the lists units, top (2)
+  aster::DBuf<uint32_t> above;                     // lengths of the lists units, top, big, crown (4)
   aster::DBuf<int32_t> units;                      // largest nodes above the groups of at most kUnit leaves
   aster::DBuf<int32_t> top;                        // nodes of more than kUnit leaves (n)
+  aster::DBuf<int32_t> big;                        // largest of those of at most kBigUnit leaves
+  aster::DBuf<int32_t> crown;                      // nodes of more than kBigUnit leaves
   aster::DBuf<int2> grange;                        // sorted-position range of internal node n+i
   aster::DBuf<uint8_t> gflag;                      // 1 where a group starts (n, to a multiple of 16)
   aster::DBuf<uint32_t> gpart;                     // groups per chunk of positions (k_group_counts)

@@ -37,6 +37,8 @@ constexpr int kMaxLevels = 128;
 // 93.6, 50000 155.7 / 155.9 / 149.4 / 154.1, 2^20 974 / 917 / 904 / 923, 2^21 1845 /
 // 1769 / 1697 / 1695.
 constexpr int kUnit = 8192;
+// Leaves per unit of the nodes above those, where there are more (k_moments_above).
+constexpr int kBigUnit = 1 << 21;
 // Traversal groups (and the moment kernel's per-wavefront subtrees): subtrees
 // of at most kGroup leaves whose parent has more.
 constexpr int kGroup = 64;
@@ -474,6 +476,9 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const uint32_t* __res
   }
 }
 
+// Lengths of the lists that k_build writes.
+enum { ABOVE_UNITS = 0, ABOVE_TOP = 1, ABOVE_BIG = 2, ABOVE_CROWN = 3, ABOVE_COUNT = 4 };
+
 // Also packs {x, y, z, m} of each body into one 32-byte record, so the leaf
 // initialisation gathers one record through the sort permutation instead of
 // four scattered planes. A workgroup takes a tile of the sort: it counts its
@@ -488,7 +493,7 @@ __global__ __launch_bounds__(kRsThreads) void k_morton(int n, const double* __re
   constexpr int T = kRsThreads;
   __shared__ uint32_t cnt[kRsWords];
   const int t = threadIdx.x, base = blockIdx.x * (T * K);
-  if (blockIdx.x == 0 && t < 2) above[t] = 0u;  // lengths of the lists that k_build writes
+  if (blockIdx.x == 0 && t < ABOVE_COUNT) above[t] = 0u;  // lengths of the lists that k_build writes
   for (int i = t; i < kRsWords; i += T) cnt[i] = 0u;
   double4 p[K];
 #pragma unroll
@@ -620,7 +625,9 @@ __device__ __forceinline__ int kdelta(const uint32_t* __restrict__ codes, int n,
 // gflag marks the position behind its split as a group's first (every
 // boundary is one node's split). Nodes of more than kUnit leaves are listed in
 // `top`, the largest nodes of at most kUnit leaves above the groups in
-// `units`, in any order (lengths above[1] and above[0]; k_moments_above).
+// `units`, those of more than kBigUnit leaves in `crown` too, the largest
+// between both sizes in `big`, in any order (lengths in `above`;
+// k_moments_above).
 template <bool VEL>
 __global__ __launch_bounds__(256) void k_build(int n, const uint32_t* __restrict__ codes,
                                                const uint32_t* __restrict__ perm, const double4* __restrict__ xm,
@@ -632,6 +639,7 @@ __global__ __launch_bounds__(256) void k_build(int n, const uint32_t* __restrict
                                                float4* __restrict__ gsh, int32_t* __restrict__ splitnode,
                                                uint8_t* __restrict__ gflag, uint32_t* __restrict__ above,
                                                int32_t* __restrict__ units, int32_t* __restrict__ top,
+                                               int32_t* __restrict__ big, int32_t* __restrict__ crown,
                                                uint32_t* __restrict__ flags, int leaf_records) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
@@ -654,7 +662,7 @@ __global__ __launch_bounds__(256) void k_build(int n, const uint32_t* __restrict
   if (k == 0) {
     if (leaf_records) parent[n] = -1;
     gflag[0] = 1;
-    if (n > kGroup && n <= kUnit) units[atomicAdd(&above[0], 1u)] = n;
+    if (n > kGroup && n <= kUnit) units[atomicAdd(&above[ABOVE_UNITS], 1u)] = n;
   }
   if (k >= n - 1) return;
   const int i = k;
@@ -692,10 +700,15 @@ __global__ __launch_bounds__(256) void k_build(int n, const uint32_t* __restrict
   splitnode[gamma] = n + i;  // every split position belongs to exactly one internal node
   gflag[gamma + 1] = l + 1 > kGroup ? 1 : 0;
   if (l + 1 > kUnit) {
-    top[atomicAdd(&above[1], 1u)] = n + i;
+    top[atomicAdd(&above[ABOVE_TOP], 1u)] = n + i;
     const int cl = gamma - lo + 1, cr = hi - gamma;
-    if (cl > kGroup && cl <= kUnit) units[atomicAdd(&above[0], 1u)] = L;
-    if (cr > kGroup && cr <= kUnit) units[atomicAdd(&above[0], 1u)] = R;
+    if (cl > kGroup && cl <= kUnit) units[atomicAdd(&above[ABOVE_UNITS], 1u)] = L;
+    if (cr > kGroup && cr <= kUnit) units[atomicAdd(&above[ABOVE_UNITS], 1u)] = R;
+    if (l + 1 > kBigUnit) {
+      crown[atomicAdd(&above[ABOVE_CROWN], 1u)] = n + i;
+      if (cl > kUnit && cl <= kBigUnit) big[atomicAdd(&above[ABOVE_BIG], 1u)] = L;
+      if (cr > kUnit && cr <= kBigUnit) big[atomicAdd(&above[ABOVE_BIG], 1u)] = R;
+    }
   }
 }
 
@@ -922,15 +935,18 @@ __global__ __launch_bounds__(256) void k_group_moments(int n, const int32_t* __r
 }
 
 // Moments of the nodes above the groups, a workgroup per unit: first the nodes
-// of the subtrees of at most kUnit leaves (TOP = false; their splits are the
+// of the subtrees of at most kUnit leaves (MOM_UNITS; their splits are the
 // boundaries between the groups inside), then all larger nodes in one workgroup
-// (TOP = true, from the list `top`). A thread takes a node, loads the records
-// of its children that are complete (group roots, leaves, units' roots) and
-// polls the other children's flags, one barrier per sweep; records pass through
-// LDS. A flag holds the sweep its node was formed in, and only earlier sweeps
-// count, so a sweep needs no second barrier and the records' order never
-// depends on timing. More nodes than threads (a unit of many small groups, more
-// than ~2.7 million bodies): the threads take turns and the records pass
+// (MOM_TOP, from the list `top`). Above kBigUnit bodies, where these are more
+// than the workgroup has threads, those of the subtrees of at most kBigUnit
+// leaves come before (MOM_BIG, each workgroup picks its own out of `top`), and
+// the last workgroup takes what is left (`crown`). A thread takes a node, loads
+// the records of its children that are complete (group roots, leaves, units'
+// roots) and polls the other children's flags, one barrier per sweep; records
+// pass through LDS. A flag holds the sweep its node was formed in, and only
+// earlier sweeps count, so a sweep needs no second barrier and the records'
+// order never depends on timing. More nodes than threads (a unit of many small
+// groups, a very uneven tree): the threads take turns and the records pass
 // through global memory. Bound: latency, ~4 dependent loads and a sweep per
 // level (at most 47 levels up to 2^17 bodies: 30 code bits, 17 of position).
 // Neither the host nor a level census is needed to order the launches: against
@@ -938,7 +954,9 @@ __global__ __launch_bounds__(256) void k_group_moments(int n, const int32_t* __r
 // pass, the tree's part of a step falls from 167 to 127 us at 50000 bodies
 // (these two launches 16 + 9 us) and from 331 to 280 us at 2^20 (15 + 30 us).
 // With the records stored after the sweeps 12 + 7 and 12 + 23 us (units of 4096
-// leaves), with units of 8192 13 + 16 us at 2^20.
+// leaves), with units of 8192 13 + 16 us at 2^20. All moments without / with the
+// big units, us: 2.2 10^6 bodies 148 / 149, 3 10^6 235 / 192, 2^22 315 / 261, 2^24
+// 1097 / 890, 2^26 4333 / 3491 (bands of levels 294, 984 and 3789 at the last three).
 template <bool VEL, int CAP>
 struct MomLds {
   double4 com[CAP];
@@ -962,39 +980,73 @@ struct MomLds {
 constexpr int kUnitThreads = 512;
 constexpr int kTopThreads = 512;
 
-template <bool VEL, bool TOP>
-__global__ __launch_bounds__(TOP ? kTopThreads : kUnitThreads) void k_moments_above(
-    int n, const uint32_t* __restrict__ above, const int32_t* __restrict__ units, const int32_t* __restrict__ top,
-    const int32_t* __restrict__ gstart, const uint32_t* __restrict__ gcount, const uint32_t* __restrict__ gscan,
-    const int32_t* __restrict__ splitnode, const int32_t* __restrict__ left, const int32_t* __restrict__ right,
-    const int2* __restrict__ grange, double4* nmc, double4* nvel, float4* nbox, float4* __restrict__ nrec,
-    double theta, float4* __restrict__ kids, int32_t* topslot, uint32_t* __restrict__ flags) {
-  constexpr int T = TOP ? kTopThreads : kUnitThreads;
+// What a launch forms: the units' nodes, the big units' nodes above units, or
+// every node of more than `small` leaves (kUnit: all of `top`, kBigUnit: `crown`).
+enum { MOM_UNITS = 0, MOM_BIG = 1, MOM_TOP = 2 };
+struct MomLists {
+  const int32_t* units;  // MOM_UNITS, MOM_BIG: the roots
+  const uint32_t* nunits;
+  const int32_t* top;  // MOM_BIG, MOM_TOP: the nodes
+  const uint32_t* ntop;
+  int small;  // children of at most so many leaves are complete
+};
+
+template <bool VEL, int KIND>
+__global__ __launch_bounds__(KIND == MOM_TOP ? kTopThreads : kUnitThreads) void k_moments_above(
+    int n, MomLists lists, const int32_t* __restrict__ gstart, const uint32_t* __restrict__ gcount,
+    const uint32_t* __restrict__ gscan, const int32_t* __restrict__ splitnode, const int32_t* __restrict__ left,
+    const int32_t* __restrict__ right, const int2* __restrict__ grange, double4* nmc, double4* nvel, float4* nbox,
+    float4* __restrict__ nrec, double theta, float4* __restrict__ kids, int32_t* topslot,
+    uint32_t* __restrict__ flags) {
+  constexpr bool UNITS = KIND == MOM_UNITS, BIG = KIND == MOM_BIG;
+  constexpr int T = KIND == MOM_TOP ? kTopThreads : kUnitThreads;
   constexpr int kNever = 0xFFFF;
-  constexpr int kSmall = TOP ? kUnit : kGroup;  // children of at most so many leaves are complete
   __shared__ MomLds<VEL, T> lds;
-  __shared__ uint16_t uslot[TOP ? 1 : kUnit];  // unit: node - n - lo -> thread, or its sweep
+  __shared__ uint16_t uslot[UNITS ? kUnit : 1];  // unit: node - n - lo -> thread, or its sweep
+  __shared__ int mine_of[BIG ? T : 1];           // big unit: its nodes, while they are at most T
+  __shared__ int mine_count;
   __shared__ int rslot;
   const int t = threadIdx.x;
-  const int nunits = TOP ? 1 : (int)above[0];
+  const int nunits = KIND == MOM_TOP ? 1 : (int)*lists.nunits;
+  const int ntop = UNITS ? 0 : (int)*lists.ntop;
   for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
-    int root = n, ulo = 0, g0 = 0, m = 0;
-    if (TOP) {
-      m = (int)above[1];
-    } else {
-      root = units[u];
+    int root = n, ulo = 0, uhi = 0, g0 = 0, m = ntop;
+    if (KIND != MOM_TOP) {
+      root = lists.units[u];
       const int2 r = grange[root - n];
       ulo = r.x;
-      g0 = (int)gscan[r.x];
-      m = (r.y + 1 < n ? (int)gscan[r.y + 1] : (int)*gcount) - g0 - 1;
+      uhi = r.y;
     }
-    // a node's entry: TOP in global memory, otherwise in LDS
+    if (UNITS) {
+      g0 = (int)gscan[ulo];
+      m = (uhi + 1 < n ? (int)gscan[uhi + 1] : (int)*gcount) - g0 - 1;
+    }
+    // Entry e of the big unit's list: a node of `top` inside it, or -1. (Node
+    // n + i covers position i; a larger node may cover the unit's first or last.)
+    auto in_big = [&](int e) -> int {
+      const int node = lists.top[e], i = node - n;
+      if (i < ulo || i > uhi) return -1;
+      const int2 r = grange[i];
+      return r.x >= ulo && r.y <= uhi ? node : -1;
+    };
+    if (BIG) {
+      if (t == 0) mine_count = 0;
+      __syncthreads();
+      for (int e = t; e < ntop; e += T) {
+        const int node = in_big(e);
+        if (node < 0) continue;
+        const int at = atomicAdd(&mine_count, 1);
+        if (at < T) mine_of[at] = node;
+      }
+      __syncthreads();
+      m = mine_count;
+    }
+    // a node's entry: a unit's in LDS, the others' in global memory
     auto state_put = [&](int node, int v) {
-      if (TOP) topslot[node - n] = v;
+      if (!UNITS) topslot[node - n] = v;
       else uslot[node - n - ulo] = (uint16_t)v;
     };
-    auto state_get = [&](int node) -> int { return TOP ? topslot[node - n] : (int)uslot[node - n - ulo]; };
-    auto node_at = [&](int e) { return TOP ? top[e] : splitnode[gstart[g0 + e + 1] - 1]; };
+    auto state_get = [&](int node) -> int { return !UNITS ? topslot[node - n] : (int)uslot[node - n - ulo]; };
     struct Kids {
       int L, R;
       bool inL, inR;  // formed here
@@ -1005,8 +1057,8 @@ __global__ __launch_bounds__(TOP ? kTopThreads : kUnitThreads) void k_moments_ab
       k.R = right[node];
       const int2 r = grange[node - n];  // children cover [r.x, gamma] and [gamma + 1, r.y]
       const int gamma = k.L < n ? k.L : k.L - n;
-      k.inL = k.L >= n && gamma - r.x + 1 > kSmall;
-      k.inR = k.R >= n && r.y - gamma > kSmall;
+      k.inL = k.L >= n && gamma - r.x + 1 > lists.small;
+      k.inR = k.R >= n && r.y - gamma > lists.small;
       return k;
     };
     auto store = [&](int node, const Kids& k, const MomRec& cl, const MomRec& cr, const MomRec& me) {
@@ -1028,7 +1080,7 @@ __global__ __launch_bounds__(TOP ? kTopThreads : kUnitThreads) void k_moments_ab
       Kids k{};
       MomRec cl{}, cr{}, me{};
       if (mine) {
-        node = node_at(t);
+        node = BIG ? mine_of[t] : UNITS ? splitnode[gstart[g0 + t + 1] - 1] : lists.top[t];
         state_put(node, t);
         if (node == root) rslot = t;
         k = kids_of(node);
@@ -1061,12 +1113,17 @@ __global__ __launch_bounds__(TOP ? kTopThreads : kUnitThreads) void k_moments_ab
       }
       if (mine) store(node, k, cl, cr, me);  // not in the sweeps: a barrier waits for stores
     } else {
-      for (int e = t; e < m; e += T) state_put(node_at(e), kNever);
+      const int entries = BIG ? ntop : m;  // (a big unit's list does not fit: all of `top` every time)
+      auto node_at = [&](int e) { return BIG ? in_big(e) : UNITS ? splitnode[gstart[g0 + e + 1] - 1] : lists.top[e]; };
+      for (int e = t; e < entries; e += T) {
+        const int node = node_at(e);
+        if (node >= 0) state_put(node, kNever);
+      }
       __syncthreads();
       for (int it = 1;; ++it) {
-        for (int e = t; e < m; e += T) {
+        for (int e = t; e < entries; e += T) {
           const int node = node_at(e);
-          if (state_get(node) != kNever) continue;
+          if (node < 0 || state_get(node) != kNever) continue;
           const Kids k = kids_of(node);
           if ((k.inL && state_get(k.L) >= it) || (k.inR && state_get(k.R) >= it)) continue;
           const MomRec cl = load_moments<VEL>(n, k.L, nmc, nvel, nbox);
@@ -1821,7 +1878,7 @@ static int reserve_sort(aster_ctx* c) {
   ASTER_HIP(c, c->idx.reserve(n));
   ASTER_HIP(c, c->kv.reserve(2 * n));
   ASTER_HIP(c, c->xm4.reserve(n));
-  ASTER_HIP(c, c->above.reserve(2));
+  ASTER_HIP(c, c->above.reserve(ABOVE_COUNT));
   ASTER_HIP(c, c->rows.reserve(tiles * kRsWords));
   ASTER_HIP(c, c->rowsum.reserve((tiles / kRsGroup + 2) * kRsWords));
   return ASTER_OK;
@@ -1857,6 +1914,8 @@ static int reserve_tree(aster_ctx* c, bool full) {
   ASTER_HIP(c, c->splitnode.reserve(n));
   ASTER_HIP(c, c->units.reserve(n / kGroup + 1));
   ASTER_HIP(c, c->top.reserve(n));
+  ASTER_HIP(c, c->big.reserve(n / kUnit + 1));
+  ASTER_HIP(c, c->crown.reserve(kMaxLevels * (n / kBigUnit + 1)));  // disjoint at each level
   ASTER_HIP(c, c->topslot.reserve(n));
   ASTER_HIP(c, c->gflag.reserve((n + 15) / 16 * 16));  // read 16 at a time
   ASTER_HIP(c, c->gpart.reserve(n / kGsChunk + 1));
@@ -1954,7 +2013,8 @@ static int build_tree(aster_ctx* c, int mac, bool vel, bool full) {
   auto build = vel ? k_build<true> : k_build<false>;
   hipLaunchKernelGGL(build, dim3((n + 255) / 256), dim3(256), 0, c->stream, n, c->codes.p, c->idx.p, c->xm4.p,
                      c->v.p, c->left.p, c->right.p, c->parent.p, c->grange.p, c->nmc.p, c->nvel.p, c->nbox.p,
-                     c->nrec.p, c->gsh.p, c->splitnode.p, c->gflag.p, c->above.p, c->units.p, c->top.p, c->flags.p,
+                     c->nrec.p, c->gsh.p, c->splitnode.p, c->gflag.p, c->above.p, c->units.p, c->top.p, c->big.p,
+                     c->crown.p, c->flags.p,
                      full ? 1 : 0);
   ASTER_HIP(c, hipGetLastError());
   // Groups of the wavefront traversal, also the subtrees of the first moment
@@ -1969,14 +2029,23 @@ static int build_tree(aster_ctx* c, int mac, bool vel, bool full) {
   auto gmom = vel ? k_group_moments<true> : k_group_moments<false>;
   hipLaunchKernelGGL(gmom, dim3(gblocks), dim3(256), 0, c->stream, n, c->gstart.p, c->gcount.p, c->grange.p, c->left.p,
                      c->right.p, c->nmc.p, c->nvel.p, c->nbox.p, c->nrec.p, c->P.theta, kids);
-  auto above = [&](auto kern, int blocks, int threads) {
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(threads), 0, c->stream, n, c->above.p, c->units.p, c->top.p,
-                       c->gstart.p, c->gcount.p, c->gscan.p, c->splitnode.p, c->left.p, c->right.p, c->grange.p,
-                       c->nmc.p, c->nvel.p, c->nbox.p, c->nrec.p, c->P.theta, kids, c->topslot.p, c->flags.p);
+  const uint32_t* len = c->above.p;
+  auto above = [&](auto kern, int blocks, int threads, const MomLists& lists) {
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(threads), 0, c->stream, n, lists, c->gstart.p, c->gcount.p, c->gscan.p,
+                       c->splitnode.p, c->left.p, c->right.p, c->grange.p, c->nmc.p, c->nvel.p, c->nbox.p, c->nrec.p,
+                       c->P.theta, kids, c->topslot.p, c->flags.p);
   };
-  const int ublocks = n / 1024 + 1;  // units hold ~2700 leaves each; the workgroups loop over more
-  if (n > kGroup) above(vel ? k_moments_above<true, false> : k_moments_above<false, false>, ublocks, kUnitThreads);
-  if (n > kUnit) above(vel ? k_moments_above<true, true> : k_moments_above<false, true>, 1, kTopThreads);
+  // (units hold ~5400 leaves each, big units ~1.4 million; the workgroups loop over more)
+  if (n > kGroup)
+    above(vel ? k_moments_above<true, MOM_UNITS> : k_moments_above<false, MOM_UNITS>, n / 1024 + 1, kUnitThreads,
+          MomLists{c->units.p, len + ABOVE_UNITS, nullptr, nullptr, kGroup});
+  if (n > kBigUnit)
+    above(vel ? k_moments_above<true, MOM_BIG> : k_moments_above<false, MOM_BIG>, n / (kBigUnit / 4) + 1, kUnitThreads,
+          MomLists{c->big.p, len + ABOVE_BIG, c->top.p, len + ABOVE_TOP, kUnit});
+  if (n > kUnit)
+    above(vel ? k_moments_above<true, MOM_TOP> : k_moments_above<false, MOM_TOP>, 1, kTopThreads,
+          n > kBigUnit ? MomLists{nullptr, nullptr, c->crown.p, len + ABOVE_CROWN, kBigUnit}
+                       : MomLists{nullptr, nullptr, c->top.p, len + ABOVE_TOP, kUnit});
   ASTER_HIP(c, hipGetLastError());
   phase_end(c, ASTER_PHASE_MOMENTS);
   phase_begin(c, ASTER_PHASE_LINKS);
