@@ -653,7 +653,9 @@ __global__ __launch_bounds__(64 * (W + 1)) void k_allpairs_f64(int n, int lower,
 // with d_ij = x_j - x_i, phi_i = sum_{k != i} mu_k / r_ik and aN the
 // Newtonian accelerations. For two bodies it is the pairwise 1PN law.
 // Pass 1 forms phi and aN, pass 2 the accelerations; one thread per body,
-// sources in index order (the oracle's order, so the two agree bit for bit).
+// sources in index order (the oracle's order, so the two agree bit for bit). One
+// wavefront per SIMD at most below 65536 bodies: inv_sqrt64, whose range check
+// ends the overlap of the unrolled pairs, was slower (2000 bodies 3.01 -> 3.20 ms).
 __global__ __launch_bounds__(256) void k_eih_pass1(int n, const double* __restrict__ x, const double* __restrict__ m,
                                                    double G, double soft, double* __restrict__ phi,
                                                    double* __restrict__ an) {
@@ -666,7 +668,7 @@ __global__ __launch_bounds__(256) void k_eih_pass1(int n, const double* __restri
     if (j == i) continue;
     const double dx = x[j] - p1x, dy = x[n + j] - p1y, dz = x[2 * n + j] - p1z;
     const double r2 = dx * dx + dy * dy + dz * dz + soft;
-    const double inv_r = inv_sqrt64(r2);
+    const double inv_r = 1.0 / sqrt(r2);
     const double inv_r3 = inv_r * inv_r * inv_r;
     const double mu = G * m[j];
     ph += mu * inv_r;
@@ -697,7 +699,7 @@ __global__ __launch_bounds__(256) void k_eih_pass2(int n, const double* __restri
     if (j == i) continue;
     const double dx = x[j] - p1x, dy = x[n + j] - p1y, dz = x[2 * n + j] - p1z;
     const double r2 = dx * dx + dy * dy + dz * dz + soft;
-    const double inv_r = inv_sqrt64(r2);
+    const double inv_r = 1.0 / sqrt(r2);
     const double inv_r3 = inv_r * inv_r * inv_r;
     const double mu = G * m[j];
     const double v2x = v[j], v2y = v[n + j], v2z = v[2 * n + j];
