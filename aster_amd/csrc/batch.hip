@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <cmath>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -58,43 +59,58 @@ struct BatchArgs {
 // step of 1000 / 8192 systems of 3-64 bodies, against IEEE square root and
 // division: Newtonian 15.0 -> 11.5 / 46.5 -> 31.8 us, 1PN 61 -> 59 / 163 -> 156,
 // EIH 75 -> 65.5 / 168 -> 146. (kU = 4: 11.3 / 33, 61 / 164, 65 / 152; the 1PN
-// force's division by div64_fast, after a look at its size: 63 / 145.)
+// force's division by div64_fast, after a look at its size: 63 / 145.) An odd last
+// source goes by itself: 16384 systems of 3 / 5 bodies with 1PN terms 4.2 -> 3.4 /
+// 9.4 -> 8.0 us (3.5 / 8.5 with one source at a time and IEEE operations). Up to
+// two bodies the look at the ranges costs more than it saves, and so does the
+// overlap (16384 pairs of bodies 0.74 -> 0.68 us).
 constexpr int kU = 2;
 
-// Separations and 1 / r of sources base + j0 .. base + j0 + kU - 1. FAST: every
-// input within the ranges of inv_sqrt64_fast and div64_fast.
-template <bool FAST>
+// The sources of a wavefront's systems, kU at a time and the odd one by itself;
+// none where every system is a single body, two one after the other.
+template <class F>
+__device__ __forceinline__ void batch_each_source(int maxcnt, F sources) {
+  if (maxcnt < 2) return;
+  int j0 = 0;
+  if (maxcnt > 2)
+    for (; j0 + kU <= maxcnt; j0 += kU) sources(j0, std::integral_constant<int, kU>{});
+  for (; j0 < maxcnt; ++j0) sources(j0, std::integral_constant<int, 1>{});
+}
+
+// Separations and 1 / r of sources first .. first + N - 1. FAST: every input
+// within the ranges of inv_sqrt64_fast and div64_fast.
+template <bool FAST, int N>
 __device__ __forceinline__ void batch_separations(int first, const double* lx, const double* ly, const double* lz,
                                                   const double* X, double soft, double (*d)[3], double* inv) {
 #pragma clang fp contract(off)
-  double r2[kU];
+  double r2[N];
 #pragma unroll
-  for (int u = 0; u < kU; ++u) {
+  for (int u = 0; u < N; ++u) {
     const int src = min(first + u, 63);
     d[u][0] = lx[src] - X[0];
     d[u][1] = ly[src] - X[1];
     d[u][2] = lz[src] - X[2];
     r2[u] = d[u][0] * d[u][0] + d[u][1] * d[u][1] + d[u][2] * d[u][2] + soft;
   }
-  if (!FAST || __builtin_expect(__any(inv_sqrt64_fast<kU>(r2, inv)), 0)) {
+  if (!FAST || __builtin_expect(__any(inv_sqrt64_fast<N>(r2, inv)), 0)) {
 #pragma unroll
-    for (int u = 0; u < kU; ++u) inv[u] = 1.0 / sqrt(r2[u]);
+    for (int u = 0; u < N; ++u) inv[u] = 1.0 / sqrt(r2[u]);
   }
 }
 
-// The accelerations f of the lane's body by sources j0 .. j0 + kU - 1 of its
+// The accelerations f of the lane's body by sources j0 .. j0 + N - 1 of its
 // system; 0 for a pair that does not count.
-template <bool PN, bool FAST>
+template <bool PN, bool FAST, int N>
 __device__ __forceinline__ void batch_exact_pairs(int lane, int base, int cnt, int j0, bool live, const double* lx,
                                                   const double* ly, const double* lz, const double* lm,
                                                   const double* lvx, const double* lvy, const double* lvz,
                                                   const double* X, const double* V, const Divisor64& mi, double G,
                                                   double ic, int pnf, double soft, double (*f)[3]) {
 #pragma clang fp contract(off)
-  double d[kU][3], inv[kU];
-  batch_separations<FAST>(base + j0, lx, ly, lz, X, soft, d, inv);
+  double d[N][3], inv[N];
+  batch_separations<FAST, N>(base + j0, lx, ly, lz, X, soft, d, inv);
 #pragma unroll
-  for (int u = 0; u < kU; ++u) {
+  for (int u = 0; u < N; ++u) {
     const int src = min(base + j0 + u, 63);
     const double m2 = lm[src];
     const double scal = G * m2 * mi.b * (inv[u] * inv[u]);
@@ -110,15 +126,15 @@ __device__ __forceinline__ void batch_exact_pairs(int lane, int base, int cnt, i
     }
   }
   if (FAST && !PN) {  // the post-Newtonian terms have no bounds of their own
-    div64_fast<3 * kU>(&f[0][0], mi);
+    div64_fast<3 * N>(&f[0][0], mi);
   } else {
 #pragma unroll
-    for (int u = 0; u < kU; ++u)
+    for (int u = 0; u < N; ++u)
 #pragma unroll
       for (int c = 0; c < 3; ++c) f[u][c] = f[u][c] / mi.b;
   }
 #pragma unroll
-  for (int u = 0; u < kU; ++u) {
+  for (int u = 0; u < N; ++u) {
     const int src = min(base + j0 + u, 63);
     const bool valid = live && j0 + u < cnt && src != lane;
 #pragma unroll
@@ -134,15 +150,17 @@ __device__ __forceinline__ void batch_exact(int lane, int base, int cnt, int max
                                             double* A) {
 #pragma clang fp contract(off)
   double a[3] = {0.0, 0.0, 0.0};
-  for (int j0 = 0; j0 < maxcnt; j0 += kU) {
-    double f[kU][3];
-    batch_exact_pairs<PN, FAST>(lane, base, cnt, j0, live, lx, ly, lz, lm, lvx, lvy, lvz, X, V, mi, G, ic, pnf, soft,
-                                f);
+  auto sources = [&](int j0, auto count) {
+    constexpr int N = count();
+    double f[N][3];
+    batch_exact_pairs<PN, FAST, N>(lane, base, cnt, j0, live, lx, ly, lz, lm, lvx, lvy, lvz, X, V, mi, G, ic, pnf,
+                                   soft, f);
 #pragma unroll
-    for (int u = 0; u < kU; ++u)
+    for (int u = 0; u < N; ++u)
 #pragma unroll
       for (int c = 0; c < 3; ++c) a[c] += f[u][c];
-  }
+  };
+  batch_each_source(maxcnt, sources);
 #pragma unroll
   for (int c = 0; c < 3; ++c) A[c] = a[c];
 }
@@ -266,11 +284,12 @@ __device__ __forceinline__ void batch_eih(int lane, int base, int cnt, int maxcn
                                           double* lanz, double* A) {
 #pragma clang fp contract(off)
   double ph = 0.0, nx = 0.0, ny = 0.0, nz = 0.0;
-  for (int j0 = 0; j0 < maxcnt; j0 += kU) {
-    double d[kU][3], inv[kU];
-    batch_separations<FAST>(base + j0, lx, ly, lz, X, soft, d, inv);
+  batch_each_source(maxcnt, [&](int j0, auto count) {
+    constexpr int N = count();
+    double d[N][3], inv[N];
+    batch_separations<FAST, N>(base + j0, lx, ly, lz, X, soft, d, inv);
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
+    for (int u = 0; u < N; ++u) {
       const int j = j0 + u, src = min(base + j, 63);
       const bool valid = live && j < cnt && src != lane;
       const double dx = d[u][0], dy = d[u][1], dz = d[u][2];
@@ -284,7 +303,7 @@ __device__ __forceinline__ void batch_eih(int lane, int base, int cnt, int maxcn
         nz += mu * dz * inv_r3;
       }
     }
-  }
+  });
   lphi[lane] = ph;
   lanx[lane] = nx;
   lany[lane] = ny;
@@ -293,11 +312,12 @@ __device__ __forceinline__ void batch_eih(int lane, int base, int cnt, int maxcn
   const double ic2 = ic * ic;
   const double vi2 = V[0] * V[0] + V[1] * V[1] + V[2] * V[2];
   double ax = 0.0, ay = 0.0, az = 0.0;
-  for (int j0 = 0; j0 < maxcnt; j0 += kU) {
-    double d[kU][3], inv[kU];
-    batch_separations<FAST>(base + j0, lx, ly, lz, X, soft, d, inv);
+  batch_each_source(maxcnt, [&](int j0, auto count) {
+    constexpr int N = count();
+    double d[N][3], inv[N];
+    batch_separations<FAST, N>(base + j0, lx, ly, lz, X, soft, d, inv);
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
+    for (int u = 0; u < N; ++u) {
       const int j = j0 + u, src = min(base + j, 63);
       const bool valid = live && j < cnt && src != lane;
       const double dx = d[u][0], dy = d[u][1], dz = d[u][2];
@@ -328,7 +348,7 @@ __device__ __forceinline__ void batch_eih(int lane, int base, int cnt, int maxcn
         az += anz * s3;
       }
     }
-  }
+  });
   wave_sync();  // the next evaluation rewrites the LDS potentials
   A[0] = ax;
   A[1] = ay;
@@ -428,7 +448,7 @@ __global__ __launch_bounds__(256) void k_batch(BatchArgs P) {
   };
   const bool eih = PN && EXACT && (P.pnf & ASTER_EIH);
   auto in_ranges = [&]() {
-    return EXACT && ranges &&
+    return EXACT && ranges && maxcnt > 2 &&
            __all(!live || (coord_in_range64(X[0]) && coord_in_range64(X[1]) && coord_in_range64(X[2])));
   };
   auto accel = [&]() {
@@ -535,10 +555,10 @@ __global__ __launch_bounds__(64 * (W + 3)) void k_batch_team(BatchArgs P) {
     const double* vz = PN ? p + 6 * 64 : p;
     if constexpr (EXACT) {
       if (j0 < maxcnt && fast)
-        batch_exact_pairs<PN, true>(lane, base, cnt, j0, live, p, p + 64, p + 128, p + 192, vx, vy, vz, X, V, md, P.G,
+        batch_exact_pairs<PN, true, kU>(lane, base, cnt, j0, live, p, p + 64, p + 128, p + 192, vx, vy, vz, X, V, md, P.G,
                                     P.ic, P.pnf, P.soft, f);
       else if (j0 < maxcnt)
-        batch_exact_pairs<PN, false>(lane, base, cnt, j0, live, p, p + 64, p + 128, p + 192, vx, vy, vz, X, V, md, P.G,
+        batch_exact_pairs<PN, false, kU>(lane, base, cnt, j0, live, p, p + 64, p + 128, p + 192, vx, vy, vz, X, V, md, P.G,
                                      P.ic, P.pnf, P.soft, f);
     } else if (j0 < sources) {
       const double v11 = V[0] * V[0] + V[1] * V[1] + V[2] * V[2];
