@@ -769,15 +769,21 @@ __global__ __launch_bounds__(256) void k_batch_wh(WhArgs P) {
   const double h = 0.5 * P.dt;
 
   // interaction accelerations of the planets at the positions in X (with the
-  // sums below read ahead: step of systems up to 64 bodies 40 -> 35 us; the
-  // Kepler drift, up to ~50 iterations in some lane, is ~20 us of it)
+  // sums below by every lane, two reads at a time: step of systems up to 64 bodies
+  // 40 -> 33 us; the Kepler drift, up to ~50 iterations in some lane, is ~20 us of
+  // it and all of it for a few bodies)
   auto interaction = [&]() {
+    if (maxcnt < 3) {  // no pair of planets
+      A[0] = A[1] = A[2] = 0.0;
+      return;
+    }
     lx[lane] = X[0];
     ly[lane] = X[1];
     lz[lane] = X[2];
     wave_sync();
     const bool fast =
-        ranges && __all(!live || (coord_in_range64(X[0]) && coord_in_range64(X[1]) && coord_in_range64(X[2])));
+        ranges && maxcnt > 3 &&
+        __all(!live || (coord_in_range64(X[0]) && coord_in_range64(X[1]) && coord_in_range64(X[2])));
     if (fast)
       batch_exact<false, true>(lane, base + 1, cnt - 1, maxcnt - 1, planet, lx, ly, lz, lm, nullptr, nullptr, nullptr,
                                X, V, md, P.G, 0.0, 0, P.soft, A);
@@ -786,43 +792,33 @@ __global__ __launch_bounds__(256) void k_batch_wh(WhArgs P) {
                                 X, V, md, P.G, 0.0, 0, P.soft, A);
     wave_sync();
   };
-  // sum over the system's planets of m_j w_j (j order), by the head lane
+  // sum over the system's planets of m_j w_j (j order), by every lane itself
   auto planet_sum = [&](const double* W, double* out) {
     ux[lane] = planet ? mi * W[0] : 0.0;
     uy[lane] = planet ? mi * W[1] : 0.0;
     uz[lane] = planet ? mi * W[2] : 0.0;
     wave_sync();
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-    if (head)
-      for (int j0 = 1; j0 < cnt; j0 += 8) {  // 8 reads at a time; past the system: 0
-        double w[8][3];
+    for (int j0 = 1; j0 < cnt; j0 += 2) {  // past the system: 0
+      double w[2][3];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int src = min(base + j0 + u, 63);
-          w[u][0] = ux[src];
-          w[u][1] = uy[src];
-          w[u][2] = uz[src];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const bool in = j0 + u < cnt;
-          s0 += in ? w[u][0] : 0.0;
-          s1 += in ? w[u][1] : 0.0;
-          s2 += in ? w[u][2] : 0.0;
-        }
+      for (int u = 0; u < 2; ++u) {
+        const int src = min(base + j0 + u, 63);
+        w[u][0] = ux[src];
+        w[u][1] = uy[src];
+        w[u][2] = uz[src];
       }
-    wave_sync();
-    if (head) {
-      ux[lane] = s0;
-      uy[lane] = s1;
-      uz[lane] = s2;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const bool in = j0 + u < cnt;
+        s0 += in ? w[u][0] : 0.0;
+        s1 += in ? w[u][1] : 0.0;
+        s2 += in ? w[u][2] : 0.0;
+      }
     }
-    wave_sync();
-    if (live) {
-      out[0] = ux[base];
-      out[1] = uy[base];
-      out[2] = uz[base];
-    }
+    out[0] = s0;
+    out[1] = s1;
+    out[2] = s2;
     wave_sync();
   };
   auto jump = [&]() {
