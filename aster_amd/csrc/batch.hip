@@ -35,6 +35,7 @@
 namespace aster {
 
 constexpr int kBatchMaxWpb = 4;
+constexpr int kBatchSimds = 1024;
 
 struct BatchArgs {
   int nwaves;
@@ -63,18 +64,22 @@ struct BatchArgs {
 // source goes by itself: 16384 systems of 3 / 5 bodies with 1PN terms 4.2 -> 3.4 /
 // 9.4 -> 8.0 us (3.5 / 8.5 with one source at a time and IEEE operations). Up to
 // two bodies the look at the ranges costs more than it saves, and so does the
-// overlap (16384 pairs of bodies 0.74 -> 0.68 us).
+// overlap (16384 pairs of bodies 0.74 -> 0.68 us), as long as a wavefront has a
+// SIMD to itself (32800 pairs 0.87 us against 1.09).
 constexpr int kU = 2;
 
 // The sources of a wavefront's systems, kU at a time and the odd one by itself;
-// none where every system is a single body, two one after the other.
-template <class F>
+// none where every system is a single body. !FAST: two one after the other, and
+// with post-Newtonian terms no code for a single one (k_batch with both is over
+// 64 KB as it is, and another 4000 lines cost 4% with many wavefronts).
+template <bool PN, bool FAST, class F>
 __device__ __forceinline__ void batch_each_source(int maxcnt, F sources) {
   if (maxcnt < 2) return;
   int j0 = 0;
-  if (maxcnt > 2)
-    for (; j0 + kU <= maxcnt; j0 += kU) sources(j0, std::integral_constant<int, kU>{});
-  for (; j0 < maxcnt; ++j0) sources(j0, std::integral_constant<int, 1>{});
+  if (FAST || PN || maxcnt > 2)
+    for (; j0 + (PN && !FAST ? 1 : kU) <= maxcnt; j0 += kU) sources(j0, std::integral_constant<int, kU>{});
+  if constexpr (FAST || !PN)
+    for (; j0 < maxcnt; ++j0) sources(j0, std::integral_constant<int, 1>{});
 }
 
 // Separations and 1 / r of sources first .. first + N - 1. FAST: every input
@@ -160,7 +165,7 @@ __device__ __forceinline__ void batch_exact(int lane, int base, int cnt, int max
 #pragma unroll
       for (int c = 0; c < 3; ++c) a[c] += f[u][c];
   };
-  batch_each_source(maxcnt, sources);
+  batch_each_source<PN, FAST>(maxcnt, sources);
 #pragma unroll
   for (int c = 0; c < 3; ++c) A[c] = a[c];
 }
@@ -284,7 +289,7 @@ __device__ __forceinline__ void batch_eih(int lane, int base, int cnt, int maxcn
                                           double* lanz, double* A) {
 #pragma clang fp contract(off)
   double ph = 0.0, nx = 0.0, ny = 0.0, nz = 0.0;
-  batch_each_source(maxcnt, [&](int j0, auto count) {
+  batch_each_source<true, FAST>(maxcnt, [&](int j0, auto count) {
     constexpr int N = count();
     double d[N][3], inv[N];
     batch_separations<FAST, N>(base + j0, lx, ly, lz, X, soft, d, inv);
@@ -312,7 +317,7 @@ __device__ __forceinline__ void batch_eih(int lane, int base, int cnt, int maxcn
   const double ic2 = ic * ic;
   const double vi2 = V[0] * V[0] + V[1] * V[1] + V[2] * V[2];
   double ax = 0.0, ay = 0.0, az = 0.0;
-  batch_each_source(maxcnt, [&](int j0, auto count) {
+  batch_each_source<true, FAST>(maxcnt, [&](int j0, auto count) {
     constexpr int N = count();
     double d[N][3], inv[N];
     batch_separations<FAST, N>(base + j0, lx, ly, lz, X, soft, d, inv);
@@ -448,7 +453,7 @@ __global__ __launch_bounds__(256) void k_batch(BatchArgs P) {
   };
   const bool eih = PN && EXACT && (P.pnf & ASTER_EIH);
   auto in_ranges = [&]() {
-    return EXACT && ranges && maxcnt > 2 &&
+    return EXACT && ranges && (maxcnt > 2 || P.nwaves > kBatchSimds) &&
            __all(!live || (coord_in_range64(X[0]) && coord_in_range64(X[1]) && coord_in_range64(X[2])));
   };
   auto accel = [&]() {
