@@ -980,7 +980,8 @@ static int upload_plan(aster_ctx* c) {
         while (used + sz <= 64 && next[sz] < by_size[sz].size()) used = place(by_size[sz][next[sz]++], used);
   }
   B.nwaves = (int)wm.size();
-  B.max_size = *std::max_element(wm.begin(), wm.end());
+  for (int r = 0; r < kTeamRounds; ++r)  // (the wavefronts are in descending order of their largest system)
+    B.round_max[r] = (size_t)r * kTeamRound < wm.size() ? wm[(size_t)r * kTeamRound] : 0;
   B.lane_slots = 0;
   for (int32_t mx : wm) B.lane_slots += 64 * (int64_t)mx;
   ASTER_HIP(c, B.lane_body.reserve(lb.size()));
@@ -1034,26 +1035,43 @@ static BatchArgs make_args(aster_ctx* c, int64_t nsteps, int nsub, const double*
 
 // Workers per wavefront of systems (k_batch_team), 0 for k_batch: while the
 // chip has more SIMDs than such wavefronts, their serial chains are what a step
-// waits for; small systems leave workers without sources. Leapfrog step, us,
-// k_batch / 4 / 8 workers, by the largest system and the wavefronts. Exact mode,
-// Newtonian: 64 bodies, 36 wavefronts 11.5 / 4.5 / 3.6, 520 12.0 / 6.3 / 6.3, 1045
-// 12.6 / 10.7 / 11.0, 4276 31.9 / 39 / 46; 16, 148 3.35 / 1.58 / 1.33, 604 3.47 /
-// 2.21 / 2.61, 1213 3.74 / 4.14; 8, 703 2.05 / 1.65; 4, 224 1.28 / 1.05, 448
-// 1.29 / 1.29. 1PN: 64, 520 58 / 39 / 33, 1045 67 / 67 / 57, 2126 107 / 124 / 105;
-// 32, 546 29.9 / 20.6 / 18.7, 1111 31.3 / 37 / 32.6; 16, 604 15.5 / 13.9 / 12.8; 8,
-// 350 8.2 / 6.4, 703 8.5 / 9.7; 4, 224 4.5 / 3.3, 448 4.6 / 6.3. Fast mode,
-// Newtonian: 64, 153 4.4 / 3.5 / 3.0, 412 4.5 / 4.2 / 4.1, 520 4.6 / 4.6 / 5.3; 16,
-// 148 1.46 / 1.21 / 1.12, 296 1.48 / 1.29 / 1.47, 441 1.50 / 1.59; 8, 172 0.99 /
-// 0.83, 256 1.00 / 0.98; 4 0.72 / 0.80. 1PN: 64, 153 18.3 / 12.3, 412 18.7 / 16.7,
-// 520 18.8 / 20.2; 16, 296 5.2 / 4.9, 441 5.3 / 6.2; 8, 172 3.0 / 2.9, 256 3.0 /
-// 3.8; 4 1.8 / 2.6.
-static int team_size(int nwaves, int largest, bool pn, bool exact) {
-  int most;
-  if (exact) most = largest <= 4 ? 256 : !pn || largest > 32 ? 1024 : largest > 8 ? 768 : 512;
-  else most = largest <= 4 ? 0 : largest <= 8 ? 192 : largest <= 16 ? 320 : 416;
-  if (nwaves > most) return 0;
-  const bool wide = exact && pn ? true : nwaves <= 256 && !pn;
-  return largest > 8 && wide ? 8 : 4;
+// waits for. The 256 CUs take a workgroup each, the wavefronts with the largest
+// systems first, so the time grows with every 256 wavefronts by what the largest
+// system behind them needs: chunks of 8 sources per 4 workers. Step times of
+// the teams over k_batch's, systems of one size, by the number of such rounds.
+// Exact mode with post-Newtonian terms (the rounds add up): 3 bodies 0.88 / 1.75,
+// 5 0.57 / 1.13, 6 0.49 / 0.97 / 1.45, 9 0.47 / 0.95 / 1.41, 16 0.28 / 0.57 / 0.85 /
+// 1.11, 17 0.39 / 0.79 / 1.18, 33 0.31 / 0.63 / 0.95 / 1.25, 64 0.24 / 0.49 / 0.73 /
+// 0.96. Exact Newtonian: 2 1.16, 3 0.90 / 1.15, 5 0.67 / 0.84 / 1.06, 8 0.48 / 0.62 /
+// 0.77 / 1.08, 16 0.35 / 0.52 / 0.73 / 1.0, 25 0.39 / 0.57 / 0.85 / 1.17, 64 0.30 / 0.47 /
+// 0.71 / 0.95; sizes 3..64 mixed 0.30 / 0.40 / 0.55 / 0.75. Fast Newtonian: 6 1.15, 7 0.95,
+// 8 0.79 / 1.05, 10 1.11, 12 0.90 / 1.3, 16 0.72 / 1.05, 64 0.65 / 1.0; 3..64 mixed 0.66 / 0.8.
+// Fast with 1PN: 7 1.07, 8 0.93 / 1.37, 10 1.19, 12 0.98 / 1.44, 16 0.79 / 1.18, 64 0.65 /
+// 1.0; mixed 0.66 / 0.8.
+static int team_size(int nwaves, const int* largest, int pnf, bool exact) {
+  const bool pn = pnf != 0;
+  const int n = largest[0], rounds = (nwaves + kTeamRound - 1) / kTeamRound;
+  if (rounds > kTeamRounds) return 0;
+  if (exact && pn) {
+    int cost = 0;  // in hundredths of a source of k_batch
+    for (int r = 0; r < rounds; ++r) {
+      const int k = (largest[r] + 7) / 8;
+      if (pnf == ASTER_PN1) cost += n > 8 ? std::max(310, 70 + 185 * k) : 290;
+      else cost += n > 8 ? std::max(265, 60 + 180 * k) : 245;
+    }
+    return cost > 100 * n ? 0 : n > 8 ? 8 : 4;
+  }
+  const int last = 32 * largest[rounds - 1];  // of the round that would be added
+  if (exact) {
+    const bool team = rounds == 1   ? n >= 3
+                      : rounds == 2 ? n >= 5
+                      : rounds == 3 ? n >= 6
+                                    : n >= 58 || (n >= 12 && last <= 24 * n);
+    return !team ? 0 : n > 8 && rounds == 1 ? 8 : 4;
+  }
+  const bool team = rounds == 1 ? n >= (pn ? 8 : 7) && n != 10
+                                : rounds == 2 && n >= 16 && last <= (n >= 32 ? 26 : 21) * n;
+  return !team ? 0 : n > 9 && rounds == 1 && !pn ? 8 : 4;
 }
 
 static int launch_batch(aster_ctx* c, const BatchArgs& P) {
@@ -1063,7 +1081,7 @@ static int launch_batch(aster_ctx* c, const BatchArgs& P) {
   const dim3 grid((P.nwaves + wpb - 1) / wpb), block(64 * wpb);
   const bool pn = (c->P.pn_flags & ASTER_PN_TERMS) != 0;
   const bool exact = c->P.precision == ASTER_FP64;
-  const int team = P.pnf & ASTER_EIH ? 0 : team_size(P.nwaves, c->batch.max_size, pn, exact);
+  const int team = P.pnf & ASTER_EIH ? 0 : team_size(P.nwaves, c->batch.round_max, P.pnf, exact);
   if (team) {
     auto kern = exact ? (team == 8 ? (pn ? k_batch_team<true, true, 8> : k_batch_team<false, true, 8>)
                                    : (pn ? k_batch_team<true, true, 4> : k_batch_team<false, true, 4>))

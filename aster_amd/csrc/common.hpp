@@ -43,6 +43,9 @@ enum : uint32_t { FLAG_OUT_OF_BOX = 1u, FLAG_NONFINITE = 2u, FLAG_TREE = 4u, FLA
 // Sizes of the Barnes-Hut counters block (ctx->bh_counters, u64).
 enum { BHC_INTERACTIONS = 0, BHC_VISITS = 1, BHC_COUNT = 4 };
 
+constexpr int kTeamRound = 256;  // wavefronts of systems that the CUs take at once as teams
+constexpr int kTeamRounds = 4;
+
 struct BatchState {
   int64_t nsys = 0, nbodies = 0;
   bool triples = false;              // every system has three bodies
@@ -56,7 +59,7 @@ struct BatchState {
   int waves_per_block = 4;
   int steps_per_launch = 0;          // 0: not tuned yet
   int nwaves = 0;
-  int max_size = 0;                  // bodies of the largest system
+  int round_max[kTeamRounds] = {};   // bodies of the largest system from each kTeamRound-th wavefront on
   int64_t lane_slots = 0;            // sum over wavefronts of 64 x its largest system: lane-pair slots per evaluation
   DBuf<int32_t> lane_body, lane_seg, wave_max;
   bool a_valid = false;
