@@ -655,7 +655,8 @@ __global__ __launch_bounds__(64 * (W + 1)) void k_allpairs_f64(int n, int lower,
 // Pass 1 forms phi and aN, pass 2 the accelerations; one thread per body,
 // sources in index order (the oracle's order, so the two agree bit for bit). One
 // wavefront per SIMD at most below 65536 bodies: inv_sqrt64, whose range check
-// ends the overlap of the unrolled pairs, was slower (2000 bodies 3.01 -> 3.20 ms).
+// ends the overlap of the unrolled pairs, was slower (leapfrog step of 2000 bodies,
+// two evaluations, 3.01 -> 3.20 ms).
 __global__ __launch_bounds__(256) void k_eih_pass1(int n, const double* __restrict__ x, const double* __restrict__ m,
                                                    double G, double soft, double* __restrict__ phi,
                                                    double* __restrict__ an) {

@@ -12,7 +12,8 @@
 //
 // Two arithmetic modes:
 //   fast  (precision != ASTER_FP64): FP64 with an rsqrt estimate refined by
-//         two Newton steps; contraction allowed.
+//         one Newton step (1/r to 4.1e-15), terms grouped for fused
+//         multiply-adds.
 //   exact (precision == ASTER_FP64): compute_gravitational in the reference's
 //         operation order and j order (src/physics/tool_chain_impl.cpp:120-137,
 //         Parallelized::compute_forces, src/utils/builder_endpoint.cpp:729-757),
@@ -514,7 +515,7 @@ __global__ __launch_bounds__(256) void k_batch(BatchArgs P) {
 // pair forces, kU sources each at a time, and pass them through LDS to three
 // adding wavefronts, one per coordinate, which sum them in j order and advance
 // the bodies; the workers are a chunk of W kU sources ahead. Same operations as
-// batch_accel in the same order, so the same bits (the fast mode passes the
+// k_batch's in the same order, so the same bits (the fast mode passes the
 // factors of its last fused multiply-adds).
 template <bool PN, bool EXACT, int W>
 __global__ __launch_bounds__(64 * (W + 3)) void k_batch_team(BatchArgs P) {

@@ -325,8 +325,6 @@ __device__ __forceinline__ void kahan_add32(float& s, float& c, float t) {
   s = u;
 }
 
-// Compiler and memory ordering point for LDS traffic between the lanes of one
-// wavefront (no cross-wave synchronisation).
 // Stumpff functions c0..c3 of z: quarter z until |z| <= 0.1, 8-term nested
 // series (multiplying by reciprocal constants folded at compile time, no
 // division), then c3 = (c2 + c0 c3)/4, c2 = c1^2/2, c1 = c0 c1,
@@ -439,7 +437,8 @@ __device__ __forceinline__ float uniform_f32(float x) {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
 }
 
-
+// Compiler and memory ordering point for LDS traffic between the lanes of one
+// wavefront (no cross-wave synchronisation).
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();

@@ -359,8 +359,9 @@ int launch_post(aster_ctx* c, const StepPost& post, bool box) {
 int launch_energy(aster_ctx* c, double* out7) {
   const int n = (int)c->n;
   const int ntiles = (n + 63) / 64;
-  // one tile per wavefront up to 128 tiles; above, strips that keep about 16384
-  // of the 32768 blocks busy (half of them lie past the last tile)
+  // one tile per wavefront up to 128 tiles; above, strips that make about 32768
+  // blocks, half of them past the last tile and at once done; from 32768 tiles on
+  // one strip per tile, the longest first
   const int strip = ntiles <= 128 ? 1 : (int)(((int64_t)ntiles * ntiles + 32767) / 32768);
   const int ny = (ntiles + strip - 1) / strip;
   const size_t slots = (size_t)ny * ntiles;

@@ -1,5 +1,5 @@
 // LBVH Barnes-Hut on CDNA4: Morton codes -> LDS radix sort -> Karras radix
-// tree -> level-synchronous bottom-up moments -> escape links -> stackless or
+// tree -> moments by subtrees, bottom-up -> escape links -> stackless or
 // wavefront-cooperative traversal.
 //
 // Tree layout follows the reference's NodesArray indexing
@@ -794,18 +794,6 @@ __device__ __forceinline__ MomRec unite_moments(const MomRec& cl, const MomRec& 
   me.lo = make_float4(fminf(cl.lo.x, cr.lo.x), fminf(cl.lo.y, cr.lo.y), fminf(cl.lo.z, cr.lo.z), 0.f);
   me.hi = make_float4(fmaxf(cl.hi.x, cr.hi.x), fmaxf(cl.hi.y, cr.hi.y), fmaxf(cl.hi.z, cr.hi.z), 0.f);
   return me;
-}
-
-template <bool VEL>
-__device__ __forceinline__ MomRec shfl_xor_rec(const MomRec& r, int m) {
-  MomRec o;
-  o.com = make_double4(__shfl_xor(r.com.x, m, 64), __shfl_xor(r.com.y, m, 64), __shfl_xor(r.com.z, m, 64),
-                       __shfl_xor(r.com.w, m, 64));
-  o.vel = VEL ? make_double4(__shfl_xor(r.vel.x, m, 64), __shfl_xor(r.vel.y, m, 64), __shfl_xor(r.vel.z, m, 64), 0.0)
-              : make_double4(0.0, 0.0, 0.0, 0.0);
-  o.lo = make_float4(__shfl_xor(r.lo.x, m, 64), __shfl_xor(r.lo.y, m, 64), __shfl_xor(r.lo.z, m, 64), 0.f);
-  o.hi = make_float4(__shfl_xor(r.hi.x, m, 64), __shfl_xor(r.hi.y, m, 64), __shfl_xor(r.hi.z, m, 64), 0.f);
-  return o;
 }
 
 // Moments of every internal node inside a traversal group, one wavefront per

@@ -295,16 +295,19 @@ int aster_timer_elapsed(aster_ctx* ctx, int a, int b, float* ms);
  * ASTER_NUM_PHASES) and clears the record. */
 enum aster_phase {
   ASTER_PHASE_MORTON = 0,   /* box reduction + Morton codes */
-  ASTER_PHASE_SORT = 1,     /* 4-pass LDS radix sort */
-  ASTER_PHASE_BUILD = 2,    /* Karras split + leaf init */
+  ASTER_PHASE_SORT = 1,     /* 3-pass LDS radix sort */
+  ASTER_PHASE_BUILD = 2,    /* Karras split + leaf init + traversal groups */
   ASTER_PHASE_MOMENTS = 3,  /* bottom-up moments */
   ASTER_PHASE_LINKS = 4,    /* escape links + opening thresholds */
   ASTER_PHASE_TRAVERSE = 5, /* Barnes-Hut traversal */
-  ASTER_PHASE_ALLPAIRS = 6, /* all-pairs pair kernel */
-  ASTER_PHASE_COMBINE = 7,  /* slice combine / 1PN add */
-  ASTER_PHASE_KICKDRIFT = 8,/* kick/drift update */
-  ASTER_PHASE_ADJOINT = 9,  /* fused force + adjoint kernel (its sources: TILES, its slice sums: COMBINE) */
-  ASTER_PHASE_TILES = 10,   /* anchored FP32 source tiles for all-pairs */
+  ASTER_PHASE_ALLPAIRS = 6, /* all-pairs pair kernel; with it the kick/drift update that follows, FP32 methods up
+                             * to 4096 bodies and Newtonian FP64 up to 16384 */
+  ASTER_PHASE_COMBINE = 7,  /* slice combine / 1PN add with the update that follows and the next sources (FP32
+                             * methods above 4096 bodies), and the adjoint's slice sums with its update */
+  ASTER_PHASE_KICKDRIFT = 8,/* kick/drift updates in launches of their own: Barnes-Hut, the opening one of an
+                             * all-pairs call and where the two above do not take it; the adjoint's first half step */
+  ASTER_PHASE_ADJOINT = 9,  /* fused force + adjoint kernel (up to 4096 bodies with the backward step's update) */
+  ASTER_PHASE_TILES = 10,   /* FP32/FP64 source records for all-pairs, where no update before left them */
   ASTER_NUM_PHASES = 12
 };
 int aster_profile(aster_ctx* ctx, int enable);
@@ -319,10 +322,11 @@ int aster_batch_get(aster_ctx* ctx, double* pos, double* vel);
 /* Integrate every system nsteps with all-pairs FP64 forces (Newton, plus
  * pairwise 1PN if pn_flags has ASTER_PN1, Plummer-softened by softening) in a
  * persistent kernel: each system lives in the lanes of one wavefront (several
- * small systems may share one). precision ASTER_FP64 evaluates
+ * small systems may share one; while there are few such wavefronts, each has a
+ * team of 7 or 11 to form and sum its forces). precision ASTER_FP64 evaluates
  * compute_gravitational in the reference's operation order (bit-identical to
  * the CPU path per system); ASTER_FP32 selects the fast FP64 path (rsqrt
- * estimate + Newton steps). Launches of steps_per_launch steps (0 = tuned) are
+ * estimate + one Newton step). Launches of steps_per_launch steps (0 = tuned) are
  * captured once in a HIP graph and replayed when use_graph != 0.
  * integrator: ASTER_LEAPFROG, ASTER_YOSHIDA4, or ASTER_WH_PLANETARY, which
  * replaces update_WH_planetary (src/physics/tool_chain_impl.cpp:235-274):
@@ -338,8 +342,9 @@ int aster_batch_step(aster_ctx* ctx, int integrator, double dt, int64_t nsteps, 
  * momentum: e[nsys], L[3 nsys]; either may be NULL. */
 int aster_batch_energy(aster_ctx* ctx, double* e, double* L);
 /* Time candidate launch shapes (packed or one system per wavefront; 1, 2 or
- * 4 wavefronts per block) on the loaded batch, restoring its state, and keep
- * the fastest. Writes the chosen wavefronts per block and steps per launch. */
+ * 4 wavefronts per block, which counts where no teams are used) on the loaded
+ * batch, restoring its state, and keep the fastest. Writes the chosen
+ * wavefronts per block and steps per launch. */
 int aster_batch_autotune(aster_ctx* ctx, int integrator, double dt, int32_t* systems_per_block,
                          int32_t* steps_per_launch);
 
@@ -357,7 +362,9 @@ int aster_batch_info(aster_ctx* ctx, int64_t* pair_interactions, int64_t* lane_s
  * nbodies, AoS-d3) go to snap_pos if not NULL. The backward pass takes
  * dLoss/d(snapshot positions) and writes dLoss/d(initial positions,
  * velocities) (3 * nbodies each) and d(masses) (nbodies) for every system at
- * once, then restores the initial state. */
+ * once, then restores the initial state. It uses the forward pass's G and
+ * softening whatever was set since; loading systems drops the trajectory
+ * (ASTER_ERR_STATE). Steps after the forward pass evaluate their own forces. */
 int aster_batch_traj_forward(aster_ctx* ctx, double dt, int64_t nsteps, int32_t nsnap, const int64_t* snap_steps,
                              double* snap_pos);
 int aster_batch_traj_backward(aster_ctx* ctx, const double* grad_snap_pos, double* g_pos, double* g_vel,
@@ -375,7 +382,9 @@ int aster_traj_forward(aster_ctx* ctx, double dt, int64_t nsteps, int64_t ckpt_e
  * dLoss/d(initial positions) (3n), d(initial velocities) (3n) and d(masses)
  * (n) by the hand-written adjoint (transposed pair-force Jacobian-vector
  * product fused with force recomputation, time-reversed recomputation,
- * re-anchored at checkpoints). Restores the initial state on return. */
+ * re-anchored at checkpoints) with the forward pass's parameters and
+ * accelerations, whatever was set or evaluated since. Restores the initial
+ * state on return. */
 int aster_traj_backward(aster_ctx* ctx, const double* grad_snap_pos, double* g_pos, double* g_vel,
                         double* g_mass);
 
