@@ -714,7 +714,7 @@ __global__ void k_batch_sum(int64_t nsys, const int64_t* __restrict__ off, int64
 // call the batch buffers hold the heliocentric state (planets: Q, u, and
 // their interaction accelerations; body 0: the barycentre and its velocity),
 // so launches can split the steps anywhere without changing a bit. Segment
-// sums are taken by the head lane in body order, and pair forces are
+// sums are taken by every lane of a system in body order, and pair forces are
 // compute_gravitational (tool_chain_impl.cpp:120-137) in j order, Newtonian,
 // so every system is bit-identical to the CPU restatement.
 enum { WH_ENTER = 0, WH_STEPS = 1, WH_EXIT = 2 };
